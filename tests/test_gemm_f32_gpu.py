@@ -1,0 +1,47 @@
+"""The float32 product on the matrix cores (csrc/gemm_f32.hip): every kernel its dispatch can choose, at the edges of tiles,
+chunks and runs of k, against a float64 product, and bit for bit the same row whatever rows ride along."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# (rows, weight rows, columns): rows on both sides of every bound of the dispatch (8, 16, 32 rows; one round of 16-, 32-row and
+# tiled workgroups on 256 compute units, two to three, four, six of the large tiles)
+CASES = [(1, 7, 4), (8, 33, 36), (9, 16, 32), (16, 300, 260), (17, 1030, 100), (17, 5000, 68), (33, 2050, 64), (48, 130, 1540),
+         (65, 2060, 1500), (130, 1536, 8960), (449, 1500, 320), (450, 2048, 1536), (1025, 2051, 72), (500, 17920, 48)]
+
+
+@pytest.mark.parametrize("M,N,K", CASES)
+def test_float32_product(M, N, K):
+    from zedinfer_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(M * 31 + N)
+    x, w = (torch.randn(s, generator=g, device="cuda") for s in ((M, K), (N, K)))
+    b = torch.randn(N, generator=g, device="cuda")
+    got = ops.linear(x, w, b)
+    ref = x.double() @ w.double().t() + b.double()
+    # an output is chains of at most 16 multiply-adds for every chunk of 32 in an eighth of k (rounded up), then ten additions:
+    # so many roundings, each at most 2^-24 of a partial sum, which is at most sum |x w| + |b|
+    roundings = 16 * -(-(-(-K // 32)) // 8) + 10
+    bound = roundings * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + b.double().abs())
+    assert bool(((got.double() - ref).abs() <= bound).all()), float(((got.double() - ref).abs() / bound).max())
+    # the same bits in other company: alone, among few, from rows that lie apart, into a slice of a wider result
+    for rows in (slice(M - 1, M), slice(max(0, M - 11), M), slice(max(0, M - 40), M)):
+        assert torch.equal(ops.linear(x[rows].contiguous(), w, b), got[rows])
+    apart, wide = torch.full((M, K + 8), float("nan"), device="cuda"), torch.zeros((M, N + 6), device="cuda")
+    apart[:, 4:K + 4] = x
+    ops.linear(apart[:, 4:K + 4], w, b, out=wide[:, 3:N + 3])
+    assert torch.equal(wide[:, 3:N + 3], got) and not wide[:, :3].any() and not wide[:, N + 3:].any()
+
+
+def test_float32_product_keeps_infinities_and_rows_apart():
+    """A row of x with an infinity or a NaN, and a weight row with one, change their own row and column and nothing else; columns
+    that are no multiple of a chunk are not read past their end."""
+    from zedinfer_amd import ops
+    for M in (3, 12, 20, 200):
+        x, w = torch.ones(M, 36, device="cuda"), torch.ones(70, 36, device="cuda")
+        x[1, 35], w[5, 0], x[2, 3] = float("inf"), float("nan"), 1e-40
+        y = ops.linear(x, w)
+        cols = [i for i in range(70) if i != 5]
+        assert bool(torch.isinf(y[1, cols]).all()) and bool(torch.isnan(y[:, 5]).all())
+        rest = [i for i in range(M) if i not in (1, 2)]
+        assert bool((y[rest][:, cols] == 36).all()) and bool((y[2, cols] == 35).all())

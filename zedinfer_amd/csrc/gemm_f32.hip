@@ -1,0 +1,336 @@
+// out[M,N] = x[M,K] . w[N,K]^T (+ bias[N]), everything float32, on the matrix cores' float32 instruction
+// (v_mfma_f32_16x16x4_f32: float32 products and float32 accumulation, no reduced precision).
+//
+// One order of the sums, the same in every kernel here, so that a row's result does not depend on M, on the tile it
+// falls in or on the rest of the batch: k is cut into GF_PARTS runs of whole chunks of 32 (a function of K alone); within
+// a run the first and the second 16 of every chunk are two chains, each 16 summed as four instructions whose lanes hold
+// k = 4 g + j (instruction j, lane group g); a run's sum is first + second chain; the sums of each half of the runs
+// are added in rising order, then the two halves, then the bias.
+//
+// gemm_f32_stream_kernel, for few rows, is bound by the one pass over the weights.  A workgroup owns 16 weight rows (8 for up
+// to 8 rows of x) and its eight wavefronts take a run of k each, so N / 16 workgroups of eight wavefronts share the stream
+// however few rows the matrix has, with nothing left to add outside the workgroup.  Operands come straight from memory in
+// the matrix cores' layout, several chunks ahead in registers; loads past the end are out of the buffer's range and give
+// zeros without a branch.  For up to 8 rows the 16 x 16 instruction holds 8 weight rows twice, at the two halves of a
+// chunk, beside the 8 rows of x twice: an instruction's load takes eight whole 128-byte lines, and two of the result's
+// four quadrants are the two chains.
+// gemm_f32_tile_kernel, for many rows, is bound by the instruction's rate (152 TFLOP/s in a large library product): tiles
+// through LDS (two buffers, one barrier a chunk of 32 k, two or four more chunks on their way in registers).  The
+// scheduling barriers keep the loads ahead of the products: without them the compiler moves a loop's loads to its end and
+// waits for all of them at its head.
+//
+// Measured, weights from memory, against the plain kernel (gemm_generic.hip: a chain of multiply-adds an output, scalar
+// loads), us, launch included: 8 rows 2,048 x 1,536 (N x K) 165 to 9; 1,536 x 8,960 914 to 19; 17,920 x 1,536 212 to 32 (3.5
+// TB/s); 151,936 x 1,536 761 to 250 (3.7 TB/s; one row 190, 4.9 TB/s).  448 rows: 2,048 x 1,536 189 to 33, 1,536 x 8,960
+// 1,050 to 147 (84 TFLOP/s), 17,920 x 1,536 975 to 219 (113 TFLOP/s).
+#include "zi_common.h"
+
+typedef __attribute__((ext_vector_type(4))) float gf_f32x4_t;
+typedef __attribute__((ext_vector_type(4))) unsigned gf_u32x4_t;
+
+#define GF_PARTS 8           // runs of k; the wavefronts of the stream kernel
+#define GF_KB 32             // k of a chunk
+#define GF_OUT 0x7fffffff    // an offset past the end of every buffer: the load gives zeros and fetches nothing
+
+union gf_pack {
+    gf_u32x4_t u;
+    gf_f32x4_t f;
+};
+
+// Rows base .. base + rows - 1 of a row-major matrix as a buffer whose range ends with the last row's K values.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t gf_rows(const float* base, int64_t ld, int rows, int K) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, (int)(((int64_t)(rows - 1) * ld + K) * 4), 0x00020000);
+}
+
+template <int AUX>
+__device__ __forceinline__ gf_f32x4_t gf_load(__amdgpu_buffer_rsrc_t rows, int offset) {
+    gf_pack p;
+    p.u = __builtin_amdgcn_raw_buffer_load_b128(rows, offset, 0, AUX);
+    return p.f;
+}
+
+// Four outputs of one row of x, columns n .. n + 3.
+__device__ __forceinline__ void gf_store4(float* __restrict__ out, const float* __restrict__ bias, gf_f32x4_t s, int n, int N, int vec_out) {
+    if (bias) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] += n + e < N ? bias[n + e] : 0.f;
+    }
+    if (vec_out && n + 3 < N) {
+        *reinterpret_cast<gf_f32x4_t*>(out + n) = s;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (n + e < N) out[n + e] = s[e];
+    }
+}
+
+// PAIR: 8 weight rows and up to 8 rows of x; else 16 weight rows and up to 16 * MT rows of x a workgroup.  RING chunks are
+// on their way while one is worked on.
+template <int MT, bool PAIR, int RING>
+__global__ void __launch_bounds__(GF_PARTS* ZI_WAVE)
+gemm_f32_stream_kernel(float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,
+                       const float* __restrict__ bias, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int per, int vec_out) {
+    constexpr int NR = PAIR ? 8 : 16, MR = PAIR ? 8 : 16 * MT, H = PAIR ? 1 : 2;
+    __shared__ __attribute__((aligned(16))) gf_f32x4_t part[GF_PARTS][MT][ZI_WAVE];
+    const int lane = threadIdx.x & (ZI_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / ZI_WAVE);
+    const int r = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * NR, m0 = blockIdx.y * MR;
+    const int rows_w = N - n0 < NR ? N - n0 : NR, rows_x = M - m0 < MR ? M - m0 : MR;
+    const __amdgpu_buffer_rsrc_t wb = gf_rows(w + (int64_t)n0 * ldw, ldw, rows_w, K), xb = gf_rows(x + (int64_t)m0 * ldx, ldx, rows_x, K);
+    const int row = PAIR ? r & 7 : r;
+    const int k_lane = (PAIR ? (r >> 3) * 64 : 0) + g * 16;       // byte of a chunk that this lane starts at
+    const int w_row = row < rows_w ? (int)(row * ldw * 4) : GF_OUT;
+    int x_row[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) x_row[t] = t * 16 + row < rows_x ? (int)((t * 16 + row) * ldx * 4) : GF_OUT;
+    const int chunks = (K + GF_KB - 1) / GF_KB;
+    const int c0 = wave * per, c1 = c0 + per < chunks ? c0 + per : chunks;
+
+    gf_f32x4_t wr[RING][H], xr[RING][H][MT];
+    auto fetch = [&](const int slot, int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+            const int k = c * (GF_KB * 4) + h * 64 + k_lane;
+            const bool in = c < c1 && k < K * 4;
+#pragma unroll
+            for (int t = 0; t < MT; ++t) xr[slot][h][t] = gf_load<0>(xb, in && x_row[t] != GF_OUT ? x_row[t] + k : GF_OUT);
+            // a weight is read once by one workgroup: past L2, where an instruction takes whole lines
+            wr[slot][h] = gf_load<PAIR ? 2 : 0>(wb, in && w_row != GF_OUT ? w_row + k : GF_OUT);
+        }
+    };
+    gf_f32x4_t acc[H][MT];
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[h][t] = gf_f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < RING; ++s) {
+        fetch(s, c0 + s);
+        __builtin_amdgcn_sched_barrier(0);         // in this order: the loop waits for the oldest only
+    }
+    for (int c = c0; c < c1; c += RING) {
+#pragma unroll
+        for (int s = 0; s < RING; ++s) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int h = 0; h < H; ++h)
+#pragma unroll
+                    for (int t = 0; t < MT; ++t)
+                        acc[h][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wr[s][h][j], xr[s][h][t][j], acc[h][t], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);     // the loads stay this far ahead of their use
+            fetch(s, c + s + RING);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    // lane (r, g) holds rows 4 g .. 4 g + 3 of column r; PAIR: the first chain in the quadrant of rows and columns 0 .. 7, the
+    // second in the one of 8 .. 15 (the others mix the halves and are dropped)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        gf_f32x4_t s = acc[0][t];
+        if (PAIR) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] += __shfl(acc[0][t][e], (lane + 40) & 63, ZI_WAVE);
+        } else {
+            s += acc[H - 1][t];
+        }
+        part[wave][t][lane] = s;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < MT * ZI_WAVE; i += GF_PARTS * ZI_WAVE) {
+        const int t = i / ZI_WAVE, l = i % ZI_WAVE, m = t * 16 + (l & 15), n = (l >> 4) * 4;
+        gf_f32x4_t s = part[0][t][l], s2 = part[GF_PARTS / 2][t][l];
+#pragma unroll
+        for (int p = 1; p < GF_PARTS / 2; ++p) {
+            s += part[p][t][l];
+            s2 += part[GF_PARTS / 2 + p][t][l];
+        }
+        s += s2;
+        if (m < rows_x && n < rows_w) gf_store4(out + (int64_t)(m0 + m) * ldo, bias, s, n0 + n, N, vec_out);
+    }
+}
+
+// TM x 64 outputs a workgroup; GROUPS (1 or 2) groups of four wavefronts, each over half of the runs of k when there are
+// two; TM/2 x 32 outputs a wavefront.  RING chunks of operands are on their way in registers.
+template <int TM, int NT, int GROUPS, int RING>
+__global__ void __launch_bounds__(256 * GROUPS)
+gemm_f32_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,
+                     const float* __restrict__ bias, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int per, int vec_out,
+                     int m_tiles, int tiles) {
+    constexpr int TN = 32 * NT, XP = TM / 32, WP = TN / 32, MT = TM / 32;     // pieces a thread loads; 16 x 16 tiles a wavefront
+    __shared__ __attribute__((aligned(16))) gf_f32x4_t lds[GROUPS][2][(TM + TN) * 8];
+    // the tiles that share weight rows follow each other on one XCD (workgroup i runs on XCD i mod 8)
+    const int per_xcd = (tiles + 7) / 8, tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if (tile >= tiles) return;
+    const int m0 = (tile % m_tiles) * TM, n0 = (tile / m_tiles) * TN;
+    const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x / ZI_WAVE), group = wave_all / 4, wave = wave_all & 3;
+    const int tid = threadIdx.x & 255, lane = tid & (ZI_WAVE - 1);
+    const int r = lane & 15, g = lane >> 4;
+    const int rows_w = N - n0 < TN ? N - n0 : TN, rows_x = M - m0 < TM ? M - m0 : TM;
+    const __amdgpu_buffer_rsrc_t wb = gf_rows(w + (int64_t)n0 * ldw, ldw, rows_w, K), xb = gf_rows(x + (int64_t)m0 * ldx, ldx, rows_x, K);
+    // a thread loads piece tid % 8 (16 bytes) of rows tid / 8, + 32, ...; piece c of row q lies at place c xor (q / 2 mod 8)
+    const int pc = tid & 7, pr = tid >> 3;
+    const int place = pc ^ ((pr >> 1) & 7);            // the same for rows 32 apart
+    int x_row[XP], w_row[WP];
+#pragma unroll
+    for (int p = 0; p < XP; ++p) x_row[p] = pr + 32 * p < rows_x ? (int)((pr + 32 * p) * ldx * 4) : GF_OUT;
+#pragma unroll
+    for (int p = 0; p < WP; ++p) w_row[p] = pr + 32 * p < rows_w ? (int)((pr + 32 * p) * ldw * 4) : GF_OUT;
+    const int chunks = (K + GF_KB - 1) / GF_KB, half = per * (GF_PARTS / 2);
+    const int c0 = group * half, c1 = GROUPS == 2 && c0 + half < chunks ? c0 + half : chunks;
+    const int steps = GROUPS == 2 ? half : chunks;      // the same for both groups: they share the barriers
+    gf_f32x4_t xr[RING][XP], wr[RING][WP];
+    auto fetch = [&](const int slot, int c) __attribute__((always_inline)) {
+        const int k = c * (GF_KB * 4) + pc * 16;
+        const bool in = c < c1 && k < K * 4;
+#pragma unroll
+        for (int p = 0; p < XP; ++p) xr[slot][p] = gf_load<0>(xb, in && x_row[p] != GF_OUT ? x_row[p] + k : GF_OUT);
+#pragma unroll
+        for (int p = 0; p < WP; ++p) wr[slot][p] = gf_load<0>(wb, in && w_row[p] != GF_OUT ? w_row[p] + k : GF_OUT);
+    };
+    auto stash = [&](const int slot, const int b) __attribute__((always_inline)) {
+        gf_f32x4_t* xs = lds[group][b], *ws = xs + TM * 8;
+#pragma unroll
+        for (int p = 0; p < XP; ++p) xs[(pr + 32 * p) * 8 + place] = xr[slot][p];
+#pragma unroll
+        for (int p = 0; p < WP; ++p) ws[(pr + 32 * p) * 8 + place] = wr[slot][p];
+    };
+    const int wm = (wave & 1) * (TM / 2), wn = (wave >> 1) * (TN / 2);
+    const gf_f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+    gf_f32x4_t acc[2][MT][NT], sum[MT][NT], first[MT][NT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int u = 0; u < NT; ++u) acc[0][t][u] = acc[1][t][u] = sum[t][u] = first[t][u] = zero;
+    int in_part = 0, parts = 0;
+    auto step = [&](const int slot, const int b, int c) __attribute__((always_inline)) {
+        fetch(slot, c + RING);                          // this slot's registers went to LDS a step ago
+        const gf_f32x4_t* xs = lds[group][b], *ws = xs + TM * 8;
+        const int sw = (r >> 1) & 7;
+        __builtin_amdgcn_sched_barrier(0);              // the loads stay this far ahead of their use
+        gf_f32x4_t va[2][NT], vb[2][MT];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int u = 0; u < NT; ++u) va[h][u] = ws[(wn + u * 16 + r) * 8 + ((h * 4 + g) ^ sw)];
+#pragma unroll
+            for (int t = 0; t < MT; ++t) vb[h][t] = xs[(wm + t * 16 + r) * 8 + ((h * 4 + g) ^ sw)];
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int t = 0; t < MT; ++t)
+#pragma unroll
+                    for (int u = 0; u < NT; ++u)
+                        acc[h][t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[h][u][j], vb[h][t][j], acc[h][t][u], 0, 0, 0);
+        if (++in_part == per) {                         // a run of k ends
+            in_part = 0;
+            ++parts;
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+                for (int u = 0; u < NT; ++u) {
+                    sum[t][u] += acc[0][t][u] + acc[1][t][u];
+                    acc[0][t][u] = acc[1][t][u] = zero;
+                    if (GROUPS == 1 && parts == GF_PARTS / 2) {
+                        first[t][u] = sum[t][u];
+                        sum[t][u] = zero;
+                    }
+                }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        stash((slot + 1) % RING, b ^ 1);                // the next chunk
+        __syncthreads();
+    };
+#pragma unroll
+    for (int s = 0; s < RING; ++s) {
+        fetch(s, c0 + s);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    stash(0, 0);
+    __syncthreads();
+    static_assert(RING % 2 == 0, "an LDS buffer a step");
+    for (int c = 0; c < steps; c += RING) {             // (steps past the end add zeros)
+#pragma unroll
+        for (int s = 0; s < RING; ++s) step(s, s & 1, c0 + c + s);
+    }
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int u = 0; u < NT; ++u) sum[t][u] += acc[0][t][u] + acc[1][t][u];       // (zeros where the last run ended)
+    if (GROUPS == 2) {
+        // the second half's sums go through LDS to the first group's wavefronts
+        gf_f32x4_t* hand = lds[0][0];
+        static_assert(GROUPS == 1 || (int)(sizeof(lds) / 16) >= 4 * MT * NT * ZI_WAVE, "the sums of four wavefronts fit");
+        if (group == 1) {
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+                for (int u = 0; u < NT; ++u) hand[((wave * MT + t) * NT + u) * ZI_WAVE + lane] = sum[t][u];
+        }
+        __syncthreads();
+        if (group == 1) return;
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int u = 0; u < NT; ++u) {
+                first[t][u] = sum[t][u];
+                sum[t][u] = hand[((wave * MT + t) * NT + u) * ZI_WAVE + lane];
+            }
+    }
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        const int m = m0 + wm + t * 16 + r;
+        if (m >= M) continue;
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+            const int n = n0 + wn + u * 16 + g * 4;
+            if (n < N) gf_store4(out + (int64_t)m * ldo, bias, first[t][u] + sum[t][u], n, N, vec_out);
+        }
+    }
+}
+
+// Whether these kernels take the operands (all float32): whole 16-byte pieces of every row, and rows of a tile within a
+// buffer's range.
+bool zi_gemm_f32_takes(const void* x, const void* w, int K, int64_t ldx, int64_t ldw) {
+    return K % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 && ldx < (1 << 21) && ldw < (1 << 21);
+}
+
+// The launch; the sizes are checked by the caller (zi_gemm_generic).
+int zi_gemm_f32_launch(float* out, const float* x, const float* w, const float* bias, int M, int N, int K, int64_t ldx, int64_t ldw,
+                       int64_t ldo, hipStream_t stream) {
+    const int chunks = (K + GF_KB - 1) / GF_KB, per = (chunks + GF_PARTS - 1) / GF_PARTS;
+    ZI_REQUIRE((int64_t)((M + 31) / 32) * ((N + 31) / 32) < (1ll << 30), "gemm: M=%d N=%d is too large for one launch", M, N);
+    const int vec_out = ldo % 4 == 0 && (uintptr_t)out % 16 == 0;
+#define ZI_GF_STREAM(MT, PAIR, RING)                                                                                                     \
+    gemm_f32_stream_kernel<MT, PAIR, RING><<<dim3((N + (PAIR ? 7 : 15)) / (PAIR ? 8 : 16), (M + (PAIR ? 8 : 16 * MT) - 1) / (PAIR ? 8 : 16 * MT)), \
+                                             GF_PARTS * ZI_WAVE, 0, stream>>>(out, x, w, bias, M, N, K, ldx, ldw, ldo, per, vec_out)
+#define ZI_GF_TILE(TM, NT, G, R)                                                                                                              \
+    do {                                                                                                                                  \
+        const int mt = (M + TM - 1) / TM, tiles = mt * ((N + 32 * NT - 1) / (32 * NT));                                                                   \
+        gemm_f32_tile_kernel<TM, NT, G, R><<<(tiles + 7) / 8 * 8, 256 * G, 0, stream>>>(out, x, w, bias, M, N, K, ldx, ldw, ldo, per, vec_out, mt, tiles); \
+    } while (0)
+    // Which kernel is a matter of filling the compute units only; all give the same bits.  Up to 8 rows the paired form of the
+    // stream (one row of a 151,936-row head 190 against 233 us); 16 rows a workgroup while that gives no unit a second
+    // workgroup (32 rows, 1,536 x 8,960: 34 against 52 us), 32 rows up to 32 rows and then while the same holds (64 rows:
+    // 52 against 92 us for the tiles).  Beyond, tiles of 32 x 64 in two halves of k while they are one round of workgroups
+    // (256 rows, 1,536 x 8,960: 96 us, one group 123, tiles of 64 x 64 194), of 32 x 96 where those make one round of what
+    // would be two (448 rows: 148 against 157); from six rounds of 64 x 64 tiles on those (17,920 x 1,536 at 448 rows 219
+    // against 226 us, at 256 rows, 4.4 rounds, 141 against 133); else 32 x 64, in two halves up to three rounds (448
+    // rows, 2,048 x 1,536: 33 against 37; 1,024 rows, four rounds: 61 against 60).
+    const int64_t cus = zi_compute_units(), n16 = (N + 15) / 16, m32 = (M + 31) / 32;
+    const int64_t t32 = m32 * ((N + 63) / 64), t96 = m32 * ((N + 95) / 96), t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
+    if (M <= 8) ZI_GF_STREAM(1, true, 6);
+    else if (M <= 16 || n16 * ((M + 15) / 16) <= cus) ZI_GF_STREAM(1, false, 4);
+    else if (M <= 32 || n16 * m32 <= cus) ZI_GF_STREAM(2, false, 3);
+    else if (t32 <= cus) ZI_GF_TILE(32, 2, 2, 4);
+    else if (t96 <= cus) ZI_GF_TILE(32, 3, 2, 2);
+    else if (t64 >= 6 * cus) ZI_GF_TILE(64, 2, 1, 2);
+    else if (t32 <= 3 * cus) ZI_GF_TILE(32, 2, 2, 4);
+    else ZI_GF_TILE(32, 2, 1, 4);
+#undef ZI_GF_STREAM
+#undef ZI_GF_TILE
+    return zi_check_launch("gemm_f32");
+}

@@ -4,8 +4,9 @@
 // size; products and sums in float32 FMA, no matrix cores, no reduced-precision
 // mode.  Each output element is one thread's sequential sum over k in rising
 // order, so its value does not depend on M, on the tile it falls in or on the
-// rest of the batch.  This is the matrix product of the float32 path, and of
-// any layer whose checkpoint tensor is stored in 32-bit.
+// rest of the batch.  It serves layers whose checkpoint tensor is stored in 32-bit
+// beside bfloat16 activations, and float32 operands whose rows are no whole 16-byte
+// pieces; the entry point hands all other float32 products to gemm_f32.hip.
 // (reference: src/backend/ops/linear/cpu/linear_cpu.cpp:26-85.)
 #include "zi_common.h"
 #include "zi_api.h"
@@ -67,12 +68,19 @@ gemm_generic_kernel(TO* __restrict__ out, const TX* __restrict__ x, const TW* __
     }
 }
 
+bool zi_gemm_f32_takes(const void* x, const void* w, int K, int64_t ldx, int64_t ldw);
+int zi_gemm_f32_launch(float* out, const float* x, const float* w, const float* bias, int M, int N, int K, int64_t ldx, int64_t ldw,
+                       int64_t ldo, hipStream_t stream);
+
 extern "C" int zi_gemm_generic(void* out, int out_dt, const void* x, int x_dt, const void* w, int w_dt,
                                const void* bias, int bias_dt, int M, int N, int K, int64_t ldx, int64_t ldw,
                                int64_t ldo, hipStream_t stream) {
     ZI_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm: bad sizes M=%d N=%d K=%d", M, N, K);
     ZI_REQUIRE(ldx >= K && ldw >= K && ldo >= N, "gemm: leading dimension too small");
     if (M == 0) return 0;
+    // all float32 and whole 16-byte pieces a row: the matrix cores' float32 instruction (gemm_f32.hip), whatever M is
+    if (x_dt == ZI_F32 && w_dt == ZI_F32 && out_dt == ZI_F32 && (!bias || bias_dt == ZI_F32) && zi_gemm_f32_takes(x, w, K, ldx, ldw))
+        return zi_gemm_f32_launch((float*)out, (const float*)x, (const float*)w, (const float*)bias, M, N, K, ldx, ldw, ldo, stream);
     const dim3 grid((N + GT - 1) / GT, (M + GT - 1) / GT);
     ZI_REQUIRE(grid.y <= 65535, "gemm: M=%d is too large for one launch", M);
     if (!bias) bias_dt = ZI_F32;

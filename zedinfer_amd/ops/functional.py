@@ -902,8 +902,9 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
 
     bfloat16 inputs with bfloat16 weights and output (or float32 output and more than 64 rows) go
     to the library matrix product, as the reference sends them to its vendor library (reference:
-    src/backend/ops/linear/nvidia/linear_cublas.cu:134-231); every other pairing, and all of
-    the float32 path, runs the plain FMA kernel, which has no reduced-precision mode."""
+    src/backend/ops/linear/nvidia/linear_cublas.cu:134-231); float32 operands go to the
+    matrix cores' float32 instruction (products and sums in float32, one order of the sums whatever the number of
+    rows); every other pairing, and float32 rows that are no whole 16-byte pieces, to the plain FMA kernel."""
     _gpu("linear", x, weight, bias, out)
     ldx, K = _rows(x, "linear x")
     ldw, Kw = _rows(weight, "linear weight")
