@@ -1,0 +1,100 @@
+"""Float32 attention on the matrix cores (csrc/attention_f32.hip) against float64 softmax attention: head sizes, groups, pages,
+windows, portions beside single tokens, sinks; the two ways a token can come give the same bits, in any company; what lies in
+masked places does not matter."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def paged(lens, nkv, d, ps, g):
+    """Keys and values of sequences in pages taken in a random order, with NaN wherever no position lies."""
+    pages = [-(-n // ps) for n in lens]
+    order = torch.randperm(sum(pages) + 2, generator=g)
+    kc = torch.full((len(order), nkv, ps, d), float("nan"))
+    vc = torch.full((len(order), nkv, d, ps), float("nan"))
+    table = torch.full((len(lens), max(pages) + 1), -1, dtype=torch.int32)
+    ks, vs, at = [], [], 0
+    for i, n in enumerate(lens):
+        k, v = torch.randn(n, nkv, d, generator=g), torch.randn(n, nkv, d, generator=g)
+        for j in range(pages[i]):
+            p = int(order[at])
+            at += 1
+            table[i, j] = p
+            part = slice(j * ps, min((j + 1) * ps, n))
+            m = part.stop - part.start
+            kc[p, :, :m] = k[part].transpose(0, 1)
+            vc[p, :, :, :m] = v[part].permute(1, 2, 0)
+        ks.append(k.double())
+        vs.append(v.double())
+    return kc.cuda(), vc.cuda(), table.cuda(), ks, vs
+
+
+def reference(q, ks, vs, seqs, poss, nh, nkv, d, scale, window, sinks):
+    out = torch.empty(q.shape[0], nh, d, dtype=torch.float64)
+    for t, (s, p) in enumerate(zip(seqs, poss)):
+        lo = max(0, p - window + 1) if window else 0
+        for h in range(nh):
+            kv = h // (nh // nkv)
+            sc = ks[s][lo:p + 1, kv] @ q[t, h * d:(h + 1) * d].double() * scale
+            if sinks is not None:
+                sc = torch.cat([sc, sinks[h:h + 1].double()])
+            w = torch.softmax(sc, 0)
+            out[t, h] = w[:p + 1 - lo] @ vs[s][lo:p + 1, kv]
+    return out.view(q.shape[0], nh * d)
+
+
+# heads, key/value heads, head size, page, tokens before and brought by each sequence, window
+CASES = [(12, 2, 128, 16, [(0, 1)], 0), (4, 4, 16, 16, [(0, 17), (15, 1), (16, 2)], 0), (6, 2, 80, 32, [(130, 1), (0, 33), (200, 40)], 0),
+         (16, 1, 64, 48, [(300, 5), (31, 1), (0, 16)], 40), (20, 1, 32, 16, [(127, 1), (128, 1), (129, 20)], 1), (2, 1, 112, 16, [(0, 300)], 100)]
+
+
+@pytest.mark.parametrize("nh,nkv,d,ps,entries,window", CASES)
+@pytest.mark.parametrize("with_sinks", [False, True])
+def test_float32_attention(nh, nkv, d, ps, entries, window, with_sinks):
+    from zedinfer_amd import ops
+    g = torch.Generator().manual_seed(nh * d + len(entries))
+    kc, vc, table, ks, vs = paged([a + b for a, b in entries], nkv, d, ps, g)
+    seqs = [s for s, (a, b) in enumerate(entries) for _ in range(b)]
+    poss = [a + j for a, b in entries for j in range(b)]
+    n = len(seqs)
+    q = torch.randn(n, nh * d, generator=g)
+    sinks = torch.randn(nh, generator=g) if with_sinks else None
+    scale = 1.0 / math.sqrt(d)
+    args = (kc, vc, torch.tensor(seqs, dtype=torch.int32).cuda(), torch.tensor(poss, dtype=torch.int32).cuda(), table, nh, nkv, d, scale, window)
+    kw = dict(sinks=sinks.cuda()) if with_sinks else {}
+    got = ops.attention(q.cuda(), *args, **kw)
+    ref = reference(q, ks, vs, seqs, poss, nh, nkv, d, scale, window, sinks)
+    # the scores, about 5 at most here, carry d roundings of 2^-24 of a sum of |q k| (about 0.64 d, scaled); a probability is off
+    # by as much, relatively, and an output of size up to about 4 by twice that; 4e-6 for 128 dims and 2e-6 for the rest
+    assert float((got.cpu().double() - ref).abs().max()) <= 2e-5
+    # a token a workgroup, and any subset of the tokens: the same bits
+    assert torch.equal(ops.attention(q.cuda(), *args, decoded=True, **kw), got)
+    some = torch.arange(n - 1, -1, -3, dtype=torch.int32).flip(0).cuda()
+    part = torch.zeros_like(got)
+    ops.attention(q.cuda(), *args, out=part, tok_index=some, **kw)
+    assert torch.equal(part[some.long()], got[some.long()]) and int((part != 0).any(1).sum()) == some.numel()
+    # a query row among wider ones
+    wide = torch.zeros(n, nh * d + 8, device="cuda")
+    wide[:, 4:-4] = q.cuda()
+    assert torch.equal(ops.attention(wide[:, 4:-4], *args, **kw), got)
+
+
+def test_float32_attention_sees_no_later_token():
+    """A later token's infinities and NaN stay out of an earlier token's result, also in the block and the workgroup they share."""
+    from zedinfer_amd import ops
+    nh, nkv, d, ps, n = 6, 2, 64, 16, 45
+    g = torch.Generator().manual_seed(3)
+    kc, vc, table, ks, vs = paged([n, n], nkv, d, ps, g)
+    q = torch.randn(2 * n, nh * d, generator=g).cuda()
+    seq = torch.arange(2, dtype=torch.int32).repeat_interleave(n).cuda()
+    pos = torch.arange(n, dtype=torch.int32).repeat(2).cuda()
+    clean = ops.attention(q, kc, vc, seq, pos, table, nh, nkv, d, 0.1)
+    assert bool(torch.isfinite(clean).all())
+    at, page = 37, int(table[0, 37 // ps])
+    vc[page, 1, 3, at % ps], kc[page, 0, at % ps, 5] = float("nan"), float("inf")
+    got = ops.attention(q, kc, vc, seq, pos, table, nh, nkv, d, 0.1)
+    assert torch.allclose(got[:at], clean[:at], rtol=1e-5, atol=1e-6) and torch.equal(got[n:], clean[n:])
+    assert bool(torch.isnan(got[at:n].view(-1, nh, d)[:, 3:, 3]).all())

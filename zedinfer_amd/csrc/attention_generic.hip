@@ -17,8 +17,8 @@
 // It takes every head size up to 512, any number of heads and groups, any page
 // size, both storage types, prompts and decoded tokens alike, and its result
 // for a token depends only on that token's position and keys, not on the
-// batch.  The faster kernels cover the common shapes; this one covers the rest
-// and the float32 path.
+// batch.  The faster kernels cover the common shapes (attention_f32.hip the float32
+// ones); this one covers the rest.
 #include "zi_common.h"
 #include "zi_api.h"
 

@@ -29,6 +29,11 @@ int zi_attention_generic(void* out, const void* q, int dt, int n, int64_t ldq, i
     void* vcache, const int32_t* tok_index, const int32_t* tok_seq, const int32_t* tok_pos, const int32_t*
     block_tables, int max_pages, int num_pages, int nh, int nkv, int d, int page_size, int window, float scale,
     hipStream_t stream);
+// attention_f32.hip
+int zi_attention_f32(void* out, const void* q, int n, int64_t ldq, int64_t ldo, const void* kcache, const void* vcache, const
+    int32_t* tok_index, const int32_t* tok_seq, const int32_t* tok_pos, const int32_t* block_tables, int max_pages, int
+    num_pages, int nh, int nkv, int d, int page_size, int window, float scale, const float* sinks, int by_heads, hipStream_t
+    stream);
 // attention_prefill.hip
 int zi_attention_prefill_maps(void* out, const void* q, int dt, int num_tiles, int64_t ldq, int64_t ldo, const void* kcache,
     const void* vcache, const int32_t* tile_entry, const int32_t* tile_off, const int32_t* entry_start, const int32_t* entry_len,
@@ -394,6 +399,7 @@ int zi_sample(int32_t* out, const float* logits, int64_t ld, float* work, int ro
     X(zi_attention_decode) \
     X(zi_attention_decode_fused) \
     X(zi_attention_decode_project) \
+    X(zi_attention_f32) \
     X(zi_attention_generic) \
     X(zi_attention_prefill) \
     X(zi_decode_layer) \

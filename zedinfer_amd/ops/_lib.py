@@ -28,6 +28,8 @@ _PROTOTYPES = {
     "zi_add_rmsnorm": [P, I, P, P, I, I, L, P, I, I, I, F, I, P],
     "zi_rope_kv_store": [P, P, P, I, I, L, L, L, P, P, P, P, L, I, I, I, I, I, I, P],
     "zi_rope": [P, P, I, I, L, L, P, P, I, I, I, P],
+    "zi_attention_f32": [P, P, I, L, L, P, P, P, P, P, P, I, I, I, I, I, I, I, F, P, I, P],
+    "zi_attention_f32_supported": [I, I, I, I],
     "zi_attention_generic": [P, P, I, I, L, L, P, P, P, P, P, P, I, I, I, I, I, I, I, F, P],
     "zi_attention_decode": [P, P, I, I, L, L, P, P, P, P, P, P, I, I, I, I, I, I, I, F, I, P, L, P],
     "zi_attention_decode_supported": [I, I, I, I, I],

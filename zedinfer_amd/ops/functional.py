@@ -367,17 +367,26 @@ def _attention_args(what, q, kcache, vcache, tok_seq, tok_pos, block_tables, nh,
 def attention(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, tok_seq: torch.Tensor,
               tok_pos: torch.Tensor, block_tables: torch.Tensor, nh: int, nkv: int, d: int, scale: float,
               window: int = 0, out: Optional[torch.Tensor] = None, tok_index: Optional[torch.Tensor] = None,
-              sinks: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """Causal grouped-query attention of q [n, nh*d] over the paged cache: the plain kernel, for
-    every shape and both storage types.
+              sinks: Optional[torch.Tensor] = None, decoded: bool = False) -> torch.Tensor:
+    """Causal grouped-query attention of q [n, nh*d] over the paged cache, for every shape and both storage types:
+    the plain kernel, or, in float32 where the shape allows, the matrix cores' float32 instruction
+    (``attention_f32_supported``).
 
     Token i belongs to row ``tok_seq[i]`` of ``block_tables`` [seqs, max_pages] and sits at
     absolute position ``tok_pos[i]``; it sees the cached keys at positions
     [max(0, pos - window + 1), pos] (window 0: all of them).  With ``tok_index`` only the listed
     tokens are computed (the other rows of ``out`` are left alone).  ``sinks`` (float32 [nh]): the softmax of
-    head h also counts exp(sinks[h]) in its denominator, a term with no key and no value.  Returns [n, nh*d]."""
+    head h also counts exp(sinks[h]) in its denominator, a term with no key and no value.  ``decoded``: the tokens are
+    single tokens of their sequences, which the float32 kernel then takes a token a workgroup instead of 16 (the same
+    result).  Returns [n, nh*d]."""
     out, n, count, ldq, ldo, pages, ps = _attention_args("attention", q, kcache, vcache, tok_seq, tok_pos,
                                                          block_tables, nh, nkv, d, tok_index, out)
+    if attention_f32_supported(q, nh, nkv, d, ps) and kcache.data_ptr() % 16 == 0 and vcache.data_ptr() % 16 == 0:
+        _lib.call("zi_attention_f32", _p(out), _p(q), count, ldq, ldo, _p(kcache), _p(vcache), _p(tok_index), _p(tok_seq),
+                  _p(tok_pos), _p(block_tables), block_tables.shape[1], pages, nh, nkv, d, ps, int(window), float(scale),
+                  _p(_sinks(sinks, nh, q, "attention")) if sinks is not None else c_void_p(0),
+                  int(bool(decoded) and nh // nkv <= 16), _stream())
+        return out
     args = (_p(out), _p(q), _code(q, "attention"), count, ldq, ldo, _p(kcache), _p(vcache),
             _p(tok_index), _p(tok_seq), _p(tok_pos), _p(block_tables), block_tables.shape[1], pages, nh, nkv, d,
             ps, int(window), float(scale))
@@ -386,6 +395,13 @@ def attention(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, tok_s
     else:
         _lib.call("zi_attention_generic", *args, _stream())
     return out
+
+
+def attention_f32_supported(q: torch.Tensor, nh: int, nkv: int, d: int, page_size: int) -> bool:
+    """Whether ``attention`` takes these queries by the float32 matrix-core kernel: float32, head sizes a multiple of 16 up to
+    128, pages a multiple of 16 positions, 16-byte aligned rows."""
+    return (q.dtype == torch.float32 and q.stride(0) % 4 == 0 and q.data_ptr() % 16 == 0
+            and bool(_lib.load().zi_attention_f32_supported(int(nh), int(nkv), int(d), int(page_size))))
 
 
 def _sinks(sinks: torch.Tensor, nh: int, q: torch.Tensor, what: str) -> torch.Tensor:

@@ -234,6 +234,9 @@ class Attention(Mixer):
                 ops.attention_decode(q, *args, plan.sizes["max_short_keys"], self.window, out=att,
                                      tok_index=plan.dev["short_idx"] if n_short < N else None, workspace=ws,
                                      sinks=self.sinks, **extras)
+            elif plain is ops.attention and ops.attention_f32_supported(q, self.nh, self.nkv, self.d, kc.shape[2]):
+                plain(q, *args, self.window, out=att, tok_index=plan.dev["short_idx"] if n_short < N else None,
+                      sinks=self.sinks, decoded=True)      # (and the portions below)
             else:
                 n_long = -1      # everything through the plain kernel
         if n_long < 0:
