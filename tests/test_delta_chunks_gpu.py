@@ -1,0 +1,85 @@
+"""The delta rule in chunks (csrc/delta_chunks.hip) against the rule token by token in float64: entries around the bound and the
+chunk's edges beside short ones, head sizes, decays down to zero, keys alike, and values that are not finite."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(lens, heads, kvh, dim, vdim, seed, alike=0.0, decay=0.2):
+    n, g = sum(lens), torch.Generator().manual_seed(seed)
+    unit = lambda t: t / t.norm(dim=-1, keepdim=True)  # noqa: E731
+    q = unit(torch.randn(n, kvh, dim, generator=g)) * dim ** -0.5
+    k = unit(torch.randn(n, kvh, dim, generator=g) + alike * torch.randn(1, kvh, dim, generator=g))
+    v, beta = torch.randn(n, heads, vdim, generator=g), torch.rand(n, heads, generator=g)
+    gate = torch.exp(-decay * torch.rand(n, heads, generator=g) ** 4)
+    state = torch.randn(len(lens) + 1, heads * dim * vdim + 12, generator=g) * 0.2
+    return q, k, v, beta, gate, state
+
+
+def _run(ops, lens, q, k, v, beta, gate, state, chunked):
+    n, kvh, dim = q.shape
+    heads, vdim, E = v.shape[1], v.shape[2], len(lens)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    qk, bg = torch.cat([q.reshape(n, -1), k.reshape(n, -1)], 1).cuda(), torch.stack([beta, gate], 1).cuda()
+    need = ops.delta_rule_workspace(n, E, heads, dim, vdim)
+    assert bool(need) == (n - (E - 1) >= 64) or dim % 16 or vdim % 16
+    ws = torch.full((need,), float("nan"), device="cuda") if chunked and need else None
+    out, st = torch.full((n, heads * vdim), 7.0, device="cuda"), state.cuda()
+    ops.delta_rule(qk, v.reshape(n, -1).cuda(), bg, st, i32([sum(lens[:e]) for e in range(E)]), i32(lens), i32(list(range(E, 0, -1))),
+                   heads, kvh, dim, vdim, out=out, workspace=ws)
+    return out.cpu().view(n, heads, vdim), st.cpu()
+
+
+def _plain(lens, q, k, v, beta, gate, state):
+    n, kvh, dim = q.shape
+    heads, vdim, at = v.shape[1], v.shape[2], 0
+    out, left = torch.empty(n, heads, vdim, dtype=torch.float64), state.double().clone()
+    q, k = (t.double().repeat_interleave(heads // kvh, 1) for t in (q, k))
+    for e, ln in enumerate(lens):
+        S = left[len(lens) - e, :heads * dim * vdim].view(heads, dim, vdim)      # (a view: updated in place)
+        for t in range(at, at + ln):
+            S *= gate[t].double()[:, None, None]
+            u = beta[t].double()[:, None] * (v[t].double() - torch.einsum("hdv,hd->hv", S, k[t]))
+            S += k[t][:, :, None] * u[:, None]
+            out[t] = torch.einsum("hdv,hd->hv", S, q[t])
+        at += ln
+    return out, left
+
+
+# entries, heads, key heads, dim, vdim, keys alike, decay
+CASES = [([64], 1, 1, 16, 16, 0.0, 0.2), ([63, 1, 65], 2, 1, 32, 48, 0.0, 3.0), ([127, 3, 128, 1, 129], 3, 3, 112, 16, 0.0, 0.05),
+         ([200, 70], 12, 6, 128, 128, 3.0, 0.02), ([256], 9, 3, 64, 144, 0.0, 300.0), ([1] * 70 + [100], 2, 2, 48, 32, 1.0, 0.5)]
+
+
+@pytest.mark.parametrize("lens,heads,kvh,dim,vdim,alike,decay", CASES)
+def test_delta_rule_in_chunks(lens, heads, kvh, dim, vdim, alike, decay):
+    from zedinfer_amd import ops
+    x = _inputs(lens, heads, kvh, dim, vdim, seed=dim + vdim, alike=alike, decay=decay)
+    want, left = _plain(lens, *x)
+    got, state = _run(ops, lens, *x, chunked=True)
+    alone, alone_state = _run(ops, lens, *x, chunked=False)
+    # token by token in float32 shows what rounding does to these inputs; another order of the same sums may be off by a few times
+    # that (T's entries are bounded by one, so nothing grows in between)
+    for a, b, ref in ((got, alone, want), (state, alone_state, left)):
+        own = float((b.double() - ref).norm() / ref.norm())
+        assert own < 2e-6 and float((a.double() - ref).norm() / ref.norm()) <= 3 * own + 2e-7
+    assert torch.equal(state[0], x[5][0]) and torch.equal(state[:, heads * dim * vdim:], x[5][:, heads * dim * vdim:])      # others' memory
+
+
+def test_a_decay_of_zero_and_values_that_are_not_finite():
+    """A decay of zero forgets all at once; a NaN or an infinity reaches its own and later tokens of its head and no earlier ones."""
+    from zedinfer_amd import ops
+    lens = [150, 90]
+    q, k, v, beta, gate, state = _inputs(lens, 4, 2, 32, 32, seed=3)
+    gate[70], gate[100, 1] = 0.0, 0.0
+    want, left = _plain(lens, q, k, v, beta, gate, state)
+    got, st = _run(ops, lens, q, k, v, beta, gate, state, True)
+    assert float((got.double() - want).norm() / want.norm()) < 1e-6 and float((st.double() - left).norm() / left.norm()) < 1e-6
+    k[140, 0, 3], v[60, 3, 5] = float("nan"), float("inf")       # heads 0 and 1 read key head 0
+    bad, _ = _run(ops, lens, q, k, v, beta, gate, state, True)
+    plain, _ = _run(ops, lens, q, k, v, beta, gate, state, False)
+    assert torch.equal(torch.isnan(bad), torch.isnan(plain)) and torch.equal(torch.isinf(bad), torch.isinf(plain))
+    fine = torch.isfinite(plain)
+    assert bool(fine[:60].all()) and bool(fine[:140, :3].all()) and not bool(fine[140:150, :2].any()) and bool(fine[150:].all())
+    assert float((bad - got)[fine & torch.isfinite(bad)].abs().max()) < 1e-5

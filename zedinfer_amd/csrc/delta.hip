@@ -152,6 +152,7 @@ extern "C" int zi_delta_conv_state(float* state, int64_t state_stride, int64_t c
 #define DELTA_COLS 8
 #define DELTA_PARTS 8
 #define DELTA_TOKS 8
+#define DELTA_CHUNK 64
 
 // x of the lane that `ctrl` names within this lane's row of 16 (quad permutations, mirrors)
 template <int CTRL>
@@ -172,7 +173,8 @@ __global__ void __launch_bounds__(ZI_WAVE)
 delta_rule_kernel(float* __restrict__ out, const float* __restrict__ qk, const float* __restrict__ v,
                   const float* __restrict__ beta_g, float* __restrict__ state, int64_t state_stride,
                   const int32_t* __restrict__ entry_start, const int32_t* __restrict__ entry_len,
-                  const int32_t* __restrict__ entry_slot, int heads, int kvh, int dim, int vdim) {
+                  const int32_t* __restrict__ entry_slot, int heads, int kvh, int dim, int vdim, int shortest,
+                  const int32_t* __restrict__ marks) {
     constexpr int D = DELTA_PARTS * R, PRE = DELTA_TOKS * D * 2 / ZI_WAVE;
     __shared__ __attribute__((aligned(16))) float qks[2][2][DELTA_TOKS][D];      // [buffer][q, k][token][d]
     __shared__ float vs[2][DELTA_TOKS][DELTA_COLS];
@@ -183,6 +185,17 @@ delta_rule_kernel(float* __restrict__ out, const float* __restrict__ qk, const f
     const bool live = col < vdim;
     const int kh = h / (heads / kvh), qkc = 2 * kvh * dim;
     const int start = entry_start[e], len = entry_len[e];
+    if (marks && len >= shortest) {
+        // an entry that is done in chunks of DELTA_CHUNK tokens (delta_chunks.hip; numbered entry by entry), unless one of its
+        // chunks is marked for this head
+        int id = 0;
+        for (int i = lane; i < e; i += ZI_WAVE) id += entry_len[i] >= shortest ? (entry_len[i] + DELTA_CHUNK - 1) / DELTA_CHUNK : 0;
+#pragma unroll
+        for (int o = ZI_WAVE / 2; o > 0; o >>= 1) id += __shfl_xor(id, o, ZI_WAVE);
+        bool left = false;
+        for (int i = lane; i < (len + DELTA_CHUNK - 1) / DELTA_CHUNK; i += ZI_WAVE) left |= marks[(int64_t)(id + i) * heads + h] != 0;
+        if (!__ballot(left)) return;
+    }
     float* S = state + (int64_t)entry_slot[e] * state_stride + (int64_t)h * dim * vdim;
     float s[R];
 #pragma unroll
@@ -289,10 +302,10 @@ delta_rule_kernel(float* __restrict__ out, const float* __restrict__ qk, const f
     }
 }
 
-extern "C" int zi_delta_rule(float* out, const float* qk, const float* v, const float* beta_g, float* state,
-                             int64_t state_stride, const int32_t* entry_start, const int32_t* entry_len,
-                             const int32_t* entry_slot, int entries, int heads, int kvh, int dim, int vdim,
-                             hipStream_t stream) {
+// `marks` (or null): entries of at least `shortest` tokens are done only for heads with a mark (see delta_chunks.hip).
+int zi_delta_rule_launch(float* out, const float* qk, const float* v, const float* beta_g, float* state, int64_t state_stride,
+                         const int32_t* entry_start, const int32_t* entry_len, const int32_t* entry_slot, int entries, int heads,
+                         int kvh, int dim, int vdim, int shortest, const int32_t* marks, hipStream_t stream) {
     ZI_REQUIRE(entries >= 0 && entries <= 65535 && heads > 0 && heads <= 65535 && kvh > 0 && heads % kvh == 0 && dim > 0 &&
                vdim > 0, "delta_rule: bad sizes");
     ZI_REQUIRE(dim <= 256, "delta_rule: dim %d is more than the 256 rows a wavefront holds", dim);
@@ -301,13 +314,21 @@ extern "C" int zi_delta_rule(float* out, const float* qk, const float* v, const 
     const dim3 grid((vdim + DELTA_COLS - 1) / DELTA_COLS, heads, entries);
 #define ZI_DELTA_RULE(R)                                                                                         \
     delta_rule_kernel<R><<<grid, ZI_WAVE, 0, stream>>>(out, qk, v, beta_g, state, state_stride, entry_start,      \
-                                                       entry_len, entry_slot, heads, kvh, dim, vdim)
+                                                       entry_len, entry_slot, heads, kvh, dim, vdim, shortest, marks)
     if (dim <= 32) ZI_DELTA_RULE(4);
     else if (dim <= 64) ZI_DELTA_RULE(8);
     else if (dim <= 128) ZI_DELTA_RULE(16);
     else ZI_DELTA_RULE(32);
 #undef ZI_DELTA_RULE
     return zi_check_launch("delta_rule");
+}
+
+extern "C" int zi_delta_rule(float* out, const float* qk, const float* v, const float* beta_g, float* state,
+                             int64_t state_stride, const int32_t* entry_start, const int32_t* entry_len,
+                             const int32_t* entry_slot, int entries, int heads, int kvh, int dim, int vdim,
+                             hipStream_t stream) {
+    return zi_delta_rule_launch(out, qk, v, beta_g, state, state_stride, entry_start, entry_len, entry_slot, entries, heads, kvh, dim,
+                                vdim, 0, nullptr, stream);
 }
 
 // o [rows][vdim] (a row per token and head) divided by its root mean square, times a weight [vdim], times

@@ -86,6 +86,7 @@ _PROTOTYPES = {
     "zi_delta_prepare": [P, P, P, P, L, I, P, P, P, I, P, L, L, P, P, P, I, I, I, I, I, P],
     "zi_delta_conv_state": [P, L, L, P, L, P, P, P, I, I, I, P],
     "zi_delta_rule": [P, P, P, P, P, L, P, P, P, I, I, I, I, I, P],
+    "zi_delta_rule_chunked": [P, P, P, P, P, L, P, P, P, I, I, I, I, I, I, P, L, P],
     "zi_gated_rmsnorm": [P, I, P, P, I, P, L, I, I, I, F, P],
     "zi_moe_route": [P, P, P, P, I, I, I, F, P],
     "zi_moe_group": [P, P, P, P, I, I, I, P],
@@ -194,6 +195,8 @@ def load() -> ctypes.CDLL:
             fn.restype = c_int
         lib.zi_gemm_skinny_workspace.argtypes = [I, I, I]
         lib.zi_gemm_skinny_workspace.restype = c_int64
+        lib.zi_delta_rule_workspace.argtypes = [I, I, I, I, I]
+        lib.zi_delta_rule_workspace.restype = c_int64
         lib.zi_attention_decode_workspace.argtypes = [I, I, I]
         lib.zi_attention_decode_workspace.restype = c_int64
         lib.zi_attention_prefill_workspace.argtypes = [I, I, I, I]

@@ -367,9 +367,11 @@ def delta_conv_state(state: torch.Tensor, proj: torch.Tensor, entry_start: torch
 
 def delta_rule(qk: torch.Tensor, v: torch.Tensor, beta_g: torch.Tensor, state: torch.Tensor, entry_start: torch.Tensor,
                entry_len: torch.Tensor, entry_slot: torch.Tensor, heads: int, kv_heads: int, dim: int, vdim: int,
-               out: torch.Tensor) -> torch.Tensor:
+               out: torch.Tensor, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Every entry's tokens in order, per head: S <- g S; u = beta (v - S^T k); S <- S + k u^T; o = S^T q, with S
-    read from and left in ``state`` [slots, ...]; out [n, heads * vdim] float32."""
+    read from and left in ``state`` [slots, ...]; out [n, heads * vdim] float32.  With a ``workspace`` of
+    ``delta_rule_workspace`` floats long entries are done in chunks on the matrix cores' float32 instruction (the products
+    regrouped: another rounding of the same size)."""
     _gpu("delta_rule", qk, v, beta_g, state, entry_start, entry_len, entry_slot, out)
     n = qk.shape[0]
     _f32(qk, "delta_rule qk", (n, 2 * kv_heads * dim))
@@ -384,9 +386,21 @@ def delta_rule(qk: torch.Tensor, v: torch.Tensor, beta_g: torch.Tensor, state: t
     E = entry_start.numel()
     for t in (entry_start, entry_len, entry_slot):
         _i32(t, "delta_rule entries", E)
+    if workspace is not None and workspace.numel() and qk.data_ptr() % 16 == 0 and v.data_ptr() % 16 == 0:
+        _gpu("delta_rule", workspace)
+        _f32(workspace, "delta_rule workspace")
+        _lib.call("zi_delta_rule_chunked", _p(out), _p(qk), _p(v), _p(beta_g), _p(state), int(state.shape[1]), _p(entry_start),
+                  _p(entry_len), _p(entry_slot), n, E, heads, kv_heads, dim, vdim, _p(workspace), workspace.numel(), _stream())
+        return out
     _lib.call("zi_delta_rule", _p(out), _p(qk), _p(v), _p(beta_g), _p(state), int(state.shape[1]), _p(entry_start),
               _p(entry_len), _p(entry_slot), E, heads, kv_heads, dim, vdim, _stream())
     return out
+
+
+def delta_rule_workspace(n: int, entries: int, heads: int, dim: int, vdim: int) -> int:
+    """Floats of workspace with which ``delta_rule`` does n tokens of so many entries in chunks; 0 where it does not (no entry
+    can be long enough, or head sizes that are no multiples of 16)."""
+    return int(_lib.load().zi_delta_rule_workspace(int(n), int(entries), int(heads), int(dim), int(vdim)))
 
 
 def gated_rms_norm(o: torch.Tensor, weight: torch.Tensor, gate: torch.Tensor, heads: int, vdim: int, eps: float,

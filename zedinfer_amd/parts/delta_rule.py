@@ -92,7 +92,9 @@ class GatedDeltaRule(Mixer):
         ops.delta_conv_state(state, proj, batch.entry_start, batch.entry_len, batch.entry_slot, nh, kvh, dim, vdim,
                              self.taps)
         o = rt.buffer("delta_read", (n, nh * vdim), torch.float32)
-        ops.delta_rule(qk, v, beta_g, state, batch.entry_start, batch.entry_len, batch.entry_slot, nh, kvh, dim, vdim, out=o)
+        need = ops.delta_rule_workspace(n, batch.entry_start.numel(), nh, dim, vdim)
+        ops.delta_rule(qk, v, beta_g, state, batch.entry_start, batch.entry_len, batch.entry_slot, nh, kvh, dim, vdim, out=o,
+                       workspace=rt.buffer("delta_chunks", (need,), torch.float32) if need else None)
         y = rt.buffer("delta_heads", (n, nh * vdim))
         ops.gated_rms_norm(o, self.norm, proj[:, self.gate_at:self.gate_at + nh * vdim], nh, vdim, self.eps, out=y)
         if out is None:
