@@ -44,46 +44,45 @@ __device__ __forceinline__ gm_u32x4_t gm_keep(gm_u32x4_t v, bool keep) {
     return v & mask;
 }
 
-// What a wavefront does with its sums: C[n = n0 + j*4 + e][m = t*16 + r] in acc[t][e].
+// What a wavefront does with its sums: C[n = n0 + j*4 + e][m = m0 + t*16 + r] in acc[t][e].
 template <int MT>
 __device__ __forceinline__ void gm_epilogue(const gm_f32x4_t (&acc)[MT], void* __restrict__ out, int mode, int out_f32,
                                             const zi_bf16* __restrict__ bias_in, int M, int N, int64_t ldo, int split,
-                                            int n0, int r, int j, int vec_out, float limit) {
+                                            int n0, int r, int j, int vec_out, float limit, int m0 = 0) {
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
         gm_f32x4_t s = acc[t];
         const zi_bf16* bias = bias_in;
-        const int m = t * 16 + r;
+        const int m = m0 + t * 16 + r;
         if (mode == GM_MODE_SWIGLU || mode == GM_MODE_CLAMPED) {
             if (mode == GM_MODE_CLAMPED && bias && n0 < N) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) s[e] += zi_load(bias + n0 + j * 4 + e);
             }
-            // lanes j = 0,1 hold gate rows j*4 + e, lanes j = 2,3 the up rows of the same columns
-            gm_f32x4_t up;
-            up[0] = __shfl_xor(s[0], 32, ZI_WAVE); up[1] = __shfl_xor(s[1], 32, ZI_WAVE);
-            up[2] = __shfl_xor(s[2], 32, ZI_WAVE); up[3] = __shfl_xor(s[3], 32, ZI_WAVE);
-            if (j >= 2 || m >= M || n0 >= N) continue;
-            const int col = (n0 / 16) * 8 + j * 4;     // N / 2 columns of output; N % 16 == 0
-            float act[4];
+            // lanes j = 0,1 hold gate rows j*4 + e, lanes j = 2,3 the up rows of the same columns: they trade halves, so that each
+            // lane makes two columns (nothing overlaps the exponentials at a product's end: 19.7 us for gate/up of 80 rows at the
+            // 1.5B sizes, 21.5 when lanes 0, 1 made four)
+            const bool low = j < 2;
+            const float t0 = __shfl_xor(low ? s[2] : s[0], 32, ZI_WAVE), t1 = __shfl_xor(low ? s[3] : s[1], 32, ZI_WAVE);
+            if (m >= M || n0 >= N) continue;
+            const int col = (n0 / 16) * 8 + (j & 1) * 4 + (low ? 0 : 2);     // N / 2 columns of output; N % 16 == 0
+            float act[2];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
+            for (int e = 0; e < 2; ++e) {
+                const float gate = low ? s[e] : e ? t1 : t0, other = low ? (e ? t1 : t0) : s[2 + e];
                 if (mode == GM_MODE_SWIGLU) {
-                    act[e] = up[e] * (s[e] / (1.f + expf(-s[e])));
+                    act[e] = other * (gate / (1.f + expf(-gate)));
                 } else {
-                    const float g = fminf(s[e], limit), u = fminf(fmaxf(up[e], -limit), limit);
+                    const float g = fminf(gate, limit), u = fminf(fmaxf(other, -limit), limit);
                     act[e] = g / (1.f + expf(-1.702f * g)) * (u + 1.f);
                 }
             }
             zi_bf16* dst = (zi_bf16*)out + (int64_t)m * ldo + col;
             if (vec_out) {
-                uint2 pk;
-                pk.x = zi_pack_bf16x2(act[0], act[1]);
-                pk.y = zi_pack_bf16x2(act[2], act[3]);
-                *reinterpret_cast<uint2*>(dst) = pk;
+                *reinterpret_cast<uint32_t*>(dst) = zi_pack_bf16x2(act[0], act[1]);
             } else {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) zi_store(dst + e, act[e]);
+                for (int e = 0; e < 2; ++e) zi_store(dst + e, act[e]);
             }
             continue;
         }
@@ -269,122 +268,141 @@ gemm_mid_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* __
     gm_epilogue<MT>(acc, out, mode, out_f32, bias, M, N, ldo, split, n0, r, j, vec_out, limit);
 }
 
-// The same product for 65 .. 128 rows of x (MT = 5 .. 8 tiles of 16 rows): one pass over the weights where two
-// launches of the kernel above would make two, and where the library's products of so few rows stay far from the
-// weights' stream.  The registers that the kernel above spends on rings of x and on all of a block's x operands
-// do not stretch to eight tiles, so here a block's x is requested one step ahead only (it comes from the cache;
-// the weights keep their ring of three), it lies in LDS once (two barriers a block instead of one; a second
-// buffer for it, 96 KB of LDS in all, was measured and changed nothing), and the x operands
-// are read a k-step at a time, just before their matrix instructions.  The cut, the order of the sums and the
-// epilogues are the kernel's above: a row's result does not depend on which of the two kernels makes it.
-template <int MT, int GM_WAVES>
-__global__ void __launch_bounds__(GM_WAVES* ZI_WAVE)
+// The same product for 65 .. 128 rows of x (MT = 5 .. 8 tiles of 16 rows): one pass over the weights where two launches of the
+// kernel above would make two.  With that many rows the reads of x from LDS bind a workgroup whose wavefronts each take all of
+// them for 16 weight rows (16.3 us for a down product of 27 MB), so here four wavefronts take 32 rows of x each and all of
+// the workgroup's NT x 16 weight rows: 2 + NT operands read for 2 NT products.  Both operands go straight into LDS
+// (global_load_lds_dwordx4, 1 KB an instruction, rows of 128 bytes with piece c of row q at place c xor (q / 2 mod 8)), k in
+// steps of 64 through four buffers, three steps on their way while one is worked on (six buffers were no faster); every wavefront issues as many loads a step
+// as every other, so that each can wait for its own by count before the step's one barrier.  The cut, the order of the
+// sums and the epilogues are the kernel's above: a row's result does not depend on which of the two kernels makes it.
+// Measured at 128 rows, weights from memory, against wavefronts of 16 weight rows: 1.5B sizes down 16.3 to 13.5 us, q/k/v 7.3 to
+// 7.2, output 7.4 to 6.9; 7B sizes down 53 to 36, q/k/v 20 to 15, output 16 to 13.  With the SwiGLU epilogue 25.2 us at 128 rows
+// and 19.7 at 80 (1.5B gate/up), where the library's product and the activation's launch take 23 + 4.8, and 76 against 72 +
+// 6 at the 7B sizes.  A step's instructions were what bound it first: loads whose addresses cost nothing (a buffer, a lane's
+// offset and a step's) took 80 rows of the 1.5B gate/up from 20.6 to 18.0 us.
+#define GW_KB 64
+
+#define GW_STAGES 4
+
+// the wavefront's loads but for the newest `n` have arrived (n counts loads; LDS and scalar counters are not waited for)
+template <int n>
+__device__ __forceinline__ void gw_wait() {
+    static_assert(n < 64, "the counter has six bits");
+    __builtin_amdgcn_s_waitcnt((n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14));
+}
+
+// 16 bytes a lane from a buffer into LDS, lane after lane from `to` on; what lies past the buffer's end gives zeros.
+template <int AUX>
+__device__ __forceinline__ void gw_to_lds(__amdgpu_buffer_rsrc_t from, gm_u32x4_t* to, int lane_at, int at) {
+#ifdef __HIP_DEVICE_COMPILE__       // (the host's pass knows loads of this size for no target)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, to, 16, lane_at, at, 0, AUX);
+#endif
+}
+
+template <int MT, int NT>
+__global__ void __launch_bounds__(4 * ZI_WAVE)
 gemm_wide_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* __restrict__ x,
                  const zi_bf16* __restrict__ w, const zi_bf16* __restrict__ bias, int M, int N, int K, int64_t ldx,
                  int64_t ldw, int64_t ldo, int kb_per_split, int vec_out, float limit) {
-    constexpr int RING = 3;
-    __shared__ __attribute__((aligned(16))) uint16_t xs[MT * 16 * GM_XS];
-    __shared__ __attribute__((aligned(16))) uint16_t wt[GM_WAVES][16 * GM_XS];
-    const int tid = threadIdx.x, lane = tid & (ZI_WAVE - 1), wave = tid / ZI_WAVE;
+    constexpr int XI = 2 * MT, LOADS = XI + 2 * NT, PW = (LOADS + 3) / 4;       // 1 KB loads of x, of a step; a wavefront's share
+    constexpr int PIECES = LOADS * ZI_WAVE;
+    // (arrays of their own, so that the compiler can tell a buffer that is read from those that loads are on their way to)
+    __shared__ __attribute__((aligned(16))) gm_u32x4_t s0[PIECES], s1[PIECES], s2[PIECES], s3[PIECES], spare[ZI_WAVE];       // (spare: where loads go that nobody needs)
+    const int tid = threadIdx.x, lane = tid & (ZI_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(tid / ZI_WAVE);
     const int r = lane & 15, j = lane >> 4;
     const int split = blockIdx.y;
-    const int kb_total = (K + GM_KB - 1) / GM_KB;
-    const int kb_lo = split * kb_per_split;
-    const int kb_hi = (kb_lo + kb_per_split < kb_total) ? kb_lo + kb_per_split : kb_total;
-    const int n0 = (blockIdx.x * GM_WAVES + wave) * 16;
-    const int wq = lane & 15;
-    const zi_bf16* wrow[4];
+    const int k_lo = split * kb_per_split * GM_KB, k_hi = k_lo + kb_per_split * GM_KB < K ? k_lo + kb_per_split * GM_KB : K;
+    const int steps = (k_hi - k_lo + GW_KB - 1) / GW_KB;
+    const int n0 = blockIdx.x * NT * 16;
+    // Load i of a step takes 8 rows: lane l row l / 8 of them, the piece that belongs at place l % 8.  A step's place along k is the
+    // same for all lanes and loads, so that a load costs no arithmetic (with one wavefront a SIMD every instruction counts).
+    // Rows past M or N are past the buffers' ends and zero; columns past K are the next row's, and masked when they are used.
+    const int rows_w = N - n0 < NT * 16 ? N - n0 : NT * 16;
+    const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc(const_cast<zi_bf16*>(x), 0, (int)(((M - 1) * ldx + K) * 2), 0x00020000);
+    const __amdgpu_buffer_rsrc_t wb = __builtin_amdgcn_make_buffer_rsrc(const_cast<zi_bf16*>(w + (int64_t)n0 * ldw), 0,
+                                                                        (int)(((rows_w - 1) * ldw + K) * 2), 0x00020000);
+    int lane_at[PW];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const int n = n0 + c * 4 + j;
-        wrow[c] = w + (int64_t)(n < N ? n : N - 1) * ldw;
+    for (int i = 0; i < PW; ++i) {
+        const int L = i * 4 + wave;
+        const int q = (L < XI ? L : L - XI) * 8 + lane / 8;
+        lane_at[i] = (int)(q * (L < XI ? ldx : ldw) * 2) + ((lane & 7) ^ ((q >> 1) & 7)) * 16;
     }
-    uint16_t* const wt_w = &wt[wave][0];
-    // the block's x slice is dealt out over all the workgroup's threads (see the kernel above)
-    constexpr int THREADS = GM_WAVES * ZI_WAVE, XP = (MT * 256 + THREADS - 1) / THREADS;
-    const int spc = tid % 16;
-    int srow[XP];
+    auto issue = [&](gm_u32x4_t* buf, int t) {
+        const int at = t < steps ? (k_lo + t * GW_KB) * 2 : 0x7fffffff;       // (steps past the end: past the buffers' ends, nothing is fetched)
 #pragma unroll
-    for (int p = 0; p < XP; ++p) srow[p] = p * (THREADS / 16) + tid / 16;
-    gm_u32x4_t ring[RING][4], xnext[XP];
-    const zi_bf16* xrow[XP];
-#pragma unroll
-    for (int p = 0; p < XP; ++p) xrow[p] = x + (int64_t)(srow[p] < M ? srow[p] : M - 1) * ldx;
-    // a block's x is requested before the weights that are requested in the same step: loads return in order,
-    // and x is wanted first.  The block index is clamped: the last step asks for its own block again.
-    auto fetch_x = [&](int kb) __attribute__((always_inline)) {
-        const int k0 = (kb < kb_hi ? kb : kb_hi - 1) * GM_KB;
-        const int kx = k0 + spc * 8 < K ? k0 + spc * 8 : K - 8;
-#pragma unroll
-        for (int p = 0; p < XP; ++p) xnext[p] = *reinterpret_cast<const gm_u32x4_t*>(xrow[p] + kx);
-    };
-    auto fetch_w = [&](const int slot, int kb) __attribute__((always_inline)) {
-        const int k = kb * GM_KB + wq * 8;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) ring[slot][c] = __builtin_nontemporal_load(reinterpret_cast<const gm_u32x4_t*>(wrow[c] + (k < K ? k : K - 8)));
-    };
-    auto stash = [&]() __attribute__((always_inline)) {
-#pragma unroll
-        for (int p = 0; p < XP; ++p)
-            if ((p + 1) * (THREADS / 16) <= MT * 16 || srow[p] < MT * 16)
-                *reinterpret_cast<gm_u32x4_t*>(&xs[srow[p] * GM_XS + (spc ^ (srow[p] & 15)) * 8]) = xnext[p];
-    };
-    gm_f32x4_t acc[MT];
-#pragma unroll
-    for (int t = 0; t < MT; ++t) acc[t] = gm_f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-    auto step = [&](const int slot, int kb, const bool request) __attribute__((always_inline)) {
-        fetch_x(kb + 1);
-        if (request) fetch_w((slot + RING - 1) % RING, kb + RING - 1);
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-            *reinterpret_cast<gm_u32x4_t*>(wt_w + (c * 4 + j) * GM_XS + (wq ^ (c * 4 + j)) * 8) =
-                gm_keep(ring[slot][c], kb * GM_KB + wq * 8 < K);
-        gm_pack a[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) a[c].u = *reinterpret_cast<const gm_u32x4_t*>(wt_w + r * GM_XS + ((c * 4 + j) ^ r) * 8);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            gm_pack bb[MT];
-#pragma unroll
-            for (int t = 0; t < MT; ++t)
-                bb[t].u = *reinterpret_cast<const gm_u32x4_t*>(&xs[(t * 16 + r) * GM_XS + ((c * 4 + j) ^ r) * 8]);
-#pragma unroll
-            for (int t = 0; t < MT; ++t)
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[c].b, bb[t].b, acc[t], 0, 0, 0);
+        for (int i = 0; i < PW; ++i) {
+            const int L = i * 4 + wave;
+            gm_u32x4_t* to = L < LOADS ? buf + L * ZI_WAVE : spare;
+            if (i * 4 + 3 < XI) gw_to_lds<0>(xb, to, lane_at[i], at);
+            else if (i * 4 >= XI) gw_to_lds<2>(wb, to, lane_at[i], at);       // weights are read once: past L2
+            else gw_to_lds<0>(L < XI ? xb : wb, to, lane_at[i], at);
         }
-        __syncthreads();        // every wavefront has read this block's x
-        stash();                // the next block's (after the last block: something nobody reads)
-        __syncthreads();
     };
-    auto ending = [&](auto left_c, int kb0) __attribute__((always_inline)) {
-        constexpr int LEFT = decltype(left_c)::value;
+    gm_f32x4_t acc[NT][2];
 #pragma unroll
-        for (int i = 0; i < LEFT + RING - 1; ++i) step(i % RING, kb0 + i, i < LEFT);
-    };
-    fetch_x(kb_lo);
+    for (int n = 0; n < NT; ++n)
 #pragma unroll
-    for (int b = 0; b < RING - 1; ++b) fetch_w(b, kb_lo + b < kb_hi ? kb_lo + b : kb_hi - 1);
-    stash();
-    __syncthreads();
-    int kb0 = kb_lo;
-    for (; kb0 + 2 * RING - 1 <= kb_hi; kb0 += RING) {
+        for (int t = 0; t < 2; ++t) acc[n][t] = gm_f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const int sw = (r >> 1) & 7;
+    int tile_at[2];         // (past the rows: the last tile again, not stored)
 #pragma unroll
-        for (int b = 0; b < RING; ++b) step(b, kb0 + b, true);
-    }
-    const int left = kb_hi - kb0 - (RING - 1);
-    if (left < 0) {
+    for (int m = 0; m < 2; ++m) tile_at[m] = ((wave * 2 + m < MT ? wave * 2 + m : MT - 1) * 16 + r) * 8;
+    auto step = [&](const gm_u32x4_t* buf, gm_u32x4_t* free, int t) __attribute__((always_inline)) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        gw_wait<(GW_STAGES - 2) * PW>();
+        __builtin_amdgcn_s_barrier();          // all wavefronts' loads of the step are there, and all are done with `free`
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        issue(free, t + GW_STAGES - 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (t >= steps) return;
+        // all of the step's operands are asked for before the first product: their way is paid once
+        gm_pack a[2][NT], b[2][2];
 #pragma unroll
-        for (int b = 0; b < RING - 1; ++b)
-            if (kb0 + b < kb_hi) step(b, kb0 + b, false);
-    } else {
-        switch (left) {
-            case 0: ending(std::integral_constant<int, 0>{}, kb0); break;
-            case 1: ending(std::integral_constant<int, 1>{}, kb0); break;
-            default: ending(std::integral_constant<int, 2>{}, kb0); break;
+        for (int kk = 0; kk < 2; ++kk) {
+            const int at = (kk * 4 + j) ^ sw;
+#pragma unroll
+            for (int m = 0; m < 2; ++m) b[kk][m].u = buf[tile_at[m] + at];
+#pragma unroll
+            for (int n = 0; n < NT; ++n) a[kk][n].u = buf[XI * ZI_WAVE + (n * 16 + r) * 8 + at];
         }
+        const int left = K - (k_lo + t * GW_KB);
+        if (left < GW_KB) {
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+                for (int n = 0; n < NT; ++n) a[kk][n].u = gm_keep(a[kk][n].u, kk * 32 + j * 8 < left);
+#pragma unroll
+                for (int m = 0; m < 2; ++m) b[kk][m].u = gm_keep(b[kk][m].u, kk * 32 + j * 8 < left);
+            }
+        }
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int m = 0; m < 2; ++m)
+                    acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kk][n].b, b[kk][m].b, acc[n][m], 0, 0, 0);
+    };
+    issue(s0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    issue(s1, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    issue(s2, 2);
+    __builtin_amdgcn_sched_barrier(0);
+    for (int t = 0; t < steps; t += GW_STAGES) {
+        step(s0, s3, t);
+        step(s1, s0, t + 1);
+        step(s2, s1, t + 2);
+        step(s3, s2, t + 3);
     }
-    gm_epilogue<MT>(acc, out, mode, out_f32, bias, M, N, ldo, split, n0, r, j, vec_out, limit);
+    gw_wait<0>();       // (no load may arrive after the workgroup's LDS is another's)
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+        gm_epilogue<2>(acc[n], out, mode, out_f32, bias, wave * 32 < MT * 16 ? M : 0, N, ldo, split, n0 + n * 16, r, j, vec_out, limit, wave * 32);
 }
 
 // How the product with a weight matrix [N, K] is cut: wavefronts a workgroup (16 weight rows each), splits
@@ -430,7 +448,7 @@ int64_t zi_gemm_mid_plan(int N, int K, int whole, int* splits, int* kb_per_split
 int zi_gemm_mid_launch(void* out, int out_f32, int mode, const zi_bf16* x, const zi_bf16* w, const zi_bf16* bias, int M,
                        int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int vec_out, float limit, hipStream_t stream) {
     int splits, per, waves;
-    zi_gemm_mid_plan(N, K, mode >= GM_MODE_ACT, &splits, &per, &waves);
+    zi_gemm_mid_plan(N, K, mode >= GM_MODE_ACT || (mode == GM_MODE_SWIGLU && M > 64), &splits, &per, &waves);
     const int tiles = (N + 15) / 16;
     const dim3 grid((tiles + waves - 1) / waves, splits);
     const int mt = (M + 15) / 16;
@@ -446,7 +464,7 @@ int zi_gemm_mid_launch(void* out, int out_f32, int mode, const zi_bf16* x, const
         default: ZI_GM2(MT, 8); break;          \
     }
 #define ZI_GW2(MT, WV)                                                                                         \
-    gemm_wide_kernel<MT, WV><<<grid, WV * ZI_WAVE, 0, stream>>>(out, mode, out_f32, x, w, bias, M, N, K, ldx, ldw, ldo, \
+    gemm_wide_kernel<MT, WV><<<grid, 4 * ZI_WAVE, 0, stream>>>(out, mode, out_f32, x, w, bias, M, N, K, ldx, ldw, ldo, \
                                                                per, vec_out, limit)
 #define ZI_GW(MT)                               \
     switch (waves) {                            \

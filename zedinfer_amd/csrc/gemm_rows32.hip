@@ -1,10 +1,10 @@
-// out[M,N] = x[M,K] . w[N,K]^T for 65 .. 256 rows of x: large decode batches, still bound by the one pass over
+// out[M,N] = x[M,K] . w[N,K]^T for 129 .. 256 rows of x: large decode batches, still bound by the one pass over
 // the weights, where the kernels of gemm_mid.hip (16 weight rows a wavefront) are bound by their reads of x from
 // LDS: every operand of x they read serves 16 weight rows.  Here a wavefront owns 32 weight rows and multiplies
 // with v_mfma_f32_32x32x16_bf16 (a 32 x 32 tile of sums in 16 registers a lane), so an operand of x serves
 // twice the weights, and a workgroup reads half as much of x for the same weights.
 //
-// A workgroup of 4 or 8 wavefronts walks its range of k in blocks of 64.  The block's slice of x (up to 256
+// A workgroup of 4 wavefronts walks its range of k in blocks of 64.  The block's slice of x (up to 256
 // rows x 64 values) lies in LDS, in one of two buffers: the next block's slice is stored while this one is
 // read, one barrier a block.  Each wavefront reads its 32 weight rows from memory as whole lines of 128 bytes
 // (an instruction takes 8 rows), several blocks ahead (a ring of register buffers; loads are issued without
@@ -229,19 +229,18 @@ gemm_rows32_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16*
 }
 
 // How the product with a weight matrix [N, K] is cut for this kernel: wavefronts a workgroup (32 weight rows
-// each), splits of k over workgroups (at most 16) and blocks of 64 per split; a function of N and K and of
-// whether there are more than 128 rows (`many_rows`: the sums of so many rows leave a wavefront registers
-// enough only when a SIMD holds one wavefront, so the workgroups are of four).  As in zi_gemm_mid_plan what
+// each; four, as the sums of so many rows leave a wavefront registers enough only when a SIMD holds one), splits of k
+// over workgroups (at most 16) and blocks of 64 per split; a function of N and K.  As in zi_gemm_mid_plan what
 // counts is the most work any compute unit gets when workgroups are dealt out in turn; `whole` forbids a split
 // (the SwiGLU epilogue needs whole sums).
-void zi_gemm_rows32_plan(int N, int K, int many_rows, int whole, int* splits, int* kb_per_split, int* waves) {
+void zi_gemm_rows32_plan(int N, int K, int whole, int* splits, int* kb_per_split, int* waves) {
     const int tiles = (N + 31) / 32;
     const int kb_total = (K + G32_KB - 1) / G32_KB;
     const int cus = zi_compute_units();
     int64_t best_cost = -1;
     int best_s = 1, best_w = 4, best_per = kb_total;
-    for (int w = 4; w <= (many_rows ? 4 : 8); w *= 2) {
-        const int groups = (tiles + w - 1) / w;
+    {
+        const int w = 4, groups = (tiles + w - 1) / w;
         for (int s0 = 1; s0 <= (whole ? 1 : 16) && s0 <= (kb_total > 1 ? kb_total / 2 : 1); ++s0) {
             const int per = (kb_total + s0 - 1) / s0;
             const int s = (kb_total + per - 1) / per;
@@ -259,34 +258,25 @@ void zi_gemm_rows32_plan(int N, int K, int many_rows, int whole, int* splits, in
     *waves = best_w;
 }
 
-// The launch; the checks are the caller's (zi_gemm_skinny).  M is 1 .. 256.
+// The launch; the checks are the caller's (zi_gemm_skinny).  M is 129 .. 256.
 int zi_gemm_rows32_launch(void* out, int out_f32, int mode, const zi_bf16* x, const zi_bf16* w, const zi_bf16* bias, int M,
                           int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int vec_out, float limit, hipStream_t stream) {
     (void)limit;      // (these products have no clamped epilogue)
     int splits, per, waves;
-    zi_gemm_rows32_plan(N, K, M > 128, mode == G32_MODE_SWIGLU, &splits, &per, &waves);
+    zi_gemm_rows32_plan(N, K, mode == G32_MODE_SWIGLU, &splits, &per, &waves);
     const int tiles = (N + 31) / 32;
     const dim3 grid((tiles + waves - 1) / waves, splits);
     const int mt = (M + 31) / 32;
-    // Workgroups of four wavefronts (a wavefront a SIMD, all 512 registers its own) keep four blocks of weights
-    // in flight; of eight, as many as the 256 registers beside the sums allow.
-#define ZI_G32W(MT, WV, RG)                                                                                            \
-    gemm_rows32_kernel<MT, WV, RG><<<grid, WV * ZI_WAVE, 0, stream>>>(out, mode, out_f32, x, w, bias, M, N, K, ldx, ldw, \
-                                                                     ldo, per, vec_out)
-#define ZI_G32(MT, RG8)                         \
-    if (waves == 4) ZI_G32W(MT, 4, 4);          \
-    else ZI_G32W(MT, 8, RG8)
+    // (a wavefront a SIMD, all 512 registers its own, keeps four blocks of weights in flight)
+#define ZI_G32(MT)                                                                                                  \
+    gemm_rows32_kernel<MT, 4, 4><<<grid, 4 * ZI_WAVE, 0, stream>>>(out, mode, out_f32, x, w, bias, M, N, K, ldx, ldw, \
+                                                                  ldo, per, vec_out)
     switch (mt) {
-        case 1: ZI_G32(1, 4); break;
-        case 2: ZI_G32(2, 4); break;
-        case 3: ZI_G32(3, 3); break;
-        case 4: ZI_G32(4, 3); break;
-        case 5: ZI_G32W(5, 4, 4); break;
-        case 6: ZI_G32W(6, 4, 4); break;
-        case 7: ZI_G32W(7, 4, 4); break;
-        default: ZI_G32W(8, 4, 4); break;
+        case 5: ZI_G32(5); break;
+        case 6: ZI_G32(6); break;
+        case 7: ZI_G32(7); break;
+        default: ZI_G32(8); break;
     }
 #undef ZI_G32
-#undef ZI_G32W
     return zi_check_launch("gemm_rows32");
 }

@@ -2,7 +2,7 @@
 // one pass over the weights.  This file holds their entry points, the cut's bookkeeping and the kernel that
 // adds partial sums; the product kernels are in gemm_mid.hip (up to 128 rows: x staged in LDS, a workgroup's
 // wavefronts take 16 weight rows each, the cut over workgroups balanced over the compute units) and in
-// gemm_rows32.hip (more rows, and the SwiGLU epilogue from 65 rows on: 32 weight rows a wavefront).
+// gemm_rows32.hip (more rows: 32 weight rows a wavefront).
 //
 // When the weight matrix gives too few workgroups the k dimension is cut over several of them (gridDim.y
 // "splits"); those write float32 partial sums [split][M][N] that the consumer adds in rising order (the next
@@ -43,7 +43,7 @@ __global__ void gemm_skinny_reduce_kernel(void* __restrict__ out, int out_f32, c
 
 #define SK_MAX_ROWS 256
 #define SK_MID_MAX_ROWS 128        // up to here the kernels of gemm_mid.hip, beyond gemm_rows32.hip
-#define SK_MID_MAX_ROWS_SWIGLU 64  // ... with the SwiGLU epilogue (measured: see gemm_rows32.hip)
+#define SK_MAX_ROWS_ACT 64         // ... with the epilogues that only products of few rows have
 
 extern "C" int zi_gemm_skinny_supported(int M, int N, int K, int64_t ldx, int64_t ldw) {
     return M >= 1 && M <= SK_MAX_ROWS && N >= 1 && K >= 8 && K % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0;
@@ -68,17 +68,17 @@ int64_t zi_gemm_mid_plan(int N, int K, int whole, int* splits, int* kb_per_split
 int zi_gemm_mid_launch(void* out, int out_f32, int mode, const zi_bf16* x, const zi_bf16* w, const zi_bf16* bias, int M,
                        int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int vec_out, float limit, hipStream_t stream);
 
-void zi_gemm_rows32_plan(int N, int K, int many_rows, int whole, int* splits, int* kb_per_split, int* waves);
+void zi_gemm_rows32_plan(int N, int K, int whole, int* splits, int* kb_per_split, int* waves);
 int zi_gemm_rows32_launch(void* out, int out_f32, int mode, const zi_bf16* x, const zi_bf16* w, const zi_bf16* bias, int M,
                           int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int vec_out, float limit, hipStream_t stream);
 
-static bool sk_rows32(int M, int mode) { return M > (mode >= SK_MODE_SWIGLU ? SK_MID_MAX_ROWS_SWIGLU : SK_MID_MAX_ROWS); }
+static bool sk_rows32(int M) { return M > SK_MID_MAX_ROWS; }
 
 // Splits of k for a weight matrix [N, K]: the leading dimension of the partial sums.  A function of N and K and
 // of which of the two kernels the rows go to (up to 128, or more).
 extern "C" int zi_gemm_skinny_splits(int M, int N, int K) {
     int s, per, waves;
-    if (sk_rows32(M, SK_MODE_PARTIAL)) zi_gemm_rows32_plan(N, K, M > 128, 0, &s, &per, &waves);
+    if (sk_rows32(M)) zi_gemm_rows32_plan(N, K, 0, &s, &per, &waves);
     else zi_gemm_mid_plan(N, K, 0, &s, &per, &waves);
     return s;
 }
@@ -93,7 +93,7 @@ extern "C" int64_t zi_gemm_skinny_workspace(int M, int N, int K) {
 // activation's launch after it: a launch is worth about as much as this many of the cut's wavefront-blocks.
 #define SK_LAUNCH_COST 32
 extern "C" int zi_gemm_skinny_act_pays(int M, int N, int K) {
-    if (M < 1 || M > SK_MID_MAX_ROWS_SWIGLU) return 0;
+    if (M < 1 || M > SK_MAX_ROWS_ACT) return 0;
     int s, per, waves;
     const int64_t whole = zi_gemm_mid_plan(N, K, 1, &s, &per, &waves);
     return whole <= zi_gemm_mid_plan(N, K, 0, &s, &per, &waves) + SK_LAUNCH_COST;
@@ -114,15 +114,15 @@ extern "C" int zi_gemm_skinny_act(void* out, int out_dt, int mode, const void* x
                "gemm_skinny: unsupported sizes M=%d N=%d K=%d (1 <= M <= 256, K and row strides multiples of 8)", M, N, K);
     ZI_REQUIRE(out_dt == ZI_F32 || out_dt == ZI_BF16, "gemm_skinny: unknown output dtype %d", out_dt);
     ZI_REQUIRE(mode >= 0 && mode <= SK_MODE_ACT + ZI_ACT_RELU2 && mode != SK_MODE_ACT + ZI_ACT_GELU_ERF, "gemm_skinny: unknown mode %d", mode);
-    ZI_REQUIRE(mode < SK_MODE_ACT || (M <= SK_MID_MAX_ROWS_SWIGLU && out_dt == ZI_BF16 && ldo >= N),
-               "gemm_skinny: an activation takes up to %d rows and a bfloat16 out of N columns", SK_MID_MAX_ROWS_SWIGLU);
-    ZI_REQUIRE(mode != SK_MODE_CLAMPED || (limit > 0.f && M <= SK_MID_MAX_ROWS_SWIGLU), "gemm_skinny: the clamped epilogue takes up to %d rows and a positive limit", SK_MID_MAX_ROWS_SWIGLU);
+    ZI_REQUIRE(mode < SK_MODE_ACT || (M <= SK_MAX_ROWS_ACT && out_dt == ZI_BF16 && ldo >= N),
+               "gemm_skinny: an activation takes up to %d rows and a bfloat16 out of N columns", SK_MAX_ROWS_ACT);
+    ZI_REQUIRE(mode != SK_MODE_CLAMPED || (limit > 0.f && M <= SK_MAX_ROWS_ACT), "gemm_skinny: the clamped epilogue takes up to %d rows and a positive limit", SK_MAX_ROWS_ACT);
     ZI_REQUIRE(ldx >= K && ldw >= K, "gemm_skinny: leading dimension too small");
     ZI_REQUIRE(((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0, "gemm_skinny: x and w must be 16-byte aligned");
     int splits, per, waves;
-    const bool rows32 = sk_rows32(M, mode);
-    if (rows32) zi_gemm_rows32_plan(N, K, M > 128, mode == SK_MODE_SWIGLU, &splits, &per, &waves);
-    else zi_gemm_mid_plan(N, K, mode >= SK_MODE_ACT, &splits, &per, &waves);
+    const bool rows32 = sk_rows32(M);
+    if (rows32) zi_gemm_rows32_plan(N, K, mode == SK_MODE_SWIGLU, &splits, &per, &waves);
+    else zi_gemm_mid_plan(N, K, mode >= SK_MODE_ACT || (mode == SK_MODE_SWIGLU && M > 64), &splits, &per, &waves);       // (whole from 65 rows on)
     void* dst = out;
     int kmode = mode;
     if (mode == SK_MODE_PLAIN) {

@@ -1159,18 +1159,15 @@ def reduce_sums(sums: torch.Tensor, bias: Optional[torch.Tensor] = None, out: Op
 SKINNY_MAX_ROWS = 64   # rows ``linear`` gives the few-rows kernels in one launch
 FEW_ROWS = 64          # up to here they beat the library product: the weights stream once, x stays on the chip
 # Products that leave partial sums (q/k/v, output, down: few weight rows, k cut over workgroups) go to the
-# few-rows kernel up to this many rows: measured at 128 rows with the weights coming from memory, 1.5B sizes,
-# 6.2 / 5.6 / 17.5 us against the library's 9.7 / 8.1 / 24.5; 7B sizes 20 / 16 / 55 against 20 / 16 / 92.  The
-# gate/up product with its activation does not (37 against 24 + 5 us at the 1.5B sizes: every wavefront reads
-# all of x from LDS for its 16 weight rows, and with 128 rows those reads bound it): FEW_ROWS stays its limit.
+# few-rows kernels up to this many rows: measured at 128 rows with the weights coming from memory, 1.5B sizes,
+# 7.2 / 6.9 / 13.5 us against the library's 9.7 / 8.1 / 24.5; 7B sizes 15 / 13 / 36 against 20 / 16 / 92.
 # Beyond 128 rows and up to 256 a kernel with 32 weight rows a wavefront (gemm_rows32.hip) takes the products whose
 # weights have at least twice as many columns as rows (the down projection; the library decides,
-# ``zi_gemm_skinny_pays``).  With the SwiGLU epilogue it loses to the library from 65 rows on (1.5B sizes at 128
-# rows 32.5 against 26.7 us with the activation's own launch: 560 wavefronts of 32 rows are too few for the
-# chip, and the epilogue forbids a cut of k): SWIGLU_MAX_ROWS stays at FEW_ROWS.
+# ``zi_gemm_skinny_pays``).  With the SwiGLU epilogue the limit is 128 rows: 25 us at 128 rows of the 1.5B sizes
+# against the library's 23 and the activation's launch of 5; beyond, the library's product.
 # (ZEDINFER_SUMS_MAX_ROWS=64 gives such products of more than 64 rows back to the library.)
 SUMS_MAX_ROWS = max(FEW_ROWS, min(256, int(os.environ.get("ZEDINFER_SUMS_MAX_ROWS", "256") or 256)))
-SWIGLU_MAX_ROWS = max(FEW_ROWS, min(256, int(os.environ.get("ZEDINFER_SWIGLU_MAX_ROWS", "64") or 64)))
+SWIGLU_MAX_ROWS = max(FEW_ROWS, min(256, int(os.environ.get("ZEDINFER_SWIGLU_MAX_ROWS", "128") or 128)))
 _WORKSPACES = {}
 _OUTGROWN_WORKSPACES: list = []
 
