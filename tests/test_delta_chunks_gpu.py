@@ -83,3 +83,31 @@ def test_a_decay_of_zero_and_values_that_are_not_finite():
     fine = torch.isfinite(plain)
     assert bool(fine[:60].all()) and bool(fine[:140, :3].all()) and not bool(fine[140:150, :2].any()) and bool(fine[150:].all())
     assert float((bad - got)[fine & torch.isfinite(bad)].abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("heads,kvh,dim,vdim", [(1, 1, 16, 4), (4, 2, 40, 64), (3, 3, 128, 68), (6, 2, 130, 128), (2, 1, 256, 100)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_a_step_of_single_tokens(heads, kvh, dim, vdim, dtype):
+    """Single tokens with the read-out's norm and gate in one launch against float64; entries of more tokens are left alone."""
+    from zedinfer_amd import ops
+    lens = [1] * 7
+    q, k, v, beta, gate, state = _inputs(lens, heads, kvh, dim, vdim, seed=dim)
+    want, left = _plain(lens, q, k, v, beta, gate, state)
+    w, z = torch.randn(vdim) + 1, torch.randn(7, heads * vdim + 8)
+    want = want / torch.sqrt((want * want).mean(-1, keepdim=True) + 1e-5) * w.double()
+    zz = z[:, 4:-4].double().view(7, heads, vdim)
+    want = (want * zz / (1 + torch.exp(-zz))).reshape(7, -1)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    qk, bg = torch.cat([q.reshape(7, -1), k.reshape(7, -1)], 1).cuda(), torch.stack([beta, gate], 1).cuda()
+    st, out = state.cuda(), torch.full((7, heads * vdim), 7.0, dtype=dtype, device="cuda")
+    assert ops.delta_rule_steps(dim, vdim, st) and not ops.delta_rule_steps(dim, 132, st) and not ops.delta_rule_steps(dim, 6, st)
+    lens_dev = i32([1, 1, 1, 0, 1, 1, 1])
+    ops.delta_rule_step(qk, v.reshape(7, -1).cuda(), bg, st, i32(list(range(7))), lens_dev, i32(list(range(7, 0, -1))), heads, kvh, dim, vdim,
+                        w.cuda(), z.cuda()[:, 4:-4], 1e-5, out=out)
+    rows = [0, 1, 2, 4, 5, 6]
+    # dot products of dim float32 terms, one after the other in 16 chains: a few 2^-24 of their sums; bfloat16 rounds once
+    tol = 2e-5 if dtype == torch.float32 else 2.0 ** -8
+    assert bool(((out.cpu().double() - want).abs()[rows] <= tol * want.abs()[rows] + 2e-5).all())
+    assert bool((out[3] == 7.0).all()) and torch.equal(st[4].cpu(), state[4]) and torch.equal(st[0].cpu(), state[0])
+    others = [1, 2, 3, 5, 6, 7]
+    assert float((st.cpu().double() - left)[others].abs().max()) < 5e-6

@@ -527,15 +527,17 @@ delta_channel_kernel(float* __restrict__ out, const float* __restrict__ qk, cons
 // once: a load instruction of a wavefront covers four rows x 64 columns (lane: row l / 16, columns 4 (l % 16) .. + 3),
 // all loads issued before the first is used.  S^T k and S^T q of the decayed state are summed over rows together, and the read-out of the updated
 // state is (S^T q) + (k . q) u.  Where a workgroup holds the whole head it can finish it: y = o / rms(o) * w *
-// sigmoid(gate), and o itself is then not written.
+// sigmoid(gate) (or SiLU), and o itself is then not written.  The rule with one decay a head (delta.hip) takes its decoded
+// tokens here too (g_channel 0): 32 requests of 12 heads of 128 x 128, 50 MB read and written, 47.7 us by delta_rule_kernel,
+// whose lanes read the state in pieces of 32 bytes, and 4.8 for the norm and gate; 14.2 us here with both, 3.5 TB/s.
 template <typename TY, int P, int CB>      // passes of 16 rows: dim <= 16 P
 __global__ void __launch_bounds__(256 * CB)
 delta_channel_step_kernel(TY* __restrict__ y, const float* __restrict__ norm, const float* __restrict__ gate, float eps,
                           float* __restrict__ out, const float* __restrict__ qk, const float* __restrict__ v,
-                          const float* __restrict__ beta, int64_t ld_beta, const float* __restrict__ g,
-                          float* __restrict__ state, int64_t state_stride, const int32_t* __restrict__ entry_start,
-                          const int32_t* __restrict__ entry_len, const int32_t* __restrict__ entry_slot, int heads, int kvh,
-                          int dim, int vdim) {
+                          const float* __restrict__ beta, int64_t ld_beta, const float* __restrict__ g, int64_t ld_g,
+                          int g_channel, int64_t ld_gate, int silu, float* __restrict__ state, int64_t state_stride,
+                          const int32_t* __restrict__ entry_start, const int32_t* __restrict__ entry_len,
+                          const int32_t* __restrict__ entry_slot, int heads, int kvh, int dim, int vdim) {
     __shared__ float ks[16 * P], qs[16 * P], gs[16 * P];
     __shared__ float4 pa[CB][4][16], pb[CB][4][16];
     __shared__ float red[16];
@@ -561,7 +563,7 @@ delta_channel_step_kernel(TY* __restrict__ y, const float* __restrict__ norm, co
         const float kk = in ? qk[t * qkc + (int64_t)(kvh + kh) * dim + d] : 0.f, qq = in ? qk[t * qkc + (int64_t)kh * dim + d] : 0.f;
         ks[d] = kk;
         qs[d] = qq;
-        gs[d] = in ? g[(t * heads + h) * dim + d] : 0.f;
+        gs[d] = in ? g[t * ld_g + (g_channel ? (int64_t)h * dim + d : h)] : 0.f;
         kq += kk * qq;
     }
     kq = zi_block_sum(kq, red);
@@ -602,11 +604,11 @@ delta_channel_step_kernel(TY* __restrict__ y, const float* __restrict__ norm, co
         const float ss = zi_block_sum(one ? o.x * o.x + o.y * o.y + o.z * o.z + o.w * o.w : 0.f, red);
         if (one) {
             const float rstd = 1.f / sqrtf(ss / (float)vdim + eps);
-            const float* gr = gate + (t * heads + h) * vdim + cc;
+            const float* gr = gate + t * ld_gate + (int64_t)h * vdim + cc;
             TY* dst = y + (t * heads + h) * vdim + cc;
             const float ov[4] = {o.x, o.y, o.z, o.w};
 #pragma unroll
-            for (int i = 0; i < 4; ++i) zi_store(dst + i, ov[i] * rstd * norm[cc + i] / (1.f + expf(-gr[i])));
+            for (int i = 0; i < 4; ++i) zi_store(dst + i, ov[i] * rstd * norm[cc + i] * (silu ? gr[i] : 1.f) / (1.f + expf(-gr[i])));
         }
     } else if (wave == 0 && rr == 0 && live) {
         *reinterpret_cast<float4*>(out + (t * heads + h) * vdim + cc) = o;
@@ -649,7 +651,7 @@ extern "C" int zi_delta_channel(float* out, const float* qk, const float* v, con
         ZI_REQUIRE(!y || (grid.x == 1 && norm && gate && eps > 0.f), "delta_channel: a head of %d values is not finished here", vdim);
 #define ZI_DCS2(P, CB)                                                                                                 \
     delta_channel_step_kernel<TY, P, CB><<<grid, 256 * CB, 0, stream>>>((TY*)y, norm, gate, eps, out, qk, v, beta, ld_beta, g, \
-        state, state_stride, entry_start, entry_len, entry_slot, heads, kvh, dim, vdim)
+        (int64_t)heads * dim, 1, (int64_t)heads * vdim, 0, state, state_stride, entry_start, entry_len, entry_slot, heads, kvh, dim, vdim)
 #define ZI_DCS(P)                  \
     do {                           \
         if (cb == 2) ZI_DCS2(P, 2); \
@@ -681,4 +683,41 @@ extern "C" int zi_delta_channel(float* out, const float* qk, const float* v, con
 #undef ZI_DC
 #undef ZI_DC2
     return zi_check_launch("delta_channel");
+}
+
+// Whether zi_delta_rule_step takes a state of this row stride and heads of these sizes.
+extern "C" int zi_delta_rule_steps(int dim, int vdim, int64_t state_stride) {
+    return dim > 0 && dim <= 256 && zi_delta_channel_finishes(vdim, state_stride);
+}
+
+// A step of entries of one token each under the rule with one decay a head (delta.hip): beta_g [n][2][heads], gate rows of stride
+// ld_gate, y [n][heads*vdim] (type y_dt) = o / rms(o) * norm [vdim] * SiLU(gate).
+extern "C" int zi_delta_rule_step(void* y, int y_dt, const float* qk, const float* v, const float* beta_g, float* state, int64_t state_stride,
+                                  const int32_t* entry_start, const int32_t* entry_len, const int32_t* entry_slot, int entries, int heads,
+                                  int kvh, int dim, int vdim, const float* norm, const float* gate, int64_t ld_gate, float eps,
+                                  hipStream_t stream) {
+    ZI_REQUIRE(entries >= 0 && entries <= 65535 && heads > 0 && heads <= 65535 && kvh > 0 && heads % kvh == 0 && eps > 0.f &&
+               ld_gate >= (int64_t)heads * vdim, "delta_rule_step: bad sizes");
+    ZI_REQUIRE(zi_delta_rule_steps(dim, vdim, state_stride), "delta_rule_step: a head of %d x %d is not taken", dim, vdim);
+    ZI_REQUIRE(state_stride >= (int64_t)heads * dim * vdim, "delta_rule_step: the state row is too short");
+    ZI_REQUIRE(((uintptr_t)state | (uintptr_t)v) % 16 == 0, "delta_rule_step: the state and v must be 16-byte aligned");
+    if (entries == 0) return 0;
+#define ZI_DRS2(P, CB)                                                                                                              \
+    delta_channel_step_kernel<TY, P, CB><<<dim3(1, heads, entries), 256 * CB, 0, stream>>>(                                          \
+        (TY*)y, norm, gate, eps, nullptr, qk, v, beta_g, 2 * (int64_t)heads, beta_g + heads, 2 * (int64_t)heads, 0, ld_gate, 1, state, \
+        state_stride, entry_start, entry_len, entry_slot, heads, kvh, dim, vdim)
+#define ZI_DRS(P)                       \
+    do {                                \
+        if (vdim > 64) ZI_DRS2(P, 2);   \
+        else ZI_DRS2(P, 1);             \
+    } while (0)
+    ZI_DISPATCH_DTYPE(y_dt, TY, {
+        if (dim <= 32) ZI_DRS(2);
+        else if (dim <= 64) ZI_DRS(4);
+        else if (dim <= 128) ZI_DRS(8);
+        else ZI_DRS(16);
+    });
+#undef ZI_DRS
+#undef ZI_DRS2
+    return zi_check_launch("delta_rule_step");
 }

@@ -184,6 +184,10 @@ int zi_delta_rule(float* out, const float* qk, const float* v, const float* beta
 int zi_delta_rule_chunked(float* out, const float* qk, const float* v, const float* beta_g, float* state, int64_t
     state_stride, const int32_t* entry_start, const int32_t* entry_len, const int32_t* entry_slot, int n, int entries, int
     heads, int kvh, int dim, int vdim, float* workspace, int64_t workspace_floats, hipStream_t stream);
+// delta_channel.hip
+int zi_delta_rule_step(void* y, int y_dt, const float* qk, const float* v, const float* beta_g, float* state, int64_t
+    state_stride, const int32_t* entry_start, const int32_t* entry_len, const int32_t* entry_slot, int entries, int heads, int
+    kvh, int dim, int vdim, const float* norm, const float* gate, int64_t ld_gate, float eps, hipStream_t stream);
 // delta.hip
 int zi_gated_rmsnorm(void* out, int out_dt, const float* o, const void* w, int w_dt, const float* gate, int64_t
     ld_gate, int n, int heads, int vdim, float eps, hipStream_t stream);
@@ -435,6 +439,7 @@ int zi_sample(int32_t* out, const float* logits, int64_t ld, float* work, int ro
     X(zi_delta_conv_state) \
     X(zi_delta_rule) \
     X(zi_delta_rule_chunked) \
+    X(zi_delta_rule_step) \
     X(zi_gated_rmsnorm) \
     X(zi_moe_route) \
     X(zi_moe_group) \

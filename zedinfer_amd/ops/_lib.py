@@ -86,6 +86,8 @@ _PROTOTYPES = {
     "zi_delta_prepare": [P, P, P, P, L, I, P, P, P, I, P, L, L, P, P, P, I, I, I, I, I, P],
     "zi_delta_conv_state": [P, L, L, P, L, P, P, P, I, I, I, P],
     "zi_delta_rule": [P, P, P, P, P, L, P, P, P, I, I, I, I, I, P],
+    "zi_delta_rule_step": [P, I, P, P, P, P, L, P, P, P, I, I, I, I, I, P, P, L, F, P],
+    "zi_delta_rule_steps": [I, I, L],
     "zi_delta_rule_chunked": [P, P, P, P, P, L, P, P, P, I, I, I, I, I, I, P, L, P],
     "zi_gated_rmsnorm": [P, I, P, P, I, P, L, I, I, I, F, P],
     "zi_moe_route": [P, P, P, P, I, I, I, F, P],

@@ -403,6 +403,39 @@ def delta_rule_workspace(n: int, entries: int, heads: int, dim: int, vdim: int) 
     return int(_lib.load().zi_delta_rule_workspace(int(n), int(entries), int(heads), int(dim), int(vdim)))
 
 
+def delta_rule_steps(dim: int, vdim: int, state: torch.Tensor) -> bool:
+    """Whether ``delta_rule_step`` takes heads of these sizes in rows of this state."""
+    return state.data_ptr() % 16 == 0 and bool(_lib.load().zi_delta_rule_steps(int(dim), int(vdim), int(state.stride(0))))
+
+
+def delta_rule_step(qk: torch.Tensor, v: torch.Tensor, beta_g: torch.Tensor, state: torch.Tensor, entry_start: torch.Tensor,
+                    entry_len: torch.Tensor, entry_slot: torch.Tensor, heads: int, kv_heads: int, dim: int, vdim: int,
+                    weight: torch.Tensor, gate: torch.Tensor, eps: float, out: torch.Tensor) -> torch.Tensor:
+    """``delta_rule`` and ``gated_rms_norm`` of its read-out in one launch, for steps in which every entry brings one token
+    (entries that do not are left alone): out [n, heads * vdim]."""
+    _gpu("delta_rule_step", qk, v, beta_g, state, entry_start, entry_len, entry_slot, weight, gate, out)
+    n = qk.shape[0]
+    _f32(qk, "delta_rule_step qk", (n, 2 * kv_heads * dim))
+    _f32(v, "delta_rule_step v", (n, heads * vdim))
+    _f32(beta_g, "delta_rule_step beta_g", (n, 2, heads))
+    _f32(state, "delta_rule_step state")
+    _f32(weight, "delta_rule_step weight", (vdim,))
+    ldg, gw = _rows(gate, "delta_rule_step gate")
+    if state.dim() != 2 or state.shape[1] < heads * dim * vdim:
+        raise ValueError("delta_rule_step: the state row is too short")
+    if gate.dtype != torch.float32 or gw != heads * vdim or gate.shape[0] != n:
+        raise ValueError("delta_rule_step: the gate must be float32 [n, heads * vdim]")
+    if tuple(out.shape) != (n, heads * vdim) or not out.is_contiguous():
+        raise ValueError("delta_rule_step: out must be contiguous [n, heads * vdim]")
+    E = entry_start.numel()
+    for t in (entry_start, entry_len, entry_slot):
+        _i32(t, "delta_rule_step entries", E)
+    _lib.call("zi_delta_rule_step", _p(out), _code(out, "delta_rule_step out"), _p(qk), _p(v), _p(beta_g), _p(state),
+              int(state.shape[1]), _p(entry_start), _p(entry_len), _p(entry_slot), E, heads, kv_heads, dim, vdim, _p(weight),
+              _p(gate), ldg, float(eps), _stream())
+    return out
+
+
 def gated_rms_norm(o: torch.Tensor, weight: torch.Tensor, gate: torch.Tensor, heads: int, vdim: int, eps: float,
                    out: torch.Tensor) -> torch.Tensor:
     """out [n, heads * vdim] = o / rms(o over each head's vdim values) * weight [vdim] * silu(gate), gate

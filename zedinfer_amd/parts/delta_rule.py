@@ -91,12 +91,16 @@ class GatedDeltaRule(Mixer):
                           batch.entry_slot, nh, kvh, dim, vdim, self.taps, qk, v, beta_g)
         ops.delta_conv_state(state, proj, batch.entry_start, batch.entry_len, batch.entry_slot, nh, kvh, dim, vdim,
                              self.taps)
-        o = rt.buffer("delta_read", (n, nh * vdim), torch.float32)
-        need = ops.delta_rule_workspace(n, batch.entry_start.numel(), nh, dim, vdim)
-        ops.delta_rule(qk, v, beta_g, state, batch.entry_start, batch.entry_len, batch.entry_slot, nh, kvh, dim, vdim, out=o,
-                       workspace=rt.buffer("delta_chunks", (need,), torch.float32) if need else None)
-        y = rt.buffer("delta_heads", (n, nh * vdim))
-        ops.gated_rms_norm(o, self.norm, proj[:, self.gate_at:self.gate_at + nh * vdim], nh, vdim, self.eps, out=y)
+        y, gate = rt.buffer("delta_heads", (n, nh * vdim)), proj[:, self.gate_at:self.gate_at + nh * vdim]
+        entries = (batch.entry_start, batch.entry_len, batch.entry_slot)
+        if batch.single_tokens and ops.delta_rule_steps(dim, vdim, state):
+            ops.delta_rule_step(qk, v, beta_g, state, *entries, nh, kvh, dim, vdim, self.norm, gate, self.eps, out=y)
+        else:
+            o = rt.buffer("delta_read", (n, nh * vdim), torch.float32)
+            need = ops.delta_rule_workspace(n, batch.entry_start.numel(), nh, dim, vdim)
+            ops.delta_rule(qk, v, beta_g, state, *entries, nh, kvh, dim, vdim, out=o,
+                           workspace=rt.buffer("delta_chunks", (need,), torch.float32) if need else None)
+            ops.gated_rms_norm(o, self.norm, gate, nh, vdim, self.eps, out=y)
         if out is None:
             out = rt.buffer("delta_out", (n, self.hidden))
         return ops.linear(y, self.o, out=out)
