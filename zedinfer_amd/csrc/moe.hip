@@ -251,7 +251,8 @@ __device__ __forceinline__ float moe_act(float z, int act) {
     return act == MOE_ACT_GELU_ERF ? 0.5f * z * (1.f + erff(z * 0.70710678118654752440f)) : z;
 }
 
-// The plain product: a workgroup of 256 threads makes 16 rows x 64 columns, k in blocks of 32 through LDS.
+// The plain product: a workgroup of 256 threads makes 16 rows (of a larger tile: the blockIdx.z-th) x 64 columns, k in blocks
+// of 32 through LDS.
 #define MOE_TM 16
 #define MOE_TN 64
 #define MOE_KC 32
@@ -265,7 +266,8 @@ moe_linear_kernel(TO* __restrict__ out, int64_t ldo, const TX* __restrict__ x, i
     __shared__ int src[MOE_TM];
     const int tile = blockIdx.y;
     if (tile >= plan[0]) return;
-    const int e = plan[1 + 3 * tile], r0 = plan[2 + 3 * tile], rows = plan[3 + 3 * tile];
+    const int e = plan[1 + 3 * tile], r0 = plan[2 + 3 * tile] + blockIdx.z * MOE_TM, rows = plan[3 + 3 * tile] - (int)blockIdx.z * MOE_TM;
+    if (rows <= 0) return;
     const int n0 = blockIdx.x * MOE_TN;
     if (threadIdx.x < MOE_TM) {
         const int r = r0 + (threadIdx.x < rows ? threadIdx.x : 0);
@@ -300,10 +302,17 @@ moe_linear_kernel(TO* __restrict__ out, int64_t ldo, const TX* __restrict__ x, i
     }
 }
 
-// The same on the matrix cores (bfloat16 operands, float32 sums): a wavefront makes 16 columns of RT tiles of 16
-// rows; the expert's weight rows are the first operand (lane: row l % 16, eight k from 8 (l / 16)), the tokens'
-// rows the second, so a lane ends with four neighbouring columns of one row.  Operands come straight from memory:
-// the weights are read once per tile of rows.
+// The same on the matrix cores (bfloat16 operands, float32 sums): a workgroup of four wavefronts makes a tile of RT x 16 rows
+// and 64 CT columns, a wavefront all of the rows and 16 CT of the columns; the expert's weight rows are the first operand (lane:
+// row l % 16, eight k from 8 (l / 16)), the tokens' rows the second, so a lane ends with four neighbouring columns of one row.
+// Both operands go straight into LDS in whole lines of 128 bytes (1 KB an instruction; piece c of row q at place c xor (q / 2
+// mod 8), so that a wavefront's reads meet no bank twice), k in steps of 64 through a ring of ST buffers; every wavefront
+// issues as many loads a step as every other, so that each can wait for its own by count before the step's one barrier.
+// Workgroups are dealt out so that an XCD takes neighbouring tiles: an expert's weights are then fetched into one L2.
+// What it replaced read the operands' fragments from memory, 16 rows x 64 bytes an instruction, a quarter of the rate of whole
+// lines.  Measured with 32 experts of 1536 x 1536 (151 MB of weights), the first product and the second: 8,000 pairs 203 and
+// 195 to 98 and 87 us (two buffers, so that a unit holds two workgroups: with four buffers and one workgroup 141 and 115), 128
+// pairs 41 and 40 to 24.8 and 24.6 us (6.1 TB/s; with four buffers 26.5 and 25.3).
 typedef __attribute__((ext_vector_type(8))) __bf16 moe_bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float moe_f32x4_t;
 typedef __attribute__((ext_vector_type(4))) unsigned moe_u32x4_t;
@@ -312,51 +321,141 @@ union moe_pack {
     moe_bf16x8_t b;
 };
 
-template <typename TO, int RT, int CT>      // a wavefront makes RT tiles of 16 rows x CT tiles of 16 columns
-__global__ void __launch_bounds__(256)
+#define MOE_KB 64
+#define MOE_XCDS 8
+// the longest row of weights whose tile of rows a buffer's 31-bit offsets reach
+#define MOE_MAX_K (1 << 21)
+
+// the wavefront's loads but for the newest `n` have arrived (n counts loads; LDS and scalar counters are not waited for)
+template <int n>
+__device__ __forceinline__ void moe_wait() {
+    static_assert(n < 64, "the counter has six bits");
+    __builtin_amdgcn_s_waitcnt((n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14));
+}
+
+// 16 bytes a lane into LDS, lane after lane from `to` on: from an address, or from a buffer (zeros past its end).
+__device__ __forceinline__ void moe_to_lds(const zi_bf16* from, moe_u32x4_t* to) {
+#ifdef __HIP_DEVICE_COMPILE__       // (the host's pass knows loads of this size for no target)
+    __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
+#endif
+}
+template <int AUX>
+__device__ __forceinline__ void moe_to_lds(__amdgpu_buffer_rsrc_t from, moe_u32x4_t* to, int lane_at, int at) {
+#ifdef __HIP_DEVICE_COMPILE__
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, to, 16, lane_at, at, 0, AUX);
+#endif
+}
+
+template <typename TO, int RT, int CT, int ST>
+__global__ void __launch_bounds__(4 * ZI_WAVE)
 moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restrict__ x, int64_t ldx,
                        const zi_bf16* __restrict__ w, const int32_t* __restrict__ plan,
                        const int32_t* __restrict__ source, int source_div, int N, int K, int act) {
-    const int tile = blockIdx.y;
-    if (tile >= plan[0]) return;
+    constexpr int XI = 2 * RT, WI = 8 * CT, XW = (XI + 3) / 4, WW = WI / 4, PW = XW + WW;      // loads of a step; a wavefront's share
+    constexpr int PIECES = (4 * XW + WI) * ZI_WAVE;
+    // (arrays of their own, so that the compiler can tell a buffer that is read from those that loads are on their way to)
+    __shared__ __attribute__((aligned(16))) moe_u32x4_t s0[PIECES], s1[PIECES], s2[ST > 2 ? PIECES : 1], s3[ST > 3 ? PIECES : 1];
+    const int blocks = (N + 64 * CT - 1) / (64 * CT), total = plan[0] * blocks, share = (total + MOE_XCDS - 1) / MOE_XCDS;
+    const int at_share = blockIdx.x / MOE_XCDS, job = (int)(blockIdx.x % MOE_XCDS) * share + at_share;
+    if (at_share >= share || job >= total) return;
+    const int tile = job / blocks, n0 = job % blocks * 64 * CT;
     const int e = plan[1 + 3 * tile], r0 = plan[2 + 3 * tile], rows = plan[3 + 3 * tile];
-    const int lane = threadIdx.x % ZI_WAVE, wave = threadIdx.x / ZI_WAVE;
-    const int r = lane % 16, j = lane / 16;
-    const int n0 = (blockIdx.x * 4 + wave) * 16 * CT;
-    if (n0 >= N) return;
-    const zi_bf16* wrow[CT];
+    const int lane = threadIdx.x % ZI_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / ZI_WAVE);
+    const int r = lane & 15, j = lane >> 4;
+    // Load i takes 8 rows: lane l row l / 8 of them, the piece that belongs at place l % 8.  (Rows of the tokens past the
+    // tile's are its first row again, not stored; weight rows past N are past the buffer's end.)
+    const int rows_w = N - n0 < 64 * CT ? N - n0 : 64 * CT;
+    const __amdgpu_buffer_rsrc_t wb = __builtin_amdgcn_make_buffer_rsrc(const_cast<zi_bf16*>(w + ((int64_t)e * N + n0) * K), 0,
+                                                                        rows_w * K * 2, 0x00020000);
+    const zi_bf16* xrow[XW];
+    int xpiece[XW], w_at[WW], wpiece[WW];
 #pragma unroll
-    for (int c = 0; c < CT; ++c) {
-        const int wn = n0 + 16 * c + r < N ? n0 + 16 * c + r : N - 1;
-        wrow[c] = w + ((int64_t)e * N + wn) * K;
+    for (int i = 0; i < XW; ++i) {
+        const int q = (i * 4 + wave) * 8 + lane / 8, rr = q < rows ? q : 0;
+        xrow[i] = x + (int64_t)(source ? source[r0 + rr] / source_div : r0 + rr) * ldx;
+        xpiece[i] = ((lane & 7) ^ ((q >> 1) & 7)) * 8;
     }
-    const zi_bf16* xrow[RT];
 #pragma unroll
-    for (int t = 0; t < RT; ++t) {
-        const int rr = t * 16 + r < rows ? t * 16 + r : 0;
-        xrow[t] = x + (int64_t)(source ? source[r0 + rr] / source_div : r0 + rr) * ldx;
+    for (int i = 0; i < WW; ++i) {
+        const int q = (i * 4 + wave) * 8 + lane / 8;
+        wpiece[i] = ((lane & 7) ^ ((q >> 1) & 7)) * 8;
+        w_at[i] = (q < rows_w ? q * K + wpiece[i] : rows_w * K) * 2;
     }
+    const int steps = (K + MOE_KB - 1) / MOE_KB;
+    // (columns past K, a multiple of 8: the tokens' are the row's first again, the weights' the next row's or zeros; both masked)
+    auto issue = [&](moe_u32x4_t* buf, int t) {
+        const int k0 = t * MOE_KB;
+        const bool whole = k0 + MOE_KB <= K;
+#pragma unroll
+        for (int i = 0; i < XW; ++i)
+            moe_to_lds(xrow[i] + (whole || k0 + xpiece[i] < K ? k0 + xpiece[i] : 0), buf + (i * 4 + wave) * ZI_WAVE);
+#pragma unroll
+        for (int i = 0; i < WW; ++i)
+            moe_to_lds<RT == 1 ? 2 : 0>(wb, buf + (4 * XW + i * 4 + wave) * ZI_WAVE,
+                                        whole || k0 + wpiece[i] < K ? w_at[i] + k0 * 2 : rows_w * K * 2, 0);
+    };
     moe_f32x4_t acc[RT][CT];
 #pragma unroll
     for (int t = 0; t < RT; ++t)
 #pragma unroll
         for (int c = 0; c < CT; ++c) acc[t][c] = (moe_f32x4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-    for (int k0 = 0; k0 < K; k0 += 32) {
-        const int k = k0 + 8 * j;
-        const bool in = k < K;      // K is a multiple of 8: a piece of eight lies inside or outside
-        const int kc = in ? k : 0;
-        const unsigned mask = 0u - (unsigned)in;
-        moe_pack a[CT], b[RT];
+    const int sw = (r >> 1) & 7;
+    auto step = [&](const moe_u32x4_t* buf, moe_u32x4_t* free, int t) __attribute__((always_inline)) {
+        if (t >= steps) return;
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        const int after = steps - 1 - t;       // steps whose loads may still be on their way
+        if (after >= ST - 2) moe_wait<(ST - 2) * PW>();
+        else if (ST > 3 && after == 1) moe_wait<PW>();
+        else moe_wait<0>();
+        __builtin_amdgcn_s_barrier();          // all wavefronts' loads of the step are there, and all are done with `free`
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        if (t + ST - 1 < steps) issue(free, t + ST - 1);
+        __builtin_amdgcn_sched_barrier(0);
+        const int left = K - t * MOE_KB;
 #pragma unroll
-        for (int c = 0; c < CT; ++c) a[c].u = *reinterpret_cast<const moe_u32x4_t*>(wrow[c] + kc) & mask;
+        for (int kk = 0; kk < 2; ++kk) {
+            const int at = (kk * 4 + j) ^ sw;
+            moe_pack a[CT], b[RT];
 #pragma unroll
-        for (int t = 0; t < RT; ++t) b[t].u = *reinterpret_cast<const moe_u32x4_t*>(xrow[t] + kc) & mask;
+            for (int c = 0; c < CT; ++c) a[c].u = buf[(4 * XW * 8 + (wave * CT + c) * 16 + r) * 8 + at];
 #pragma unroll
-        for (int t = 0; t < RT; ++t)
+            for (int m = 0; m < RT; ++m) b[m].u = buf[(m * 16 + r) * 8 + at];
+            if (left < MOE_KB) {
+                const unsigned mask = 0u - (unsigned)(kk * 32 + j * 8 < left);
 #pragma unroll
-            for (int c = 0; c < CT; ++c)
-                acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[c].b, b[t].b, acc[t][c], 0, 0, 0);
+                for (int c = 0; c < CT; ++c) a[c].u &= mask;
+#pragma unroll
+                for (int m = 0; m < RT; ++m) b[m].u &= mask;
+            }
+#pragma unroll
+            for (int m = 0; m < RT; ++m)
+#pragma unroll
+                for (int c = 0; c < CT; ++c)
+                    acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[c].b, b[m].b, acc[m][c], 0, 0, 0);
+        }
+    };
+    issue(s0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (ST > 2) if (steps > 1) issue(s1, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (ST > 3) if (steps > 2) issue(s2, 2);
+    __builtin_amdgcn_sched_barrier(0);
+    for (int t = 0; t < steps; t += ST) {
+        if constexpr (ST == 2) {
+            step(s0, s1, t);
+            step(s1, s0, t + 1);
+        } else if constexpr (ST == 3) {
+            step(s0, s2, t);
+            step(s1, s0, t + 1);
+            step(s2, s1, t + 2);
+        } else {
+            step(s0, s3, t);
+            step(s1, s0, t + 1);
+            step(s2, s1, t + 2);
+            step(s3, s2, t + 3);
+        }
     }
     // a lane holds four consecutive columns of a row: one store of 16 (float32) or 8 bytes (bfloat16) where the rows
     // allow it
@@ -367,7 +466,7 @@ moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restr
         if (row >= rows) continue;
 #pragma unroll
         for (int c = 0; c < CT; ++c) {
-            const int n = n0 + 16 * c + 4 * j;
+            const int n = n0 + (wave * CT + c) * 16 + 4 * j;
             TO* dst = out + (int64_t)(r0 + row) * ldo + n;
             if (whole && n + 3 < N) {
                 moe_store4(dst, moe_act(acc[t][c][0], act), moe_act(acc[t][c][1], act), moe_act(acc[t][c][2], act),
@@ -388,24 +487,25 @@ extern "C" int zi_moe_linear(void* out, int out_dt, int64_t ldo, const void* x, 
                "moe_linear: bad sizes");
     ZI_REQUIRE(act == MOE_ACT_NONE || act == MOE_ACT_GELU_ERF, "moe_linear: unknown activation %d", act);
     if (max_tiles == 0) return 0;
-    const dim3 grid((N + MOE_TN - 1) / MOE_TN, max_tiles);
+    const dim3 grid((N + MOE_TN - 1) / MOE_TN, max_tiles, (tile_rows + MOE_TM - 1) / MOE_TM);
     const bool cores = x_dt == ZI_BF16 && w_dt == ZI_BF16 && K % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)x % 16) == 0 &&
                        ((uintptr_t)w % 16) == 0 && (tile_rows == 16 || tile_rows == 32 || tile_rows == 64);
-    // tiles of 64 rows (many rows an expert: prompts): a wavefront makes 64 columns of them, so that an operand of
-    // the tokens serves four of the weights'; smaller tiles (decoded tokens) are bound by the weights' stream
-#define ZI_MOE_CORES(RT, CT)                                                                                       \
-    moe_linear_mfma_kernel<TO, RT, CT><<<dim3((N + 64 * CT - 1) / (64 * CT), max_tiles), 256, 0, stream>>>(         \
-        (TO*)out, ldo, (const zi_bf16*)x, ldx, (const zi_bf16*)w, plan, source, source_div, N, K, act)
-    if (cores) {
+    // tiles of 64 rows (many rows an expert: prompts) are 256 columns wide, for a workgroup's reads of LDS: 8 operands for 16
+    // products; smaller ones (decoded tokens) are bound by the weights' stream: narrow, so that every unit has several workgroups
+    if (cores && K <= MOE_MAX_K) {
+#define ZI_MOE_CORES(RT, CT, ST)                                                                                                   \
+    moe_linear_mfma_kernel<TO, RT, CT, ST><<<dim3((((N + 64 * CT - 1) / (64 * CT)) * (int64_t)max_tiles + MOE_XCDS - 1) / MOE_XCDS * \
+                                             MOE_XCDS), 256, 0, stream>>>((TO*)out, ldo, (const zi_bf16*)x, ldx,                      \
+                                                                          (const zi_bf16*)w, plan, source, source_div, N, K, act)
         ZI_DISPATCH_DTYPE(out_dt, TO, {
-            if (tile_rows == 16) ZI_MOE_CORES(1, 1);
-            else if (tile_rows == 32) ZI_MOE_CORES(2, 2);
-            else ZI_MOE_CORES(4, 4);
+            if (tile_rows == 16) ZI_MOE_CORES(1, 1, 3);
+            else if (tile_rows == 32) ZI_MOE_CORES(2, 2, 3);
+            else ZI_MOE_CORES(4, 4, 2);
         });
         return zi_check_launch("moe_linear");
     }
 #undef ZI_MOE_CORES
-    ZI_REQUIRE(tile_rows == MOE_TM, "moe_linear: the plain product walks tiles of %d rows, not %d", MOE_TM, tile_rows);
+    ZI_REQUIRE(cores || tile_rows == MOE_TM, "moe_linear: the plain product walks tiles of %d rows, not %d", MOE_TM, tile_rows);
     ZI_DISPATCH_DTYPE(x_dt, TX, ZI_DISPATCH_DTYPE(w_dt, TW, ZI_DISPATCH_DTYPE(out_dt, TO, {
         moe_linear_kernel<TX, TW, TO><<<grid, 256, 0, stream>>>((TO*)out, ldo, (const TX*)x, ldx, (const TW*)w, plan,
                                                                  source, source_div, N, K, act);
