@@ -111,3 +111,39 @@ def test_a_step_of_single_tokens(heads, kvh, dim, vdim, dtype):
     assert bool((out[3] == 7.0).all()) and torch.equal(st[4].cpu(), state[4]) and torch.equal(st[0].cpu(), state[0])
     others = [1, 2, 3, 5, 6, 7]
     assert float((st.cpu().double() - left)[others].abs().max()) < 5e-6
+
+
+@pytest.mark.parametrize("heads,kvh,dim,vdim", [(2, 1, 4, 6), (4, 2, 64, 20), (3, 3, 128, 128), (2, 1, 256, 258), (2, 2, 8, 1024)])
+@pytest.mark.parametrize("lens", [[1], [3, 1, 2], [1] * 5 + [1018, 4, 7], [2050]])
+def test_preparing_four_channels_a_thread(heads, kvh, dim, vdim, lens):
+    """Convolution over the kept tail, SiLU and unit vectors against float64, with runs of tokens that cross entries; few
+    tokens and enough for four a thread."""
+    from zedinfer_amd import ops
+    g = torch.Generator().manual_seed(dim + len(lens))
+    n, E, C = sum(lens), len(lens), 2 * kvh * dim + heads * vdim
+    width, off = C + heads * vdim + 2 * heads, heads * dim * vdim
+    proj = torch.randn(n, width + (-width) % 4, generator=g)
+    conv, a_log, dt = torch.randn(C, 4, generator=g), torch.randn(heads, generator=g), torch.randn(heads, generator=g)
+    state = torch.randn(E + 1, ops.delta_state_floats(heads, dim, vdim, kvh, 4), generator=g)
+    starts = [sum(lens[:e]) for e in range(E)]
+    slots = list(range(E, 0, -1))
+    x = torch.empty(n, C, dtype=torch.float64)
+    for s, length, slot in zip(starts, lens, slots):
+        rows = torch.cat([state[slot, off:off + 3 * C].view(3, C), proj[s:s + length, :C]]).double()
+        y = sum(rows[j:j + length] * conv[:, j].double() for j in range(4))
+        x[s:s + length] = y / (1 + torch.exp(-y))
+    unit = x[:, :2 * kvh * dim].view(n, 2, kvh, dim)
+    unit = unit / torch.sqrt((unit * unit).sum(-1, keepdim=True) + 1e-6)
+    unit[:, 0] *= dim ** -0.5
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device="cuda")  # noqa: E731
+    qk, v, bg = (torch.full(s, 7.0, device="cuda") for s in ((n, 2 * kvh * dim), (n, heads * vdim), (n, 2, heads)))
+    seq = i32([e for e, length in enumerate(lens) for _ in range(length)])
+    ops.delta_prepare(proj.cuda()[:, :width], conv.cuda(), a_log.cuda(), dt.cuda(), state.cuda(), seq, i32(starts), i32(slots), heads, kvh,
+                      dim, vdim, 4, qk, v, bg)
+    # four products and their sum, an exponential and a quotient: some ten roundings of values of a few units; near-zero heads lose more
+    assert float((v.cpu().double() - x[:, 2 * kvh * dim:]).abs().max()) < 1e-5
+    assert float((qk.cpu().double().view_as(unit) - unit).abs().max()) < 1e-4
+    b, a = proj[:, width - 2 * heads:width - heads].double(), proj[:, width - heads:width].double()
+    assert float((bg[:, 0].cpu().double() - torch.sigmoid(b)).abs().max()) < 1e-6
+    decay = torch.exp(-torch.exp(a_log.double()) * torch.nn.functional.softplus(a + dt.double()))
+    assert float((bg[:, 1].cpu().double() - decay).abs().max()) < 1e-5
