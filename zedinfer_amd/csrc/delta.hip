@@ -9,7 +9,8 @@
 //
 // Everything here is float32 arithmetic.  Three launches a step: `zi_delta_prepare` (convolution, SiLU, unit
 // vectors, beta, g, for every token at once), `zi_delta_conv_state` (the new tail of the convolution's input),
-// `zi_delta_rule` (the recurrence, token by token within an entry, entries and heads and columns in parallel).
+// `zi_delta_rule` (the recurrence, token by token within an entry, entries and heads and columns in parallel; long
+// portions in chunks: delta_chunks.hip; steps of single tokens: delta_channel.hip).
 #include "zi_common.h"
 #include "zi_api.h"
 
