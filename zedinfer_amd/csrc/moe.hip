@@ -492,7 +492,10 @@ extern "C" int zi_moe_linear(void* out, int out_dt, int64_t ldo, const void* x, 
                        ((uintptr_t)w % 16) == 0 && (tile_rows == 16 || tile_rows == 32 || tile_rows == 64);
     // tiles of 64 rows (many rows an expert: prompts) are 256 columns wide, for a workgroup's reads of LDS: 8 operands for 16
     // products; smaller ones (decoded tokens) are bound by the weights' stream: narrow, so that every unit has several workgroups
-    if (cores && K <= MOE_MAX_K) {
+    // (and what neither a buffer's offsets nor a grid of one dimension, 2^32 threads, reaches is left to the plain kernel)
+    const int wide = cores ? 64 * (tile_rows / 16) : 64;       // columns of a workgroup
+    const int64_t most = ((int64_t)N + wide - 1) / wide * max_tiles + MOE_XCDS;
+    if (cores && K <= MOE_MAX_K && most * 256 < (1LL << 32)) {
 #define ZI_MOE_CORES(RT, CT, ST)                                                                                                   \
     moe_linear_mfma_kernel<TO, RT, CT, ST><<<dim3((((N + 64 * CT - 1) / (64 * CT)) * (int64_t)max_tiles + MOE_XCDS - 1) / MOE_XCDS * \
                                              MOE_XCDS), 256, 0, stream>>>((TO*)out, ldo, (const zi_bf16*)x, ldx,                      \
