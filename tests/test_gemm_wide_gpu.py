@@ -1,0 +1,47 @@
+"""The products of 65 to 128 rows (csrc/gemm_mid.hip, both operands by buffer loads straight into LDS) where their addressing can
+go wrong: rows that lie apart, columns past K, weight rows past a workgroup's, the last row at the end of its memory."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _inside(rows, cols, ld, at, g):
+    """[rows, cols] bfloat16 of row stride ld in memory that holds NaN wherever it does not lie, and ends with its last value."""
+    store = torch.full((at + (rows - 1) * ld + cols,), float("nan"), dtype=torch.bfloat16, device="cuda")
+    t = store.as_strided((rows, cols), (ld, 1), at)
+    t.copy_(torch.randn(rows, cols, generator=g, device="cuda"))
+    return t
+
+
+def _check(ops, x, w, monkeypatch):
+    from zedinfer_amd.ops import functional
+    from zedinfer_amd.parts.feed_forward import GATE_UP_BLOCK
+    monkeypatch.setattr(functional, "SWIGLU_MAX_ROWS", 128)
+    M, K, N = x.shape[0], x.shape[1], w.shape[0]
+    sums = ops.linear_sums(x, w)
+    ref, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    # exact products, at most K + 16 roundings of running sums that are at most `size`
+    bound = (K + 16) * 2.0 ** -24 * size
+    assert bool(((sums.double().sum(0) - ref).abs() <= bound).all())
+    # the kernel for up to 64 rows: the same sums in the same order
+    for rows in (slice(0, 64), slice(M - 33, M)):
+        assert torch.equal(ops.linear_sums(x[rows], w), sums[:, rows])
+    if N % 16 == 0:
+        wide = torch.full((M, N // 2 + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+        ops.linear_swiglu(x, w, out=wide[:, :N // 2])
+        gu = ref.view(M, -1, 2, GATE_UP_BLOCK)
+        want = (gu[:, :, 1] * torch.nn.functional.silu(gu[:, :, 0])).reshape(M, N // 2)
+        # gate and up each off by `bound`, and one rounding to bfloat16 (silu's slope is below 1.1)
+        off = bound.view(M, -1, 2, GATE_UP_BLOCK)
+        slack = 1.1 * off[:, :, 0] * gu[:, :, 1].abs() + off[:, :, 1] * gu[:, :, 0].abs()
+        assert bool(((wide[:, :N // 2].double() - want).abs() <= 2.0 ** -8 * want.abs() + 2 * slack.reshape(M, -1) + 1e-30).all())
+        assert bool((wide[:, N // 2:] == 7.0).all())
+
+
+@pytest.mark.parametrize("M", [65, 80, 97, 128])
+@pytest.mark.parametrize("N,K,padx,padw", [(1, 8, 0, 0), (16, 72, 8, 16), (130, 200, 24, 8), (304, 1000, 0, 40), (1024, 1544, 56, 0), (7, 4096, 8, 8)])
+def test_rows_that_lie_apart(M, N, K, padx, padw, monkeypatch):
+    from zedinfer_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(M * N + K)
+    _check(ops, _inside(M, K, K + padx, padx // 8 * 8, g), _inside(N, K, K + padw, padw // 8 * 8, g), monkeypatch)

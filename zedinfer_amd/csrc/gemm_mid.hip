@@ -294,10 +294,16 @@ __device__ __forceinline__ void gw_wait() {
 
 // 16 bytes a lane from a buffer into LDS, lane after lane from `to` on; what lies past the buffer's end gives zeros.
 template <int AUX>
-__device__ __forceinline__ void gw_to_lds(__amdgpu_buffer_rsrc_t from, gm_u32x4_t* to, int lane_at, int at) {
+__device__ __forceinline__ void gw_to_lds(__amdgpu_buffer_rsrc_t from, gm_u32x4_t* to, int lane_at) {
 #ifdef __HIP_DEVICE_COMPILE__       // (the host's pass knows loads of this size for no target)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, to, 16, lane_at, at, 0, AUX);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, to, 16, lane_at, 0, 0, AUX);
 #endif
+}
+
+// Column k (a multiple of 8) and all that follows of `rows` rows as a buffer: it ends with the last row's K values, and past
+// the last column it holds nothing.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t gw_rows(const zi_bf16* base, int64_t ld, int rows, int K, int k) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<zi_bf16*>(base + k), 0, k < K ? (int)(((rows - 1) * ld + K - k) * 2) : 0, 0x00020000);
 }
 
 template <int MT, int NT>
@@ -315,13 +321,13 @@ gemm_wide_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* _
     const int k_lo = split * kb_per_split * GM_KB, k_hi = k_lo + kb_per_split * GM_KB < K ? k_lo + kb_per_split * GM_KB : K;
     const int steps = (k_hi - k_lo + GW_KB - 1) / GW_KB;
     const int n0 = blockIdx.x * NT * 16;
-    // Load i of a step takes 8 rows: lane l row l / 8 of them, the piece that belongs at place l % 8.  A step's place along k is the
-    // same for all lanes and loads, so that a load costs no arithmetic (with one wavefront a SIMD every instruction counts).
+    // Load i of a step takes 8 rows: lane l row l / 8 of them, the piece that belongs at place l % 8.  A step's place along k is in
+    // the buffers it loads from (scalar registers), so that a load costs no arithmetic of the lanes (with one wavefront a SIMD every
+    // instruction counts) and every address is checked by the lane's offset alone, the one part of an address that the buffer's
+    // range is sure to be held against.
     // Rows past M or N are past the buffers' ends and zero; columns past K are the next row's, and masked when they are used.
     const int rows_w = N - n0 < NT * 16 ? N - n0 : NT * 16;
-    const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc(const_cast<zi_bf16*>(x), 0, (int)(((M - 1) * ldx + K) * 2), 0x00020000);
-    const __amdgpu_buffer_rsrc_t wb = __builtin_amdgcn_make_buffer_rsrc(const_cast<zi_bf16*>(w + (int64_t)n0 * ldw), 0,
-                                                                        (int)(((rows_w - 1) * ldw + K) * 2), 0x00020000);
+    const zi_bf16* const w0 = w + (int64_t)n0 * ldw;
     int lane_at[PW];
 #pragma unroll
     for (int i = 0; i < PW; ++i) {
@@ -330,14 +336,15 @@ gemm_wide_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* _
         lane_at[i] = (int)(q * (L < XI ? ldx : ldw) * 2) + ((lane & 7) ^ ((q >> 1) & 7)) * 16;
     }
     auto issue = [&](gm_u32x4_t* buf, int t) {
-        const int at = t < steps ? (k_lo + t * GW_KB) * 2 : 0x7fffffff;       // (steps past the end: past the buffers' ends, nothing is fetched)
+        const int k = t < steps ? k_lo + t * GW_KB : K;       // (steps past the end: nothing is fetched)
+        const __amdgpu_buffer_rsrc_t xb = gw_rows(x, ldx, M, K, k), wb = gw_rows(w0, ldw, rows_w, K, k);
 #pragma unroll
         for (int i = 0; i < PW; ++i) {
             const int L = i * 4 + wave;
             gm_u32x4_t* to = L < LOADS ? buf + L * ZI_WAVE : spare;
-            if (i * 4 + 3 < XI) gw_to_lds<0>(xb, to, lane_at[i], at);
-            else if (i * 4 >= XI) gw_to_lds<2>(wb, to, lane_at[i], at);       // weights are read once: past L2
-            else gw_to_lds<0>(L < XI ? xb : wb, to, lane_at[i], at);
+            if (i * 4 + 3 < XI) gw_to_lds<0>(xb, to, lane_at[i]);
+            else if (i * 4 >= XI) gw_to_lds<2>(wb, to, lane_at[i]);       // weights are read once: past L2
+            else gw_to_lds<0>(L < XI ? xb : wb, to, lane_at[i]);
         }
     };
     gm_f32x4_t acc[NT][2];
