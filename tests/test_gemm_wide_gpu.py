@@ -45,3 +45,12 @@ def test_rows_that_lie_apart(M, N, K, padx, padw, monkeypatch):
     from zedinfer_amd import ops
     g = torch.Generator(device="cuda").manual_seed(M * N + K)
     _check(ops, _inside(M, K, K + padx, padx // 8 * 8, g), _inside(N, K, K + padw, padw // 8 * 8, g), monkeypatch)
+
+
+@pytest.mark.parametrize("ldx,ldw", [(1 << 22, 1 << 22), ((1 << 22) + 8, 264), (264, (1 << 22) + 8), ((1 << 24) + (1 << 23), 1 << 24)])
+def test_rows_further_apart_than_offsets_of_31_bits_reach(ldx, ldw, monkeypatch):
+    """128 rows of 2^23 elements and more are 2^31 bytes apart and more: the kernel with addresses of 64 bits takes them."""
+    from zedinfer_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(ldx % 1000 + ldw % 1000)
+    for M, N, K in ((128, 80, 264), (77, 16, 72)):
+        _check(ops, _inside(M, K, ldx, 0, g), _inside(N, K, ldw, 0, g), monkeypatch)

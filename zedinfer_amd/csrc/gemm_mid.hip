@@ -132,7 +132,8 @@ __device__ __forceinline__ void gm_epilogue(const gm_f32x4_t (&acc)[MT], void* _
     }
 }
 
-template <int MT, int GM_RING, int GM_WAVES>
+// APART: rows blockIdx.z * 16 MT .. of x.
+template <int MT, int GM_RING, int GM_WAVES, bool APART = false>
 __global__ void __launch_bounds__(GM_WAVES* ZI_WAVE)
 gemm_mid_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* __restrict__ x,
                 const zi_bf16* __restrict__ w, const zi_bf16* __restrict__ bias, int M, int N, int K, int64_t ldx,
@@ -145,7 +146,7 @@ gemm_mid_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* __
     const int kb_total = (K + GM_KB - 1) / GM_KB;
     const int kb_lo = split * kb_per_split;
     const int kb_hi = (kb_lo + kb_per_split < kb_total) ? kb_lo + kb_per_split : kb_total;
-    const int n0 = (blockIdx.x * GM_WAVES + wave) * 16;
+    const int n0 = (blockIdx.x * GM_WAVES + wave) * 16, m0 = APART ? blockIdx.z * MT * 16 : 0;
     // Weights are read as whole cache lines: a load instruction takes 4 rows x 256 bytes (lane l: row
     // l / 16 of the four, 16-byte piece l % 16), four instructions a tile of 16 rows x 128 values.
     // Loads in the matrix-core operand layout (16 rows x 64 bytes an instruction) were measured a fifth
@@ -179,7 +180,7 @@ gemm_mid_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* __
     // comes from the cache and is wanted a step earlier, must not queue behind weights from memory.
     const zi_bf16* xrow[XP];
 #pragma unroll
-    for (int p = 0; p < XP; ++p) xrow[p] = x + (int64_t)(srow[p] < M ? srow[p] : M - 1) * ldx;
+    for (int p = 0; p < XP; ++p) xrow[p] = x + (int64_t)(m0 + srow[p] < M ? m0 + srow[p] : M - 1) * ldx;
     auto fetch = [&](const int slot, int kb) __attribute__((always_inline)) {
         const int k0 = kb * GM_KB;
         const int kx = k0 + spc * 8 < K ? k0 + spc * 8 : K - 8;
@@ -265,7 +266,7 @@ gemm_mid_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* __
             default: if (GM_RING > 3) ending(std::integral_constant<int, 3>{}, kb0); break;
         }
     }
-    gm_epilogue<MT>(acc, out, mode, out_f32, bias, M, N, ldo, split, n0, r, j, vec_out, limit);
+    gm_epilogue<MT>(acc, out, mode, out_f32, bias, M, N, ldo, split, n0, r, j, vec_out, limit, m0);
 }
 
 // The same product for 65 .. 128 rows of x (MT = 5 .. 8 tiles of 16 rows): one pass over the weights where two launches of the
@@ -284,6 +285,10 @@ gemm_mid_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* __
 #define GW_KB 64
 
 #define GW_STAGES 4
+
+// Rows further apart than this (in elements; 128 of them then span 2^30 bytes) are past what the kernel's 31-bit offsets reach:
+// they go to the kernel above, whose addresses have 64 bits, 64 rows a workgroup.
+#define GW_MAX_LD (1 << 22)
 
 // the wavefront's loads but for the newest `n` have arrived (n counts loads; LDS and scalar counters are not waited for)
 template <int n>
@@ -458,10 +463,21 @@ int zi_gemm_mid_launch(void* out, int out_f32, int mode, const zi_bf16* x, const
     zi_gemm_mid_plan(N, K, mode >= GM_MODE_ACT || (mode == GM_MODE_SWIGLU && M > 64), &splits, &per, &waves);
     const int tiles = (N + 15) / 16;
     const dim3 grid((tiles + waves - 1) / waves, splits);
-    const int mt = (M + 15) / 16;
-#define ZI_GM2(MT, WV)                                                                                            \
-    gemm_mid_kernel<MT, 3, WV><<<grid, WV * ZI_WAVE, 0, stream>>>(out, mode, out_f32, x, w, bias, M, N, K, ldx, ldw, \
-                                                                  ldo, per, vec_out, limit)
+    const bool apart = M > 64 && (ldx > GW_MAX_LD || ldw > GW_MAX_LD);
+    const int mt = apart ? 0 : (M + 15) / 16;
+#define ZI_GM3(MT, WV, APART, GRID)                                                                                            \
+    gemm_mid_kernel<MT, 3, WV, APART><<<GRID, WV * ZI_WAVE, 0, stream>>>(out, mode, out_f32, x, w, bias, M, N, K, ldx, ldw, \
+                                                                         ldo, per, vec_out, limit)
+#define ZI_GM2(MT, WV) ZI_GM3(MT, WV, false, grid)
+#define ZI_GA2(MT, WV) ZI_GM3(MT, WV, true, dim3(grid.x, grid.y, (M + 16 * MT - 1) / (16 * MT)))
+#define ZI_GA(MT)                               \
+    switch (waves) {                            \
+        case 4: ZI_GA2(MT, 4); break;           \
+        case 5: ZI_GA2(MT, 5); break;           \
+        case 6: ZI_GA2(MT, 6); break;           \
+        case 7: ZI_GA2(MT, 7); break;           \
+        default: ZI_GA2(MT, 8); break;          \
+    }
 #define ZI_GM(MT)                               \
     switch (waves) {                            \
         case 4: ZI_GM2(MT, 4); break;           \
@@ -482,6 +498,7 @@ int zi_gemm_mid_launch(void* out, int out_f32, int mode, const zi_bf16* x, const
         default: ZI_GW2(MT, 8); break;          \
     }
     switch (mt) {
+        case 0: ZI_GA(4); break;
         case 1: ZI_GM(1); break;
         case 2: ZI_GM(2); break;
         case 3: ZI_GM(3); break;
@@ -493,6 +510,9 @@ int zi_gemm_mid_launch(void* out, int out_f32, int mode, const zi_bf16* x, const
     }
 #undef ZI_GM
 #undef ZI_GM2
+#undef ZI_GM3
+#undef ZI_GA
+#undef ZI_GA2
 #undef ZI_GW
 #undef ZI_GW2
     return zi_check_launch("gemm_mid");
