@@ -98,3 +98,32 @@ def test_float32_attention_sees_no_later_token():
     got = ops.attention(q, kc, vc, seq, pos, table, nh, nkv, d, 0.1)
     assert torch.allclose(got[:at], clean[:at], rtol=1e-5, atol=1e-6) and torch.equal(got[n:], clean[n:])
     assert bool(torch.isnan(got[at:n].view(-1, nh, d)[:, 3:, 3]).all())
+
+
+@pytest.mark.parametrize("n,window", [(17, 0), (33, 0), (150, 0), (40, 3)])
+@pytest.mark.parametrize("with_sinks", [False, True])
+def test_a_seen_key_of_minus_infinite_score_has_no_weight(n, window, with_sinks):
+    """A key with an infinite component against the query's sign scores minus infinity: weight zero, also where it is all that a
+    wavefront sees; a column that sees nothing else is NaN (without a sink), and so is one that sees a NaN."""
+    from zedinfer_amd import ops
+    nh, nkv, d, ps = 4, 2, 32, 16
+    g = torch.Generator().manual_seed(n)
+    kc, vc, table, ks, vs = paged([n], nkv, d, ps, g)
+    q = torch.rand(n, nh * d, generator=g) + 0.1                # every query positive
+    sinks = torch.randn(nh, generator=g) if with_sinks else None
+    at = [n - 1, 0] + [j for j in range(n) if 16 <= j < 32]     # the 17th token alone in its block, then all of the block; the first
+    for j in at:
+        kc[table[0, j // ps].long(), 0, j % ps, 5] = float("-inf")
+        ks[0][j, 0, 5] = float("-inf")
+    seq, pos = torch.zeros(n, dtype=torch.int32), torch.arange(n, dtype=torch.int32)
+    args = (kc, vc, seq.cuda(), pos.cuda(), table, nh, nkv, d, 0.2, window)
+    kw = dict(sinks=sinks.cuda()) if with_sinks else {}
+    ref = reference(q, ks, vs, seq.tolist(), pos.tolist(), nh, nkv, d, 0.2, window, sinks)
+    assert with_sinks or bool(torch.isnan(ref[0, :d]).all())
+    for decoded in (False, True):
+        got = ops.attention(q.cuda(), *args, decoded=decoded, **kw).cpu().double()
+        assert torch.equal(torch.isnan(got), torch.isnan(ref))
+        assert float((got - ref)[~torch.isnan(ref)].abs().max()) <= 2e-5      # (as in test_float32_attention)
+    kc[table[0, (n - 1) // ps].long(), 1, (n - 1) % ps, 0] = float("nan")
+    got = ops.attention(q.cuda(), *args, **kw)
+    assert bool(torch.isnan(got[n - 1, 2 * d:]).all()) and not bool(torch.isnan(got[:n - 1, 2 * d:]).any())

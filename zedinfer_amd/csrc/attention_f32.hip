@@ -122,10 +122,12 @@ attention_f32_kernel(float* __restrict__ out, const float* __restrict__ q, int64
             top = fmaxf(top, __shfl_xor(top, 32, ZI_WAVE));
             const float m_new = fmaxf(m, top), corr = m == -INFINITY ? 0.f : expf(m - m_new);
             m = m_new;
+            // (where all that was seen scores minus infinity, its weight is zero; a NaN stays one)
+            const float from = m_new == -INFINITY ? 0.f : m_new;
             float sum = 0.f;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                s0[e] = seen[e] ? expf(s0[e] - m_new) : 0.f;
+                s0[e] = seen[e] ? expf(s0[e] - from) : 0.f;
                 sum += s0[e];
             }
             l = l * corr + sum;
