@@ -127,3 +127,28 @@ def test_a_seen_key_of_minus_infinite_score_has_no_weight(n, window, with_sinks)
     kc[table[0, (n - 1) // ps].long(), 1, (n - 1) % ps, 0] = float("nan")
     got = ops.attention(q.cuda(), *args, **kw)
     assert bool(torch.isnan(got[n - 1, 2 * d:]).all()) and not bool(torch.isnan(got[:n - 1, 2 * d:]).any())
+
+
+@pytest.mark.parametrize("d", [16, 80, 128])
+def test_what_lies_in_cells_that_are_not_seen_changes_no_bit(d):
+    """Cells past a sequence's end hold NaN, or what a sequence left that had the page before: the same bits as with zeros there;
+    and the same for a token before one whose values are not finite, in its block and workgroup."""
+    from zedinfer_amd import ops
+    nh, nkv, ps, lens = 4, 2, 16, [37, 5, 70]
+    g = torch.Generator().manual_seed(d)
+    kc, vc, table, ks, vs = paged(lens, nkv, d, ps, g)
+    q = torch.randn(sum(lens), nh * d, generator=g).cuda()
+    seq = torch.repeat_interleave(torch.arange(3), torch.tensor(lens)).to(torch.int32).cuda()
+    pos = torch.cat([torch.arange(n) for n in lens]).to(torch.int32).cuda()
+    run = lambda k, v, decoded=False: ops.attention(q, k, v, seq, pos, table, nh, nkv, d, 0.1, decoded=decoded)  # noqa: E731
+    want = run(kc.nan_to_num(0.0), vc.nan_to_num(0.0))
+    assert bool(torch.isfinite(want).all())
+    for k, v in ((kc, vc), (kc.nan_to_num(3.0), vc.nan_to_num(-5.0))):
+        assert torch.equal(run(k, v), want) and torch.equal(run(k, v, True), want)
+    vc[int(table[0, 2]), 1, 3, 35 % ps], vc[int(table[0, 2]), 1, 4, 36 % ps] = float("nan"), float("-inf")
+    got = run(kc, vc)
+    assert torch.equal(got[:35], want[:35]) and torch.equal(got[37:], want[37:])
+    bad = got[35:37].view(2, nh, d)[:, 2:]
+    assert bool(torch.isnan(bad[:, :, 3]).all()) and bool(torch.isinf(bad[1, :, 4]).all())
+    rest = [i for i in range(d) if i not in (3, 4)]
+    assert torch.equal(bad[:, :, rest], want[35:37].view(2, nh, d)[:, 2:][:, :, rest])

@@ -14,7 +14,8 @@
 //
 // Tokens of several sequences among the 16 are done sequence by sequence.  A masked probability is zero, but zero times
 // an infinity or a NaN is not: where a block is not seen whole by all columns and one of its values is not finite, the
-// second product is made key by key with the masked ones left out.
+// second product is made with zeros in the place of such values, and their terms are added afterwards to the columns that
+// see them.  A column that sees none keeps its bits, whatever lies in masked cells.
 //
 // Bound, for prompts, by the instruction's rate and the trips to the cache (16 queries share a pass over the keys); for
 // decoded tokens by the trips that follow each other, one a block and wavefront.  Measured against the plain kernel
@@ -143,6 +144,16 @@ attention_f32_kernel(float* __restrict__ out, const float* __restrict__ q, int64
                 by_key = __ballot(odd) != 0;
             }
             if (by_key) {
+#pragma unroll
+                for (int i = 0; i < DT; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) vr[i][e] = fabsf(vr[i][e]) < INFINITY ? vr[i][e] : 0.f;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < DT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[i][j], s0[j], acc[i], 0, 0, 0);
+            if (by_key) {
                 const float* v = vcache + cell(page) + (b * 16) % page_size + (int64_t)g * 4 * page_size;
 #pragma unroll 1
                 for (int kk = 0; kk < 16; ++kk) {
@@ -156,18 +167,13 @@ attention_f32_kernel(float* __restrict__ out, const float* __restrict__ q, int64
                     for (int i = 0; i < DT; ++i) {
 #pragma unroll
                         for (int x = 0; x < 4; ++x) {
-                            const float term = pk * *vk;
-                            acc[i][x] += sk ? term : 0.f;
+                            const float val = *vk;
+                            acc[i][x] += sk && !(fabsf(val) < INFINITY) ? pk * val : 0.f;
                             vk += x < 3 ? page_size : 13 * page_size;
                             asm volatile("" : "+v"(vk));      // (32 addresses held for a path hardly ever taken cost registers)
                         }
                     }
                 }
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-#pragma unroll
-                    for (int i = 0; i < DT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[i][j], s0[j], acc[i], 0, 0, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
             fetch_v(next, page_next);
