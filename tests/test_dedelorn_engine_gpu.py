@@ -229,3 +229,46 @@ def test_configurations_drawn_at_random(tmp_path, seed):
                             ("whole", traces.whole(requests))):
             out = traces.run_in_process(engine, steps)
             _check(steps, out, ref, requests, dtype, (what, seed, json.dumps(cfg)))
+
+
+@pytest.mark.parametrize("name", ["delta", "wide"])
+def test_in_float32_a_position_has_one_set_of_bits(tmp_path, name):
+    """Whole, in portions, token by token and beside others, with portions on both sides of the lengths at which the bfloat16
+    engine changes kernels (64 tokens of an entry, 1,024 of a step, steps of single tokens): the same logits to the last bit."""
+    import json
+    from zedinfer_amd.config import SchedulerConfig
+    from zedinfer_amd.engine import Engine
+    from zedinfer_amd.weights.safetensors_io import write_safetensors
+    cfg = models.CONFIGS.get(name) or dict(
+        architecture="Dedelorn", width=64, vocab=120, norm=dict(eps=1e-6),
+        layers=[dict(type="delta", mixer=dict(heads=4, kv_heads=2, dim=32, vdim=48, conv=4), mlp=dict(kind="dense", ff=96)),
+                dict(type="latent_attention", mixer=dict(heads=2, dim=16, rot_dim=16, vdim=16, kv_rank=32, scale=0.25,
+                                                         mask=dict(size=90), rot=dict(base=100.0, dims=16)), mlp=dict(kind="dense", ff=96)),
+                dict(type="delta", mixer=dict(heads=2, kv_heads=2, dim=128, vdim=128, conv=4),
+                     mlp=dict(kind="moe", expert=dict(ff=32), router=dict(experts=4, top=2, scale=1.0)))])
+    folder = str(tmp_path / "m")
+    os.makedirs(folder)
+    with open(os.path.join(folder, "config.json"), "w") as f:
+        json.dump(cfg, f)
+    write_safetensors(os.path.join(folder, "model.safetensors"), models.make_weights(cfg, 3, torch.float32), metadata={"format": "pt"})
+    engine = Engine.from_folder(folder, "float32", SchedulerConfig(num_kv_blocks=400, kv_block_size=16, max_batch_requests=4,
+                                                                   max_batch_tokens=4096, max_seq_len=4096))
+    requests = {f"r{i}": traces.random_tokens(cfg["vocab"], n, seed=60 + i) for i, n in enumerate([1100, 150, 64, 70, 3])}
+    ref = {}
+    for what, steps in (("whole", traces.whole(requests)), ("decode", traces.last_decoded(requests, tail=40)),
+                        ("portions", traces.portions(requests, seed=1, sizes=(200, 63, 64, 65, 1, 2, 129, 31, 300))),
+                        ("mixed", traces.mixed(requests, max_live=4, seed=3, decode_tail=60, max_portion=260))):
+        out, fed = traces.run_in_process(engine, steps), {}
+        for st in steps:
+            row = 0
+            for e in st["entries"]:
+                base = fed.get(e["id"], 0)
+                for wpos in e["want"]:
+                    got = out[st["step"]][row]
+                    row += 1
+                    at = (e["id"], base + wpos)
+                    assert np.array_equal(ref.setdefault(at, got), got), (what, at, float(np.abs(ref[at] - got).max()))
+                fed[e["id"]] = base + len(e["tokens"])
+            for rid in st["end"]:
+                fed.pop(rid, None)
+    assert len(ref) == sum(len(t) for t in requests.values())

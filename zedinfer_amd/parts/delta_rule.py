@@ -93,11 +93,15 @@ class GatedDeltaRule(Mixer):
                              self.taps)
         y, gate = rt.buffer("delta_heads", (n, nh * vdim)), proj[:, self.gate_at:self.gate_at + nh * vdim]
         entries = (batch.entry_start, batch.entry_len, batch.entry_slot)
-        if batch.single_tokens and ops.delta_rule_steps(dim, vdim, state):
+        # The recurrence token by token, in chunks and by the single-token kernel are three orders of the sums.  A float32 model,
+        # whose products and attention have one order each, keeps to the first: a position's logits are the same bits however its
+        # prompt is cut and whatever rides along.  In bfloat16 the products' kernels differ by the number of rows anyway.
+        one_order = rt.dtype == torch.float32
+        if not one_order and batch.single_tokens and ops.delta_rule_steps(dim, vdim, state):
             ops.delta_rule_step(qk, v, beta_g, state, *entries, nh, kvh, dim, vdim, self.norm, gate, self.eps, out=y)
         else:
             o = rt.buffer("delta_read", (n, nh * vdim), torch.float32)
-            need = ops.delta_rule_workspace(n, batch.entry_start.numel(), nh, dim, vdim)
+            need = 0 if one_order else ops.delta_rule_workspace(n, batch.entry_start.numel(), nh, dim, vdim)
             ops.delta_rule(qk, v, beta_g, state, *entries, nh, kvh, dim, vdim, out=o,
                            workspace=rt.buffer("delta_chunks", (need,), torch.float32) if need else None)
             ops.gated_rms_norm(o, self.norm, gate, nh, vdim, self.eps, out=y)
