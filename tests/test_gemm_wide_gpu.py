@@ -54,3 +54,18 @@ def test_rows_further_apart_than_offsets_of_31_bits_reach(ldx, ldw, monkeypatch)
     g = torch.Generator(device="cuda").manual_seed(ldx % 1000 + ldw % 1000)
     for M, N, K in ((128, 80, 264), (77, 16, 72)):
         _check(ops, _inside(M, K, ldx, 0, g), _inside(N, K, ldw, 0, g), monkeypatch)
+
+
+@pytest.mark.parametrize("I,K,many", [(8960, 1536, True), (3072, 1024, True), (18944, 3584, False), (2048, 7168, False), (512, 8192, False),
+                                      (256, 7168, False), (2048, 2048, False)])
+def test_which_products_take_the_swiglu_epilogue_beyond_64_rows(I, K, many):
+    """Those that would not be cut for more than a launch is worth and whose workgroups are one round on 256 compute units (up to 64
+    rows: those that are never cut)."""
+    from zedinfer_amd import ops
+    w = torch.empty(2 * I, K, dtype=torch.bfloat16, device="cuda")
+    for M in (64, 65, 100, 128, 129):
+        x = torch.empty(M, K, dtype=torch.bfloat16, device="cuda")
+        if M > 64:
+            assert ops.linear_swiglu_pays(x, w) == (many and M <= 128), M
+        else:
+            assert ops.linear_swiglu_pays(x, w) == ops.linear_swiglu_supported(x, w) == (ops.linear_splits(M, 2 * I, K) == 1)

@@ -278,10 +278,10 @@ gemm_mid_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* __
 // as every other, so that each can wait for its own by count before the step's one barrier.  The cut, the order of the
 // sums and the epilogues are the kernel's above: a row's result does not depend on which of the two kernels makes it.
 // Measured at 128 rows, weights from memory, against wavefronts of 16 weight rows: 1.5B sizes down 16.3 to 13.5 us, q/k/v 7.3 to
-// 7.2, output 7.4 to 6.9; 7B sizes down 53 to 36, q/k/v 20 to 15, output 16 to 13.  With the SwiGLU epilogue 25.2 us at 128 rows
-// and 19.7 at 80 (1.5B gate/up), where the library's product and the activation's launch take 23 + 4.8, and 76 against 72 +
-// 6 at the 7B sizes.  A step's instructions were what bound it first: loads whose addresses cost nothing (a buffer, a lane's
-// offset and a step's) took 80 rows of the 1.5B gate/up from 20.6 to 18.0 us.
+// 7.2, output 7.4 to 6.9; 7B sizes down 53 to 36, q/k/v 20 to 15, output 16 to 13.  With the SwiGLU epilogue 21.1 us at 128 rows
+// and 17.2 at 80 (1.5B gate/up), where the library's product and the activation's launch take 25.5 and 21.7 together (for which
+// products it pays: zi_gemm_skinny_swiglu_pays).  A step's instructions were what bound it first: loads whose addresses cost the
+// lanes nothing took 80 rows of the 1.5B gate/up from 20.6 to 18.0 us.
 #define GW_KB 64
 
 #define GW_STAGES 4

@@ -99,6 +99,20 @@ extern "C" int zi_gemm_skinny_act_pays(int M, int N, int K) {
     return whole <= zi_gemm_mid_plan(N, K, 0, &s, &per, &waves) + SK_LAUNCH_COST;
 }
 
+// 1 when the SwiGLU epilogue of 65 to 128 rows beats the library's product and the activation's launch.  It makes the product
+// whole, so it does where a cut would gain no more than a launch is worth and where the workgroups are one round on the compute
+// units.  Measured with weights from memory, columns I of output x K, epilogue against library and launch, at 65 and at 128 rows: one
+// round 8,960 x 1,536 16.8 against 21.4 us and 21.1 against 25.5, 13,824 x 5,120 57 against 62 and 65 against 70, 3,072 x 1,024
+// 10.4 against 15.0 and 11.7 against 15.1; two rounds 18,944 x 3,584 60 against 64 but 73 against 65, 27,648 x 5,120 112 against
+// 116 but 134 against 124; a product that wants its cut 2,048 x 7,168 39 against 26 and 50 against 30, 512 x 8,192 42 against 15
+// and 50 against 17, 4,096 x 4,096 25 against 23 and 31 against 25.
+extern "C" int zi_gemm_skinny_swiglu_pays(int M, int N, int K) {
+    if (M <= 64 || M > SK_MID_MAX_ROWS) return 0;
+    int s, per, waves;
+    const int64_t cut = zi_gemm_mid_plan(N, K, 0, &s, &per, &waves), whole = zi_gemm_mid_plan(N, K, 1, &s, &per, &waves);
+    return whole <= cut + SK_LAUNCH_COST && ((N + 15) / 16 + waves - 1) / waves <= zi_compute_units();
+}
+
 // mode 0: out[M,N] (+ bias), reduced through `workspace` when the product is split.
 // mode 1: out = float32 partial sums [splits][M][N] (splits from zi_gemm_skinny_splits; the bias, if any, is in the first).
 // mode 2: w holds gate and up rows interleaved in blocks of 8; out[M, N/2] (bfloat16) =

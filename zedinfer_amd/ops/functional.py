@@ -1098,6 +1098,16 @@ def linear_swiglu_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
             and (x.shape[0] > FEW_ROWS or linear_splits(x.shape[0], weight.shape[0], weight.shape[1]) == 1))
 
 
+def linear_swiglu_pays(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether ``linear_swiglu`` takes this product and is the faster way to it: always up to FEW_ROWS rows, beyond them for
+    shapes at which it was measured to be (the kernel library says), or as ZEDINFER_SWIGLU_MAX_ROWS says."""
+    if not linear_swiglu_supported(x, weight):
+        return False
+    M = int(x.shape[0])
+    return M <= FEW_ROWS or _SWIGLU_ROWS_GIVEN or bool(
+        _lib.load().zi_gemm_skinny_swiglu_pays(M, int(weight.shape[0]), int(weight.shape[1])))
+
+
 def linear_swiglu(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """up * silu(gate) of x . weight^T in one kernel, for a weight [2I, K] whose rows are 8 gate rows,
     then the 8 up rows of the same columns, and so on; out [M, I] bfloat16."""
@@ -1163,11 +1173,13 @@ FEW_ROWS = 64          # up to here they beat the library product: the weights s
 # 7.2 / 6.9 / 13.5 us against the library's 9.7 / 8.1 / 24.5; 7B sizes 15 / 13 / 36 against 20 / 16 / 92.
 # Beyond 128 rows and up to 256 a kernel with 32 weight rows a wavefront (gemm_rows32.hip) takes the products whose
 # weights have at least twice as many columns as rows (the down projection; the library decides,
-# ``zi_gemm_skinny_pays``).  With the SwiGLU epilogue the limit is 128 rows: 25 us at 128 rows of the 1.5B sizes
-# against the library's 23 and the activation's launch of 5; beyond, the library's product.
-# (ZEDINFER_SUMS_MAX_ROWS=64 gives such products of more than 64 rows back to the library.)
+# ``zi_gemm_skinny_pays``).  With the SwiGLU epilogue the limit is 128 rows, and up to there the library decides from
+# 65 rows on (``zi_gemm_skinny_swiglu_pays``); beyond, the library's product.
+# (ZEDINFER_SUMS_MAX_ROWS=64 gives such products of more than 64 rows back to the library; ZEDINFER_SWIGLU_MAX_ROWS
+# gives the SwiGLU epilogue every product of up to that many rows.)
 SUMS_MAX_ROWS = max(FEW_ROWS, min(256, int(os.environ.get("ZEDINFER_SUMS_MAX_ROWS", "256") or 256)))
 SWIGLU_MAX_ROWS = max(FEW_ROWS, min(256, int(os.environ.get("ZEDINFER_SWIGLU_MAX_ROWS", "128") or 128)))
+_SWIGLU_ROWS_GIVEN = bool(os.environ.get("ZEDINFER_SWIGLU_MAX_ROWS"))
 _WORKSPACES = {}
 _OUTGROWN_WORKSPACES: list = []
 

@@ -134,7 +134,7 @@ class SwiGLU(FeedForward):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         n, I = x.shape[0], self.inter
         act = self.rt.buffer("ffn_act", (n, I))
-        if self.interleave and ops.linear_swiglu_supported(x, self.gate_up):
+        if self.interleave and ops.linear_swiglu_pays(x, self.gate_up):
             ops.linear_swiglu(x, self.gate_up, out=act)
         elif self.interleave and ops.linear_sums_supported(x, self.gate_up, ops.FEW_ROWS):
             S = ops.linear_splits(n, 2 * I, self.hidden)
