@@ -45,3 +45,17 @@ def test_float32_product_keeps_infinities_and_rows_apart():
         assert bool(torch.isinf(y[1, cols]).all()) and bool(torch.isnan(y[:, 5]).all())
         rest = [i for i in range(M) if i not in (1, 2)]
         assert bool((y[rest][:, cols] == 36).all()) and bool((y[2, cols] == 35).all())
+
+
+def test_float32_products_too_large_for_a_launch():
+    """More rows than the entry point takes are refused, whichever kernel; more weight rows than a launch of one dimension has
+    workgroups for go to the plain kernel."""
+    from zedinfer_amd import ops
+    x, w = torch.zeros(65535 * 64 + 1, 4, device="cuda"), torch.ones(1, 4, device="cuda")
+    with pytest.raises(RuntimeError):
+        ops.linear(x, w)
+    x[:, 1] = torch.arange(x.shape[0], device="cuda")
+    assert torch.equal(ops.linear(x[:-1], w)[:, 0], x[:-1, 1])
+    many = torch.zeros((1 << 26) + 9, 4, device="cuda")
+    many[:, 0] = torch.arange(many.shape[0], device="cuda") % 1021
+    assert torch.equal(ops.linear(torch.full((2, 4), 3.0, device="cuda"), many)[1], 3 * many[:, 0])

@@ -150,8 +150,8 @@ gemm_f32_stream_kernel(float* __restrict__ out, const float* __restrict__ x, con
     }
 }
 
-// TM x 64 outputs a workgroup; GROUPS (1 or 2) groups of four wavefronts, each over half of the runs of k when there are
-// two; TM/2 x 32 outputs a wavefront.  RING chunks of operands are on their way in registers.
+// TM x 32 NT outputs a workgroup; GROUPS (1 or 2) groups of four wavefronts, each over half of the runs of k when there are
+// two; TM/2 x 16 NT outputs a wavefront.  RING chunks of operands are on their way in registers.
 template <int TM, int NT, int GROUPS, int RING>
 __global__ void __launch_bounds__(256 * GROUPS)
 gemm_f32_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,
@@ -292,32 +292,38 @@ gemm_f32_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const
     }
 }
 
-// Whether these kernels take the operands (all float32): whole 16-byte pieces of every row, and rows of a tile within a
-// buffer's range.
-bool zi_gemm_f32_takes(const void* x, const void* w, int K, int64_t ldx, int64_t ldw) {
-    return K % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 && ldx < (1 << 21) && ldw < (1 << 21);
+// Whether these kernels take the operands (all float32): whole 16-byte pieces of every row, rows of a tile within a buffer's
+// range, and weight rows whose workgroups fit a launch of one dimension (2^32 threads; 64 a row for up to 8 rows of x).
+bool zi_gemm_f32_takes(const void* x, const void* w, int N, int K, int64_t ldx, int64_t ldw) {
+    return K % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 && ldx < (1 << 21) && ldw < (1 << 21) &&
+           N <= (1 << 25);
 }
 
 // The launch; the sizes are checked by the caller (zi_gemm_generic).
 int zi_gemm_f32_launch(float* out, const float* x, const float* w, const float* bias, int M, int N, int K, int64_t ldx, int64_t ldw,
                        int64_t ldo, hipStream_t stream) {
     const int chunks = (K + GF_KB - 1) / GF_KB, per = (chunks + GF_PARTS - 1) / GF_PARTS;
-    ZI_REQUIRE((int64_t)((M + 31) / 32) * ((N + 31) / 32) < (1ll << 30), "gemm: M=%d N=%d is too large for one launch", M, N);
     const int vec_out = ldo % 4 == 0 && (uintptr_t)out % 16 == 0;
 #define ZI_GF_STREAM(MT, PAIR, RING)                                                                                                     \
     gemm_f32_stream_kernel<MT, PAIR, RING><<<dim3((N + (PAIR ? 7 : 15)) / (PAIR ? 8 : 16), (M + (PAIR ? 8 : 16 * MT) - 1) / (PAIR ? 8 : 16 * MT)), \
                                              GF_PARTS * ZI_WAVE, 0, stream>>>(out, x, w, bias, M, N, K, ldx, ldw, ldo, per, vec_out)
+    // (rows in as many launches as 2^32 threads of one make necessary: a row's result does not depend on them)
 #define ZI_GF_TILE(TM, NT, G, R)                                                                                                              \
     do {                                                                                                                                  \
-        const int mt = (M + TM - 1) / TM, tiles = mt * ((N + 32 * NT - 1) / (32 * NT));                                                                   \
-        gemm_f32_tile_kernel<TM, NT, G, R><<<(tiles + 7) / 8 * 8, 256 * G, 0, stream>>>(out, x, w, bias, M, N, K, ldx, ldw, ldo, per, vec_out, mt, tiles); \
+        const int64_t nt = (N + 32 * NT - 1) / (32 * NT), most = ((1ll << 31) / (256 * G)) / nt * TM;                                              \
+        for (int64_t m = 0; m < M; m += most) {                                                                                           \
+            const int rows = (int)(M - m < most ? M - m : most), mt = (rows + TM - 1) / TM, tiles = (int)(mt * nt);                              \
+            gemm_f32_tile_kernel<TM, NT, G, R><<<(tiles + 7) / 8 * 8, 256 * G, 0, stream>>>(out + m * ldo, x + m * ldx, w, bias, rows, N, K, ldx, \
+                                                                                            ldw, ldo, per, vec_out, mt, tiles);               \
+        }                                                                                                                                 \
     } while (0)
     // Which kernel is a matter of filling the compute units only; all give the same bits.  Up to 8 rows the paired form of the
     // stream (one row of a 151,936-row head 190 against 233 us); 16 rows a workgroup while that gives no unit a second
     // workgroup (32 rows, 1,536 x 8,960: 34 against 52 us), 32 rows up to 32 rows and then while the same holds (64 rows:
     // 52 against 92 us for the tiles).  Beyond, tiles of 32 x 64 in two halves of k while they are one round of workgroups
     // (256 rows, 1,536 x 8,960: 96 us, one group 123, tiles of 64 x 64 194), of 32 x 96 where those make one round of what
-    // would be two (448 rows: 148 against 157); from six rounds of 64 x 64 tiles on those (17,920 x 1,536 at 448 rows 219
+    // would be two (448 rows: 148 against 158, 2,560 x 2,560 at 288 rows 48 against 53, 2,816 x 1,024 at 256 20.8 against 23.9, 6,144 x
+    // 2,048 at 128 38 against 42: 6 to 16 % at 17 shapes); from six rounds of 64 x 64 tiles on those (17,920 x 1,536 at 448 rows 219
     // against 226 us, at 256 rows, 4.4 rounds, 141 against 133); else 32 x 64, in two halves up to three rounds (448
     // rows, 2,048 x 1,536: 33 against 37; 1,024 rows, four rounds: 61 against 60).
     const int64_t cus = zi_compute_units(), n16 = (N + 15) / 16, m32 = (M + 31) / 32;

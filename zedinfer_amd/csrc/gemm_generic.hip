@@ -68,7 +68,7 @@ gemm_generic_kernel(TO* __restrict__ out, const TX* __restrict__ x, const TW* __
     }
 }
 
-bool zi_gemm_f32_takes(const void* x, const void* w, int K, int64_t ldx, int64_t ldw);
+bool zi_gemm_f32_takes(const void* x, const void* w, int N, int K, int64_t ldx, int64_t ldw);
 int zi_gemm_f32_launch(float* out, const float* x, const float* w, const float* bias, int M, int N, int K, int64_t ldx, int64_t ldw,
                        int64_t ldo, hipStream_t stream);
 
@@ -78,11 +78,11 @@ extern "C" int zi_gemm_generic(void* out, int out_dt, const void* x, int x_dt, c
     ZI_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm: bad sizes M=%d N=%d K=%d", M, N, K);
     ZI_REQUIRE(ldx >= K && ldw >= K && ldo >= N, "gemm: leading dimension too small");
     if (M == 0) return 0;
-    // all float32 and whole 16-byte pieces a row: the matrix cores' float32 instruction (gemm_f32.hip), whatever M is
-    if (x_dt == ZI_F32 && w_dt == ZI_F32 && out_dt == ZI_F32 && (!bias || bias_dt == ZI_F32) && zi_gemm_f32_takes(x, w, K, ldx, ldw))
-        return zi_gemm_f32_launch((float*)out, (const float*)x, (const float*)w, (const float*)bias, M, N, K, ldx, ldw, ldo, stream);
     const dim3 grid((N + GT - 1) / GT, (M + GT - 1) / GT);
     ZI_REQUIRE(grid.y <= 65535, "gemm: M=%d is too large for one launch", M);
+    // all float32 and whole 16-byte pieces a row: the matrix cores' float32 instruction (gemm_f32.hip), whatever M is
+    if (x_dt == ZI_F32 && w_dt == ZI_F32 && out_dt == ZI_F32 && (!bias || bias_dt == ZI_F32) && zi_gemm_f32_takes(x, w, N, K, ldx, ldw))
+        return zi_gemm_f32_launch((float*)out, (const float*)x, (const float*)w, (const float*)bias, M, N, K, ldx, ldw, ldo, stream);
     if (!bias) bias_dt = ZI_F32;
     ZI_DISPATCH_DTYPE(x_dt, TX, ZI_DISPATCH_DTYPE(w_dt, TW, ZI_DISPATCH_DTYPE(bias_dt, TB, ZI_DISPATCH_DTYPE(out_dt, TO, {
         gemm_generic_kernel<TX, TW, TB, TO><<<grid, 256, 0, stream>>>(
