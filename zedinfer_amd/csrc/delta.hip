@@ -13,6 +13,7 @@
 // portions in chunks: delta_chunks.hip; steps of single tokens: delta_channel.hip).
 #include "zi_common.h"
 #include "zi_api.h"
+#include "zi_delta.h"
 
 __device__ __forceinline__ float delta_silu(float z) { return z / (1.f + expf(-z)); }
 __device__ __forceinline__ float delta_softplus(float z) { return z > 30.f ? z : log1pf(expf(z)); }
@@ -237,7 +238,6 @@ extern "C" int zi_delta_conv_state(float* state, int64_t state_stride, int64_t c
 #define DELTA_COLS 8
 #define DELTA_PARTS 8
 #define DELTA_TOKS 8
-#define DELTA_CHUNK 64
 
 // x of the lane that `ctrl` names within this lane's row of 16 (quad permutations, mirrors)
 template <int CTRL>
@@ -271,15 +271,9 @@ delta_rule_kernel(float* __restrict__ out, const float* __restrict__ qk, const f
     const int kh = h / (heads / kvh), qkc = 2 * kvh * dim;
     const int start = entry_start[e], len = entry_len[e];
     if (marks && len >= shortest) {
-        // an entry that is done in chunks of DELTA_CHUNK tokens (delta_chunks.hip; numbered entry by entry), unless one of its
-        // chunks is marked for this head
-        int id = 0;
-        for (int i = lane; i < e; i += ZI_WAVE) id += entry_len[i] >= shortest ? (entry_len[i] + DELTA_CHUNK - 1) / DELTA_CHUNK : 0;
-#pragma unroll
-        for (int o = ZI_WAVE / 2; o > 0; o >>= 1) id += __shfl_xor(id, o, ZI_WAVE);
-        bool left = false;
-        for (int i = lane; i < (len + DELTA_CHUNK - 1) / DELTA_CHUNK; i += ZI_WAVE) left |= marks[(int64_t)(id + i) * heads + h] != 0;
-        if (!__ballot(left)) return;
+        // an entry that is done in chunks (delta_chunks.hip), unless one of them is marked for this head
+        const int chunks = delta_chunks_of(len, shortest);
+        if (delta_first_mark(delta_first_chunk(e, entry_len, shortest), chunks, marks, heads, h) == chunks) return;
     }
     float* S = state + (int64_t)entry_slot[e] * state_stride + (int64_t)h * dim * vdim;
     float s[R];
@@ -387,7 +381,6 @@ delta_rule_kernel(float* __restrict__ out, const float* __restrict__ qk, const f
     }
 }
 
-// `marks` (or null): entries of at least `shortest` tokens are done only for heads with a mark (see delta_chunks.hip).
 int zi_delta_rule_launch(float* out, const float* qk, const float* v, const float* beta_g, float* state, int64_t state_stride,
                          const int32_t* entry_start, const int32_t* entry_len, const int32_t* entry_slot, int entries, int heads,
                          int kvh, int dim, int vdim, int shortest, const int32_t* marks, hipStream_t stream) {

@@ -24,11 +24,12 @@
 // A NaN or an infinity would pass, as zero times it, from a token to earlier ones of its chunk.  Chunks with a value that
 // is not finite are marked, and the entry's head with one is left to delta_rule_kernel.
 #include "zi_common.h"
+#include "zi_delta.h"
 #include <type_traits>
 
 typedef __attribute__((ext_vector_type(4))) float dc_f32x4_t;
 
-#define DC_TOKS 64
+#define DC_TOKS DELTA_CHUNK
 #define DC_LD (DC_TOKS + 4)
 
 __device__ __forceinline__ dc_f32x4_t dc_mfma(dc_f32x4_t a, dc_f32x4_t b, dc_f32x4_t c) {
@@ -58,8 +59,6 @@ __device__ __forceinline__ dc_f32x4_t dc_dot(const dc_f32x4_t (&held)[N], const 
     return dc_total<N>(s);
 }
 
-__device__ __forceinline__ int dc_chunks(int len, int shortest) { return len >= shortest ? (len + DC_TOKS - 1) / DC_TOKS : 0; }
-
 // Chunks are numbered entry by entry.  All lanes of a wavefront: the entry and the chunk within it that number `id` stands for
 // (entry -1: none).
 __device__ __forceinline__ void dc_find(int id, const int32_t* __restrict__ entry_len, int entries, int shortest, int* entry, int* chunk) {
@@ -67,7 +66,7 @@ __device__ __forceinline__ void dc_find(int id, const int32_t* __restrict__ entr
     int before = 0;
     *entry = -1;
     for (int e0 = 0; e0 < entries; e0 += ZI_WAVE) {
-        const int own = e0 + lane < entries ? dc_chunks(entry_len[e0 + lane], shortest) : 0;
+        const int own = e0 + lane < entries ? delta_chunks_of(entry_len[e0 + lane], shortest) : 0;
         int upto = own;
 #pragma unroll
         for (int o = 1; o < ZI_WAVE; o <<= 1) {
@@ -83,15 +82,6 @@ __device__ __forceinline__ void dc_find(int id, const int32_t* __restrict__ entr
         }
         before += __builtin_amdgcn_readlane(upto, ZI_WAVE - 1);
     }
-}
-
-// the number of entry e's first chunk
-__device__ __forceinline__ int dc_first(int e, const int32_t* __restrict__ entry_len, int shortest) {
-    int sum = 0;
-    for (int i = threadIdx.x & (ZI_WAVE - 1); i < e; i += ZI_WAVE) sum += dc_chunks(entry_len[i], shortest);
-#pragma unroll
-    for (int o = ZI_WAVE / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, ZI_WAVE);
-    return __builtin_amdgcn_readfirstlane(sum);
 }
 
 // What a (chunk, head) is given in the workspace, in floats: W [64][dim], r q [64][dim], the keys [dim][64], U [64][vdim], A [64][64],
@@ -332,12 +322,10 @@ delta_chunk_walk_kernel(float* __restrict__ out, const float* __restrict__ ws, c
     const int blocks = vdim / 16, in_xcd = blockIdx.x / 8;
     const int e = blockIdx.z, h = blockIdx.x % 8 + in_xcd / blocks * 8, col = in_xcd % blocks * 16 + c;
     if (h >= heads) return;
-    const int len = entry_len[e], chunks = dc_chunks(len, shortest);
+    const int len = entry_len[e], chunks = delta_chunks_of(len, shortest);
     if (chunks == 0) return;
-    const int id0 = dc_first(e, entry_len, shortest);
-    bool bad = false;
-    for (int i = lane; i < chunks; i += ZI_WAVE) bad |= marks[(int64_t)(id0 + i) * heads + h] != 0;
-    if (__ballot(bad)) return;
+    const int id0 = delta_first_chunk(e, entry_len, shortest);
+    if (delta_first_mark(id0, chunks, marks, heads, h) < chunks) return;
     const int start = entry_start[e];
     const int64_t cell = dc_cell(D, vdim);
     const float* const base = ws + ((int64_t)id0 * heads + h) * cell;
@@ -479,10 +467,6 @@ delta_chunk_walk_kernel(float* __restrict__ out, const float* __restrict__ ws, c
         }
     }
 }
-
-int zi_delta_rule_launch(float* out, const float* qk, const float* v, const float* beta_g, float* state, int64_t state_stride,
-                         const int32_t* entry_start, const int32_t* entry_len, const int32_t* entry_slot, int entries, int heads,
-                         int kvh, int dim, int vdim, int shortest, const int32_t* marks, hipStream_t stream);
 
 // Tokens of an entry from which it is done in chunks: one chunk's launches take 32 us, as delta_rule_kernel does for 64 tokens.
 #define DC_SHORTEST 64
