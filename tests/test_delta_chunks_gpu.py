@@ -147,3 +147,34 @@ def test_preparing_four_channels_a_thread(heads, kvh, dim, vdim, lens):
     assert float((bg[:, 0].cpu().double() - torch.sigmoid(b)).abs().max()) < 1e-6
     decay = torch.exp(-torch.exp(a_log.double()) * torch.nn.functional.softplus(a + dt.double()))
     assert float((bg[:, 1].cpu().double() - decay).abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("heads,kvh,dim,vdim,lens", [(120, 4, 128, 128, [70, 1, 300, 64, 500, 3]), (600, 300, 128, 128, [200, 129]), (64, 2, 64, 16, [6000])])
+def test_chunks_in_rounds(heads, kvh, dim, vdim, lens):
+    """Heads and tokens whose chunks are more than one round's workspace: the rule token by token, and a value that is not finite in
+    a later round or an earlier one."""
+    from zedinfer_amd import ops
+    x = _inputs(lens, heads, kvh, dim, vdim, seed=heads)
+    n, E = sum(lens), len(lens)
+    need = ops.delta_rule_workspace(n, E, heads, dim, vdim)
+    cell = 64 * (3 * dim + vdim + 65)
+    assert 0 < need <= (128 << 18) + heads * (n // 64 + E) and need < heads * cell * (n // 64)
+    alone, alone_state = _run(ops, lens, *x, chunked=False)
+    got, state = _run(ops, lens, *x, chunked=True)
+    for a, b in ((got, alone), (state, alone_state)):       # (each within 2e-6 of float64, see above)
+        assert float((a.double() - b.double()).norm() / b.double().norm()) < 4e-6
+    for bad in (n - 5, 40):                                 # of the last and of the first long entry
+        v = x[2].clone()
+        v[bad, 3, 1] = float("inf")
+        args = (*x[:2], v, *x[3:])
+        odd, odd_state = _run(ops, lens, *args, chunked=True)
+        plain, plain_state = _run(ops, lens, *args, chunked=False)
+        assert torch.equal(torch.isfinite(odd), torch.isfinite(plain)) and torch.equal(torch.isfinite(odd_state), torch.isfinite(plain_state))
+        at = torch.isfinite(plain)
+        assert not bool(at.all()) and torch.equal(odd[:bad // 64 * 64 if E == 1 else 0], got[:bad // 64 * 64 if E == 1 else 0])
+        assert float((odd - plain)[at].abs().max()) < 2e-5 * float(plain[at].abs().max())
+
+
+def test_more_heads_than_a_round_holds():
+    from zedinfer_amd import ops
+    assert ops.delta_rule_workspace(200, 1, 908, 128, 128) > 0 and ops.delta_rule_workspace(200, 1, 909, 128, 128) == 0

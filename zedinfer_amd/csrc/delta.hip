@@ -269,11 +269,14 @@ delta_rule_kernel(float* __restrict__ out, const float* __restrict__ qk, const f
     const int col0 = blockIdx.x * DELTA_COLS, col = col0 + lane / DELTA_PARTS, part = lane % DELTA_PARTS;
     const bool live = col < vdim;
     const int kh = h / (heads / kvh), qkc = 2 * kvh * dim;
-    const int start = entry_start[e], len = entry_len[e];
+    int start = entry_start[e], len = entry_len[e];
     if (marks && len >= shortest) {
-        // an entry that is done in chunks (delta_chunks.hip), unless one of them is marked for this head
+        // an entry that is done in chunks (delta_chunks.hip), up to the first that is marked for this head
         const int chunks = delta_chunks_of(len, shortest);
-        if (delta_first_mark(delta_first_chunk(e, entry_len, shortest), chunks, marks, heads, h) == chunks) return;
+        const int done = delta_first_mark(delta_first_chunk(e, entry_len, shortest), chunks, marks, heads, h);
+        if (done == chunks) return;
+        start += done * DELTA_CHUNK;
+        len -= done * DELTA_CHUNK;
     }
     float* S = state + (int64_t)entry_slot[e] * state_stride + (int64_t)h * dim * vdim;
     float s[R];

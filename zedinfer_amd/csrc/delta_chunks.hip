@@ -21,8 +21,13 @@
 // do, against 992 us token by token.  Against 64 bits, on the tensors of a model's six such layers, the read-out is 1.7e-7 off
 // (token by token 1.8e-7) and the state 1.5e-7 (2.1e-7): the long sums are made of a sum for every 16 values.
 //
+// The two take DC_ROUND bytes' worth of chunks in turn, so that the workspace has a bound whatever the step: 148 KB a (chunk, head)
+// at those sizes, where a round is 75 chunks.  A round more costs its launches and the end of a chain: 8,192 tokens 397 us against
+// 387 in one round of 229 MB, 28 heads 531 against 527 (534 MB), eight prompts of 1,000 294 against 265; with half of DC_ROUND 414,
+// 575 and 329.
+//
 // A NaN or an infinity would pass, as zero times it, from a token to earlier ones of its chunk.  Chunks with a value that
-// is not finite are marked, and the entry's head with one is left to delta_rule_kernel.
+// is not finite are marked, and an entry's head is left to delta_rule_kernel from its first marked chunk on.
 #include "zi_common.h"
 #include "zi_delta.h"
 #include <type_traits>
@@ -93,7 +98,7 @@ template <int DT>        // dim / 16
 __global__ void __launch_bounds__(512)
 delta_chunk_kernel(float* __restrict__ ws, int32_t* __restrict__ marks, const float* __restrict__ qk, const float* __restrict__ v,
                    const float* __restrict__ beta_g, const int32_t* __restrict__ entry_start, const int32_t* __restrict__ entry_len,
-                   int entries, int shortest, int heads, int kvh, int vdim) {
+                   int entries, int shortest, int heads, int kvh, int vdim, int id0) {
     constexpr int D = DT * 16, LDK = D + 4, VP = (DC_TOKS * D / 4 + 511) / 512;
     __shared__ __attribute__((aligned(16))) float ks[DC_TOKS * LDK];      // keys; then dim columns of v at a time
     __shared__ __attribute__((aligned(16))) float rt[DC_TOKS * DC_LD], ms[DC_TOKS * DC_LD];        // r_ij, then T; M
@@ -102,7 +107,7 @@ delta_chunk_kernel(float* __restrict__ ws, int32_t* __restrict__ marks, const fl
     const int tid = threadIdx.x, lane = tid & (ZI_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(tid / ZI_WAVE);
     const int c = lane & 15, g = lane >> 4;
     int e, chunk;
-    dc_find(blockIdx.x, entry_len, entries, shortest, &e, &chunk);
+    dc_find(id0 + blockIdx.x, entry_len, entries, shortest, &e, &chunk);
     if (e < 0) return;
     const int h = blockIdx.y, kh = h / (heads / kvh), qkc = 2 * kvh * D;
     const int len = entry_len[e], cnt = len - chunk * DC_TOKS < DC_TOKS ? len - chunk * DC_TOKS : DC_TOKS;
@@ -305,15 +310,16 @@ delta_chunk_kernel(float* __restrict__ ws, int32_t* __restrict__ marks, const fl
     }
     if (bad) odd = 1;
     __syncthreads();
-    if (tid == 0) marks[(int64_t)blockIdx.x * heads + h] = odd;
+    if (tid == 0) marks[(int64_t)(id0 + blockIdx.x) * heads + h] = odd;
 }
 
+// The chunks id_lo .. id_hi - 1 (of all entries; those of the round), as far as no mark of an entry's head comes before them.
 template <int DT>        // dim / 16, at most 8: a wavefront holds 16 rows of the state
 __global__ void __launch_bounds__(512)
 delta_chunk_walk_kernel(float* __restrict__ out, const float* __restrict__ ws, const int32_t* __restrict__ marks,
                         float* __restrict__ state, int64_t state_stride, const int32_t* __restrict__ entry_start,
                         const int32_t* __restrict__ entry_len, const int32_t* __restrict__ entry_slot, int shortest, int heads,
-                        int vdim) {
+                        int vdim, int id_lo, int id_hi) {
     constexpr int D = DT * 16;
     __shared__ __attribute__((aligned(16))) float st[16 * (D + 4)], xt[16 * DC_LD];      // [column][row of S], [column][token]
     const int lane = threadIdx.x & (ZI_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / ZI_WAVE);
@@ -322,13 +328,18 @@ delta_chunk_walk_kernel(float* __restrict__ out, const float* __restrict__ ws, c
     const int blocks = vdim / 16, in_xcd = blockIdx.x / 8;
     const int e = blockIdx.z, h = blockIdx.x % 8 + in_xcd / blocks * 8, col = in_xcd % blocks * 16 + c;
     if (h >= heads) return;
-    const int len = entry_len[e], chunks = delta_chunks_of(len, shortest);
-    if (chunks == 0) return;
+    const int len_all = entry_len[e], chunks_all = delta_chunks_of(len_all, shortest);
+    if (chunks_all == 0) return;
     const int id0 = delta_first_chunk(e, entry_len, shortest);
-    if (delta_first_mark(id0, chunks, marks, heads, h) < chunks) return;
-    const int start = entry_start[e];
+    const int first = id_lo > id0 ? id_lo - id0 : 0, before = id_hi - id0 < chunks_all ? id_hi - id0 : chunks_all;
+    if (first >= before) return;
+    const int chunks = delta_first_mark(id0, before, marks, heads, h) - first;       // (the marks of earlier rounds are there)
+    if (chunks <= 0) return;
+    // from here on the entry is this round's part of it
+    const int start = entry_start[e] + first * DC_TOKS;
+    const int len = len_all - first * DC_TOKS < chunks * DC_TOKS ? len_all - first * DC_TOKS : chunks * DC_TOKS;
     const int64_t cell = dc_cell(D, vdim);
-    const float* const base = ws + ((int64_t)id0 * heads + h) * cell;
+    const float* const base = ws + ((int64_t)(id0 + first - id_lo) * heads + h) * cell;
     float* const S = state + (int64_t)entry_slot[e] * state_stride + (int64_t)h * D * vdim;
     const dc_f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
     const int rb = wave & 3;                                  // the block of tokens
@@ -471,13 +482,23 @@ delta_chunk_walk_kernel(float* __restrict__ out, const float* __restrict__ ws, c
 // Tokens of an entry from which it is done in chunks: one chunk's launches take 32 us, as delta_rule_kernel does for 64 tokens.
 #define DC_SHORTEST 64
 
+// Bytes of workspace that a round of chunks may take (marks apart).
+#define DC_ROUND (128 << 20)
+
 static int64_t dc_most_chunks(int n, int entries) { return n / DC_TOKS + (entries < n / DC_SHORTEST ? entries : n / DC_SHORTEST); }
 
+// Chunks of a round; 0: not even one chunk's heads fit.
+static int64_t dc_round(int n, int entries, int heads, int dim, int vdim) {
+    const int64_t fit = DC_ROUND / 4 / (heads * dc_cell(dim, vdim)), most = dc_most_chunks(n, entries);
+    return fit < most ? fit : most;
+}
+
 // Floats of workspace with which zi_delta_rule_chunked takes n tokens of so many entries in chunks; 0: it would not, the
-// entries are too short or the head sizes no multiples of 16.
+// entries are too short, the head sizes no multiples of 16 or the heads too many for a round.
 extern "C" int64_t zi_delta_rule_workspace(int n, int entries, int heads, int dim, int vdim) {
     if (entries < 1 || n - (entries - 1) < DC_SHORTEST || (int64_t)heads * vdim > (1 << 20) || dim % 16 || dim < 16 || dim > 128 || vdim % 16 || vdim < 16) return 0;
-    return dc_most_chunks(n, entries) * heads * (dc_cell(dim, vdim) + 1);
+    const int64_t round = dc_round(n, entries, heads, dim, vdim);
+    return round > 0 ? heads * (round * dc_cell(dim, vdim) + dc_most_chunks(n, entries)) : 0;
 }
 
 extern "C" int zi_delta_rule_chunked(float* out, const float* qk, const float* v, const float* beta_g, float* state, int64_t state_stride,
@@ -491,14 +512,17 @@ extern "C" int zi_delta_rule_chunked(float* out, const float* qk, const float* v
     ZI_REQUIRE(need > 0 && workspace && workspace_floats >= need, "delta_rule: workspace of %lld floats is too small (%lld needed)",
                (long long)workspace_floats, (long long)need);
     ZI_REQUIRE(((uintptr_t)qk | (uintptr_t)v | (uintptr_t)workspace) % 16 == 0, "delta_rule: rows must be 16-byte aligned");
-    const int64_t chunks = dc_most_chunks(n, entries);
-    int32_t* marks = (int32_t*)(workspace + chunks * heads * dc_cell(dim, vdim));
+    const int64_t chunks = dc_most_chunks(n, entries), round = dc_round(n, entries, heads, dim, vdim);
+    int32_t* marks = (int32_t*)(workspace + round * heads * dc_cell(dim, vdim));
 #define ZI_DC(DT)                                                                                                                       \
     case DT:                                                                                                                            \
-        delta_chunk_kernel<DT><<<dim3(chunks, heads), 512, 0, stream>>>(workspace, marks, qk, v, beta_g, entry_start, entry_len, entries, \
-                                                                        DC_SHORTEST, heads, kvh, vdim);                                 \
-        delta_chunk_walk_kernel<DT><<<dim3((heads + 7) / 8 * 8 * (vdim / 16), 1, entries), 512, 0, stream>>>(                            \
-            out, workspace, marks, state, state_stride, entry_start, entry_len, entry_slot, DC_SHORTEST, heads, vdim);                   \
+        for (int64_t lo = 0; lo < chunks; lo += round) {                                                                                \
+            const int hi = (int)(lo + round < chunks ? lo + round : chunks);                                                             \
+            delta_chunk_kernel<DT><<<dim3(hi - lo, heads), 512, 0, stream>>>(workspace, marks, qk, v, beta_g, entry_start, entry_len,    \
+                                                                             entries, DC_SHORTEST, heads, kvh, vdim, (int)lo);          \
+            delta_chunk_walk_kernel<DT><<<dim3((heads + 7) / 8 * 8 * (vdim / 16), 1, entries), 512, 0, stream>>>(                        \
+                out, workspace, marks, state, state_stride, entry_start, entry_len, entry_slot, DC_SHORTEST, heads, vdim, (int)lo, hi);  \
+        }                                                                                                                               \
         break
     switch (dim / 16) {
         ZI_DC(1); ZI_DC(2); ZI_DC(3); ZI_DC(4); ZI_DC(5); ZI_DC(6); ZI_DC(7); ZI_DC(8);
@@ -506,7 +530,7 @@ extern "C" int zi_delta_rule_chunked(float* out, const float* qk, const float* v
 #undef ZI_DC
     const int rc = zi_check_launch("delta_rule_chunked");
     if (rc) return rc;
-    // the short entries, and the heads of long ones that a mark left undone
+    // the short entries, and the heads of long ones from a mark on
     return zi_delta_rule_launch(out, qk, v, beta_g, state, state_stride, entry_start, entry_len, entry_slot, entries, heads, kvh, dim,
                                 vdim, DC_SHORTEST, marks, stream);
 }

@@ -28,7 +28,8 @@ __device__ __forceinline__ int delta_first_mark(int first, int chunks, const int
     return chunks;
 }
 
-// The recurrence token by token.  `marks` (or null): entries of at least `shortest` tokens are done only for heads with a mark.
+// The recurrence token by token.  `marks` (or null): of entries of at least `shortest` tokens only a head's tokens from its first
+// marked chunk on are done, from the state that the chunks before it left.
 int zi_delta_rule_launch(float* out, const float* qk, const float* v, const float* beta_g, float* state, int64_t state_stride,
                          const int32_t* entry_start, const int32_t* entry_len, const int32_t* entry_slot, int entries, int heads,
                          int kvh, int dim, int vdim, int shortest, const int32_t* marks, hipStream_t stream);
