@@ -178,3 +178,24 @@ def test_chunks_in_rounds(heads, kvh, dim, vdim, lens):
 def test_more_heads_than_a_round_holds():
     from zedinfer_amd import ops
     assert ops.delta_rule_workspace(200, 1, 908, 128, 128) > 0 and ops.delta_rule_workspace(200, 1, 909, 128, 128) == 0
+
+
+def test_finite_values_whose_sums_are_not():
+    """Two tokens whose values are near the largest float32 make an infinity between them: it reaches them and later tokens of their
+    head and no earlier one of their chunk."""
+    from zedinfer_amd import ops
+    lens = [150]
+    q, k, v, beta, gate, state = _inputs(lens, 2, 1, 32, 32, seed=5)
+    k[101] = k[100]
+    beta[100:102], gate[100:102] = 0.99, 1.0
+    v[100, 1, 4], v[101, 1, 4] = 3e38, -3e38
+    got, _ = _run(ops, lens, q, k, v, beta, gate, state, True)
+    plain, _ = _run(ops, lens, q, k, v, beta, gate, state, False)
+    assert bool(torch.isfinite(plain[:100]).all()) and not bool(torch.isfinite(plain[101:, 1, 4]).any())
+    assert torch.equal(torch.isfinite(got), torch.isfinite(plain))
+    at = torch.isfinite(plain) & (plain.abs() < 1e30)
+    assert float((got - plain)[at].abs().max()) < 1e-5
+    gate[60] = 1.5                                              # no decay: the rule token by token
+    got, _ = _run(ops, lens, q, k, v.clamp(-3, 3), beta, gate, state, True)
+    plain, _ = _run(ops, lens, q, k, v.clamp(-3, 3), beta, gate, state, False)
+    assert torch.equal(got, plain)

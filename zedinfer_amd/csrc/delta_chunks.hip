@@ -27,7 +27,7 @@
 // 575 and 329.
 //
 // A NaN or an infinity would pass, as zero times it, from a token to earlier ones of its chunk.  Chunks with a value that
-// is not finite are marked, and an entry's head is left to delta_rule_kernel from its first marked chunk on.
+// is not finite, or so large that sums of them may not be (DC_LARGEST; a decay above one, which grows), are marked, and an entry's head is left to delta_rule_kernel from its first marked chunk on.
 #include "zi_common.h"
 #include "zi_delta.h"
 #include <type_traits>
@@ -36,6 +36,7 @@ typedef __attribute__((ext_vector_type(4))) float dc_f32x4_t;
 
 #define DC_TOKS DELTA_CHUNK
 #define DC_LD (DC_TOKS + 4)
+#define DC_LARGEST 0x1p60f        // (keys are unit vectors, T's entries at most one: sums of a chunk's values stay far from infinity)
 
 __device__ __forceinline__ dc_f32x4_t dc_mfma(dc_f32x4_t a, dc_f32x4_t b, dc_f32x4_t c) {
 #pragma unroll
@@ -120,7 +121,7 @@ delta_chunk_kernel(float* __restrict__ ws, int32_t* __restrict__ marks, const fl
     bool bad = false;
     auto check = [&](const dc_f32x4_t& x) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) bad |= !(fabsf(x[j]) < INFINITY);
+        for (int j = 0; j < 4; ++j) bad |= !(fabsf(x[j]) < DC_LARGEST);
     };
     // The blocks of K K^T (wavefronts 0 .. 3) and Q K^T (4 .. 7) on and below the diagonal, a row of blocks a wavefront, the long
     // rows of one beside the short ones of the other on a SIMD.  Queries go straight into registers (rows past the end repeat
@@ -144,7 +145,7 @@ delta_chunk_kernel(float* __restrict__ ws, int32_t* __restrict__ marks, const fl
         const float* row = beta_g + (int64_t)(t0 + (tid < cnt ? tid : 0)) * 2 * heads + h;
         bs[tid] = tid < cnt ? row[0] : 0.f;
         gs[tid] = tid < cnt ? row[heads] : 1.f;
-        bad |= !(fabsf(bs[tid]) < INFINITY) || !(fabsf(gs[tid]) < INFINITY);
+        bad |= !(fabsf(bs[tid]) < DC_LARGEST) || !(fabsf(gs[tid]) <= 1.f);
     }
     __syncthreads();
     // r_ij for i >= j: a thread has column j and 8 rows i0 ..; what comes before them is the rest of j's own 8, then whole 8s
