@@ -24,6 +24,7 @@ typedef __attribute__((ext_vector_type(16))) float g32_f32x16_t;
 typedef __attribute__((ext_vector_type(4))) float g32_f32x4_t;
 typedef __attribute__((ext_vector_type(4))) unsigned g32_u32x4_t;
 
+#define G32_WAVES 4         // wavefronts of a workgroup, 32 weight rows each
 #define G32_KB 64           // values of k a block
 #define G32_ROW 64          // LDS row stride in elements (128 bytes, 8 pieces of 16 bytes)
 #define G32_MODE_PLAIN 0
@@ -39,22 +40,22 @@ __device__ __forceinline__ g32_u32x4_t g32_keep(g32_u32x4_t v, bool keep) { retu
 // where the 16-byte piece c of LDS row r lies, in elements from the tile's start
 __device__ __forceinline__ int g32_at(int r, int c) { return r * G32_ROW + ((c ^ ((r >> 1) & 7)) << 3); }
 
-template <int MT, int WAVES, int RING>
-__global__ void __launch_bounds__(WAVES* ZI_WAVE)
+template <int MT>
+__global__ void __launch_bounds__(G32_WAVES* ZI_WAVE)
 gemm_rows32_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* __restrict__ x,
                    const zi_bf16* __restrict__ w, const zi_bf16* __restrict__ bias, int M, int N, int K, int64_t ldx,
                    int64_t ldw, int64_t ldo, int kb_per_split, int vec_out) {
-    constexpr int THREADS = WAVES * ZI_WAVE;
+    constexpr int THREADS = G32_WAVES * ZI_WAVE, RING = 4;      // (a wavefront a SIMD, all 512 registers its own, keeps four blocks of weights in flight)
     constexpr int XP = (MT * 32 * 8 + THREADS - 1) / THREADS;      // pieces of a block's x slice a thread stages
     __shared__ __attribute__((aligned(16))) uint16_t xs[2][MT * 32 * G32_ROW];
-    __shared__ __attribute__((aligned(16))) uint16_t wt[WAVES][32 * G32_ROW];
+    __shared__ __attribute__((aligned(16))) uint16_t wt[G32_WAVES][32 * G32_ROW];
     const int tid = threadIdx.x, lane = tid & (ZI_WAVE - 1), wave = tid / ZI_WAVE;
     const int r32 = lane & 31, kh = lane >> 5;        // operand row, and which 8 of a k-step's 16 values
     const int split = blockIdx.y;
     const int kb_total = (K + G32_KB - 1) / G32_KB;
     const int kb_lo = split * kb_per_split;
     const int kb_hi = (kb_lo + kb_per_split < kb_total) ? kb_lo + kb_per_split : kb_total;
-    const int n0 = (blockIdx.x * WAVES + wave) * 32;
+    const int n0 = (blockIdx.x * G32_WAVES + wave) * 32;
     // weights: instruction q takes rows q * 8 + lane / 8, 16-byte piece lane % 8 of the block
     const int wr = lane >> 3, wc = lane & 7;
     const zi_bf16* wrow[4];
@@ -146,12 +147,12 @@ gemm_rows32_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16*
         for (int b = 0; b < RING - 1; ++b)
             if (kb0 + b < kb_hi) step(b, kb0 + b, false);
     } else {
-        static_assert(RING >= 2 && RING <= 4, "one ending per residue");
+        static_assert(RING == 4, "one ending per residue");
         switch (left) {
             case 0: ending(std::integral_constant<int, 0>{}, kb0); break;
             case 1: ending(std::integral_constant<int, 1>{}, kb0); break;
-            case 2: if (RING > 2) ending(std::integral_constant<int, 2>{}, kb0); break;
-            default: if (RING > 3) ending(std::integral_constant<int, 3>{}, kb0); break;
+            case 2: ending(std::integral_constant<int, 2>{}, kb0); break;
+            default: ending(std::integral_constant<int, 3>{}, kb0); break;
         }
     }
 
@@ -228,50 +229,42 @@ gemm_rows32_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16*
     }
 }
 
-// How the product with a weight matrix [N, K] is cut for this kernel: wavefronts a workgroup (32 weight rows
-// each; four, as the sums of so many rows leave a wavefront registers enough only when a SIMD holds one), splits of k
-// over workgroups (at most 16) and blocks of 64 per split; a function of N and K.  As in zi_gemm_mid_plan what
-// counts is the most work any compute unit gets when workgroups are dealt out in turn; `whole` forbids a split
-// (the SwiGLU epilogue needs whole sums).
-void zi_gemm_rows32_plan(int N, int K, int whole, int* splits, int* kb_per_split, int* waves) {
-    const int tiles = (N + 31) / 32;
+// How the product with a weight matrix [N, K] is cut for this kernel (workgroups of four wavefronts, as the sums of so many rows
+// leave a wavefront registers enough only when a SIMD holds one): splits of k over workgroups (at most 16) and blocks of 64 per
+// split; a function of N and K.  As in zi_gemm_mid_plan what counts is the most work any compute unit gets when workgroups are
+// dealt out in turn; `whole` forbids a split (the SwiGLU epilogue needs whole sums).
+void zi_gemm_rows32_plan(int N, int K, int whole, int* splits, int* kb_per_split) {
+    const int groups = ((N + 31) / 32 + G32_WAVES - 1) / G32_WAVES;
     const int kb_total = (K + G32_KB - 1) / G32_KB;
     const int cus = zi_compute_units();
     int64_t best_cost = -1;
-    int best_s = 1, best_w = 4, best_per = kb_total;
-    {
-        const int w = 4, groups = (tiles + w - 1) / w;
-        for (int s0 = 1; s0 <= (whole ? 1 : 16) && s0 <= (kb_total > 1 ? kb_total / 2 : 1); ++s0) {
-            const int per = (kb_total + s0 - 1) / s0;
-            const int s = (kb_total + per - 1) / per;
-            if (s != s0) continue;
-            const int64_t wgs = (int64_t)groups * s;
-            const int64_t rounds = (wgs + cus - 1) / cus;
-            const int64_t cost = rounds * ((int64_t)w * per + 16);
-            if (best_cost < 0 || cost < best_cost || (cost == best_cost && (s < best_s || (s == best_s && w > best_w)))) {
-                best_cost = cost; best_s = s; best_w = w; best_per = per;
-            }
+    *splits = 1;
+    *kb_per_split = kb_total;
+    for (int s0 = 1; s0 <= (whole ? 1 : 16) && s0 <= (kb_total > 1 ? kb_total / 2 : 1); ++s0) {
+        const int per = (kb_total + s0 - 1) / s0;
+        const int s = (kb_total + per - 1) / per;
+        if (s != s0) continue;
+        const int64_t rounds = ((int64_t)groups * s + cus - 1) / cus;
+        const int64_t cost = rounds * ((int64_t)G32_WAVES * per + 16);
+        if (best_cost < 0 || cost < best_cost) {        // (of equals the fewest splits)
+            best_cost = cost;
+            *splits = s;
+            *kb_per_split = per;
         }
     }
-    *splits = best_s;
-    *kb_per_split = best_per;
-    *waves = best_w;
 }
 
 // The launch; the checks are the caller's (zi_gemm_skinny).  M is 129 .. 256.
 int zi_gemm_rows32_launch(void* out, int out_f32, int mode, const zi_bf16* x, const zi_bf16* w, const zi_bf16* bias, int M,
                           int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int vec_out, float limit, hipStream_t stream) {
     (void)limit;      // (these products have no clamped epilogue)
-    int splits, per, waves;
-    zi_gemm_rows32_plan(N, K, mode == G32_MODE_SWIGLU, &splits, &per, &waves);
-    const int tiles = (N + 31) / 32;
-    const dim3 grid((tiles + waves - 1) / waves, splits);
-    const int mt = (M + 31) / 32;
-    // (a wavefront a SIMD, all 512 registers its own, keeps four blocks of weights in flight)
-#define ZI_G32(MT)                                                                                                  \
-    gemm_rows32_kernel<MT, 4, 4><<<grid, 4 * ZI_WAVE, 0, stream>>>(out, mode, out_f32, x, w, bias, M, N, K, ldx, ldw, \
-                                                                  ldo, per, vec_out)
-    switch (mt) {
+    int splits, per;
+    zi_gemm_rows32_plan(N, K, mode == G32_MODE_SWIGLU, &splits, &per);
+    const dim3 grid(((N + 31) / 32 + G32_WAVES - 1) / G32_WAVES, splits);
+#define ZI_G32(MT)                                                                                                           \
+    gemm_rows32_kernel<MT><<<grid, G32_WAVES * ZI_WAVE, 0, stream>>>(out, mode, out_f32, x, w, bias, M, N, K, ldx, ldw, ldo, \
+                                                                     per, vec_out)
+    switch ((M + 31) / 32) {
         case 5: ZI_G32(5); break;
         case 6: ZI_G32(6); break;
         case 7: ZI_G32(7); break;

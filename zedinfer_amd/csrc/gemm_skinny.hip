@@ -68,7 +68,7 @@ int64_t zi_gemm_mid_plan(int N, int K, int whole, int* splits, int* kb_per_split
 int zi_gemm_mid_launch(void* out, int out_f32, int mode, const zi_bf16* x, const zi_bf16* w, const zi_bf16* bias, int M,
                        int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int vec_out, float limit, hipStream_t stream);
 
-void zi_gemm_rows32_plan(int N, int K, int whole, int* splits, int* kb_per_split, int* waves);
+void zi_gemm_rows32_plan(int N, int K, int whole, int* splits, int* kb_per_split);
 int zi_gemm_rows32_launch(void* out, int out_f32, int mode, const zi_bf16* x, const zi_bf16* w, const zi_bf16* bias, int M,
                           int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int vec_out, float limit, hipStream_t stream);
 
@@ -78,7 +78,7 @@ static bool sk_rows32(int M) { return M > SK_MID_MAX_ROWS; }
 // of which of the two kernels the rows go to (up to 128, or more).
 extern "C" int zi_gemm_skinny_splits(int M, int N, int K) {
     int s, per, waves;
-    if (sk_rows32(M)) zi_gemm_rows32_plan(N, K, 0, &s, &per, &waves);
+    if (sk_rows32(M)) zi_gemm_rows32_plan(N, K, 0, &s, &per);
     else zi_gemm_mid_plan(N, K, 0, &s, &per, &waves);
     return s;
 }
@@ -135,7 +135,7 @@ extern "C" int zi_gemm_skinny_act(void* out, int out_dt, int mode, const void* x
     ZI_REQUIRE(((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0, "gemm_skinny: x and w must be 16-byte aligned");
     int splits, per, waves;
     const bool rows32 = sk_rows32(M);
-    if (rows32) zi_gemm_rows32_plan(N, K, mode == SK_MODE_SWIGLU, &splits, &per, &waves);
+    if (rows32) zi_gemm_rows32_plan(N, K, mode == SK_MODE_SWIGLU, &splits, &per);
     else zi_gemm_mid_plan(N, K, mode >= SK_MODE_ACT || (mode == SK_MODE_SWIGLU && M > 64), &splits, &per, &waves);       // (whole from 65 rows on)
     void* dst = out;
     int kmode = mode;

@@ -340,9 +340,9 @@ __device__ __forceinline__ void moe_to_lds(const zi_bf16* from, moe_u32x4_t* to)
 #endif
 }
 template <int AUX>
-__device__ __forceinline__ void moe_to_lds(__amdgpu_buffer_rsrc_t from, moe_u32x4_t* to, int lane_at, int at) {
+__device__ __forceinline__ void moe_to_lds(__amdgpu_buffer_rsrc_t from, moe_u32x4_t* to, int lane_at) {
 #ifdef __HIP_DEVICE_COMPILE__
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, to, 16, lane_at, at, 0, AUX);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, to, 16, lane_at, 0, 0, AUX);
 #endif
 }
 
@@ -354,7 +354,8 @@ moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restr
     constexpr int XI = 2 * RT, WI = 8 * CT, XW = (XI + 3) / 4, WW = WI / 4, PW = XW + WW;      // loads of a step; a wavefront's share
     constexpr int PIECES = (4 * XW + WI) * ZI_WAVE;
     // (arrays of their own, so that the compiler can tell a buffer that is read from those that loads are on their way to)
-    __shared__ __attribute__((aligned(16))) moe_u32x4_t s0[PIECES], s1[PIECES], s2[ST > 2 ? PIECES : 1], s3[ST > 3 ? PIECES : 1];
+    __shared__ __attribute__((aligned(16))) moe_u32x4_t s0[PIECES], s1[PIECES], s2[ST > 2 ? PIECES : 1];
+    static_assert(ST == 2 || ST == 3, "two or three buffers");
     const int blocks = (N + 64 * CT - 1) / (64 * CT), total = plan[0] * blocks, share = (total + MOE_XCDS - 1) / MOE_XCDS;
     const int at_share = blockIdx.x / MOE_XCDS, job = (int)(blockIdx.x % MOE_XCDS) * share + at_share;
     if (at_share >= share || job >= total) return;
@@ -392,7 +393,7 @@ moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restr
 #pragma unroll
         for (int i = 0; i < WW; ++i)
             moe_to_lds<RT == 1 ? 2 : 0>(wb, buf + (4 * XW + i * 4 + wave) * ZI_WAVE,
-                                        whole || k0 + wpiece[i] < K ? w_at[i] + k0 * 2 : rows_w * K * 2, 0);
+                                        whole || k0 + wpiece[i] < K ? w_at[i] + k0 * 2 : rows_w * K * 2);
     };
     moe_f32x4_t acc[RT][CT];
 #pragma unroll
@@ -406,7 +407,6 @@ moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restr
         __builtin_amdgcn_sched_barrier(0);
         const int after = steps - 1 - t;       // steps whose loads may still be on their way
         if (after >= ST - 2) moe_wait<(ST - 2) * PW>();
-        else if (ST > 3 && after == 1) moe_wait<PW>();
         else moe_wait<0>();
         __builtin_amdgcn_s_barrier();          // all wavefronts' loads of the step are there, and all are done with `free`
         asm volatile("" ::: "memory");
@@ -440,21 +440,14 @@ moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restr
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (ST > 2) if (steps > 1) issue(s1, 1);
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (ST > 3) if (steps > 2) issue(s2, 2);
-    __builtin_amdgcn_sched_barrier(0);
     for (int t = 0; t < steps; t += ST) {
         if constexpr (ST == 2) {
             step(s0, s1, t);
             step(s1, s0, t + 1);
-        } else if constexpr (ST == 3) {
+        } else {
             step(s0, s2, t);
             step(s1, s0, t + 1);
             step(s2, s1, t + 2);
-        } else {
-            step(s0, s3, t);
-            step(s1, s0, t + 1);
-            step(s2, s1, t + 2);
-            step(s3, s2, t + 3);
         }
     }
     // a lane holds four consecutive columns of a row: one store of 16 (float32) or 8 bytes (bfloat16) where the rows
