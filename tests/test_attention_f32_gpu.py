@@ -152,3 +152,30 @@ def test_what_lies_in_cells_that_are_not_seen_changes_no_bit(d):
     assert bool(torch.isnan(bad[:, :, 3]).all()) and bool(torch.isinf(bad[1, :, 4]).all())
     rest = [i for i in range(d) if i not in (3, 4)]
     assert torch.equal(bad[:, :, rest], want[35:37].view(2, nh, d)[:, 2:][:, :, rest])
+
+
+@pytest.mark.parametrize("nh,nkv,d", [(40, 1, 32), (34, 2, 48), (17, 1, 128)])
+def test_groups_of_more_than_16_heads(nh, nkv, d):
+    """Decoded tokens of such a group are several workgroups, each of up to 16 of its heads: the same bits as in tiles of tokens."""
+    from zedinfer_amd import ops
+    g = torch.Generator().manual_seed(nh)
+    entries = [(30, 1), (0, 1), (64, 3), (5, 1), (15, 20)]
+    kc, vc, table, ks, vs = paged([a + b for a, b in entries], nkv, d, 16, g)
+    seqs = [s for s, (a, b) in enumerate(entries) for _ in range(b)]
+    poss = [a + j for a, b in entries for j in range(b)]
+    q = torch.randn(len(seqs), nh * d, generator=g)
+    args = (kc, vc, torch.tensor(seqs, dtype=torch.int32).cuda(), torch.tensor(poss, dtype=torch.int32).cuda(), table, nh, nkv, d, 0.2)
+    got = ops.attention(q.cuda(), *args, decoded=True)
+    assert float((got.cpu().double() - reference(q, ks, vs, seqs, poss, nh, nkv, d, 0.2, 0, None)).abs().max()) <= 2e-5
+    every = torch.arange(len(seqs), dtype=torch.int32).cuda()
+    assert torch.equal(ops.attention(q.cuda(), *args, tok_index=every), got)
+
+
+def test_which_tokens_are_taken_one_by_one():
+    """Tokens of 16 and more a sequence in tiles, single tokens one by one, in between as measured."""
+    from zedinfer_amd import ops
+    for nh, nkv in ((12, 2), (16, 16), (40, 1), (1, 1)):
+        for E in (1, 8, 64):
+            assert ops.attention_f32_by_heads(E, E, nh, nkv) and not ops.attention_f32_by_heads(16 * E, E, nh, nkv)
+    assert ops.attention_f32_by_heads(100, 20, 12, 2) and ops.attention_f32_by_heads(192, 64, 12, 2)
+    assert ops.attention_f32_by_heads(128, 64, 16, 16) and not ops.attention_f32_by_heads(256, 64, 16, 16)

@@ -394,9 +394,9 @@ def test_linear_sums_of_129_to_256_rows(ops, N, K):
 @pytest.mark.parametrize("M", [65, 96, 128, 129, 200, 256])
 @pytest.mark.parametrize("I,K", [(8960, 1536), (1000, 200), (18944, 3584)])
 def test_linear_swiglu_of_65_to_256_rows(ops, M, I, K, monkeypatch):
-    """The same kernel with the SwiGLU epilogue (gate and up rows interleaved in blocks of 8), which the engine
-    does not take beyond 64 rows (the library's product and the activation's own launch are faster there): here
-    with the limit lifted, against float32."""
+    """The SwiGLU epilogue (gate and up rows interleaved in blocks of 8) of the kernel for 65 to 128 rows, which the engine takes
+    for the products at which it pays, and of the one for 129 to 256 rows, which it does not take (the library's product and
+    the activation's own launch are faster there): here with the limit lifted, against float32."""
     from zedinfer_amd.ops import functional
     from zedinfer_amd.parts.feed_forward import GATE_UP_BLOCK, interleave_rows
     monkeypatch.setattr(functional, "SWIGLU_MAX_ROWS", 256)
@@ -410,9 +410,14 @@ def test_linear_swiglu_of_65_to_256_rows(ops, M, I, K, monkeypatch):
     got = ops.linear_swiglu(x, w)
     assert tuple(got.shape) == (M, I)
     assert float((got.float() - want).abs().max()) <= 1e-2 * float(want.abs().max())
-    # rows do not depend on each other (from 65 rows on it is this kernel, whose sums run over k in one order)
-    if M - 3 > 64:
+    # rows do not depend on each other: fewer rows of the same kernel, or, of the fewest it takes, more
+    if M in (65, 129):
+        more = torch.cat([x, rnd(9, K, dtype=torch.bfloat16, seed=6)])
+        assert torch.equal(ops.linear_swiglu(more, w)[:M], got)
+    else:
         assert torch.equal(ops.linear_swiglu(x[:M - 3].contiguous(), w), got[:M - 3])
+    if M == 129:      # the two kernels' sums run over k in one order (k in steps of 32, whole sums under this epilogue)
+        assert torch.equal(ops.linear_swiglu(x[:126].contiguous(), w), got[:126])
 
 
 def test_linear_f32_row_does_not_depend_on_batch(ops):

@@ -41,11 +41,12 @@ attention_f32_kernel(float* __restrict__ out, const float* __restrict__ q, int64
     const int group = nh / nkv;
     // this lane's column: token t, head h
     const int at = by_heads ? blockIdx.x : blockIdx.x * AF_COLS + c;
-    const bool real = by_heads ? c < group : at < n;
+    const int slices = (group + AF_COLS - 1) / AF_COLS, in_group = by_heads ? blockIdx.y % slices * AF_COLS + c : 0;
+    const bool real = by_heads ? in_group < group : at < n;
     const int place = at < n ? at : n - 1;
     const int t = tok_index ? tok_index[place] : place;
-    const int h = by_heads ? blockIdx.y * group + (c < group ? c : 0) : blockIdx.y;
-    const int kvh = by_heads ? blockIdx.y : blockIdx.y / group;
+    const int kvh = by_heads ? blockIdx.y / slices : blockIdx.y / group;
+    const int h = by_heads ? kvh * group + (real ? in_group : 0) : blockIdx.y;
     const int p = tok_pos[t], seq = tok_seq[t];
     const int lo = (window > 0 && p - window + 1 > 0) ? p - window + 1 : 0;
     const af_f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
@@ -218,19 +219,32 @@ extern "C" int zi_attention_f32_supported(int nh, int nkv, int d, int page_size)
     return nkv > 0 && nh % nkv == 0 && d >= 16 && d <= 128 && d % 16 == 0 && page_size >= 16 && page_size % 16 == 0;
 }
 
-// `by_heads`: a workgroup takes the heads of one token's group (decoded tokens; groups of at most 16 heads), else 16 listed
-// tokens of one head.  The results are the same.
+// Whether n tokens of so many sequences are the faster taken by heads than in tiles of 16 tokens.  A tile does the sequences among
+// its tokens one after the other (on average 1 + 15 / (tokens a sequence) of them), while a token by heads is a workgroup for
+// every key/value head; a launch past one workgroup a compute unit takes so many times longer.  From 16 tokens a sequence on, tiles.
+// Measured, us, by heads against tiles: 12 heads, 2 key/value heads of 128, 20 sequences of 5 tokens 6.5 against 18, 64 of 3 tokens
+// after 30 14 against 33, 16 of 8 after 1,000 53 against 74; 16 heads of 32 that share nothing, 64 sequences of 2 tokens 14 against 20,
+// of 4 tokens 26 against 11 (tiles); 28 heads, 4 key/value heads, 20 sequences of 16 tokens 29 against 20 (tiles).
+extern "C" int zi_attention_f32_by_heads(int n, int sequences, int nh, int nkv) {
+    if (n < 1 || nkv < 1 || nh < nkv || n >= 16 * (int64_t)sequences) return 0;
+    const double units = zi_compute_units();
+    const double heads = (double)n * nkv * ((nh / nkv + AF_COLS - 1) / AF_COLS) / units, tiles = (double)((n + AF_COLS - 1) / AF_COLS) * nh / units;
+    return (heads > 1 ? heads : 1) <= (tiles > 1 ? tiles : 1) * (1 + 15. * sequences / n);
+}
+
+// `by_heads`: a workgroup takes up to 16 heads of one token's group (decoded tokens), else 16 listed tokens of one head.  The
+// results are the same.
 extern "C" int zi_attention_f32(void* out, const void* q, int n, int64_t ldq, int64_t ldo, const void* kcache, const void* vcache,
                                 const int32_t* tok_index, const int32_t* tok_seq, const int32_t* tok_pos, const int32_t* block_tables,
                                 int max_pages, int num_pages, int nh, int nkv, int d, int page_size, int window, float scale,
                                 const float* sinks, int by_heads, hipStream_t stream) {
     ZI_REQUIRE(n >= 0 && max_pages > 0 && num_pages > 0 && window >= 0, "attention: bad sizes");
     ZI_REQUIRE(zi_attention_f32_supported(nh, nkv, d, page_size), "attention: unsupported heads (%d, %d), head_dim %d or page size %d", nh, nkv, d, page_size);
-    ZI_REQUIRE(nh <= 65535 && (!by_heads || nh / nkv <= AF_COLS), "attention: too many heads (%d of %d)", nh, nkv);
+    ZI_REQUIRE(nh <= 65535, "attention: too many heads (%d)", nh);
     ZI_REQUIRE(ldq >= (int64_t)nh * d && ldo >= (int64_t)nh * d, "attention: row stride too small");
     ZI_REQUIRE(ldq % 4 == 0 && ((uintptr_t)q | (uintptr_t)kcache | (uintptr_t)vcache) % 16 == 0, "attention: rows must be 16-byte aligned");
     if (n == 0) return 0;
-    const dim3 grid(by_heads ? n : (n + AF_COLS - 1) / AF_COLS, by_heads ? nkv : nh);
+    const dim3 grid(by_heads ? n : (n + AF_COLS - 1) / AF_COLS, by_heads ? nkv * ((nh / nkv + AF_COLS - 1) / AF_COLS) : nh);
 #define ZI_AF(DT)                                                                                                                  \
     case DT:                                                                                                                       \
         attention_f32_kernel<DT><<<grid, AF_WAVES * ZI_WAVE, 0, stream>>>((float*)out, (const float*)q, ldq, ldo, (const float*)kcache, \

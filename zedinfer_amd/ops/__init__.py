@@ -5,7 +5,7 @@ then launches on torch's current stream.  The op-level names follow the
 reference's Python module (reference: python/bindings/zedinfer_ops.cpp:257-291:
 add, argmax, embedding, linear, rms_norm, rope, swiglu).
 """
-from .functional import (add, add_rms_norm, argmax, attention, attention_decode, attention_f32_supported, attention_decode_chunks,
+from .functional import (add, add_rms_norm, argmax, attention, attention_decode, attention_f32_by_heads, attention_f32_supported, attention_decode_chunks,
                          attention_decode_fused,
                          attention_decode_fused_supported, attention_decode_project,
                          attention_decode_project_splits, attention_decode_project_supported,

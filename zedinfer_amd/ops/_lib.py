@@ -30,6 +30,7 @@ _PROTOTYPES = {
     "zi_rope": [P, P, I, I, L, L, P, P, I, I, I, P],
     "zi_attention_f32": [P, P, I, L, L, P, P, P, P, P, P, I, I, I, I, I, I, I, F, P, I, P],
     "zi_attention_f32_supported": [I, I, I, I],
+    "zi_attention_f32_by_heads": [I, I, I, I],
     "zi_attention_generic": [P, P, I, I, L, L, P, P, P, P, P, P, I, I, I, I, I, I, I, F, P],
     "zi_attention_decode": [P, P, I, I, L, L, P, P, P, P, P, P, I, I, I, I, I, I, I, F, I, P, L, P],
     "zi_attention_decode_supported": [I, I, I, I, I],

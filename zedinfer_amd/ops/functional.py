@@ -377,15 +377,16 @@ def attention(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, tok_s
     [max(0, pos - window + 1), pos] (window 0: all of them).  With ``tok_index`` only the listed
     tokens are computed (the other rows of ``out`` are left alone).  ``sinks`` (float32 [nh]): the softmax of
     head h also counts exp(sinks[h]) in its denominator, a term with no key and no value.  ``decoded``: the tokens are
-    single tokens of their sequences, which the float32 kernel then takes a token a workgroup instead of 16 (the same
-    result).  Returns [n, nh*d]."""
+    few of each sequence, which the float32 kernel then takes a token a workgroup instead of 16 (the same result; without
+    a ``tok_index`` it goes by the rows of the block tables, ``attention_f32_by_heads``).  Returns [n, nh*d]."""
     out, n, count, ldq, ldo, pages, ps = _attention_args("attention", q, kcache, vcache, tok_seq, tok_pos,
                                                          block_tables, nh, nkv, d, tok_index, out)
     if attention_f32_supported(q, nh, nkv, d, ps) and kcache.data_ptr() % 16 == 0 and vcache.data_ptr() % 16 == 0:
+        by_heads = bool(decoded) or (tok_index is None and attention_f32_by_heads(count, block_tables.shape[0], nh, nkv))
         _lib.call("zi_attention_f32", _p(out), _p(q), count, ldq, ldo, _p(kcache), _p(vcache), _p(tok_index), _p(tok_seq),
                   _p(tok_pos), _p(block_tables), block_tables.shape[1], pages, nh, nkv, d, ps, int(window), float(scale),
                   _p(_sinks(sinks, nh, q, "attention")) if sinks is not None else c_void_p(0),
-                  int(bool(decoded) and nh // nkv <= 16), _stream())
+                  int(by_heads), _stream())
         return out
     args = (_p(out), _p(q), _code(q, "attention"), count, ldq, ldo, _p(kcache), _p(vcache),
             _p(tok_index), _p(tok_seq), _p(tok_pos), _p(block_tables), block_tables.shape[1], pages, nh, nkv, d,
@@ -402,6 +403,11 @@ def attention_f32_supported(q: torch.Tensor, nh: int, nkv: int, d: int, page_siz
     128, pages a multiple of 16 positions, 16-byte aligned rows."""
     return (q.dtype == torch.float32 and q.stride(0) % 4 == 0 and q.data_ptr() % 16 == 0
             and bool(_lib.load().zi_attention_f32_supported(int(nh), int(nkv), int(d), int(page_size))))
+
+
+def attention_f32_by_heads(tokens: int, sequences: int, nh: int, nkv: int) -> bool:
+    """Whether so many tokens of so many sequences are few enough a sequence for ``attention``'s ``decoded`` in float32."""
+    return bool(_lib.load().zi_attention_f32_by_heads(int(tokens), int(sequences), int(nh), int(nkv)))
 
 
 def _sinks(sinks: torch.Tensor, nh: int, q: torch.Tensor, what: str) -> torch.Tensor:

@@ -236,7 +236,7 @@ class Attention(Mixer):
                                      sinks=self.sinks, **extras)
             elif plain is ops.attention and ops.attention_f32_supported(q, self.nh, self.nkv, self.d, kc.shape[2]):
                 plain(q, *args, self.window, out=att, tok_index=plan.dev["short_idx"] if n_short < N else None,
-                      sinks=self.sinks, decoded=True)      # (and the portions below)
+                      sinks=self.sinks, decoded=self._few_each(batch, n_short, True))      # (and the portions below)
             else:
                 n_long = -1      # everything through the plain kernel
         if n_long < 0:
@@ -255,8 +255,17 @@ class Attention(Mixer):
                                       workspace=ws, tile=plan.sizes["tile"], alone=plan.sizes["alone"], sinks=self.sinks,
                                       **extras)
             else:
+                if plain is ops.attention:
+                    extras = {"decoded": self._few_each(batch, n_long, False)}
                 plain(q, *args, self.window, out=att, tok_index=plan.dev["long_idx"] if n_long < N else None,
                       sinks=self.sinks, **extras)
+
+    def _few_each(self, batch, tokens: int, short: bool) -> bool:
+        """Whether the ``tokens`` tokens of the step's short (long) entries are few enough an entry to be attended token by token in
+        float32 (a matter of speed alone)."""
+        if batch.host_len is None:
+            return short
+        return ops.attention_f32_by_heads(tokens, int(((batch.host_len <= SHORT_ENTRY) == short).sum()), self.nh, self.nkv)
 
     def prompt_reads_parts(self, dtype: torch.dtype, page_size: int) -> bool:
         """Whether the prompt kernel multiplies a map's part of a query and key row alone (else a query row is zero outside
