@@ -22,9 +22,8 @@
 // (token by token 1.8e-7) and the state 1.5e-7 (2.1e-7): the long sums are made of a sum for every 16 values.
 //
 // The two take DC_ROUND bytes' worth of chunks in turn, so that the workspace has a bound whatever the step: 148 KB a (chunk, head)
-// at those sizes, where a round is 75 chunks.  A round more costs its launches and the end of a chain: 8,192 tokens 397 us against
-// 387 in one round of 229 MB, 28 heads 531 against 527 (534 MB), eight prompts of 1,000 294 against 265; with half of DC_ROUND 414,
-// 575 and 329.
+// at those sizes, where a round is 151 chunks.  A round more costs its launches and the end of a chain (with rounds of 128 MB 28
+// heads took 531 us for 8,192 tokens, against 527 in one of 534 MB; 32 heads 189 for 2,000 against 165).
 //
 // A NaN or an infinity would pass, as zero times it, from a token to earlier ones of its chunk.  Chunks with a value that
 // is not finite, or so large that sums of them may not be (DC_LARGEST; a decay above one, which grows), are marked, and an entry's head is left to delta_rule_kernel from its first marked chunk on.
@@ -484,7 +483,7 @@ delta_chunk_walk_kernel(float* __restrict__ out, const float* __restrict__ ws, c
 #define DC_SHORTEST 64
 
 // Bytes of workspace that a round of chunks may take (marks apart).
-#define DC_ROUND (128 << 20)
+#define DC_ROUND (256 << 20)
 
 static int64_t dc_most_chunks(int n, int entries) { return n / DC_TOKS + (entries < n / DC_SHORTEST ? entries : n / DC_SHORTEST); }
 
