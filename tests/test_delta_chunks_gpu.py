@@ -199,3 +199,17 @@ def test_finite_values_whose_sums_are_not():
     got, _ = _run(ops, lens, q, k, v.clamp(-3, 3), beta, gate, state, True)
     plain, _ = _run(ops, lens, q, k, v.clamp(-3, 3), beta, gate, state, False)
     assert torch.equal(got, plain)
+
+
+def test_when_chunks_pay():
+    """A long entry in chunks, many of 64 tokens with few heads token by token, steps without a long entry without the launches."""
+    import numpy as np
+    from zedinfer_amd import ops
+    pay = lambda lens, *sizes: ops.delta_rule_chunks_pay(np.array(lens, dtype=np.int32), *sizes)  # noqa: E731
+    for sizes in ((12, 128, 128), (2, 128, 128), (32, 128, 128), (6, 64, 64), (16, 32, 64)):
+        assert pay([500], *sizes) and pay([1] * 31 + [500], *sizes) and pay([300] * 8, *sizes)
+        assert not pay([63], *sizes) and not pay([2] * 64, *sizes) and not pay([1] * 200, *sizes)
+    for sizes in ((2, 128, 128), (6, 64, 64), (16, 32, 64)):
+        assert not pay([64] * 32, *sizes) and not pay([64] * 128, *sizes)
+    assert pay([64] * 32, 12, 128, 128) and pay([100] * 20, 32, 128, 128) and not pay([64], 16, 32, 64)
+    assert not pay([2000], 4, 256, 256) and not pay([2000], 6, 48, 40)       # (no multiples of 16, more than 128)

@@ -493,6 +493,25 @@ static int64_t dc_round(int n, int entries, int heads, int dim, int vdim) {
     return fit < most ? fit : most;
 }
 
+extern "C" int64_t zi_delta_rule_workspace(int n, int entries, int heads, int dim, int vdim);
+
+// Whether a step whose entries of at least DC_SHORTEST tokens are `long_entries` with `long_tokens` tokens, the longest `longest`, is the
+// faster with them in chunks than token by token.  Token by token the longest entry's chain, or, where there are more wavefronts
+// than one (two from dim 64 down) a SIMD, all tokens' share of the chip; in chunks the chain of the longest entry's chunks and the
+// walk's workgroups, 40 a microsecond past the first 256.  (Constants from one MI355X; the chip is scaled by its units.)  Measured,
+// us, token by token against chunks: 12 heads of 128 x 128 one entry of 64 tokens 40 against 31, 32 of them 237 against 168, 20 of 100
+// 241 against 124; 2 heads one of 64 39 against 30, 32 of them 46 against 90, 20 of 100 65 against 67; 16 heads of 32 x 64 one of 64
+// 20.9 against 22.5, one of 100 30 against 23, 32 of 64 45 against 63; 6 heads of 64 x 64 32 of 64 35 against 49, 8 of 300 108 against 43.
+extern "C" int zi_delta_rule_chunks_pay(int long_tokens, int longest, int long_entries, int heads, int dim, int vdim) {
+    if (long_entries < 1 || longest < DC_SHORTEST || zi_delta_rule_workspace(long_tokens, long_entries, heads, dim, vdim) == 0) return 0;
+    const double chip = zi_compute_units() / 256.;
+    const double share = (double)long_tokens * heads * ((vdim + 7) / 8) / ((dim > 64 ? 1024. : 2048.) * chip);
+    const double tokens = (0.2 + 0.003 * dim) * (share > longest ? share : longest);
+    const double groups = (double)long_entries * ((heads + 7) / 8 * 8) * (vdim / 16) - 256. * chip;
+    const double chunks = 17. + 0.09 * dim + 0.018 * dim * ((longest - 1) / DC_TOKS) + (groups > 0 ? 0.025 * groups / chip : 0.);
+    return chunks < tokens;
+}
+
 // Floats of workspace with which zi_delta_rule_chunked takes n tokens of so many entries in chunks; 0: it would not, the
 // entries are too short, the head sizes no multiples of 16 or the heads too many for a round.
 extern "C" int64_t zi_delta_rule_workspace(int n, int entries, int heads, int dim, int vdim) {

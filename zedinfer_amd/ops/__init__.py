@@ -18,7 +18,7 @@ from .functional import (add, add_rms_norm, argmax, attention, attention_decode,
                          linear_transposed, linear_tune, reduce_sums, rms_norm, rope, rope_inv_freq,
                          rope_kv_store, rope_kv_store_sums, rope_table, sample, swiglu, swiglu_t,
                          DECODE_LAYER_SPIN_LIMIT, FEW_ROWS, SUMS_MAX_ROWS)
-from .mixing import (delta_conv_state, delta_prepare, delta_rule, delta_rule_step, delta_rule_steps, delta_rule_workspace, delta_state_floats, gated_act, gated_rms_norm,
+from .mixing import (delta_conv_state, delta_prepare, delta_rule, delta_rule_chunks_pay, delta_rule_step, delta_rule_steps, delta_rule_workspace, delta_state_floats, gated_act, gated_rms_norm,
                      latent_attention, latent_attention_cores, latent_attention_cores_plan,
                      latent_attention_cores_supported, latent_attention_cores_workspace, latent_inputs, latent_query, latent_query_cores, latent_store, latent_value, latent_value_gates,
                      moe_combine, moe_group, moe_linear,
@@ -51,7 +51,7 @@ __all__ = [
     "linear", "linear_choose", "linear_splits", "linear_sums", "linear_sums_supported", "linear_swiglu",
     "linear_swiglu_pays", "linear_swiglu_supported", "linear_transposed", "linear_tune", "reduce_sums", "rms_norm", "rope",
     "rope_inv_freq", "rope_kv_store", "rope_kv_store_sums", "rope_table", "sample", "swiglu", "swiglu_t",
-    "delta_conv_state", "delta_prepare", "delta_rule", "delta_rule_step", "delta_rule_steps", "delta_rule_workspace", "delta_state_floats", "gated_act", "gated_rms_norm",
+    "delta_conv_state", "delta_prepare", "delta_rule", "delta_rule_chunks_pay", "delta_rule_step", "delta_rule_steps", "delta_rule_workspace", "delta_state_floats", "gated_act", "gated_rms_norm",
     "latent_attention", "latent_attention_cores", "latent_attention_cores_plan", "latent_attention_cores_supported",
     "latent_attention_cores_workspace", "latent_query", "latent_store", "latent_value", "moe_combine", "moe_group", "moe_linear",
     "moe_max_tiles", "moe_route", "moe_tile_rows", "rope_pairs",

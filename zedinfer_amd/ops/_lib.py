@@ -90,6 +90,7 @@ _PROTOTYPES = {
     "zi_delta_rule": [P, P, P, P, P, L, P, P, P, I, I, I, I, I, P],
     "zi_delta_rule_step": [P, I, P, P, P, P, L, P, P, P, I, I, I, I, I, P, P, L, F, P],
     "zi_delta_rule_steps": [I, I, L],
+    "zi_delta_rule_chunks_pay": [I, I, I, I, I, I],
     "zi_delta_rule_chunked": [P, P, P, P, P, L, P, P, P, I, I, I, I, I, I, P, L, P],
     "zi_gated_rmsnorm": [P, I, P, P, I, P, L, I, I, I, F, P],
     "zi_moe_route": [P, P, P, P, I, I, I, F, P],

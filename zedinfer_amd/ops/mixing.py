@@ -403,6 +403,16 @@ def delta_rule_workspace(n: int, entries: int, heads: int, dim: int, vdim: int) 
     return int(_lib.load().zi_delta_rule_workspace(int(n), int(entries), int(heads), int(dim), int(vdim)))
 
 
+DELTA_LONG_ENTRY = 64      # tokens from which an entry can be done in chunks
+
+
+def delta_rule_chunks_pay(entry_lens, heads: int, dim: int, vdim: int) -> bool:
+    """Whether ``delta_rule`` is faster with a workspace for entries that bring these numbers of tokens (a numpy array)."""
+    lens = entry_lens[entry_lens >= DELTA_LONG_ENTRY]
+    return lens.size > 0 and bool(_lib.load().zi_delta_rule_chunks_pay(int(lens.sum()), int(lens.max()), int(lens.size), int(heads),
+                                                                       int(dim), int(vdim)))
+
+
 def delta_rule_steps(dim: int, vdim: int, state: torch.Tensor) -> bool:
     """Whether ``delta_rule_step`` takes heads of these sizes in rows of this state."""
     return state.data_ptr() % 16 == 0 and bool(_lib.load().zi_delta_rule_steps(int(dim), int(vdim), int(state.stride(0))))

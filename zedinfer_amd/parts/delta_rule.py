@@ -101,7 +101,9 @@ class GatedDeltaRule(Mixer):
             ops.delta_rule_step(qk, v, beta_g, state, *entries, nh, kvh, dim, vdim, self.norm, gate, self.eps, out=y)
         else:
             o = rt.buffer("delta_read", (n, nh * vdim), torch.float32)
-            need = 0 if one_order else ops.delta_rule_workspace(n, batch.entry_start.numel(), nh, dim, vdim)
+            need = 0
+            if not one_order and ops.delta_rule_chunks_pay(batch.host_len, nh, dim, vdim):
+                need = ops.delta_rule_workspace(n, batch.entry_start.numel(), nh, dim, vdim)
             ops.delta_rule(qk, v, beta_g, state, *entries, nh, kvh, dim, vdim, out=o,
                            workspace=rt.buffer("delta_chunks", (need,), torch.float32) if need else None)
             ops.gated_rms_norm(o, self.norm, gate, nh, vdim, self.eps, out=y)
