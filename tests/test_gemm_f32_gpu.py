@@ -59,3 +59,10 @@ def test_float32_products_too_large_for_a_launch():
     many = torch.zeros((1 << 26) + 9, 4, device="cuda")
     many[:, 0] = torch.arange(many.shape[0], device="cuda") % 1021
     assert torch.equal(ops.linear(torch.full((2, 4), 3.0, device="cuda"), many)[1], 3 * many[:, 0])
+
+
+# products of few columns: one round and two of 32-row workgroups, tiles of one group (K up to 128), of 64 x 64 (K up to 64)
+@pytest.mark.parametrize("M,N,K", [(9000, 4, 4), (1024, 256, 32), (1025, 256, 32), (4100, 70, 20), (513, 250, 64), (1100, 250, 64),
+                                   (520, 250, 68), (2070, 130, 100), (4000, 128, 128), (3000, 2060, 96), (520, 250, 132)])
+def test_float32_product_of_few_columns(M, N, K):
+    test_float32_product(M, N, K)

@@ -325,12 +325,17 @@ int zi_gemm_f32_launch(float* out, const float* x, const float* w, const float* 
     // would be two (448 rows: 148 against 158, 2,560 x 2,560 at 288 rows 48 against 53, 2,816 x 1,024 at 256 20.8 against 23.9, 6,144 x
     // 2,048 at 128 38 against 42: 6 to 16 % at 17 shapes); from six rounds of 64 x 64 tiles on those (17,920 x 1,536 at 448 rows 219
     // against 226 us, at 256 rows, 4.4 rounds, 141 against 133); else 32 x 64, in two halves up to three rounds (448
-    // rows, 2,048 x 1,536: 33 against 37; 1,024 rows, four rounds: 61 against 60).
+    // rows, 2,048 x 1,536: 33 against 37; 1,024 rows, four rounds: 61 against 60).  Up to K = 128 the second half of the runs is
+    // empty, so one group (4,000 rows, 128 x 128: 5.7 against 6.8 us); up to K = 64 a workgroup is little more than its start, so the
+    // larger tiles (9,000 rows, 64 x 16: 5.4 against 9.3, 256 x 64: 9.0 against 13.2), after 32 rows a workgroup up to two a unit
+    // (1,000 rows, 256 x 32: 4.1 against 5.3 us).
     const int64_t cus = zi_compute_units(), n16 = (N + 15) / 16, m32 = (M + 31) / 32;
     const int64_t t32 = m32 * ((N + 63) / 64), t96 = m32 * ((N + 95) / 96), t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
     if (M <= 8) ZI_GF_STREAM(1, true, 6);
     else if (M <= 16 || n16 * ((M + 15) / 16) <= cus) ZI_GF_STREAM(1, false, 4);
-    else if (M <= 32 || n16 * m32 <= cus) ZI_GF_STREAM(2, false, 3);
+    else if (M <= 32 || n16 * m32 <= (chunks <= 2 ? 2 : 1) * cus) ZI_GF_STREAM(2, false, 3);
+    else if (chunks <= 2) ZI_GF_TILE(64, 2, 1, 2);
+    else if (chunks <= GF_PARTS / 2 && t64 < 6 * cus) ZI_GF_TILE(32, 2, 1, 4);
     else if (t32 <= cus) ZI_GF_TILE(32, 2, 2, 4);
     else if (t96 <= cus) ZI_GF_TILE(32, 3, 2, 2);
     else if (t64 >= 6 * cus) ZI_GF_TILE(64, 2, 1, 2);
