@@ -66,3 +66,30 @@ def test_float32_products_too_large_for_a_launch():
                                    (520, 250, 68), (2070, 130, 100), (4000, 128, 128), (3000, 2060, 96), (520, 250, 132)])
 def test_float32_product_of_few_columns(M, N, K):
     test_float32_product(M, N, K)
+
+
+# the activation in the product's end: x held in registers for up to 8 and 16 rows (every number of chunks a kernel is made for, the
+# last group of weight rows not whole, groups for every place and more), each kind of tile, and what is left to two launches
+@pytest.mark.parametrize("M,I,K", [(1, 1030, 4), (8, 1500, 512), (3, 2050, 1000), (5, 1027, 1536), (8, 1100, 2048), (7, 1029, 3000), (8, 1050, 4096),
+                                   (9, 2070, 96), (16, 2053, 1024), (12, 2100, 1500), (13, 2049, 2048), (70, 1000, 60), (70, 5000, 60), (100, 3001, 100),
+                                   (200, 530, 1500), (300, 2050, 260), (450, 4480, 200), (8, 64, 260), (40, 100, 260), (8, 5000, 4100)])
+def test_float32_product_with_the_activation(M, I, K):
+    """The bits of the product and the activation one after the other, whatever rows ride along, and nothing written beside them."""
+    from zedinfer_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(M * 31 + I)
+    x, w = (torch.randn(s, generator=g, device="cuda") for s in ((M, K), (2 * I, K)))
+    two = ops.linear(x, w)
+    # (alone, a row's product is the same bits, test_float32_product)
+    ref = two[:, :I].double()
+    ref = two[:, I:].double() * ref / (1 + torch.exp(-ref))
+    want = ops.swiglu(two[:, :I], two[:, I:])
+    assert bool(((want.double() - ref).abs() <= 1e-6 * ref.abs() + 1e-30).all())
+    if not ops.linear_swiglu_halves_supported(x, w):
+        assert (M, I) in ((70, 1000), (8, 64), (40, 100), (8, 5000))
+        return
+    wide = torch.zeros((M, I + 6), device="cuda")
+    ops.linear_swiglu_halves(x, w, out=wide[:, 3:I + 3])
+    assert torch.equal(wide[:, 3:I + 3], want) and not wide[:, :3].any() and not wide[:, I + 3:].any()
+    apart = torch.full((M, K + 8), float("nan"), device="cuda")
+    apart[:, 4:K + 4] = x
+    assert torch.equal(ops.linear_swiglu_halves(apart[:, 4:K + 4], w), want)

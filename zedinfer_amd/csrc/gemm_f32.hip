@@ -22,7 +22,8 @@
 // Measured, weights from memory, against the plain kernel (gemm_generic.hip: a chain of multiply-adds an output, scalar
 // loads), us, launch included: 8 rows 2,048 x 1,536 (N x K) 165 to 9; 1,536 x 8,960 914 to 19; 17,920 x 1,536 212 to 32 (3.5
 // TB/s); 151,936 x 1,536 761 to 250 (3.7 TB/s; one row 190, 4.9 TB/s).  448 rows: 2,048 x 1,536 189 to 33, 1,536 x 8,960
-// 1,050 to 147 (84 TFLOP/s), 17,920 x 1,536 975 to 219 (113 TFLOP/s).
+// 1,050 to 147 (84 TFLOP/s), 17,920 x 1,536 975 to 219 (113 TFLOP/s).  The gate/up product with the activation in its end against the
+// two launches: 448 rows of 17,920 x 1,536 233 to 220, 1,024 rows 502 to 486, 256 rows 153 to 144.
 #include "zi_common.h"
 
 typedef __attribute__((ext_vector_type(4))) float gf_f32x4_t;
@@ -30,6 +31,7 @@ typedef __attribute__((ext_vector_type(4))) unsigned gf_u32x4_t;
 
 #define GF_PARTS 8           // runs of k; the wavefronts of the stream kernel
 #define GF_KB 32             // k of a chunk
+#define GF_HELD_CHUNKS 16    // chunks of a run that a wavefront can hold of 8 rows of x beside as many of weights (256 registers)
 #define GF_OUT 0x7fffffff    // an offset past the end of every buffer: the load gives zeros and fetches nothing
 
 union gf_pack {
@@ -63,6 +65,9 @@ __device__ __forceinline__ void gf_store4(float* __restrict__ out, const float* 
             if (n + e < N) out[n + e] = s[e];
     }
 }
+
+// up * silu(gate), the arithmetic of the activation's own kernel (elementwise.hip).
+__device__ __forceinline__ float gf_gate(float gate, float up) { return up * (gate / (1.f + expf(-gate))); }
 
 // PAIR: 8 weight rows and up to 8 rows of x; else 16 weight rows and up to 16 * MT rows of x a workgroup.  RING chunks are
 // on their way while one is worked on.
@@ -150,9 +155,106 @@ gemm_f32_stream_kernel(float* __restrict__ out, const float* __restrict__ x, con
     }
 }
 
+// The same for up to 16 rows of x and more groups of weight rows than there are compute units: a workgroup keeps its wavefronts' runs
+// of x in registers (PER chunks a wavefront, at most) and walks over groups of 8 (PAIR) or 16 weight rows, gridDim.x apart.  As
+// soon as a chunk of weights has been used, its registers are filled with the same chunk of the next group: PER chunks are always
+// on their way, x passes the loads once a workgroup instead of once a group, as many bytes again as the weights' for 8 rows, and a
+// workgroup's start and end come once.  The eight runs' sums meet in one of two LDS buffers, so a group costs one barrier, which
+// does not wait for loads; the wavefronts take the adding and storing in turn.  GATED: a group is as many gate rows as up rows (row
+// n and row N + n of w) and the outputs are up * silu(gate).
+//
+// Bound by the stream of the weights.  Measured against the stream kernel above (weights from memory, us, launch
+// included), 1 and 8 rows: 17,920 x 1,536 29.0 to 20.6 and 35.0 to 23.8 (4.6 TB/s), 151,936 x 1,536 206 to 143 and 261 to 163 (5.7), 37,888
+// x 3,584 115 to 88 and 151 to 90 (6.0), 3,000 x 512 6.1 to 3.8 and 6.6 to 4.4; 16 rows 17,920 x 1,536 37.7 to 25.3, 151,936 x 1,536
+// 264 to 177, 5,000 x 1,000 11.7 to 11.3.  With the activation 8 rows of 17,920 x 1,536 take 23.8 us, the product and the activation's
+// launch 37.3 before.
+template <bool PAIR, int PER, bool GATED>
+__global__ void __launch_bounds__(GF_PARTS* ZI_WAVE, (PAIR ? 1 : 2) * PER <= 8 ? 4 : 2)
+gemm_f32_held_kernel(float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
+                     int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int per, int vec_out, int groups) {
+    constexpr int NR = PAIR ? 8 : 16, NC = GATED ? NR / 2 : NR, H = PAIR ? 1 : 2;
+    __shared__ __attribute__((aligned(16))) gf_f32x4_t part[2][GF_PARTS][ZI_WAVE];
+    const int lane = threadIdx.x & (ZI_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / ZI_WAVE);
+    const int r = lane & 15, g = lane >> 4, row = PAIR ? r & 7 : r;
+    const int chunks = (K + GF_KB - 1) / GF_KB, c0 = wave * per;
+    const int mine = chunks - c0 < per ? chunks - c0 : per;       // chunks of this wavefront's run (none or fewer at the end of k)
+    const int k0 = c0 * (GF_KB * 4) + (PAIR ? (r >> 3) * 64 : 0) + g * 16;      // the first byte of a row that this lane loads
+    const __amdgpu_buffer_rsrc_t xb = gf_rows(x, ldx, M, K);
+    const int x_row = row < M ? (int)(row * ldx * 4) : GF_OUT;
+    const int w_row = (int)((GATED && row >= NC ? N + row - NC : row) * ldw * 4);
+    // the weight rows of a group: what lies past the last one gives zeros (or, of a gate row past the last, an output that is not stored)
+    auto weights = [&](int group) {
+        const int64_t n0 = (int64_t)group * NC;
+        const int rows = group >= groups ? 0 : (GATED ? N : 0) + (int)(N - n0 < NC ? N - n0 : NC);
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(w + (rows ? n0 * ldw : 0)), 0,
+                                                 rows ? (int)(((int64_t)(rows - 1) * ldw + K) * 4) : 0, 0x00020000);
+    };
+    auto in = [&](int s, int h) { return s < mine && k0 + s * (GF_KB * 4) + h * 64 < K * 4; };
+    gf_f32x4_t xr[PER][H], wr[PER][H];
+    __amdgpu_buffer_rsrc_t wb = weights(blockIdx.x);
+    auto fetch = [&](const int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int h = 0; h < H; ++h)
+            wr[s][h] = gf_load<PAIR ? 2 : 0>(wb, in(s, h) ? w_row + k0 + s * (GF_KB * 4) + h * 64 : GF_OUT);
+    };
+#pragma unroll
+    for (int s = 0; s < PER; ++s) {
+#pragma unroll
+        for (int h = 0; h < H; ++h)
+            xr[s][h] = gf_load<0>(xb, in(s, h) && x_row != GF_OUT ? x_row + k0 + s * (GF_KB * 4) + h * 64 : GF_OUT);
+        fetch(s);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    int b = 0, turn = 0;
+    for (int group = blockIdx.x; group < groups; group += gridDim.x, b ^= 1, turn = (turn + 1) % GF_PARTS) {
+        wb = weights(group + (int)gridDim.x);
+        gf_f32x4_t acc[H];
+#pragma unroll
+        for (int h = 0; h < H; ++h) acc[h] = gf_f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < PER; ++s) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int h = 0; h < H; ++h) acc[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(wr[s][h][j], xr[s][h][j], acc[h], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(s);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        gf_f32x4_t sum = acc[0];
+        if (PAIR) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum[e] += __shfl(acc[0][e], (lane + 40) & 63, ZI_WAVE);
+        } else {
+            sum += acc[H - 1];
+        }
+        part[b][wave][lane] = sum;
+        // all sums are in LDS (and the buffer's reader of two groups ago is past the barrier of the last one); loads travel on
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        if (wave != turn) continue;
+        gf_f32x4_t s = part[b][0][lane], s2 = part[b][GF_PARTS / 2][lane];
+#pragma unroll
+        for (int p = 1; p < GF_PARTS / 2; ++p) {
+            s += part[b][p][lane];
+            s2 += part[b][GF_PARTS / 2 + p][lane];
+        }
+        s += s2;
+        if (GATED) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] = gf_gate(s[e], __shfl(s[e], lane + (PAIR ? 16 : 32), ZI_WAVE));
+        }
+        const int64_t n = (int64_t)group * NC + g * 4;
+        if (r < M && g * 4 < NC && n < N) gf_store4(out + (int64_t)r * ldo, bias, s, (int)n, N, vec_out);
+    }
+}
+
 // TM x 32 NT outputs a workgroup; GROUPS (1 or 2) groups of four wavefronts, each over half of the runs of k when there are
-// two; TM/2 x 16 NT outputs a wavefront.  RING chunks of operands are on their way in registers.
-template <int TM, int NT, int GROUPS, int RING>
+// two; TM/2 x 16 NT outputs a wavefront.  RING chunks of operands are on their way in registers.  GATED (NT = 2): of a wavefront's two
+// blocks of 16 weight rows one are gate rows and one the up rows of the same outputs (rows n and N + n of w), and TM x 32 outputs
+// up * silu(gate) are what the tile leaves.
+template <int TM, int NT, int GROUPS, int RING, bool GATED>
 __global__ void __launch_bounds__(256 * GROUPS)
 gemm_f32_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,
                      const float* __restrict__ bias, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int per, int vec_out,
@@ -162,12 +264,14 @@ gemm_f32_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const
     // the tiles that share weight rows follow each other on one XCD (workgroup i runs on XCD i mod 8)
     const int per_xcd = (tiles + 7) / 8, tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
     if (tile >= tiles) return;
-    const int m0 = (tile % m_tiles) * TM, n0 = (tile / m_tiles) * TN;
+    static_assert(!GATED || NT == 2, "a gate and an up block a wavefront");
+    constexpr int NC = GATED ? TN / 2 : TN;
+    const int m0 = (tile % m_tiles) * TM, n0 = (tile / m_tiles) * NC;
     const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x / ZI_WAVE), group = wave_all / 4, wave = wave_all & 3;
     const int tid = threadIdx.x & 255, lane = tid & (ZI_WAVE - 1);
     const int r = lane & 15, g = lane >> 4;
-    const int rows_w = N - n0 < TN ? N - n0 : TN, rows_x = M - m0 < TM ? M - m0 : TM;
-    const __amdgpu_buffer_rsrc_t wb = gf_rows(w + (int64_t)n0 * ldw, ldw, rows_w, K), xb = gf_rows(x + (int64_t)m0 * ldx, ldx, rows_x, K);
+    const int rows_w = N - n0 < NC ? N - n0 : NC, rows_x = M - m0 < TM ? M - m0 : TM;
+    const __amdgpu_buffer_rsrc_t wb = gf_rows(w + (int64_t)n0 * ldw, ldw, (GATED ? N : 0) + rows_w, K), xb = gf_rows(x + (int64_t)m0 * ldx, ldx, rows_x, K);
     // a thread loads piece tid % 8 (16 bytes) of rows tid / 8, + 32, ...; piece c of row q lies at place c xor (q / 2 mod 8)
     const int pc = tid & 7, pr = tid >> 3;
     const int place = pc ^ ((pr >> 1) & 7);            // the same for rows 32 apart
@@ -175,7 +279,11 @@ gemm_f32_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const
 #pragma unroll
     for (int p = 0; p < XP; ++p) x_row[p] = pr + 32 * p < rows_x ? (int)((pr + 32 * p) * ldx * 4) : GF_OUT;
 #pragma unroll
-    for (int p = 0; p < WP; ++p) w_row[p] = pr + 32 * p < rows_w ? (int)((pr + 32 * p) * ldw * 4) : GF_OUT;
+    for (int p = 0; p < WP; ++p) {
+        // GATED: row q of the tile is row q % 16 + 16 (q / 32) of the gate rows, of the up rows if q / 16 is odd
+        const int q = GATED ? 16 * p + (pr & 15) : pr + 32 * p;
+        w_row[p] = q < rows_w ? (int)((q + (GATED && (pr & 16) ? N : 0)) * ldw * 4) : GF_OUT;
+    }
     const int chunks = (K + GF_KB - 1) / GF_KB, half = per * (GF_PARTS / 2);
     const int c0 = group * half, c1 = GROUPS == 2 && c0 + half < chunks ? c0 + half : chunks;
     const int steps = GROUPS == 2 ? half : chunks;      // the same for both groups: they share the barriers
@@ -284,6 +392,15 @@ gemm_f32_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const
     for (int t = 0; t < MT; ++t) {
         const int m = m0 + wm + t * 16 + r;
         if (m >= M) continue;
+        if (GATED) {
+            const int n = n0 + wn / 2 + g * 4;
+            const gf_f32x4_t gate = first[t][0] + sum[t][0], up = first[t][NT - 1] + sum[t][NT - 1];
+            gf_f32x4_t s;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] = gf_gate(gate[e], up[e]);
+            if (n < N) gf_store4(out + (int64_t)m * ldo, nullptr, s, n, N, vec_out);
+            continue;
+        }
 #pragma unroll
         for (int u = 0; u < NT; ++u) {
             const int n = n0 + wn + u * 16 + g * 4;
@@ -299,49 +416,124 @@ bool zi_gemm_f32_takes(const void* x, const void* w, int N, int K, int64_t ldx, 
            N <= (1 << 25);
 }
 
-// The launch; the sizes are checked by the caller (zi_gemm_generic).
-int zi_gemm_f32_launch(float* out, const float* x, const float* w, const float* bias, int M, int N, int K, int64_t ldx, int64_t ldw,
-                       int64_t ldo, hipStream_t stream) {
+// The kernels a product can take; all give the same bits.
+enum gf_kernel { GF_PAIRS, GF_ROWS16, GF_ROWS32, GF_HELD_PAIRS, GF_HELD_ROWS16, GF_TILE_64, GF_TILE_32, GF_TILE_32_HALVES, GF_TILE_96_HALVES };
+
+// Which kernel M rows of x and N weight rows take is a matter of filling the compute units only.  Up to 16 rows a stream of the
+// weights, 8 or 16 of them a workgroup (one row of a 151,936-row head 190 in pairs, 233 us without), with x held in registers once
+// there are more such groups than units and k is not too long for it (see there).  9 to 16 rows go twice over groups of 8 weight rows
+// while those are one round (896 x 4,864, 16 rows: 12.2 against 20.1 us; 1,536 x 8,960 34.9 both ways; twelve chunks on their way
+// instead of six gained nothing, 21.4 against 20.9 us at 8 rows).  16 rows a workgroup while that gives no unit a
+// second workgroup (32 rows, 1,536 x 8,960: 34 against 52 us), 32 rows up to 32 rows and then while the same holds (64 rows:
+// 52 against 92 us for the tiles).  Beyond, tiles of 32 x 64 in two halves of k while they are one round of workgroups
+// (256 rows, 1,536 x 8,960: 96 us, one group 123, tiles of 64 x 64 194), of 32 x 96 where those make one round of what
+// would be two (448 rows: 148 against 158, 2,560 x 2,560 at 288 rows 48 against 53, 2,816 x 1,024 at 256 20.8 against 23.9, 6,144 x
+// 2,048 at 128 38 against 42: 6 to 16 % at 17 shapes); from six rounds of 64 x 64 tiles on those (17,920 x 1,536 at 448 rows 219
+// against 226 us, at 256 rows, 4.4 rounds, 141 against 133); else 32 x 64, in two halves up to three rounds (448
+// rows, 2,048 x 1,536: 33 against 37; 1,024 rows, four rounds: 61 against 60).  Up to K = 128 the second half of the runs is
+// empty, so one group (4,000 rows, 128 x 128: 5.7 against 6.8 us); up to K = 64 a workgroup is little more than its start, so the
+// larger tiles (9,000 rows, 64 x 16: 5.4 against 9.3, 256 x 64: 9.0 against 13.2), after 32 rows a workgroup up to two a unit
+// (1,000 rows, 256 x 32: 4.1 against 5.3 us).
+static gf_kernel gf_kernel_for(int M, int64_t N, int chunks, int per) {
+    const int64_t cus = zi_compute_units(), n16 = (N + 15) / 16, m32 = (M + 31) / 32;
+    const int64_t t32 = m32 * ((N + 63) / 64), t96 = m32 * ((N + 95) / 96), t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
+    if (M <= 8) return (N + 7) / 8 > cus && per <= GF_HELD_CHUNKS ? GF_HELD_PAIRS : GF_PAIRS;
+    if (M <= 16 && n16 > cus && per <= GF_HELD_CHUNKS / 2) return GF_HELD_ROWS16;
+    if (M <= 16) return (N + 7) / 8 <= cus ? GF_PAIRS : GF_ROWS16;
+    if (n16 * ((M + 15) / 16) <= cus) return GF_ROWS16;
+    if (M <= 32 || n16 * m32 <= (chunks <= 2 ? 2 : 1) * cus) return GF_ROWS32;
+    if (chunks <= 2) return GF_TILE_64;
+    if (chunks <= GF_PARTS / 2 && t64 < 6 * cus) return GF_TILE_32;
+    if (t32 <= cus) return GF_TILE_32_HALVES;
+    if (t96 <= cus) return GF_TILE_96_HALVES;
+    if (t64 >= 6 * cus) return GF_TILE_64;
+    return t32 <= 3 * cus ? GF_TILE_32_HALVES : GF_TILE_32;
+}
+
+template <bool GATED>
+static int gf_launch(float* out, const float* x, const float* w, const float* bias, int M, int N, int K, int64_t ldx, int64_t ldw,
+                     int64_t ldo, hipStream_t stream) {
     const int chunks = (K + GF_KB - 1) / GF_KB, per = (chunks + GF_PARTS - 1) / GF_PARTS;
     const int vec_out = ldo % 4 == 0 && (uintptr_t)out % 16 == 0;
 #define ZI_GF_STREAM(MT, PAIR, RING)                                                                                                     \
     gemm_f32_stream_kernel<MT, PAIR, RING><<<dim3((N + (PAIR ? 7 : 15)) / (PAIR ? 8 : 16), (M + (PAIR ? 8 : 16 * MT) - 1) / (PAIR ? 8 : 16 * MT)), \
                                              GF_PARTS * ZI_WAVE, 0, stream>>>(out, x, w, bias, M, N, K, ldx, ldw, ldo, per, vec_out)
+    // two workgroups a unit while a lane has registers for that (128), else one
+#define ZI_GF_HELD(PAIR, PER)                                                                                                            \
+    do {                                                                                                                                 \
+        const int nc = (PAIR ? 8 : 16) / (GATED ? 2 : 1), groups = (N + nc - 1) / nc;                                                        \
+        const int places = zi_compute_units() * ((PAIR ? 1 : 2) * PER <= 8 ? 2 : 1);                                                         \
+        gemm_f32_held_kernel<PAIR, PER, GATED><<<groups < places ? groups : places, GF_PARTS * ZI_WAVE, 0, stream>>>(                         \
+            out, x, w, bias, M, N, K, ldx, ldw, ldo, per, vec_out, groups);                                                               \
+    } while (0)
     // (rows in as many launches as 2^32 threads of one make necessary: a row's result does not depend on them)
 #define ZI_GF_TILE(TM, NT, G, R)                                                                                                              \
     do {                                                                                                                                  \
-        const int64_t nt = (N + 32 * NT - 1) / (32 * NT), most = ((1ll << 31) / (256 * G)) / nt * TM;                                              \
+        const int nc = 32 * NT / (GATED ? 2 : 1);                                                                                              \
+        const int64_t nt = (N + nc - 1) / nc, most = ((1ll << 31) / (256 * G)) / nt * TM;                                                      \
         for (int64_t m = 0; m < M; m += most) {                                                                                           \
             const int rows = (int)(M - m < most ? M - m : most), mt = (rows + TM - 1) / TM, tiles = (int)(mt * nt);                              \
-            gemm_f32_tile_kernel<TM, NT, G, R><<<(tiles + 7) / 8 * 8, 256 * G, 0, stream>>>(out + m * ldo, x + m * ldx, w, bias, rows, N, K, ldx, \
-                                                                                            ldw, ldo, per, vec_out, mt, tiles);               \
+            gemm_f32_tile_kernel<TM, NT, G, R, GATED><<<(tiles + 7) / 8 * 8, 256 * G, 0, stream>>>(out + m * ldo, x + m * ldx, w, bias, rows, N, \
+                                                                                                   K, ldx, ldw, ldo, per, vec_out, mt, tiles);  \
         }                                                                                                                                 \
     } while (0)
-    // Which kernel is a matter of filling the compute units only; all give the same bits.  Up to 8 rows the paired form of the
-    // stream (one row of a 151,936-row head 190 against 233 us); 16 rows a workgroup while that gives no unit a second
-    // workgroup (32 rows, 1,536 x 8,960: 34 against 52 us), 32 rows up to 32 rows and then while the same holds (64 rows:
-    // 52 against 92 us for the tiles).  Beyond, tiles of 32 x 64 in two halves of k while they are one round of workgroups
-    // (256 rows, 1,536 x 8,960: 96 us, one group 123, tiles of 64 x 64 194), of 32 x 96 where those make one round of what
-    // would be two (448 rows: 148 against 158, 2,560 x 2,560 at 288 rows 48 against 53, 2,816 x 1,024 at 256 20.8 against 23.9, 6,144 x
-    // 2,048 at 128 38 against 42: 6 to 16 % at 17 shapes); from six rounds of 64 x 64 tiles on those (17,920 x 1,536 at 448 rows 219
-    // against 226 us, at 256 rows, 4.4 rounds, 141 against 133); else 32 x 64, in two halves up to three rounds (448
-    // rows, 2,048 x 1,536: 33 against 37; 1,024 rows, four rounds: 61 against 60).  Up to K = 128 the second half of the runs is
-    // empty, so one group (4,000 rows, 128 x 128: 5.7 against 6.8 us); up to K = 64 a workgroup is little more than its start, so the
-    // larger tiles (9,000 rows, 64 x 16: 5.4 against 9.3, 256 x 64: 9.0 against 13.2), after 32 rows a workgroup up to two a unit
-    // (1,000 rows, 256 x 32: 4.1 against 5.3 us).
-    const int64_t cus = zi_compute_units(), n16 = (N + 15) / 16, m32 = (M + 31) / 32;
-    const int64_t t32 = m32 * ((N + 63) / 64), t96 = m32 * ((N + 95) / 96), t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
-    if (M <= 8) ZI_GF_STREAM(1, true, 6);
-    else if (M <= 16 || n16 * ((M + 15) / 16) <= cus) ZI_GF_STREAM(1, false, 4);
-    else if (M <= 32 || n16 * m32 <= (chunks <= 2 ? 2 : 1) * cus) ZI_GF_STREAM(2, false, 3);
-    else if (chunks <= 2) ZI_GF_TILE(64, 2, 1, 2);
-    else if (chunks <= GF_PARTS / 2 && t64 < 6 * cus) ZI_GF_TILE(32, 2, 1, 4);
-    else if (t32 <= cus) ZI_GF_TILE(32, 2, 2, 4);
-    else if (t96 <= cus) ZI_GF_TILE(32, 3, 2, 2);
-    else if (t64 >= 6 * cus) ZI_GF_TILE(64, 2, 1, 2);
-    else if (t32 <= 3 * cus) ZI_GF_TILE(32, 2, 2, 4);
-    else ZI_GF_TILE(32, 2, 1, 4);
+    switch (gf_kernel_for(M, (int64_t)N * (GATED ? 2 : 1), chunks, per)) {
+        case GF_HELD_PAIRS:
+            if (per <= 2) ZI_GF_HELD(true, 2);
+            else if (per <= 4) ZI_GF_HELD(true, 4);
+            else if (per <= 6) ZI_GF_HELD(true, 6);
+            else if (per <= 8) ZI_GF_HELD(true, 8);
+            else if (per <= 12) ZI_GF_HELD(true, 12);
+            else ZI_GF_HELD(true, 16);
+            break;
+        case GF_HELD_ROWS16:
+            if (per <= 2) ZI_GF_HELD(false, 2);
+            else if (per <= 4) ZI_GF_HELD(false, 4);
+            else if (per <= 6) ZI_GF_HELD(false, 6);
+            else ZI_GF_HELD(false, 8);
+            break;
+        case GF_TILE_64: ZI_GF_TILE(64, 2, 1, 2); break;
+        case GF_TILE_32: ZI_GF_TILE(32, 2, 1, 4); break;
+        case GF_TILE_32_HALVES: ZI_GF_TILE(32, 2, 2, 4); break;
+        default:
+            if constexpr (GATED) {
+                return zi_fail("gemm_f32: no gated kernel for %d rows of %d x %d", M, N, K);      // (zi_gemm_f32_swiglu_takes says so)
+            } else {
+                switch (gf_kernel_for(M, N, chunks, per)) {
+                    case GF_PAIRS: ZI_GF_STREAM(1, true, 6); break;
+                    case GF_ROWS16: ZI_GF_STREAM(1, false, 4); break;
+                    case GF_ROWS32: ZI_GF_STREAM(2, false, 3); break;
+                    default: ZI_GF_TILE(32, 3, 2, 2); break;
+                }
+            }
+    }
 #undef ZI_GF_STREAM
+#undef ZI_GF_HELD
 #undef ZI_GF_TILE
     return zi_check_launch("gemm_f32");
+}
+
+// The launch; the sizes are checked by the caller (zi_gemm_generic).
+int zi_gemm_f32_launch(float* out, const float* x, const float* w, const float* bias, int M, int N, int K, int64_t ldx, int64_t ldw,
+                       int64_t ldo, hipStream_t stream) {
+    return gf_launch<false>(out, x, w, bias, M, N, K, ldx, ldw, ldo, stream);
+}
+
+// Whether zi_gemm_f32_swiglu takes M rows of x and the [2 inter, K] weights: what the product's own kernels take, with the up rows within
+// 2^31 bytes of the gate rows they belong to, where the kernel that the product would take has the activation in its end.
+extern "C" int zi_gemm_f32_swiglu_takes(const void* x, const void* w, int M, int inter, int K, int64_t ldx, int64_t ldw) {
+    if (M < 1 || M > 65535 * 64 || inter < 1 || K < 1 || inter > (1 << 24) || ldx < K || ldw < K || !zi_gemm_f32_takes(x, w, 2 * inter, K, ldx, ldw)) return 0;
+    if (((int64_t)inter + 64) * ldw * 4 >= (1ll << 31) - 64) return 0;
+    const int chunks = (K + GF_KB - 1) / GF_KB, per = (chunks + GF_PARTS - 1) / GF_PARTS;
+    const gf_kernel k = gf_kernel_for(M, 2ll * inter, chunks, per);
+    return k == GF_HELD_PAIRS || k == GF_HELD_ROWS16 || k == GF_TILE_64 || k == GF_TILE_32 || k == GF_TILE_32_HALVES;
+}
+
+// out[M, inter] = up * silu(gate), gate and up the products of x with the first and the last inter rows of w: the bits of the product
+// and the activation one after the other.
+extern "C" int zi_gemm_f32_swiglu(float* out, const float* x, const float* w, int M, int inter, int K, int64_t ldx, int64_t ldw, int64_t ldo,
+                                  hipStream_t stream) {
+    ZI_REQUIRE(zi_gemm_f32_swiglu_takes(x, w, M, inter, K, ldx, ldw), "gemm_f32_swiglu: M=%d inter=%d K=%d is not taken", M, inter, K);
+    ZI_REQUIRE(ldo >= inter, "gemm_f32_swiglu: leading dimension too small");
+    return gf_launch<true>(out, x, w, nullptr, M, inter, K, ldx, ldw, ldo, stream);
 }

@@ -61,6 +61,8 @@ _PROTOTYPES = {
     "zi_attention_prefill_tile": [I, I],
     "zi_attention_prefill_chunk_keys": [],
     "zi_gemm_generic": [P, I, P, I, P, I, P, I, I, I, I, L, L, L, P],
+    "zi_gemm_f32_swiglu": [P, P, P, I, I, I, L, L, L, P],
+    "zi_gemm_f32_swiglu_takes": [P, P, I, I, I, L, L],
     "zi_gemm_skinny": [P, I, I, P, P, P, I, I, I, L, L, L, P, L, P],
     "zi_gemm_skinny_act": [P, I, I, P, P, P, I, I, I, L, L, L, P, L, F, P],
     "zi_clamped_glu_il8": [P, L, P, L, I, I, F, F, P],

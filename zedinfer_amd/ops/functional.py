@@ -1132,6 +1132,34 @@ def linear_swiglu(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Ten
     return out
 
 
+def linear_swiglu_halves_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether ``linear_swiglu_halves`` takes this product: float32 matrices on the GPU that the float32 kernels can load, and
+    rows whose kernel has the activation in its end (the kernel library says)."""
+    if not all(t.is_cuda and t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1 for t in (x, weight)):
+        return False
+    M, K = x.shape
+    if K != weight.shape[1] or weight.shape[0] % 2 or max(M, K, weight.shape[0]) >= 1 << 31 or min(M, K, weight.shape[0]) < 1:
+        return False
+    return bool(_lib.load().zi_gemm_f32_swiglu_takes(_p(x), _p(weight), M, weight.shape[0] // 2, K, x.stride(0), weight.stride(0)))
+
+
+def linear_swiglu_halves(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """up * silu(gate) of x . weight^T in one kernel, float32, for a weight [2I, K] of I gate rows and the I up rows; out [M, I].
+    The bits of ``linear`` and ``swiglu`` one after the other."""
+    _gpu("linear_swiglu_halves", x, weight, out)
+    if not linear_swiglu_halves_supported(x, weight):
+        raise ValueError("linear_swiglu_halves: float32 matrices with rows of whole 16-byte pieces are needed")
+    M, K = x.shape
+    inter = weight.shape[0] // 2
+    if out is None:
+        out = torch.empty((M, inter), dtype=torch.float32, device=x.device)
+    ldo, wo = _rows(out, "linear_swiglu_halves out")
+    if tuple(out.shape) != (M, inter) or out.dtype != torch.float32:
+        raise ValueError(f"linear_swiglu_halves: out must be float32 [{M}, {inter}]")
+    _lib.call("zi_gemm_f32_swiglu", _p(out), _p(x), _p(weight), M, inter, K, x.stride(0), weight.stride(0), ldo, _stream())
+    return out
+
+
 def linear_clamped_glu(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], limit: float,
                        out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """g sigmoid(1.702 g) (u + 1) with g = min(gate, limit), u = clamp(up, -limit, limit) of x . weight^T + bias in one

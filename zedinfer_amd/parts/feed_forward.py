@@ -142,6 +142,8 @@ class SwiGLU(FeedForward):
             ops.swiglu(sums, out=act, interleave=self.interleave)
         elif self.interleave == GATE_UP_BLOCK and x.dtype == torch.bfloat16:
             self._gate_up_many_rows(x, act)
+        elif not self.interleave and self.gate_up is not None and ops.linear_swiglu_halves_supported(x, self.gate_up):
+            ops.linear_swiglu_halves(x, self.gate_up, out=act)
         else:
             gu = self.rt.buffer("ffn_gate_up", (n, 2 * I))
             if self.gate_up is not None:
