@@ -179,3 +179,18 @@ def test_which_tokens_are_taken_one_by_one():
             assert ops.attention_f32_by_heads(E, E, nh, nkv) and not ops.attention_f32_by_heads(16 * E, E, nh, nkv)
     assert ops.attention_f32_by_heads(100, 20, 12, 2) and ops.attention_f32_by_heads(192, 64, 12, 2)
     assert ops.attention_f32_by_heads(128, 64, 16, 16) and not ops.attention_f32_by_heads(256, 64, 16, 16)
+
+
+@pytest.mark.parametrize("nh,nkv,d,n", [(12, 2, 128, 32), (12, 2, 128, 33), (8, 8, 64, 8), (8, 8, 64, 9), (4, 4, 64, 65), (6, 2, 112, 3)])
+def test_tokens_one_by_one_give_the_bits_of_tiles(nh, nkv, d, n):
+    """A token by heads, its dims shared by four workgroups (few workgroups, head sizes 64 and 128) or not, and in a tile of 16 tokens."""
+    from zedinfer_amd import ops
+    g = torch.Generator().manual_seed(n + d)
+    lens = [1 + 37 * i % 300 for i in range(n)]
+    kc, vc, table, _, _ = paged(lens, nkv, d, 16, g)
+    q = torch.randn(n, nh * d, generator=g).cuda()
+    seqs, poss = torch.arange(n, dtype=torch.int32).cuda(), torch.tensor([m - 1 for m in lens], dtype=torch.int32).cuda()
+    index = torch.arange(n, dtype=torch.int32).cuda()
+    args = (q, kc, vc, seqs, poss, table, nh, nkv, d, d ** -0.5)
+    one = ops.attention(*args, tok_index=index, decoded=True)
+    assert torch.equal(one, ops.attention(*args, tok_index=index, decoded=False)) and bool(torch.isfinite(one).all())

@@ -19,7 +19,7 @@
 //
 // Bound, for prompts, by the instruction's rate and the trips to the cache (16 queries share a pass over the keys); for
 // decoded tokens by the trips that follow each other, one a block and wavefront.  Measured against the plain kernel
-// (12 heads of 128, 2 key/value heads): a prompt of 450 tokens 585 to 39 us, 8 decoded tokens of 400 keys 176 to 16 us.
+// (12 heads of 128, 2 key/value heads): a prompt of 450 tokens 585 to 39 us, 8 decoded tokens of 400 keys 176 to 13 us.
 #include "zi_common.h"
 
 typedef __attribute__((ext_vector_type(4))) float af_f32x4_t;
@@ -27,14 +27,16 @@ typedef __attribute__((ext_vector_type(4))) float af_f32x4_t;
 #define AF_WAVES 8
 #define AF_COLS 16
 
-template <int DT>        // head size / 16
+// DT: head size / 16; DV: how many 16 dims of the values a workgroup makes, from blockIdx.z * DV on.
+template <int DT, int DV>
 __global__ void __launch_bounds__(AF_WAVES* ZI_WAVE)
 attention_f32_kernel(float* __restrict__ out, const float* __restrict__ q, int64_t ldq, int64_t ldo, const float* __restrict__ kcache,
                      const float* __restrict__ vcache, const int32_t* __restrict__ tok_index, const int32_t* __restrict__ tok_seq,
                      const int32_t* __restrict__ tok_pos, const int32_t* __restrict__ block_tables, int max_pages, int num_pages, int n,
                      int nh, int nkv, int page_size, int window, float scale, const float* __restrict__ sinks, int by_heads) {
     constexpr int D = DT * 16;
-    __shared__ __attribute__((aligned(16))) af_f32x4_t os[AF_WAVES][DT][ZI_WAVE];
+    const int d0 = DV == DT ? 0 : blockIdx.z * DV * 16;
+    __shared__ __attribute__((aligned(16))) af_f32x4_t os[AF_WAVES][DV][ZI_WAVE];
     __shared__ float ms[AF_WAVES][AF_COLS], ls[AF_WAVES][AF_COLS];
     const int lane = threadIdx.x & (ZI_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / ZI_WAVE);
     const int c = lane & 15, g = lane >> 4;
@@ -78,21 +80,21 @@ attention_f32_kernel(float* __restrict__ out, const float* __restrict__ q, int64
             return __builtin_amdgcn_readfirstlane(page < num_pages ? page : -1);
         };
         auto cell = [&](int page) -> int64_t { return ((int64_t)(page < 0 ? 0 : page) * nkv + kvh) * page_size * D; };
-        af_f32x4_t kr[DT], vr[DT];
+        af_f32x4_t kr[DT], vr[DV];
         auto fetch_k = [&](int b, int page) __attribute__((always_inline)) {
             const float* k = kcache + cell(page) + (int64_t)((b * 16) % page_size + c) * D + g * 4;
 #pragma unroll
             for (int i = 0; i < DT; ++i) kr[i] = *reinterpret_cast<const af_f32x4_t*>(k + i * 16);
         };
         auto fetch_v = [&](int b, int page) __attribute__((always_inline)) {
-            const float* v = vcache + cell(page) + (int64_t)c * page_size + (b * 16) % page_size + g * 4;
+            const float* v = vcache + cell(page) + (int64_t)(d0 + c) * page_size + (b * 16) % page_size + g * 4;
 #pragma unroll
-            for (int i = 0; i < DT; ++i) vr[i] = *reinterpret_cast<const af_f32x4_t*>(v + (int64_t)i * 16 * page_size);
+            for (int i = 0; i < DV; ++i) vr[i] = *reinterpret_cast<const af_f32x4_t*>(v + (int64_t)i * 16 * page_size);
         };
         float m = -INFINITY, l = 0.f;
-        af_f32x4_t acc[DT];
+        af_f32x4_t acc[DV];
 #pragma unroll
-        for (int i = 0; i < DT; ++i) acc[i] = zero;
+        for (int i = 0; i < DV; ++i) acc[i] = zero;
         int page = page_of(first), page_next = page_of(first + AF_WAVES);
         fetch_k(first <= last ? first : last, page);
         fetch_v(first <= last ? first : last, page);
@@ -134,28 +136,28 @@ attention_f32_kernel(float* __restrict__ out, const float* __restrict__ q, int64
             }
             l = l * corr + sum;
 #pragma unroll
-            for (int i = 0; i < DT; ++i) acc[i] *= corr;
+            for (int i = 0; i < DV; ++i) acc[i] *= corr;
             bool by_key = false;
             if (__ballot(mine && !(seen[0] && seen[3]))) {      // (what a column sees of a block has no gaps)
                 bool odd = false;
 #pragma unroll
-                for (int i = 0; i < DT; ++i)
+                for (int i = 0; i < DV; ++i)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) odd |= !(fabsf(vr[i][e]) < INFINITY);
                 by_key = __ballot(odd) != 0;
             }
             if (by_key) {
 #pragma unroll
-                for (int i = 0; i < DT; ++i)
+                for (int i = 0; i < DV; ++i)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) vr[i][e] = fabsf(vr[i][e]) < INFINITY ? vr[i][e] : 0.f;
             }
 #pragma unroll
             for (int j = 0; j < 4; ++j)
 #pragma unroll
-                for (int i = 0; i < DT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[i][j], s0[j], acc[i], 0, 0, 0);
+                for (int i = 0; i < DV; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[i][j], s0[j], acc[i], 0, 0, 0);
             if (by_key) {
-                const float* v = vcache + cell(page) + (b * 16) % page_size + (int64_t)g * 4 * page_size;
+                const float* v = vcache + cell(page) + (b * 16) % page_size + (int64_t)(d0 + g * 4) * page_size;
 #pragma unroll 1
                 for (int kk = 0; kk < 16; ++kk) {
                     const int e = kk & 3, from = (kk >> 2) * 16 + c;
@@ -165,7 +167,7 @@ attention_f32_kernel(float* __restrict__ out, const float* __restrict__ q, int64
                     const bool sk = __shfl((int)se, from, ZI_WAVE) != 0;
                     const float* vk = v + kk;
 #pragma unroll
-                    for (int i = 0; i < DT; ++i) {
+                    for (int i = 0; i < DV; ++i) {
 #pragma unroll
                         for (int x = 0; x < 4; ++x) {
                             const float val = *vk;
@@ -188,7 +190,7 @@ attention_f32_kernel(float* __restrict__ out, const float* __restrict__ q, int64
             ls[wave][c] = l;
         }
 #pragma unroll
-        for (int i = 0; i < DT; ++i) os[wave][i][lane] = acc[i];
+        for (int i = 0; i < DV; ++i) os[wave][i][lane] = acc[i];
         __syncthreads();
         float top = ms[0][c];
 #pragma unroll
@@ -201,12 +203,12 @@ attention_f32_kernel(float* __restrict__ out, const float* __restrict__ q, int64
         }
         if (sinks) total += expf(sinks[h] - top);
         const float inv = 1.f / total;
-        for (int i = wave; i < DT; i += AF_WAVES) {
+        for (int i = wave; i < DV; i += AF_WAVES) {
             af_f32x4_t o = os[0][i][lane] * part[0];
 #pragma unroll
             for (int u = 1; u < AF_WAVES; ++u) o += os[u][i][lane] * part[u];
             if (mine) {
-                float* dst = out + (int64_t)t * ldo + (int64_t)h * D + i * 16 + g * 4;
+                float* dst = out + (int64_t)t * ldo + (int64_t)h * D + d0 + i * 16 + g * 4;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) dst[e] = o[e] * inv;
             }
@@ -245,16 +247,25 @@ extern "C" int zi_attention_f32(void* out, const void* q, int n, int64_t ldq, in
     ZI_REQUIRE(ldq % 4 == 0 && ((uintptr_t)q | (uintptr_t)kcache | (uintptr_t)vcache) % 16 == 0, "attention: rows must be 16-byte aligned");
     if (n == 0) return 0;
     const dim3 grid(by_heads ? n : (n + AF_COLS - 1) / AF_COLS, by_heads ? nkv * ((nh / nkv + AF_COLS - 1) / AF_COLS) : nh);
-#define ZI_AF(DT)                                                                                                                  \
-    case DT:                                                                                                                       \
-        attention_f32_kernel<DT><<<grid, AF_WAVES * ZI_WAVE, 0, stream>>>((float*)out, (const float*)q, ldq, ldo, (const float*)kcache, \
-                                                                          (const float*)vcache, tok_index, tok_seq, tok_pos, block_tables, \
-                                                                          max_pages, num_pages, n, nh, nkv, page_size, window, scale,    \
-                                                                          sinks, by_heads);                                            \
-        break
-    switch (d / 16) {
+    // Few workgroups leave most units idle, and a wavefront's time is its matrix instructions (32 a block of 16 keys for the scores, 32
+    // for the values at head size 128, two wavefronts a SIMD): then four workgroups make the scores each and a quarter of the dims,
+    // the same sums of each.  us, one workgroup against four: 8 tokens of
+    // 400 keys, 12 heads of 128 on 2 key/value heads, 16.6 to 12.9, of 900 28.0 to 21.2, of 100 9.2 to 8.0; 14 heads of 64 10.6 to 9.2.
+    // (Two or four blocks of keys on their way a wavefront instead of one: 16.6 and 19.3 us at 400 keys, with the waits counted
+    // exactly; the blocks' loads are not what a wavefront waits for.)
+    const bool quarters = by_heads && d % 64 == 0 && (int64_t)grid.x * grid.y * 4 <= zi_compute_units();
+#define ZI_AF_LAUNCH(DT, DV)                                                                                                       \
+    attention_f32_kernel<DT, DV><<<dim3(grid.x, grid.y, DT / DV), AF_WAVES * ZI_WAVE, 0, stream>>>(                                 \
+        (float*)out, (const float*)q, ldq, ldo, (const float*)kcache, (const float*)vcache, tok_index, tok_seq, tok_pos, block_tables, \
+        max_pages, num_pages, n, nh, nkv, page_size, window, scale, sinks, by_heads)
+#define ZI_AF(DT)                     \
+    case DT: ZI_AF_LAUNCH(DT, DT); break
+    if (quarters && d == 64) ZI_AF_LAUNCH(4, 1);
+    else if (quarters) ZI_AF_LAUNCH(8, 2);
+    else switch (d / 16) {
         ZI_AF(1); ZI_AF(2); ZI_AF(3); ZI_AF(4); ZI_AF(5); ZI_AF(6); ZI_AF(7); ZI_AF(8);
     }
 #undef ZI_AF
+#undef ZI_AF_LAUNCH
     return zi_check_launch("attention_f32");
 }
