@@ -269,7 +269,7 @@ gemm_mid_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* __
     gm_epilogue<MT>(acc, out, mode, out_f32, bias, M, N, ldo, split, n0, r, j, vec_out, limit, m0);
 }
 
-// The same product for 65 .. 128 rows of x (MT = 5 .. 8 tiles of 16 rows): one pass over the weights where two launches of the
+// The same product for 65 .. 256 rows of x (MT = 5 .. 16 tiles of 16 rows): one pass over the weights where two launches of the
 // kernel above would make two.  With that many rows the reads of x from LDS bind a workgroup whose wavefronts each take all of
 // them for 16 weight rows (16.3 us for a down product of 27 MB), so here four wavefronts take 32 rows of x each and all of
 // the workgroup's NT x 16 weight rows: 2 + NT operands read for 2 NT products.  Both operands go straight into LDS
@@ -282,9 +282,21 @@ gemm_mid_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* __
 // and 17.2 at 80 (1.5B gate/up), where the library's product and the activation's launch take 25.5 and 21.7 together (for which
 // products it pays: zi_gemm_skinny_swiglu_pays).  A step's instructions were what bound it first: loads whose addresses cost the
 // lanes nothing took 80 rows of the 1.5B gate/up from 20.6 to 18.0 us.
+//
+// Beyond 128 rows eight wavefronts share the workgroup's products, four along the rows of x and two along the weight rows: a wavefront
+// reads (MT / 4 + NT / 2) operands for MT / 4 x NT / 2 products, and two a SIMD cover each other's waits (gate/up at the 7B sizes, 10
+// weight tiles, 160 rows 63 us; four wavefronts two by two 66, five of 32 rows each 71).  The cut is one of its own
+// (zi_gemm_many_plan); with LDS for four buffers of a step gone, three.  Weights from memory, us at 160 and 256 rows, against the
+// library's first proposal: 7B sizes q/k/v 15 and 18 against 25 and 35, output 14 and 17 against 25 and 20, down 37 and 43 against
+// 106 and 125 (a kernel of 32 weight rows a wavefront, 32 x 32 instructions, took 59 at 160 rows and is gone), gate/up with
+// the activation 63 and 79 against 83 and 88 with its launch; 1.5B gate/up 24 and 27 against 30 and 34; 32B q/k/v 24 and 30 against
+// 38 and 52, output 20 and 25 against 37 and 50, down 60 and 73 against 194 and 267.  Bound by a step's barrier and LDS
+// reads: 3.7 to 4.3 TB/s of weights where ten tiles share a slice of x.
 #define GW_KB 64
 
 #define GW_STAGES 4
+#define GW_MID_ROWS 128      // up to here the cut of the kernel above, beyond it zi_gemm_many_plan's
+#define GW_MAX_TILES 10      // 16 weight rows each, of a workgroup
 
 // Rows further apart than this (in elements; 128 of them then span 2^30 bytes) are past what the kernel's 31-bit offsets reach:
 // they go to the kernel above, whose addresses have 64 bits, 64 rows a workgroup.
@@ -312,14 +324,24 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t gw_rows(const zi_bf16* base, i
 }
 
 template <int MT, int NT>
-__global__ void __launch_bounds__(4 * ZI_WAVE)
+struct gw_shape {
+    static constexpr int WM = 4, WN = MT <= 8 ? 1 : 2;                                    // wavefronts along the rows of x and the weight rows
+    static constexpr int WAVES = WM * WN, MW = MT <= 8 ? 2 : (MT + 3) / 4, NW = (NT + WN - 1) / WN;       // a wavefront's tiles
+    static constexpr int STAGES = (MT + NT) * 8 + 1 <= 160 ? GW_STAGES : 3;       // 2 KB a tile and buffer in 160 KB of LDS
+};
+
+template <int MT, int NT>
+__global__ void __launch_bounds__((gw_shape<MT, NT>::WAVES) * ZI_WAVE)
 gemm_wide_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* __restrict__ x,
                  const zi_bf16* __restrict__ w, const zi_bf16* __restrict__ bias, int M, int N, int K, int64_t ldx,
                  int64_t ldw, int64_t ldo, int kb_per_split, int vec_out, float limit) {
-    constexpr int XI = 2 * MT, LOADS = XI + 2 * NT, PW = (LOADS + 3) / 4;       // 1 KB loads of x, of a step; a wavefront's share
+    typedef gw_shape<MT, NT> S;
+    constexpr int WAVES = S::WAVES, STAGES = S::STAGES, MW = S::MW, NW = S::NW;
+    constexpr int XI = 2 * MT, LOADS = XI + 2 * NT, PW = (LOADS + WAVES - 1) / WAVES;       // 1 KB loads of x, of a step; a wavefront's share
     constexpr int PIECES = LOADS * ZI_WAVE;
+    static_assert(STAGES * LOADS + 1 <= 160, "the buffers fit into LDS");
     // (arrays of their own, so that the compiler can tell a buffer that is read from those that loads are on their way to)
-    __shared__ __attribute__((aligned(16))) gm_u32x4_t s0[PIECES], s1[PIECES], s2[PIECES], s3[PIECES], spare[ZI_WAVE];       // (spare: where loads go that nobody needs)
+    __shared__ __attribute__((aligned(16))) gm_u32x4_t s0[PIECES], s1[PIECES], s2[PIECES], s3[STAGES > 3 ? PIECES : 1], spare[ZI_WAVE];       // (spare: where loads go that nobody needs)
     const int tid = threadIdx.x, lane = tid & (ZI_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(tid / ZI_WAVE);
     const int r = lane & 15, j = lane >> 4;
     const int split = blockIdx.y;
@@ -336,7 +358,7 @@ gemm_wide_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* _
     int lane_at[PW];
 #pragma unroll
     for (int i = 0; i < PW; ++i) {
-        const int L = i * 4 + wave;
+        const int L = i * WAVES + wave;
         const int q = (L < XI ? L : L - XI) * 8 + lane / 8;
         lane_at[i] = (int)(q * (L < XI ? ldx : ldw) * 2) + ((lane & 7) ^ ((q >> 1) & 7)) * 16;
     }
@@ -345,76 +367,88 @@ gemm_wide_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* _
         const __amdgpu_buffer_rsrc_t xb = gw_rows(x, ldx, M, K, k), wb = gw_rows(w0, ldw, rows_w, K, k);
 #pragma unroll
         for (int i = 0; i < PW; ++i) {
-            const int L = i * 4 + wave;
+            const int L = i * WAVES + wave;
             gm_u32x4_t* to = L < LOADS ? buf + L * ZI_WAVE : spare;
-            if (i * 4 + 3 < XI) gw_to_lds<0>(xb, to, lane_at[i]);
-            else if (i * 4 >= XI) gw_to_lds<2>(wb, to, lane_at[i]);       // weights are read once: past L2
+            if (i * WAVES + WAVES - 1 < XI) gw_to_lds<0>(xb, to, lane_at[i]);
+            else if (i * WAVES >= XI) gw_to_lds<2>(wb, to, lane_at[i]);       // weights are read once: past L2
             else gw_to_lds<0>(L < XI ? xb : wb, to, lane_at[i]);
         }
     };
-    gm_f32x4_t acc[NT][2];
+    gm_f32x4_t acc[NW][MW];
 #pragma unroll
-    for (int n = 0; n < NT; ++n)
+    for (int n = 0; n < NW; ++n)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) acc[n][t] = gm_f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < MW; ++t) acc[n][t] = gm_f32x4_t{0.f, 0.f, 0.f, 0.f};
     const int sw = (r >> 1) & 7;
-    int tile_at[2];         // (past the rows: the last tile again, not stored)
+    const int m_tile = wave % S::WM * MW, n_tile = wave / S::WM * NW;
+    int tile_at[MW], wtile_at[NW];         // (past the rows: the last tile again, not stored)
 #pragma unroll
-    for (int m = 0; m < 2; ++m) tile_at[m] = ((wave * 2 + m < MT ? wave * 2 + m : MT - 1) * 16 + r) * 8;
+    for (int m = 0; m < MW; ++m) tile_at[m] = ((m_tile + m < MT ? m_tile + m : MT - 1) * 16 + r) * 8;
+#pragma unroll
+    for (int n = 0; n < NW; ++n) wtile_at[n] = XI * ZI_WAVE + ((n_tile + n < NT ? n_tile + n : NT - 1) * 16 + r) * 8;
     auto step = [&](const gm_u32x4_t* buf, gm_u32x4_t* free, int t) __attribute__((always_inline)) {
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
-        gw_wait<(GW_STAGES - 2) * PW>();
+        gw_wait<(STAGES - 2) * PW>();
         __builtin_amdgcn_s_barrier();          // all wavefronts' loads of the step are there, and all are done with `free`
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
-        issue(free, t + GW_STAGES - 1);
+        issue(free, t + STAGES - 1);
         __builtin_amdgcn_sched_barrier(0);
         if (t >= steps) return;
         // all of the step's operands are asked for before the first product: their way is paid once
-        gm_pack a[2][NT], b[2][2];
+        gm_pack a[2][NW], b[2][MW];
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
             const int at = (kk * 4 + j) ^ sw;
 #pragma unroll
-            for (int m = 0; m < 2; ++m) b[kk][m].u = buf[tile_at[m] + at];
+            for (int m = 0; m < MW; ++m) b[kk][m].u = buf[tile_at[m] + at];
 #pragma unroll
-            for (int n = 0; n < NT; ++n) a[kk][n].u = buf[XI * ZI_WAVE + (n * 16 + r) * 8 + at];
+            for (int n = 0; n < NW; ++n) a[kk][n].u = buf[wtile_at[n] + at];
         }
         const int left = K - (k_lo + t * GW_KB);
         if (left < GW_KB) {
 #pragma unroll
             for (int kk = 0; kk < 2; ++kk) {
 #pragma unroll
-                for (int n = 0; n < NT; ++n) a[kk][n].u = gm_keep(a[kk][n].u, kk * 32 + j * 8 < left);
+                for (int n = 0; n < NW; ++n) a[kk][n].u = gm_keep(a[kk][n].u, kk * 32 + j * 8 < left);
 #pragma unroll
-                for (int m = 0; m < 2; ++m) b[kk][m].u = gm_keep(b[kk][m].u, kk * 32 + j * 8 < left);
+                for (int m = 0; m < MW; ++m) b[kk][m].u = gm_keep(b[kk][m].u, kk * 32 + j * 8 < left);
             }
         }
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-            for (int n = 0; n < NT; ++n)
+            for (int n = 0; n < NW; ++n)
 #pragma unroll
-                for (int m = 0; m < 2; ++m)
+                for (int m = 0; m < MW; ++m)
                     acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kk][n].b, b[kk][m].b, acc[n][m], 0, 0, 0);
     };
     issue(s0, 0);
     __builtin_amdgcn_sched_barrier(0);
     issue(s1, 1);
     __builtin_amdgcn_sched_barrier(0);
-    issue(s2, 2);
-    __builtin_amdgcn_sched_barrier(0);
-    for (int t = 0; t < steps; t += GW_STAGES) {
-        step(s0, s3, t);
-        step(s1, s0, t + 1);
-        step(s2, s1, t + 2);
-        step(s3, s2, t + 3);
+    if constexpr (STAGES == 4) {
+        issue(s2, 2);
+        __builtin_amdgcn_sched_barrier(0);
+        for (int t = 0; t < steps; t += 4) {
+            step(s0, s3, t);
+            step(s1, s0, t + 1);
+            step(s2, s1, t + 2);
+            step(s3, s2, t + 3);
+        }
+    } else {
+        for (int t = 0; t < steps; t += 3) {
+            step(s0, s2, t);
+            step(s1, s0, t + 1);
+            step(s2, s1, t + 2);
+        }
     }
     gw_wait<0>();       // (no load may arrive after the workgroup's LDS is another's)
 #pragma unroll
-    for (int n = 0; n < NT; ++n)
-        gm_epilogue<2>(acc[n], out, mode, out_f32, bias, wave * 32 < MT * 16 ? M : 0, N, ldo, split, n0 + n * 16, r, j, vec_out, limit, wave * 32);
+    for (int n = 0; n < NW; ++n)
+        if (n_tile + n < NT)
+            gm_epilogue<MW>(acc[n], out, mode, out_f32, bias, M, N, ldo, split, n0 + (n_tile + n) * 16, r, j, vec_out, limit, m_tile * 16);
 }
 
 // How the product with a weight matrix [N, K] is cut: wavefronts a workgroup (16 weight rows each), splits
@@ -456,14 +490,46 @@ int64_t zi_gemm_mid_plan(int N, int K, int whole, int* splits, int* kb_per_split
     return best_cost;
 }
 
+// How the product of 129 .. 256 rows is cut: weight tiles of 16 rows a workgroup, splits of k over workgroups (at most 16) and blocks of
+// 128 per split; a function of N and K alone.  A cut's time in ns, as measured at the 7B and 32B sizes: a round of workgroups is 3 us
+// and, a block, 500 and 150 for each tile (5 tiles 1.2 us a block, 10 tiles 1.8 to 2.1); a split's sums are written and read once
+// more, at 5 TB/s.  us at 160 rows, the model's choice and the best of all cuts: 4,608 x 3,584 15.2 and 14.2, 3,584 x 3,584 14.1 and
+// 13.1, 3,584 x 18,944 36.9 and 35.1 (10 splits), 7,168 x 5,120 24 and 23.3, 5,120 x 27,648 60.2 and 60.2.  `whole`: without a split.
+// Returns the cost.
+#define GW_PLAN_ROWS 192
+int64_t zi_gemm_many_plan(int N, int K, int whole, int* splits, int* kb_per_split, int* tiles_wg) {
+    const int tiles = (N + 15) / 16, kb_total = (K + GM_KB - 1) / GM_KB, cus = zi_compute_units();
+    int64_t best = -1;
+    for (int w = GM_MIN_WAVES; w <= GW_MAX_TILES; ++w) {
+        if (w == 9) continue;
+        const int groups = (tiles + w - 1) / w;
+        for (int s0 = 1; s0 <= (whole ? 1 : 16) && s0 <= (kb_total > 1 ? kb_total / 2 : 1); ++s0) {
+            const int per = (kb_total + s0 - 1) / s0, s = (kb_total + per - 1) / per;
+            if (s != s0) continue;      // the same cut under another name
+            const int64_t rounds = ((int64_t)groups * s + cus - 1) / cus;
+            const int64_t cost = rounds * ((int64_t)per * (150 * w + 500) + 3000) + (whole ? 0 : (int64_t)s * N * GW_PLAN_ROWS / 625);
+            if (best < 0 || cost < best) {
+                best = cost;
+                *splits = s;
+                *kb_per_split = per;
+                *tiles_wg = w;
+            }
+        }
+    }
+    return best;
+}
+
 // The launch; the checks are the caller's (zi_gemm_skinny).
 int zi_gemm_mid_launch(void* out, int out_f32, int mode, const zi_bf16* x, const zi_bf16* w, const zi_bf16* bias, int M,
                        int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int vec_out, float limit, hipStream_t stream) {
     int splits, per, waves;
-    zi_gemm_mid_plan(N, K, mode >= GM_MODE_ACT || (mode == GM_MODE_SWIGLU && M > 64), &splits, &per, &waves);
+    if (M > GW_MID_ROWS) zi_gemm_many_plan(N, K, mode == GM_MODE_SWIGLU, &splits, &per, &waves);
+    else zi_gemm_mid_plan(N, K, mode >= GM_MODE_ACT || (mode == GM_MODE_SWIGLU && M > 64), &splits, &per, &waves);
+    const int64_t most_ld = M > GW_MID_ROWS ? GW_MAX_LD / 2 : GW_MAX_LD;
+    const bool apart = M > 64 && (ldx > most_ld || ldw > most_ld);
+    if (apart && waves > GM_MAX_WAVES) waves = GM_MAX_WAVES;       // (which weight rows share a workgroup changes no sum)
     const int tiles = (N + 15) / 16;
     const dim3 grid((tiles + waves - 1) / waves, splits);
-    const bool apart = M > 64 && (ldx > GW_MAX_LD || ldw > GW_MAX_LD);
     const int mt = apart ? 0 : (M + 15) / 16;
 #define ZI_GM3(MT, WV, APART, GRID)                                                                                            \
     gemm_mid_kernel<MT, 3, WV, APART><<<GRID, WV * ZI_WAVE, 0, stream>>>(out, mode, out_f32, x, w, bias, M, N, K, ldx, ldw, \
@@ -487,7 +553,7 @@ int zi_gemm_mid_launch(void* out, int out_f32, int mode, const zi_bf16* x, const
         default: ZI_GM2(MT, 8); break;          \
     }
 #define ZI_GW2(MT, WV)                                                                                         \
-    gemm_wide_kernel<MT, WV><<<grid, 4 * ZI_WAVE, 0, stream>>>(out, mode, out_f32, x, w, bias, M, N, K, ldx, ldw, ldo, \
+    gemm_wide_kernel<MT, WV><<<grid, (gw_shape<MT, WV>::WAVES) * ZI_WAVE, 0, stream>>>(out, mode, out_f32, x, w, bias, M, N, K, ldx, ldw, ldo, \
                                                                per, vec_out, limit)
 #define ZI_GW(MT)                               \
     switch (waves) {                            \
@@ -496,6 +562,12 @@ int zi_gemm_mid_launch(void* out, int out_f32, int mode, const zi_bf16* x, const
         case 6: ZI_GW2(MT, 6); break;           \
         case 7: ZI_GW2(MT, 7); break;           \
         default: ZI_GW2(MT, 8); break;          \
+    }
+// (rows beyond 128 in tiles of 32: the engine's steps have multiples of 32)
+#define ZI_GW_MANY(MT)                          \
+    switch (waves) {                            \
+        case 10: ZI_GW2(MT, 10); break;         \
+        default: ZI_GW(MT)                      \
     }
     switch (mt) {
         case 0: ZI_GA(4); break;
@@ -506,13 +578,21 @@ int zi_gemm_mid_launch(void* out, int out_f32, int mode, const zi_bf16* x, const
         case 5: ZI_GW(5); break;
         case 6: ZI_GW(6); break;
         case 7: ZI_GW(7); break;
-        default: ZI_GW(8); break;
+        case 8: ZI_GW(8); break;
+        case 9:
+        case 10: ZI_GW_MANY(10); break;
+        case 11:
+        case 12: ZI_GW_MANY(12); break;
+        case 13:
+        case 14: ZI_GW_MANY(14); break;
+        default: ZI_GW_MANY(16); break;
     }
 #undef ZI_GM
 #undef ZI_GM2
 #undef ZI_GM3
 #undef ZI_GA
 #undef ZI_GA2
+#undef ZI_GW_MANY
 #undef ZI_GW
 #undef ZI_GW2
     return zi_check_launch("gemm_mid");

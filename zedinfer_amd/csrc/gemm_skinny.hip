@@ -1,8 +1,7 @@
 // out[M,N] = x[M,K] . w[N,K]^T (+ bias) for up to 256 rows of x: the decode-time matrix products, bound by the
 // one pass over the weights.  This file holds their entry points, the cut's bookkeeping and the kernel that
-// adds partial sums; the product kernels are in gemm_mid.hip (up to 128 rows: x staged in LDS, a workgroup's
-// wavefronts take 16 weight rows each, the cut over workgroups balanced over the compute units) and in
-// gemm_rows32.hip (more rows: 32 weight rows a wavefront).
+// adds partial sums; the product kernels are in gemm_mid.hip (x staged in LDS, a workgroup's wavefronts take 16 weight rows each, or,
+// from 65 rows on, share the rows of x, the cut over workgroups balanced over the compute units).
 //
 // When the weight matrix gives too few workgroups the k dimension is cut over several of them (gridDim.y
 // "splits"); those write float32 partial sums [split][M][N] that the consumer adds in rising order (the next
@@ -42,7 +41,7 @@ __global__ void gemm_skinny_reduce_kernel(void* __restrict__ out, int out_f32, c
 }
 
 #define SK_MAX_ROWS 256
-#define SK_MID_MAX_ROWS 128        // up to here the kernels of gemm_mid.hip, beyond gemm_rows32.hip
+#define SK_MID_MAX_ROWS 128        // up to here one cut of the weights, beyond it another
 #define SK_MAX_ROWS_ACT 64         // ... with the epilogues that only products of few rows have
 
 extern "C" int zi_gemm_skinny_supported(int M, int N, int K, int64_t ldx, int64_t ldw) {
@@ -52,33 +51,31 @@ extern "C" int zi_gemm_skinny_supported(int M, int N, int K, int64_t ldx, int64_
 // most rows the products take
 extern "C" int zi_gemm_skinny_max_rows() { return SK_MAX_ROWS; }
 
-// 1 when these kernels are the faster way to partial sums than the library's product of the same operands, as
-// measured: always up to 128 rows; beyond, for large weights with at least twice as many columns as rows (a down
-// projection: 7B sizes at 256 rows 71 against 126 us, 32B 136 against 263), not for square ones (an output
-// projection: 7B at 256 rows 24.6 against 16.9 us), and not for small ones (1.5B down at 256 rows 25.5 against
-// 31 us, which the 25 MB of partial sums that the next kernel then adds take back: the decode step of 256
-// requests got 3 % slower with it).
+// 1 when these kernels are the faster way to partial sums than the library's product of the same operands, with what the next kernel's
+// reading of the sums costs, as measured: always up to 128 rows; beyond, for weights with at least twice as many columns as
+// rows (a down projection) from 2^24 elements on (us at 160 and 256 rows against the library's 36 and 40: 2,048 x 11,008 19 and 23 with
+// 8 splits; 1,536 x 8,960 14 and 17 against 23 and 31, of which 10 splits of sums take most back), and for about square ones (q/k/v,
+// output) from 2^23 on (3,072 x 3,072 12 and 15 against 17 and 18, 4,096 x 4,096 14 and 18 against 27 and 23; 2,048 x 2,048 8 and 11
+// against 9 and 10).  Weights with many more rows than columns are whole products, whose partial sums gain nothing.
 extern "C" int zi_gemm_skinny_pays(int M, int N, int K) {
     if (M <= SK_MID_MAX_ROWS) return 1;
-    return M <= SK_MAX_ROWS && (int64_t)K >= 2 * (int64_t)N && (int64_t)N * K >= ((int64_t)1 << 25);
+    const int64_t n = N, k = K, size = n * k;
+    return M <= SK_MAX_ROWS && (k >= 2 * n ? size >= 1 << 24 : n <= 2 * k && size >= 1 << 23);
 }
 
-// The product kernel (gemm_mid.hip): its cut and its launch.
+// The product kernels (gemm_mid.hip): their cuts and their launch.
 int64_t zi_gemm_mid_plan(int N, int K, int whole, int* splits, int* kb_per_split, int* waves);
+int64_t zi_gemm_many_plan(int N, int K, int whole, int* splits, int* kb_per_split, int* tiles);
 int zi_gemm_mid_launch(void* out, int out_f32, int mode, const zi_bf16* x, const zi_bf16* w, const zi_bf16* bias, int M,
                        int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int vec_out, float limit, hipStream_t stream);
 
-void zi_gemm_rows32_plan(int N, int K, int whole, int* splits, int* kb_per_split);
-int zi_gemm_rows32_launch(void* out, int out_f32, int mode, const zi_bf16* x, const zi_bf16* w, const zi_bf16* bias, int M,
-                          int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int vec_out, float limit, hipStream_t stream);
-
-static bool sk_rows32(int M) { return M > SK_MID_MAX_ROWS; }
+static bool sk_many(int M) { return M > SK_MID_MAX_ROWS; }
 
 // Splits of k for a weight matrix [N, K]: the leading dimension of the partial sums.  A function of N and K and
-// of which of the two kernels the rows go to (up to 128, or more).
+// of whether there are more than 128 rows.
 extern "C" int zi_gemm_skinny_splits(int M, int N, int K) {
     int s, per, waves;
-    if (sk_rows32(M)) zi_gemm_rows32_plan(N, K, 0, &s, &per);
+    if (sk_many(M)) zi_gemm_many_plan(N, K, 0, &s, &per, &waves);
     else zi_gemm_mid_plan(N, K, 0, &s, &per, &waves);
     return s;
 }
@@ -113,6 +110,19 @@ extern "C" int zi_gemm_skinny_swiglu_pays(int M, int N, int K) {
     return whole <= cut + SK_LAUNCH_COST && ((N + 15) / 16 + waves - 1) / waves <= zi_compute_units();
 }
 
+// The same for 129 to 256 rows.  A launch and the sums that a cut leaves are 4 us; the workgroups have to be one round, and of ten
+// weight tiles (a slice of x is read for each of them) unless k is short.  us at 160 and 256 rows, epilogue against the library's first
+// proposal and the launch: 18,944 columns I x 3,584 63 and 79 against 84 and 88, 8,960 x 1,536 24 and 27 against 30 and 34, 11,008 x
+// 2,048 29 and 34 against 35 and 39, 4,864 x 896 13 and 16 against 17 and 20, 20,480 x 7,168 120 and 151 against 155 and 167; left to the
+// library: two rounds 27,648 x 5,120 152 and 176 against 137 and 169, seven tiles 13,824 x 5,120 77 and 94 against 79 and 95, half
+// a round 4,096 x 4,096 36 and 47 against 32 and 45.
+extern "C" int zi_gemm_skinny_swiglu_many_pays(int M, int N, int K) {
+    if (M <= SK_MID_MAX_ROWS || M > SK_MAX_ROWS) return 0;
+    int s, per, tiles, cut_tiles;
+    const int64_t cut = zi_gemm_many_plan(N, K, 0, &s, &per, &cut_tiles), whole = zi_gemm_many_plan(N, K, 1, &s, &per, &tiles);
+    return whole <= cut + 4000 && ((N + 15) / 16 + tiles - 1) / tiles <= zi_compute_units() && (tiles == 10 || K < 4096);
+}
+
 // mode 0: out[M,N] (+ bias), reduced through `workspace` when the product is split.
 // mode 1: out = float32 partial sums [splits][M][N] (splits from zi_gemm_skinny_splits; the bias, if any, is in the first).
 // mode 2: w holds gate and up rows interleaved in blocks of 8; out[M, N/2] (bfloat16) =
@@ -134,8 +144,7 @@ extern "C" int zi_gemm_skinny_act(void* out, int out_dt, int mode, const void* x
     ZI_REQUIRE(ldx >= K && ldw >= K, "gemm_skinny: leading dimension too small");
     ZI_REQUIRE(((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0, "gemm_skinny: x and w must be 16-byte aligned");
     int splits, per, waves;
-    const bool rows32 = sk_rows32(M);
-    if (rows32) zi_gemm_rows32_plan(N, K, mode == SK_MODE_SWIGLU, &splits, &per);
+    if (sk_many(M)) zi_gemm_many_plan(N, K, mode == SK_MODE_SWIGLU, &splits, &per, &waves);
     else zi_gemm_mid_plan(N, K, mode >= SK_MODE_ACT || (mode == SK_MODE_SWIGLU && M > 64), &splits, &per, &waves);       // (whole from 65 rows on)
     void* dst = out;
     int kmode = mode;
@@ -163,8 +172,7 @@ extern "C" int zi_gemm_skinny_act(void* out, int out_dt, int mode, const void* x
     else if (kmode >= SK_MODE_SWIGLU) vec_out = ldo % 4 == 0 && ((uintptr_t)dst % 8) == 0;
     else vec_out = ldo % 4 == 0 && ((uintptr_t)dst % (out_dt == ZI_F32 ? 16 : 8)) == 0;
     const int of32 = out_dt == ZI_F32;
-    const int rc = (rows32 ? zi_gemm_rows32_launch : zi_gemm_mid_launch)(dst, of32, kmode, (const zi_bf16*)x, (const zi_bf16*)w, b,
-                                                                         M, N, K, ldx, ldw, ldo, vec_out, limit, stream);
+    const int rc = zi_gemm_mid_launch(dst, of32, kmode, (const zi_bf16*)x, (const zi_bf16*)w, b, M, N, K, ldx, ldw, ldo, vec_out, limit, stream);
     if (rc) return rc;
     if (mode == SK_MODE_PLAIN && splits > 1) {
         const int64_t total = (int64_t)M * N;

@@ -1120,16 +1120,35 @@ def linear_swiglu(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Ten
     _gpu("linear_swiglu", x, weight, out)
     if not linear_swiglu_supported(x, weight):
         raise ValueError("linear_swiglu: needs an unsplit bfloat16 few-rows product with 2I a multiple of 16")
+    return _swiglu_epilogue("linear_swiglu", x, weight, out)
+
+
+def _swiglu_epilogue(what: str, x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor]) -> torch.Tensor:
     M, K = x.shape
     N = weight.shape[0]
     if out is None:
         out = torch.empty((M, N // 2), dtype=torch.bfloat16, device=x.device)
-    ldo, wo = _rows(out, "linear_swiglu out")
+    ldo, wo = _rows(out, f"{what} out")
     if tuple(out.shape) != (M, N // 2) or out.dtype != torch.bfloat16:
-        raise ValueError(f"linear_swiglu: out must be bfloat16 [{M}, {N // 2}]")
+        raise ValueError(f"{what}: out must be bfloat16 [{M}, {N // 2}]")
     _lib.call("zi_gemm_skinny", _p(out), BF16, 2, _p(x), _p(weight), c_void_p(0), M, N, K, x.stride(0), weight.stride(0),
               ldo, c_void_p(0), 0, _stream())
     return out
+
+
+def linear_swiglu_many_pays(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether ``linear_swiglu_many`` takes this product (129 .. SUMS_MAX_ROWS rows) and was measured to be the faster way to it than the
+    library's product and the activation's launch (the kernel library says)."""
+    return (_few_rows_operands(x, weight, SUMS_MAX_ROWS) and weight.shape[0] % 16 == 0
+            and bool(_lib.load().zi_gemm_skinny_swiglu_many_pays(int(x.shape[0]), int(weight.shape[0]), int(weight.shape[1]))))
+
+
+def linear_swiglu_many(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``linear_swiglu`` for the products of more than 128 rows at which it pays (``linear_swiglu_many_pays``)."""
+    _gpu("linear_swiglu_many", x, weight, out)
+    if not linear_swiglu_many_pays(x, weight):
+        raise ValueError("linear_swiglu_many: not a product of 129 rows and more that it is for")
+    return _swiglu_epilogue("linear_swiglu_many", x, weight, out)
 
 
 def linear_swiglu_halves_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -1205,10 +1224,9 @@ FEW_ROWS = 64          # up to here they beat the library product: the weights s
 # Products that leave partial sums (q/k/v, output, down: few weight rows, k cut over workgroups) go to the
 # few-rows kernels up to this many rows: measured at 128 rows with the weights coming from memory, 1.5B sizes,
 # 7.2 / 6.9 / 13.5 us against the library's 9.7 / 8.1 / 24.5; 7B sizes 15 / 13 / 36 against 20 / 16 / 92.
-# Beyond 128 rows and up to 256 a kernel with 32 weight rows a wavefront (gemm_rows32.hip) takes the products whose
-# weights have at least twice as many columns as rows (the down projection; the library decides,
-# ``zi_gemm_skinny_pays``).  With the SwiGLU epilogue the limit is 128 rows, and up to there the library decides from
-# 65 rows on (``zi_gemm_skinny_swiglu_pays``); beyond, the library's product.
+# Beyond 128 rows and up to 256 they take the down products and the about square ones of larger models (the library decides,
+# ``zi_gemm_skinny_pays``).  With the SwiGLU epilogue the library decides from 65 rows on (``zi_gemm_skinny_swiglu_pays``) and for
+# more than 128 (``linear_swiglu_many``, ``zi_gemm_skinny_swiglu_many_pays``).
 # (ZEDINFER_SUMS_MAX_ROWS=64 gives such products of more than 64 rows back to the library; ZEDINFER_SWIGLU_MAX_ROWS
 # gives the SwiGLU epilogue every product of up to that many rows.)
 SUMS_MAX_ROWS = max(FEW_ROWS, min(256, int(os.environ.get("ZEDINFER_SUMS_MAX_ROWS", "256") or 256)))

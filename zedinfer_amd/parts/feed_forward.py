@@ -141,7 +141,10 @@ class SwiGLU(FeedForward):
             sums = ops.linear_sums(x, self.gate_up, out=self.rt.buffer("ffn_gate_up_sums", (S, n, 2 * I), torch.float32))
             ops.swiglu(sums, out=act, interleave=self.interleave)
         elif self.interleave == GATE_UP_BLOCK and x.dtype == torch.bfloat16:
-            self._gate_up_many_rows(x, act)
+            if ops.linear_swiglu_many_pays(x, self.gate_up):
+                ops.linear_swiglu_many(x, self.gate_up, out=act)
+            else:
+                self._gate_up_many_rows(x, act)
         elif not self.interleave and self.gate_up is not None and ops.linear_swiglu_halves_supported(x, self.gate_up):
             ops.linear_swiglu_halves(x, self.gate_up, out=act)
         else:
