@@ -15,15 +15,17 @@
 // chunk, beside the 8 rows of x twice: an instruction's load takes eight whole 128-byte lines, and two of the result's
 // four quadrants are the two chains.
 // gemm_f32_tile_kernel, for many rows, is bound by the instruction's rate (152 TFLOP/s in a large library product): tiles
-// through LDS (two buffers, one barrier a chunk of 32 k, two or four more chunks on their way in registers).  The
-// scheduling barriers keep the loads ahead of the products: without them the compiler moves a loop's loads to its end and
-// waits for all of them at its head.
+// through LDS (three buffers, one barrier a chunk of 32 k, three more chunks on their way in registers), the operands of the next
+// half of a chunk on their way from LDS while one half is multiplied; with two buffers, and a chunk's operands asked for after
+// its barrier, 448 rows of 1,536 x 8,960 took 144 us where they take 123 now, 512 rows of 17,920 x 1,536 244 and 231, 256 rows of
+// 4,608 x 3,584 102 and 97.  The scheduling barriers keep the loads ahead of the products: without them the compiler moves a loop's
+// loads to its end and waits for all of them at its head.
 //
 // Measured, weights from memory, against the plain kernel (gemm_generic.hip: a chain of multiply-adds an output, scalar
 // loads), us, launch included: 8 rows 2,048 x 1,536 (N x K) 165 to 9; 1,536 x 8,960 914 to 19; 17,920 x 1,536 212 to 32 (3.5
-// TB/s); 151,936 x 1,536 761 to 250 (3.7 TB/s; one row 190, 4.9 TB/s).  448 rows: 2,048 x 1,536 189 to 33, 1,536 x 8,960
-// 1,050 to 147 (84 TFLOP/s), 17,920 x 1,536 975 to 219 (113 TFLOP/s).  The gate/up product with the activation in its end against the
-// two launches: 448 rows of 17,920 x 1,536 233 to 220, 1,024 rows 502 to 486, 256 rows 153 to 144.
+// TB/s); 151,936 x 1,536 761 to 250 (3.7 TB/s; one row 190, 4.9 TB/s).  448 rows: 2,048 x 1,536 189 to 32, 1,536 x 8,960
+// 1,050 to 123 (101 TFLOP/s), 17,920 x 1,536 975 to 207 (119 TFLOP/s).  With the activation in its end the gate/up product of 512 rows
+// of 17,920 x 1,536 takes 235 us, of 1,024 452, where the two launches took 258 and 504.
 #include "zi_common.h"
 
 typedef __attribute__((ext_vector_type(4))) float gf_f32x4_t;
@@ -31,6 +33,7 @@ typedef __attribute__((ext_vector_type(4))) unsigned gf_u32x4_t;
 
 #define GF_PARTS 8           // runs of k; the wavefronts of the stream kernel
 #define GF_KB 32             // k of a chunk
+#define GF_BUFFERS 3         // chunks that the tile kernel holds in LDS, and as many on their way in registers
 #define GF_HELD_CHUNKS 16    // chunks of a run that a wavefront can hold of 8 rows of x beside as many of weights (256 registers)
 #define GF_OUT 0x7fffffff    // an offset past the end of every buffer: the load gives zeros and fetches nothing
 
@@ -251,16 +254,16 @@ gemm_f32_held_kernel(float* __restrict__ out, const float* __restrict__ x, const
 }
 
 // TM x 32 NT outputs a workgroup; GROUPS (1 or 2) groups of four wavefronts, each over half of the runs of k when there are
-// two; TM/2 x 16 NT outputs a wavefront.  RING chunks of operands are on their way in registers.  GATED (NT = 2): of a wavefront's two
+// two; TM/2 x 16 NT outputs a wavefront.  GATED (NT = 2): of a wavefront's two
 // blocks of 16 weight rows one are gate rows and one the up rows of the same outputs (rows n and N + n of w), and TM x 32 outputs
 // up * silu(gate) are what the tile leaves.
-template <int TM, int NT, int GROUPS, int RING, bool GATED>
-__global__ void __launch_bounds__(256 * GROUPS)
+template <int TM, int NT, int GROUPS, bool GATED, bool SHORT>
+__global__ void __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2)     // (three workgroups a unit: 64 x 64 tiles 4 % slower with two)
 gemm_f32_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,
                      const float* __restrict__ bias, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int per, int vec_out,
                      int m_tiles, int tiles) {
     constexpr int TN = 32 * NT, XP = TM / 32, WP = TN / 32, MT = TM / 32;     // pieces a thread loads; 16 x 16 tiles a wavefront
-    __shared__ __attribute__((aligned(16))) gf_f32x4_t lds[GROUPS][2][(TM + TN) * 8];
+    __shared__ __attribute__((aligned(16))) gf_f32x4_t lds[GROUPS][GF_BUFFERS][(TM + TN) * 8];
     // the tiles that share weight rows follow each other on one XCD (workgroup i runs on XCD i mod 8)
     const int per_xcd = (tiles + 7) / 8, tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
     if (tile >= tiles) return;
@@ -287,7 +290,7 @@ gemm_f32_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const
     const int chunks = (K + GF_KB - 1) / GF_KB, half = per * (GF_PARTS / 2);
     const int c0 = group * half, c1 = GROUPS == 2 && c0 + half < chunks ? c0 + half : chunks;
     const int steps = GROUPS == 2 ? half : chunks;      // the same for both groups: they share the barriers
-    gf_f32x4_t xr[RING][XP], wr[RING][WP];
+    gf_f32x4_t xr[GF_BUFFERS][XP], wr[GF_BUFFERS][WP];
     auto fetch = [&](const int slot, int c) __attribute__((always_inline)) {
         const int k = c * (GF_KB * 4) + pc * 16;
         const bool in = c < c1 && k < K * 4;
@@ -296,8 +299,8 @@ gemm_f32_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const
 #pragma unroll
         for (int p = 0; p < WP; ++p) wr[slot][p] = gf_load<0>(wb, in && w_row[p] != GF_OUT ? w_row[p] + k : GF_OUT);
     };
-    auto stash = [&](const int slot, const int b) __attribute__((always_inline)) {
-        gf_f32x4_t* xs = lds[group][b], *ws = xs + TM * 8;
+    auto stash = [&](const int slot) __attribute__((always_inline)) {
+        gf_f32x4_t* xs = lds[group][slot], *ws = xs + TM * 8;
 #pragma unroll
         for (int p = 0; p < XP; ++p) xs[(pr + 32 * p) * 8 + place] = xr[slot][p];
 #pragma unroll
@@ -311,28 +314,38 @@ gemm_f32_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const
 #pragma unroll
         for (int u = 0; u < NT; ++u) acc[0][t][u] = acc[1][t][u] = sum[t][u] = first[t][u] = zero;
     int in_part = 0, parts = 0;
-    auto step = [&](const int slot, const int b, int c) __attribute__((always_inline)) {
-        fetch(slot, c + RING);                          // this slot's registers went to LDS a step ago
+    gf_f32x4_t va[2][NT], vb[2][MT];
+    const int sw = (r >> 1) & 7;
+    auto read = [&](const int b, const int h) __attribute__((always_inline)) {      // the operands of a half of the chunk in buffer b
         const gf_f32x4_t* xs = lds[group][b], *ws = xs + TM * 8;
-        const int sw = (r >> 1) & 7;
-        __builtin_amdgcn_sched_barrier(0);              // the loads stay this far ahead of their use
-        gf_f32x4_t va[2][NT], vb[2][MT];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int u = 0; u < NT; ++u) va[h][u] = ws[(wn + u * 16 + r) * 8 + ((h * 4 + g) ^ sw)];
 #pragma unroll
-            for (int u = 0; u < NT; ++u) va[h][u] = ws[(wn + u * 16 + r) * 8 + ((h * 4 + g) ^ sw)];
+        for (int t = 0; t < MT; ++t) vb[h][t] = xs[(wm + t * 16 + r) * 8 + ((h * 4 + g) ^ sw)];
+    };
+    auto multiply = [&](const int h) __attribute__((always_inline)) {
 #pragma unroll
-            for (int t = 0; t < MT; ++t) vb[h][t] = xs[(wm + t * 16 + r) * 8 + ((h * 4 + g) ^ sw)];
-        }
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+            for (int t = 0; t < MT; ++t)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int t = 0; t < MT; ++t)
-#pragma unroll
-                    for (int u = 0; u < NT; ++u)
-                        acc[h][t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[h][u][j], vb[h][t][j], acc[h][t][u], 0, 0, 0);
+                for (int u = 0; u < NT; ++u)
+                    acc[h][t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[h][u][j], vb[h][t][j], acc[h][t][u], 0, 0, 0);
+    };
+    // Chunk c lies in buffer and slot c mod 3.  While a half is multiplied the next one's operands are on their way from LDS; between
+    // the halves the chunk after the next goes into LDS (its buffer was last read a step ago) and its registers are asked for anew.
+    auto step = [&](const int s, int c) __attribute__((always_inline)) {
+        constexpr int B = GF_BUFFERS;
+        read(s, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(0);
+        __builtin_amdgcn_sched_barrier(0);
+        read((s + 1) % B, 0);
+        stash((s + 2) % B);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch((s + 2) % B, c + 2 + B);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(1);
         if (++in_part == per) {                         // a run of k ends
             in_part = 0;
             ++parts;
@@ -349,20 +362,32 @@ gemm_f32_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const
                 }
         }
         __builtin_amdgcn_sched_barrier(0);
-        stash((slot + 1) % RING, b ^ 1);                // the next chunk
         __syncthreads();
     };
 #pragma unroll
-    for (int s = 0; s < RING; ++s) {
+    for (int s = 0; s < GF_BUFFERS; ++s) {
         fetch(s, c0 + s);
         __builtin_amdgcn_sched_barrier(0);
     }
-    stash(0, 0);
-    __syncthreads();
-    static_assert(RING % 2 == 0, "an LDS buffer a step");
-    for (int c = 0; c < steps; c += RING) {             // (steps past the end add zeros)
 #pragma unroll
-        for (int s = 0; s < RING; ++s) step(s, s & 1, c0 + c + s);
+    for (int s = 0; s < 2; ++s) {
+        stash(s);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(s, c0 + GF_BUFFERS + s);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+    read(0, 0);
+    // (the large tiles have no registers for an ending of their own, 240 against 207 us: steps past the end add zeros; SHORT: at most two
+    // steps, 9,000 x 64 at 1,024 rows 28 us with three)
+    int c = 0;
+    for (; !SHORT && c + (TM == 64 ? 1 : GF_BUFFERS) <= steps; c += GF_BUFFERS) {
+#pragma unroll
+        for (int s = 0; s < GF_BUFFERS; ++s) step(s, c0 + c + s);
+    }
+    if (SHORT || TM < 64) {
+        if (c < steps) step(0, c0 + c);
+        if (c + 1 < steps) step(1, c0 + c + 1);
     }
 #pragma unroll
     for (int t = 0; t < MT; ++t)
@@ -467,13 +492,13 @@ static int gf_launch(float* out, const float* x, const float* w, const float* bi
             out, x, w, bias, M, N, K, ldx, ldw, ldo, per, vec_out, groups);                                                               \
     } while (0)
     // (rows in as many launches as 2^32 threads of one make necessary: a row's result does not depend on them)
-#define ZI_GF_TILE(TM, NT, G, R)                                                                                                              \
+#define ZI_GF_TILE(TM, NT, G, SHORT)                                                                                                              \
     do {                                                                                                                                  \
         const int nc = 32 * NT / (GATED ? 2 : 1);                                                                                              \
         const int64_t nt = (N + nc - 1) / nc, most = ((1ll << 31) / (256 * G)) / nt * TM;                                                      \
         for (int64_t m = 0; m < M; m += most) {                                                                                           \
             const int rows = (int)(M - m < most ? M - m : most), mt = (rows + TM - 1) / TM, tiles = (int)(mt * nt);                              \
-            gemm_f32_tile_kernel<TM, NT, G, R, GATED><<<(tiles + 7) / 8 * 8, 256 * G, 0, stream>>>(out + m * ldo, x + m * ldx, w, bias, rows, N, \
+            gemm_f32_tile_kernel<TM, NT, G, GATED, SHORT><<<(tiles + 7) / 8 * 8, 256 * G, 0, stream>>>(out + m * ldo, x + m * ldx, w, bias, rows, N, \
                                                                                                    K, ldx, ldw, ldo, per, vec_out, mt, tiles);  \
         }                                                                                                                                 \
     } while (0)
@@ -492,9 +517,12 @@ static int gf_launch(float* out, const float* x, const float* w, const float* bi
             else if (per <= 6) ZI_GF_HELD(false, 6);
             else ZI_GF_HELD(false, 8);
             break;
-        case GF_TILE_64: ZI_GF_TILE(64, 2, 1, 2); break;
-        case GF_TILE_32: ZI_GF_TILE(32, 2, 1, 4); break;
-        case GF_TILE_32_HALVES: ZI_GF_TILE(32, 2, 2, 4); break;
+        case GF_TILE_64:
+            if (chunks <= 2) ZI_GF_TILE(64, 2, 1, true);
+            else ZI_GF_TILE(64, 2, 1, false);
+            break;
+        case GF_TILE_32: ZI_GF_TILE(32, 2, 1, false); break;
+        case GF_TILE_32_HALVES: ZI_GF_TILE(32, 2, 2, false); break;
         default:
             if constexpr (GATED) {
                 return zi_fail("gemm_f32: no gated kernel for %d rows of %d x %d", M, N, K);      // (zi_gemm_f32_swiglu_takes says so)
@@ -503,7 +531,7 @@ static int gf_launch(float* out, const float* x, const float* w, const float* bi
                     case GF_PAIRS: ZI_GF_STREAM(1, true, 6); break;
                     case GF_ROWS16: ZI_GF_STREAM(1, false, 4); break;
                     case GF_ROWS32: ZI_GF_STREAM(2, false, 3); break;
-                    default: ZI_GF_TILE(32, 3, 2, 2); break;
+                    default: ZI_GF_TILE(32, 3, 2, false); break;
                 }
             }
     }
