@@ -474,7 +474,12 @@ __device__ __attribute__((aligned(16))) const unsigned pf_zero16[4] = {0u, 0u, 0
 // LOGB: slope * ln(1 + rate * distance) is taken off every score, two numbers a head (ZiScoreExtras).
 // MAPS: several softmax maps over the same values: a key row holds MAPS keys of D / MAPS values side by side, head h
 // reads the (h mod MAPS)-th of them, and only that part of its query row (the rest of the row is not read).
-template <int D, int QW, int KH, bool LOGB, int MAPS>
+// PAGED: pages of 16 positions and more, and key rows of at least 8 pieces.  A load instruction then lies in one page, whose number the
+// wavefront reads once a block, a block ahead, and moves to scalar registers: a load costs the lanes nothing but its place, which
+// does not change.  For that the values' tile holds 16 keys after 16 keys, of each every dim's two pieces (swapped for dims 8 to 15 of 16,
+// so that sixteen lanes' reads touch every bank once), as pages of 16 hold them: an instruction takes 1 KB in one run.  us a layer, the
+// same bits: 2,048 tokens of 12 heads 45.0 to 41.2, 2,048 of 28 heads 72.9 to 69.8, 1,163 tokens after 2,048 of 28 heads 113.9 to 104.2.
+template <int D, int QW, int KH, bool LOGB, int MAPS, bool PAGED>
 __global__ void __launch_bounds__(4 * KH * ZI_WAVE, KH == 1 ? 2 : 1)
 attention_prefill_dma_kernel(zi_bf16* __restrict__ out, int64_t ldo, const zi_bf16* __restrict__ q, int64_t ldq,
                              const zi_bf16* __restrict__ kcache, const zi_bf16* __restrict__ vcache,
@@ -570,6 +575,8 @@ attention_prefill_dma_kernel(zi_bf16* __restrict__ out, int64_t ldo, const zi_bf
     // What a lane loads does not change from block to block: for its KI pieces of the key tile the key
     // (as an offset into the block) and the piece of its row, for its VI pieces of the value tile the
     // dim and the eight keys.  Place L of a tile is row L / pieces-per-row; the piece there is swizzled.
+    static_assert(!PAGED || KC >= 8, "a load of keys lies within 16 of them");
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     int k_key[KI], k_piece[KI], v_dim[VI], v_key[VI];
 #pragma unroll
     for (int i = 0; i < KI; ++i) {
@@ -591,7 +598,46 @@ attention_prefill_dma_kernel(zi_bf16* __restrict__ out, int64_t ldo, const zi_bf
     const int khi8 = khi & ~7;
     __syncthreads();      // the table is in LDS
 
-    auto issue = [&](int kb, uint4* kl, uint4* vl) {
+    // PAGED: a wavefront's loads of keys take 16 rows of the tile, the keys k_first + 8 q + 0..3, q = 0 .. 3, of the block (two groups of
+    // 16 keys), and its loads of values all dims of the block's keys 16 wave .. 16 wave + 15.
+    static_assert(KI * (ZI_WAVE / KC) == 16, "16 rows of the keys' tile a wavefront");
+    const int k_first = (wave_u / 4) * PF_BN + (wave_u % 4 / 2) * 32 + (wave_u % 2) * 4;
+    const unsigned v_lane = (unsigned)(((lane >> 1) << ps_shift) + (((lane & 1) ^ ((lane >> 4) & 1)) << 3)) * 2;
+    const unsigned page_elements = (unsigned)(nkv * ps * D);      // (the launch has checked that this is below 2^31)
+    // the pages of the block's groups of 16 keys, a lane each (past the last key: the last key's)
+    auto pages_of = [&](int kb) {
+        const int key = kb + (lane & (BS / 16 - 1)) * 16;
+        return bt_lds[((key < khi ? key : khi) >> ps_shift) - pi_first];
+    };
+    int pages = PAGED ? pages_of(kb_begin) : 0;
+    auto issue_paged = [&](int kb, uint4* kl, uint4* vl) __attribute__((always_inline)) {
+        const char* group[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const unsigned pg = __builtin_amdgcn_readlane(pages, k_first / 16 + q);
+            const unsigned page = pg < (unsigned)num_pages ? pg : 0;          // not held: a window has passed it
+            group[q] = (const char*)(kbase + (uint64_t)page * page_elements + ((kb + (k_first & ~15) + q * 16) & ps_mask) * D);
+        }
+#pragma unroll
+        for (int i = 0; i < KI; ++i) {
+            const unsigned at = (unsigned)(((k_key[i] & 15) * D + k_piece[i] * 8) * 2);
+            __builtin_amdgcn_global_load_lds(group[i * 2 / KI] + at, kl + (wave_u * KI + i) * ZI_WAVE, 16, 0, 0);
+        }
+        const int key0 = kb + wave_u * 16;
+        const unsigned pg = __builtin_amdgcn_readlane(pages, wave_u);
+        const bool ok = key0 <= khi && pg < (unsigned)num_pages;
+        const char* base = ok ? (const char*)(vbase + (uint64_t)pg * page_elements + (key0 & ps_mask)) : (const char*)pf_zero16;
+        const unsigned at = ok ? v_lane : 0;
+#pragma unroll
+        for (int i = 0; i < VI; ++i)
+            __builtin_amdgcn_global_load_lds(base + (ok ? (int64_t)i << (6 + ps_shift) : 0) + at, vl + (wave_u * VI + i) * ZI_WAVE, 16, 0, 0);
+        pages = pages_of(kb + BS);
+    };
+    auto issue = [&](int kb, uint4* kl, uint4* vl) __attribute__((always_inline)) {
+        if constexpr (PAGED) {
+            issue_paged(kb, kl, vl);
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < KI; ++i) {
             const int key = kb + k_key[i];
@@ -615,7 +661,20 @@ attention_prefill_dma_kernel(zi_bf16* __restrict__ out, int64_t ldo, const zi_bf
     // The piece of every value row that holds the last key and keys past it: what lies past is cleared
     // (those slots of the page may hold anything).  Only in the block that holds the last key.
     auto clean = [&](int kb, uint4* vl) {
-        if (kb + BS - 1 > kmax && ((kmax + 1) & 7) != 0) {
+        if (PAGED && kb + BS - 1 > kmax && ((kmax + 1) & 15) != 0) {
+            if (tid < 2 * D) {
+                const int group = (kmax - kb) / 16, keep = (kmax + 1) & 15, half = (tid & 1) ^ ((tid >> 4) & 1);
+                pf_pack val;
+                uint4* at = vl + group * 2 * D + tid;
+                val.u = *at;
+#pragma unroll
+                for (int x = 0; x < 8; ++x)
+                    if (half * 8 + x >= keep) val.h[x] = 0;
+                *at = val.u;
+            }
+            __syncthreads();
+        }
+        if (!PAGED && kb + BS - 1 > kmax && ((kmax + 1) & 7) != 0) {
             if (tid < D) {
                 const int piece = (kmax - kb) / 8, keep = (kmax + 1) & 7;
                 pf_pack val;
@@ -716,7 +775,8 @@ attention_prefill_dma_kernel(zi_bf16* __restrict__ out, int64_t ldo, const zi_bf
 #pragma unroll
             for (int b = 0; b < 2; ++b) {
                 pf_pack a;
-                a.u = vl[dim * VC + ((kh * 8 + b * 4 + j) ^ ((dim / VSW) & (VC - 1)))];
+                if constexpr (PAGED) a.u = vl[((kh * 4 + b * 2 + j / 2) * D + dim) * 2 + ((j & 1) ^ ((r >> 3) & 1))];
+                else a.u = vl[dim * VC + ((kh * 8 + b * 4 + j) ^ ((dim / VSW) & (VC - 1)))];
 #pragma unroll
                 for (int u = 0; u < QW; ++u)      // and one read of the values' operand
                     o[u][dd] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.b, pb[u][b].b, o[u][dd], 0, 0, 0);
@@ -980,7 +1040,13 @@ static int pf_launch(void* out, const void* q, int dt, int num_tiles, int64_t ld
             tile_off, entry_start, entry_len, entry_past, block_tables, max_pages, num_pages, nh, nkv, ps_shift, \
             window, scale, po, pml, max_chunks, chunk_keys, sinks, ex)
 #define ZI_PF_DMA2(DD, QW, KH, LOGB, MAPS)                                                                     \
-    attention_prefill_dma_kernel<DD, QW, KH, LOGB, MAPS><<<grid, 4 * KH * ZI_WAVE, 0, stream>>>(                     \
+    do {                                                                                                       \
+        constexpr bool PG = DD / MAPS >= 64;                                                                   \
+        if (PG && page_size >= 16 && (int64_t)nkv * page_size * d < (1ll << 31)) ZI_PF_DMA3(DD, QW, KH, LOGB, MAPS, PG);                                     \
+        else ZI_PF_DMA3(DD, QW, KH, LOGB, MAPS, false);                                                        \
+    } while (0)
+#define ZI_PF_DMA3(DD, QW, KH, LOGB, MAPS, PAGED)                                                              \
+    attention_prefill_dma_kernel<DD, QW, KH, LOGB, MAPS, PAGED><<<grid, 4 * KH * ZI_WAVE, 0, stream>>>(                     \
         (zi_bf16*)out, ldo, (const zi_bf16*)q, ldq, (const zi_bf16*)kcache, (const zi_bf16*)vcache, tile_entry, \
         tile_off, entry_start, entry_len, entry_past, block_tables, max_pages, num_pages, nh, nkv, ps_shift,   \
         window, scale, po, pml, max_chunks, chunk_keys, sinks, slope, rate)
@@ -1015,6 +1081,7 @@ static int pf_launch(void* out, const void* q, int dt, int num_tiles, int64_t ld
 #undef ZI_PF
 #undef ZI_PF_DMA
 #undef ZI_PF_DMA2
+#undef ZI_PF_DMA3
     if (max_chunks > 1)
         attention_prefill_merge_kernel<<<dim3(num_tiles * tile, nh), ZI_WAVE, 0, stream>>>(
             (zi_bf16*)out, ldo, po, pml, tile_entry, tile_off, entry_start, entry_len, entry_past, nh, d, window, max_chunks,
