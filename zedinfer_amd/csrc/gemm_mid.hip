@@ -271,8 +271,8 @@ gemm_mid_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* __
 
 // The same product for 65 .. 256 rows of x (MT = 5 .. 16 tiles of 16 rows): one pass over the weights where two launches of the
 // kernel above would make two.  With that many rows the reads of x from LDS bind a workgroup whose wavefronts each take all of
-// them for 16 weight rows (16.3 us for a down product of 27 MB), so here four wavefronts take 32 rows of x each and all of
-// the workgroup's NT x 16 weight rows: 2 + NT operands read for 2 NT products.  Both operands go straight into LDS
+// them for 16 weight rows (16.3 us for a down product of 27 MB), so here eight wavefronts take 32 rows of x and half of
+// the workgroup's NT x 16 weight rows each: 2 + NT / 2 operands read for NT products.  Both operands go straight into LDS
 // (global_load_lds_dwordx4, 1 KB an instruction, rows of 128 bytes with piece c of row q at place c xor (q / 2 mod 8)), k in
 // steps of 64 through four buffers, three steps on their way while one is worked on (six buffers were no faster); every wavefront issues as many loads a step
 // as every other, so that each can wait for its own by count before the step's one barrier.  The cut, the order of the
@@ -283,8 +283,13 @@ gemm_mid_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* __
 // products it pays: zi_gemm_skinny_swiglu_pays).  A step's instructions were what bound it first: loads whose addresses cost the
 // lanes nothing took 80 rows of the 1.5B gate/up from 20.6 to 18.0 us.
 //
-// Beyond 128 rows eight wavefronts share the workgroup's products, four along the rows of x and two along the weight rows: a wavefront
-// reads (MT / 4 + NT / 2) operands for MT / 4 x NT / 2 products, and two a SIMD cover each other's waits (gate/up at the 7B sizes, 10
+// Two wavefronts a SIMD cover each other's waits: against four wavefronts of 32 rows of x and all weight rows, us at 65 and 128 rows, 2,048
+// x 1,536 5.9 to 5.2 and 6.7 to 6.2, 4,608 x 3,584 12.9 to 11.2 and 14.6 to 13.3, 2,560 x 2,048 7.0 to 6.2 and 8.2 to 7.9, gate/up of
+// 8,960 columns x 1,536 18.8 to 18.0 and 23.5 to 22.3, of 3,072 x 1,024 10.6 to 9.3 and 11.8 to 10.7; the same at 1,536 x 8,960 and
+// 5,120 x 5,120.  Five weight tiles do not halve, which a long k pays for (5,120 x 27,648 55 to 58 and 71 to 75, 18,944 columns x
+// 3,584 61 to 63): those keep the four (GW_LONG).
+//
+// Beyond 128 rows a wavefront has a quarter of the rows of x (gate/up at the 7B sizes, 10
 // weight tiles, 160 rows 63 us; four wavefronts two by two 66, five of 32 rows each 71).  The cut is one of its own
 // (zi_gemm_many_plan); with LDS for four buffers of a step gone, three.  Weights from memory, us at 160 and 256 rows, against the
 // library's first proposal: 7B sizes q/k/v 15 and 18 against 25 and 35, output 14 and 17 against 25 and 20, down 37 and 43 against
@@ -296,6 +301,7 @@ gemm_mid_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* __
 
 #define GW_STAGES 4
 #define GW_MID_ROWS 128      // up to here the cut of the kernel above, beyond it zi_gemm_many_plan's
+#define GW_LONG 20           // blocks of 128 from which five weight tiles of up to 128 rows are four wavefronts' (see above)
 #define GW_MAX_TILES 10      // 16 weight rows each, of a workgroup
 
 // Rows further apart than this (in elements; 128 of them then span 2^30 bytes) are past what the kernel's 31-bit offsets reach:
@@ -323,19 +329,20 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t gw_rows(const zi_bf16* base, i
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<zi_bf16*>(base + k), 0, k < K ? (int)(((rows - 1) * ld + K - k) * 2) : 0, 0x00020000);
 }
 
-template <int MT, int NT>
+// WN: the wavefronts along the weight rows, four times as many in all.
+template <int MT, int NT, int WN>
 struct gw_shape {
-    static constexpr int WM = 4, WN = MT <= 8 ? 1 : 2;                                    // wavefronts along the rows of x and the weight rows
-    static constexpr int WAVES = WM * WN, MW = MT <= 8 ? 2 : (MT + 3) / 4, NW = (NT + WN - 1) / WN;       // a wavefront's tiles
+    static constexpr int WM = 4, WAVES = WM * WN;                                 // wavefronts along the rows of x, of a workgroup
+    static constexpr int MW = MT <= 8 ? 2 : (MT + 3) / 4, NW = (NT + WN - 1) / WN;       // a wavefront's tiles
     static constexpr int STAGES = (MT + NT) * 8 + 1 <= 160 ? GW_STAGES : 3;       // 2 KB a tile and buffer in 160 KB of LDS
 };
 
-template <int MT, int NT>
-__global__ void __launch_bounds__((gw_shape<MT, NT>::WAVES) * ZI_WAVE)
+template <int MT, int NT, int WN>
+__global__ void __launch_bounds__((gw_shape<MT, NT, WN>::WAVES) * ZI_WAVE)
 gemm_wide_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* __restrict__ x,
                  const zi_bf16* __restrict__ w, const zi_bf16* __restrict__ bias, int M, int N, int K, int64_t ldx,
                  int64_t ldw, int64_t ldo, int kb_per_split, int vec_out, float limit) {
-    typedef gw_shape<MT, NT> S;
+    typedef gw_shape<MT, NT, WN> S;
     constexpr int WAVES = S::WAVES, STAGES = S::STAGES, MW = S::MW, NW = S::NW;
     constexpr int XI = 2 * MT, LOADS = XI + 2 * NT, PW = (LOADS + WAVES - 1) / WAVES;       // 1 KB loads of x, of a step; a wavefront's share
     constexpr int PIECES = LOADS * ZI_WAVE;
@@ -552,13 +559,17 @@ int zi_gemm_mid_launch(void* out, int out_f32, int mode, const zi_bf16* x, const
         case 7: ZI_GM2(MT, 7); break;           \
         default: ZI_GM2(MT, 8); break;          \
     }
-#define ZI_GW2(MT, WV)                                                                                         \
-    gemm_wide_kernel<MT, WV><<<grid, (gw_shape<MT, WV>::WAVES) * ZI_WAVE, 0, stream>>>(out, mode, out_f32, x, w, bias, M, N, K, ldx, ldw, ldo, \
-                                                               per, vec_out, limit)
+#define ZI_GW3(MT, WV, WN)                                                                                     \
+    gemm_wide_kernel<MT, WV, WN><<<grid, (gw_shape<MT, WV, WN>::WAVES) * ZI_WAVE, 0, stream>>>(out, mode, out_f32, x, w, bias, M, N, \
+                                                                                               K, ldx, ldw, ldo, per, vec_out, limit)
+#define ZI_GW2(MT, WV) ZI_GW3(MT, WV, 2)
 #define ZI_GW(MT)                               \
     switch (waves) {                            \
         case 4: ZI_GW2(MT, 4); break;           \
-        case 5: ZI_GW2(MT, 5); break;           \
+        case 5:                                 \
+            if (MT <= 8 && per > GW_LONG) ZI_GW3(MT, 5, (MT <= 8 ? 1 : 2)); \
+            else ZI_GW2(MT, 5);                 \
+            break;                              \
         case 6: ZI_GW2(MT, 6); break;           \
         case 7: ZI_GW2(MT, 7); break;           \
         default: ZI_GW2(MT, 8); break;          \
@@ -595,5 +606,6 @@ int zi_gemm_mid_launch(void* out, int out_f32, int mode, const zi_bf16* x, const
 #undef ZI_GW_MANY
 #undef ZI_GW
 #undef ZI_GW2
+#undef ZI_GW3
     return zi_check_launch("gemm_mid");
 }
