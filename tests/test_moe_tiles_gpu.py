@@ -46,3 +46,19 @@ def test_rows_of_weights_past_the_staged_lengths():
     out = torch.empty(rows, N, dtype=torch.float32, device="cuda")
     ops.moe_linear(x, w, plan, 64, 1, out=out)
     assert torch.equal(out, x.float() @ w[0].float().t())       # whole numbers below 2^24: exact in any order
+
+
+# tiles of eight wavefronts: a remainder of the k step, fewer steps than buffers, columns past a workgroup's
+@pytest.mark.parametrize("N,K", [(1, 8), (257, 128), (515, 200), (64, 264), (768, 1024)])
+@pytest.mark.parametrize("out_dtype,pad", [(torch.float32, 0), (torch.bfloat16, 8), (torch.float32, 1)])
+def test_products_of_sorted_rows_in_tiles_of_128(N, K, out_dtype, pad):
+    test_products_of_sorted_rows(128, N, K, out_dtype, pad)
+
+
+@pytest.mark.parametrize("mean,experts,widths,rows", [(8, 32, (1536, 1536), 16), (16, 32, (1536, 1536), 32), (48, 32, (1536, 1536), 32), (64, 32, (1536, 1536), 128),
+                                                      (128, 32, (1536, 1536), 64), (250, 32, (1536, 1536), 128), (32, 32, (2560, 3584), 64),
+                                                      (64, 8, (4096, 1024), 32), (100, 8, (4096, 1024), 64), (16, 2, (12, 8), 16)])
+def test_which_tiles_a_step_takes(mean, experts, widths, rows):
+    from zedinfer_amd import ops
+    assert ops.moe_tile_rows(torch.bfloat16, torch.bfloat16, widths, mean * experts, experts) == rows
+    assert ops.moe_tile_rows(torch.float32, torch.bfloat16, widths, mean * experts, experts) == 16

@@ -313,6 +313,9 @@ moe_linear_kernel(TO* __restrict__ out, int64_t ldo, const TX* __restrict__ x, i
 // lines.  Measured with 32 experts of 1536 x 1536 (151 MB of weights), the first product and the second: 8,000 pairs 203 and
 // 195 to 98 and 87 us (two buffers, so that a unit holds two workgroups: with four buffers and one workgroup 141 and 115), 128
 // pairs 41 and 40 to 24.8 and 24.6 us (6.1 TB/s; with four buffers 26.5 and 25.3).
+// Tiles of 128 rows x 256 columns are eight wavefronts', 64 x 64 each, with three buffers in 144 KB: three fifths of the bytes an
+// operation, and two steps on their way: 8,000 pairs 92 and 83 to 88 and 77 us; 2,048 pairs, a tile an expert, 53 and 49 (tiles of
+// 32) to 50 and 43.
 typedef __attribute__((ext_vector_type(8))) __bf16 moe_bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float moe_f32x4_t;
 typedef __attribute__((ext_vector_type(4))) unsigned moe_u32x4_t;
@@ -346,13 +349,16 @@ __device__ __forceinline__ void moe_to_lds(__amdgpu_buffer_rsrc_t from, moe_u32x
 #endif
 }
 
-template <typename TO, int RT, int CT, int ST>
-__global__ void __launch_bounds__(4 * ZI_WAVE)
+// WR: wavefronts along the rows of a tile, each with RT / WR of its sixteens; four times as many in all.
+template <typename TO, int RT, int CT, int ST, int WR>
+__global__ void __launch_bounds__(4 * WR * ZI_WAVE)
 moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restrict__ x, int64_t ldx,
                        const zi_bf16* __restrict__ w, const int32_t* __restrict__ plan,
                        const int32_t* __restrict__ source, int source_div, int N, int K, int act) {
-    constexpr int XI = 2 * RT, WI = 8 * CT, XW = (XI + 3) / 4, WW = WI / 4, PW = XW + WW;      // loads of a step; a wavefront's share
-    constexpr int PIECES = (4 * XW + WI) * ZI_WAVE;
+    constexpr int WAVES = 4 * WR, RW = RT / WR;
+    static_assert(RT % WR == 0 && 8 * CT % WAVES == 0, "whole shares");
+    constexpr int XI = 2 * RT, WI = 8 * CT, XW = (XI + WAVES - 1) / WAVES, WW = WI / WAVES, PW = XW + WW;      // loads of a step; a wavefront's share
+    constexpr int PIECES = (WAVES * XW + WI) * ZI_WAVE;
     // (arrays of their own, so that the compiler can tell a buffer that is read from those that loads are on their way to)
     __shared__ __attribute__((aligned(16))) moe_u32x4_t s0[PIECES], s1[PIECES], s2[ST > 2 ? PIECES : 1];
     static_assert(ST == 2 || ST == 3, "two or three buffers");
@@ -362,7 +368,7 @@ moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restr
     const int tile = job / blocks, n0 = job % blocks * 64 * CT;
     const int e = plan[1 + 3 * tile], r0 = plan[2 + 3 * tile], rows = plan[3 + 3 * tile];
     const int lane = threadIdx.x % ZI_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / ZI_WAVE);
-    const int r = lane & 15, j = lane >> 4;
+    const int r = lane & 15, j = lane >> 4, wave_c = wave % 4, row0 = wave / 4 * RW * 16;      // this wavefront's columns and rows
     // Load i takes 8 rows: lane l row l / 8 of them, the piece that belongs at place l % 8.  (Rows of the tokens past the
     // tile's are its first row again, not stored; weight rows past N are past the buffer's end.)
     const int rows_w = N - n0 < 64 * CT ? N - n0 : 64 * CT;
@@ -372,13 +378,13 @@ moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restr
     int xpiece[XW], w_at[WW], wpiece[WW];
 #pragma unroll
     for (int i = 0; i < XW; ++i) {
-        const int q = (i * 4 + wave) * 8 + lane / 8, rr = q < rows ? q : 0;
+        const int q = (i * WAVES + wave) * 8 + lane / 8, rr = q < rows ? q : 0;
         xrow[i] = x + (int64_t)(source ? source[r0 + rr] / source_div : r0 + rr) * ldx;
         xpiece[i] = ((lane & 7) ^ ((q >> 1) & 7)) * 8;
     }
 #pragma unroll
     for (int i = 0; i < WW; ++i) {
-        const int q = (i * 4 + wave) * 8 + lane / 8;
+        const int q = (i * WAVES + wave) * 8 + lane / 8;
         wpiece[i] = ((lane & 7) ^ ((q >> 1) & 7)) * 8;
         w_at[i] = (q < rows_w ? q * K + wpiece[i] : rows_w * K) * 2;
     }
@@ -389,15 +395,15 @@ moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restr
         const bool whole = k0 + MOE_KB <= K;
 #pragma unroll
         for (int i = 0; i < XW; ++i)
-            moe_to_lds(xrow[i] + (whole || k0 + xpiece[i] < K ? k0 + xpiece[i] : 0), buf + (i * 4 + wave) * ZI_WAVE);
+            moe_to_lds(xrow[i] + (whole || k0 + xpiece[i] < K ? k0 + xpiece[i] : 0), buf + (i * WAVES + wave) * ZI_WAVE);
 #pragma unroll
         for (int i = 0; i < WW; ++i)
-            moe_to_lds<RT == 1 ? 2 : 0>(wb, buf + (4 * XW + i * 4 + wave) * ZI_WAVE,
+            moe_to_lds<RT == 1 ? 2 : 0>(wb, buf + (WAVES * XW + i * WAVES + wave) * ZI_WAVE,
                                         whole || k0 + wpiece[i] < K ? w_at[i] + k0 * 2 : rows_w * K * 2);
     };
-    moe_f32x4_t acc[RT][CT];
+    moe_f32x4_t acc[RW][CT];
 #pragma unroll
-    for (int t = 0; t < RT; ++t)
+    for (int t = 0; t < RW; ++t)
 #pragma unroll
         for (int c = 0; c < CT; ++c) acc[t][c] = (moe_f32x4_t){0.f, 0.f, 0.f, 0.f};
     const int sw = (r >> 1) & 7;
@@ -417,20 +423,20 @@ moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restr
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
             const int at = (kk * 4 + j) ^ sw;
-            moe_pack a[CT], b[RT];
+            moe_pack a[CT], b[RW];
 #pragma unroll
-            for (int c = 0; c < CT; ++c) a[c].u = buf[(4 * XW * 8 + (wave * CT + c) * 16 + r) * 8 + at];
+            for (int c = 0; c < CT; ++c) a[c].u = buf[(WAVES * XW * 8 + (wave_c * CT + c) * 16 + r) * 8 + at];
 #pragma unroll
-            for (int m = 0; m < RT; ++m) b[m].u = buf[(m * 16 + r) * 8 + at];
+            for (int m = 0; m < RW; ++m) b[m].u = buf[(row0 + m * 16 + r) * 8 + at];
             if (left < MOE_KB) {
                 const unsigned mask = 0u - (unsigned)(kk * 32 + j * 8 < left);
 #pragma unroll
                 for (int c = 0; c < CT; ++c) a[c].u &= mask;
 #pragma unroll
-                for (int m = 0; m < RT; ++m) b[m].u &= mask;
+                for (int m = 0; m < RW; ++m) b[m].u &= mask;
             }
 #pragma unroll
-            for (int m = 0; m < RT; ++m)
+            for (int m = 0; m < RW; ++m)
 #pragma unroll
                 for (int c = 0; c < CT; ++c)
                     acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[c].b, b[m].b, acc[m][c], 0, 0, 0);
@@ -454,12 +460,12 @@ moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restr
     // allow it
     const bool whole = ldo % 4 == 0 && ((uintptr_t)out % 16) == 0;
 #pragma unroll
-    for (int t = 0; t < RT; ++t) {
-        const int row = t * 16 + r;
+    for (int t = 0; t < RW; ++t) {
+        const int row = row0 + t * 16 + r;
         if (row >= rows) continue;
 #pragma unroll
         for (int c = 0; c < CT; ++c) {
-            const int n = n0 + (wave * CT + c) * 16 + 4 * j;
+            const int n = n0 + (wave_c * CT + c) * 16 + 4 * j;
             TO* dst = out + (int64_t)(r0 + row) * ldo + n;
             if (whole && n + 3 < N) {
                 moe_store4(dst, moe_act(acc[t][c][0], act), moe_act(acc[t][c][1], act), moe_act(acc[t][c][2], act),
@@ -482,21 +488,22 @@ extern "C" int zi_moe_linear(void* out, int out_dt, int64_t ldo, const void* x, 
     if (max_tiles == 0) return 0;
     const dim3 grid((N + MOE_TN - 1) / MOE_TN, max_tiles, (tile_rows + MOE_TM - 1) / MOE_TM);
     const bool cores = x_dt == ZI_BF16 && w_dt == ZI_BF16 && K % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)x % 16) == 0 &&
-                       ((uintptr_t)w % 16) == 0 && (tile_rows == 16 || tile_rows == 32 || tile_rows == 64);
+                       ((uintptr_t)w % 16) == 0 && (tile_rows == 16 || tile_rows == 32 || tile_rows == 64 || tile_rows == 128);
     // tiles of 64 rows (many rows an expert: prompts) are 256 columns wide, for a workgroup's reads of LDS: 8 operands for 16
     // products; smaller ones (decoded tokens) are bound by the weights' stream: narrow, so that every unit has several workgroups
     // (and what neither a buffer's offsets nor a grid of one dimension, 2^32 threads, reaches is left to the plain kernel)
-    const int wide = cores ? 64 * (tile_rows / 16) : 64;       // columns of a workgroup
+    const int wide = cores ? (tile_rows < 64 ? 64 * (tile_rows / 16) : 256) : 64;       // columns of a workgroup
     const int64_t most = ((int64_t)N + wide - 1) / wide * max_tiles + MOE_XCDS;
-    if (cores && K <= MOE_MAX_K && most * 256 < (1LL << 32)) {
-#define ZI_MOE_CORES(RT, CT, ST)                                                                                                   \
-    moe_linear_mfma_kernel<TO, RT, CT, ST><<<dim3((((N + 64 * CT - 1) / (64 * CT)) * (int64_t)max_tiles + MOE_XCDS - 1) / MOE_XCDS * \
-                                             MOE_XCDS), 256, 0, stream>>>((TO*)out, ldo, (const zi_bf16*)x, ldx,                      \
+    if (cores && K <= MOE_MAX_K && most * (tile_rows == 128 ? 512 : 256) < (1LL << 32)) {
+#define ZI_MOE_CORES(RT, CT, ST, WR)                                                                                                   \
+    moe_linear_mfma_kernel<TO, RT, CT, ST, WR><<<dim3((((N + 64 * CT - 1) / (64 * CT)) * (int64_t)max_tiles + MOE_XCDS - 1) / MOE_XCDS * \
+                                             MOE_XCDS), 256 * WR, 0, stream>>>((TO*)out, ldo, (const zi_bf16*)x, ldx,                      \
                                                                           (const zi_bf16*)w, plan, source, source_div, N, K, act)
         ZI_DISPATCH_DTYPE(out_dt, TO, {
-            if (tile_rows == 16) ZI_MOE_CORES(1, 1, 3);
-            else if (tile_rows == 32) ZI_MOE_CORES(2, 2, 3);
-            else ZI_MOE_CORES(4, 4, 2);
+            if (tile_rows == 16) ZI_MOE_CORES(1, 1, 3, 1);
+            else if (tile_rows == 32) ZI_MOE_CORES(2, 2, 3, 1);
+            else if (tile_rows == 64) ZI_MOE_CORES(4, 4, 2, 1);
+            else ZI_MOE_CORES(8, 4, 3, 2);
         });
         return zi_check_launch("moe_linear");
     }

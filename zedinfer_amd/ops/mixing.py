@@ -9,10 +9,10 @@ from typing import Optional
 import torch
 
 from . import _lib
-from .functional import _code, _gpu, _i32, _p, _rows, _stream
+from .functional import _code, _gpu, _i32, _p, _rows, _stream, compute_units
 
 ACTIVATIONS = {"silu": 0, "gelu_tanh": 1, "gelu_erf": 2}
-MOE_TILE_ROWS = (16, 32, 64)
+MOE_TILE_ROWS = (16, 32, 64, 128)
 MOE_MAX_EXPERTS = 1024
 DELTA_MAX_TAPS = 17
 
@@ -500,12 +500,25 @@ def moe_group(idx: torch.Tensor, experts: int, tile_rows: int, plan: torch.Tenso
 
 def moe_tile_rows(x_dtype: torch.dtype, w_dtype: torch.dtype, widths, pairs: int, experts: int) -> int:
     """Rows of a tile of the experts' products: 16 for the plain kernel; on the matrix cores (bfloat16, every
-    inner size a multiple of 8) 16, 32 or 64, the more rows an expert gets on average the larger."""
+    inner size a multiple of 8) 16, 32, 64 or 128, the more rows an expert gets on average the larger: every tile reads the
+    expert's weights again.
+
+    Tiles of 64 rows are 256 columns wide, so from fewer rows on only where that still gives every compute unit a workgroup.  Both
+    products together, us: 32 experts of 1,536 x 1,536, 16 rows each 84 in tiles of 16, 71 of 32; 32 of 2,560 x 3,584, 32 rows
+    275 of 32, 239 of 64, 48 rows 313 and 250; 64 of 1,024 x 2,048, 32 rows 146 and 133; 8 of 4,096 x 1,024 (128 workgroups), 64 rows 64
+    and 86.  Tiles of 128 rows are a workgroup a unit, and pay unless most experts have just more than a tile: 32 of 1,536 x 1,536, 64
+    rows 102 of 32, 92 of 128, 96 rows 107 of 64 and 96, 128 rows 112 of 64 and 149, 250 rows 176 and 165; 32 of 2,560 x 3,584 96 rows 354
+    and 318, 250 rows 585 and 545."""
     cores = x_dtype == torch.bfloat16 and w_dtype == torch.bfloat16 and all(int(k) % 8 == 0 for k in widths)
     if not cores:
         return 16
-    mean = pairs / max(experts, 1)
-    return 64 if mean >= 96 else 32 if mean >= 24 else 16
+    mean, units = pairs / max(experts, 1), compute_units()
+    columns = -(-min(int(k) for k in widths) // 256)
+    if (60 <= mean <= 112 or mean >= 192) and (pairs / 128 + experts / 2) * columns >= 0.7 * units:
+        return 128
+    if mean >= 96 or (mean >= 28 and experts * columns >= units):
+        return 64
+    return 32 if mean >= 14 else 16
 
 
 def moe_linear(x: torch.Tensor, w: torch.Tensor, plan: torch.Tensor, tile_rows: int, max_tiles: int,
