@@ -1077,6 +1077,16 @@ def linear_splits(M: int, N: int, K: int) -> int:
     return int(_lib.load().zi_gemm_skinny_splits(int(M), int(N), int(K)))
 
 
+def linear_out_sums(dtype: torch.dtype, rows: int, weight: torch.Tensor) -> int:
+    """How many partial sums ``linear_sums`` leaves of ``rows`` contiguous rows of ``dtype`` and this weight where what follows adds
+    terms anyway, up to 128 rows; 1 where the whole product is to be made."""
+    N, K = weight.shape
+    if dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or not 0 < rows <= 128 or K % 8 or weight.stride(1) != 1 \
+            or weight.stride(0) % 8 or weight.data_ptr() % 16 or rows > SUMS_MAX_ROWS:
+        return 1
+    return linear_splits(rows, N, K)
+
+
 def linear_sums(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None,
                 bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x[M,K] . weight[N,K]^T for M <= SUMS_MAX_ROWS as float32 partial sums [S, M, N], S =

@@ -221,6 +221,11 @@ class Part:
         self.spec = spec
         self.rt = rt
 
+    def out_sums(self, rows: int) -> int:
+        """How many partial sums ``forward`` writes into ``out=`` [sums, rows, width] when it is handed so many places (a part with
+        ``writes_into``); 1: its whole result, into [rows, width]."""
+        return 1
+
     def tune(self, num_tokens: int) -> None:
         """Measure, outside of any step, which of several equivalent ways is faster for steps of
         ``num_tokens`` tokens and record the decision in ``rt.choices`` (``Engine.warm_up`` calls this).

@@ -79,6 +79,9 @@ class GatedDeltaRule(Mixer):
     def step_rows(self, rows: int, kind: str) -> int:
         return ProductRows.step_rows(rows, kind)
 
+    def out_sums(self, rows: int) -> int:
+        return ops.linear_out_sums(self.rt.dtype, rows, self.o)
+
     def forward(self, x: torch.Tensor, batch, memory: LayerMemory, out=None) -> torch.Tensor:
         n, rt, nh, kvh, dim, vdim = x.shape[0], self.rt, self.nh, self.kvh, self.dim, self.vdim
         state = memory.state
@@ -109,6 +112,8 @@ class GatedDeltaRule(Mixer):
             ops.gated_rms_norm(o, self.norm, gate, nh, vdim, self.eps, out=y)
         if out is None:
             out = rt.buffer("delta_out", (n, self.hidden))
+        if out.dim() == 3:
+            return ops.linear_sums(y, self.o, out=out)
         return ops.linear(y, self.o, out=out)
 
 

@@ -219,6 +219,9 @@ class GatedMLP(FeedForward):
         n = int(num_tokens)
         self.rt.tune_linear(self.rt.buffer("norm_out", (n, self.hidden)), self.gate_up)
 
+    def out_sums(self, rows: int) -> int:
+        return ops.linear_out_sums(self.rt.dtype, rows, self.down)
+
     def forward(self, x: torch.Tensor, out=None) -> torch.Tensor:
         n, I = x.shape[0], self.inter
         gu = self.rt.buffer("ffn_gate_up", (n, self.up_at + I))
@@ -227,6 +230,8 @@ class GatedMLP(FeedForward):
         ops.gated_act(gu[:, :I], gu[:, self.up_at:], self.activation, out=act)
         if out is None:
             out = self.rt.buffer("ffn_out", (n, self.hidden))
+        if out.dim() == 3:
+            return ops.linear_sums(act, self.down, out=out)
         return ops.linear(act, self.down, out=out)
 
 

@@ -183,6 +183,9 @@ class LatentAttention(Mixer):
             ops.latent_inputs(full, self.dq_norm, self.eps, cq)
         return cq, full[..., self.gate_at:self.gate_at + self.nh * self.vdim]
 
+    def out_sums(self, rows: int) -> int:
+        return ops.linear_out_sums(self.rt.dtype, rows, self.o)
+
     def forward(self, x: torch.Tensor, batch, memory: LayerMemory, out=None) -> torch.Tensor:
         n, rt = x.shape[0], self.rt
         view = batch.groups[memory.group]
@@ -232,4 +235,6 @@ class LatentAttention(Mixer):
                 S = ops.linear_splits(n, self.hidden, self.nh * self.vdim)
                 return ops.linear_sums(heads, self.o, out=rt.buffer("latent_out_sums", (S, n, self.hidden), torch.float32))
             out = rt.buffer("latent_out", (n, self.hidden))
+        if out.dim() == 3:
+            return ops.linear_sums(heads, self.o, out=out)
         return ops.linear(heads, self.o, out=out)
