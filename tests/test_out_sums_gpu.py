@@ -75,3 +75,21 @@ def test_a_parallel_blocks_stack():
         assert float((terms.sum(0) - want).norm() / want.norm()) <= 1e-6
         k = part.out_sums(5) if most <= 16 else 1
         assert torch.equal(ops.reduce_sums(terms[k:].contiguous(), out_dtype=torch.float32), mlp.forward(resid.bfloat16(), out=torch.empty(5, 1536, device="cuda")))
+
+
+@pytest.mark.parametrize("splits", [1, 2, 7, 15, 16, 17])
+@pytest.mark.parametrize("rows,width,pad", [(1, 4, 0), (3, 70, 0), (5, 1000, 8), (33, 132, 2), (2, 260, 4)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_sums_added_four_columns_at_a_time(splits, rows, width, pad, dtype):
+    """Widths and strides that are and are not whole pieces, one sum and as many as there are kernels for and one more; with a bias and
+    without: float32 additions in rising order."""
+    from zedinfer_amd import ops
+    g = torch.Generator().manual_seed(splits * width)
+    sums, bias = torch.randn(splits, rows, width, generator=g).cuda(), torch.randn(width, generator=g).bfloat16().cuda()
+    want = torch.zeros(rows, width, device="cuda")
+    for s in sums:
+        want = want + s
+    for b in (None, bias):
+        store = torch.full((rows, width + pad), 7.0, dtype=dtype, device="cuda")
+        ops.reduce_sums(sums, b, out=store[:, :width])
+        assert torch.equal(store[:, :width], (want + b.float() if b is not None else want).to(dtype)) and bool((store[:, width:] == 7.0).all())

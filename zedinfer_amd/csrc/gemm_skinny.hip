@@ -40,6 +40,63 @@ __global__ void gemm_skinny_reduce_kernel(void* __restrict__ out, int out_f32, c
     else zi_store((zi_bf16*)out + (int64_t)m * ldo + n, s);
 }
 
+// The same, four columns a thread and all of its sums on their way before the first is added: the kernel is a trip to memory that other XCDs
+// have just written, and one after the other they were as many trips.  us: 32 rows of
+// 1,536 columns and 10 sums 4.7 to 2.6, of 4,632 and 6 3.9 to 2.9, 8 of 4,632 2.9 to 2.35, 64 of 1,536 and 10 to bfloat16 4.6 to 2.9.
+template <int SPLITS>
+__global__ void __launch_bounds__(64)
+gemm_skinny_reduce4_kernel(void* __restrict__ out, int out_f32, const float* __restrict__ partial, const zi_bf16* __restrict__ bias,
+                           int N, int64_t total, int64_t ldo) {
+    const int64_t i = ((int64_t)blockIdx.x * 64 + threadIdx.x) * 4;
+    if (i >= total) return;
+    const int64_t m = i / N;
+    const int n = (int)(i - m * N);
+    float4 p[SPLITS];
+#pragma unroll
+    for (int k = 0; k < SPLITS; ++k) p[k] = *reinterpret_cast<const float4*>(partial + k * total + i);
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int k = 0; k < SPLITS; ++k) {
+        s.x += p[k].x;
+        s.y += p[k].y;
+        s.z += p[k].z;
+        s.w += p[k].w;
+    }
+    if (bias) {
+        s.x += zi_load(bias + n);
+        s.y += zi_load(bias + n + 1);
+        s.z += zi_load(bias + n + 2);
+        s.w += zi_load(bias + n + 3);
+    }
+    if (out_f32) {
+        *reinterpret_cast<float4*>((float*)out + m * ldo + n) = s;
+    } else {
+        uint2 pk;
+        pk.x = zi_pack_bf16x2(s.x, s.y);
+        pk.y = zi_pack_bf16x2(s.z, s.w);
+        *reinterpret_cast<uint2*>((zi_bf16*)out + m * ldo + n) = pk;
+    }
+}
+
+// The sums added, by the one kernel where every four columns are whole 16-byte pieces (8-byte ones of a bfloat16 result), else by the
+// other: the same order, the same bits.
+static void sk_reduce(void* out, int out_f32, const float* partial, const zi_bf16* bias, int M, int N, int64_t ldo, int splits,
+                      hipStream_t stream) {
+    const int64_t total = (int64_t)M * N;
+    if (N % 4 == 0 && ldo % 4 == 0 && (uintptr_t)partial % 16 == 0 && (uintptr_t)out % (out_f32 ? 16 : 8) == 0 && splits <= 16) {
+#define ZI_SK_REDUCE(S)                                                                                                          \
+    case S:                                                                                                                      \
+        gemm_skinny_reduce4_kernel<S><<<(unsigned)((total / 4 + 63) / 64), 64, 0, stream>>>(out, out_f32, partial, bias, N, total, ldo); \
+        return
+        switch (splits) {
+            ZI_SK_REDUCE(1); ZI_SK_REDUCE(2); ZI_SK_REDUCE(3); ZI_SK_REDUCE(4); ZI_SK_REDUCE(5); ZI_SK_REDUCE(6); ZI_SK_REDUCE(7); ZI_SK_REDUCE(8);
+            ZI_SK_REDUCE(9); ZI_SK_REDUCE(10); ZI_SK_REDUCE(11); ZI_SK_REDUCE(12); ZI_SK_REDUCE(13); ZI_SK_REDUCE(14); ZI_SK_REDUCE(15); ZI_SK_REDUCE(16);
+        }
+#undef ZI_SK_REDUCE
+    }
+    gemm_skinny_reduce_kernel<<<(int)((total + 255) / 256), 256, 0, stream>>>(out, out_f32, partial, bias, M, N, ldo, splits);
+}
+
 #define SK_MAX_ROWS 256
 #define SK_MID_MAX_ROWS 128        // up to here one cut of the weights, beyond it another
 #define SK_MAX_ROWS_ACT 64         // ... with the epilogues that only products of few rows have
@@ -174,11 +231,7 @@ extern "C" int zi_gemm_skinny_act(void* out, int out_dt, int mode, const void* x
     const int of32 = out_dt == ZI_F32;
     const int rc = zi_gemm_mid_launch(dst, of32, kmode, (const zi_bf16*)x, (const zi_bf16*)w, b, M, N, K, ldx, ldw, ldo, vec_out, limit, stream);
     if (rc) return rc;
-    if (mode == SK_MODE_PLAIN && splits > 1) {
-        const int64_t total = (int64_t)M * N;
-        gemm_skinny_reduce_kernel<<<(int)((total + 255) / 256), 256, 0, stream>>>(out, of32, workspace,
-                                                                                  (const zi_bf16*)bias, M, N, ldo, splits);
-    }
+    if (mode == SK_MODE_PLAIN && splits > 1) sk_reduce(out, of32, workspace, (const zi_bf16*)bias, M, N, ldo, splits, stream);
     return zi_check_launch("gemm_skinny");
 }
 
@@ -195,8 +248,6 @@ extern "C" int zi_reduce_splits(void* out, int out_dt, const float* sums, const 
     ZI_REQUIRE(M >= 0 && N > 0 && splits >= 1 && ldo >= N, "reduce_splits: bad sizes");
     ZI_REQUIRE(out_dt == ZI_F32 || out_dt == ZI_BF16, "reduce_splits: unknown output dtype %d", out_dt);
     if (M == 0) return 0;
-    const int64_t total = (int64_t)M * N;
-    gemm_skinny_reduce_kernel<<<(int)((total + 255) / 256), 256, 0, stream>>>(out, out_dt == ZI_F32, sums,
-                                                                              (const zi_bf16*)bias, M, N, ldo, splits);
+    sk_reduce(out, out_dt == ZI_F32, sums, (const zi_bf16*)bias, M, N, ldo, splits, stream);
     return zi_check_launch("reduce_splits");
 }
