@@ -62,3 +62,17 @@ def test_which_tiles_a_step_takes(mean, experts, widths, rows):
     from zedinfer_amd import ops
     assert ops.moe_tile_rows(torch.bfloat16, torch.bfloat16, widths, mean * experts, experts) == rows
     assert ops.moe_tile_rows(torch.float32, torch.bfloat16, widths, mean * experts, experts) == 16
+
+
+@pytest.mark.parametrize("n,top,H", [(1, 1, 4), (3, 2, 260), (7, 4, 1536), (5, 5, 256), (33, 9, 132), (4, 3, 70), (2, 8, 1001)])
+def test_pairs_results_combined(n, top, H):
+    """Widths that are and are not whole pieces, a wavefront's columns not whole, one round of four pairs, a part of one and more."""
+    from zedinfer_amd import ops
+    g = torch.Generator().manual_seed(n * H)
+    y, wt = torch.randn(n * top, H, generator=g), torch.rand(n, top, generator=g)
+    place = torch.randperm(n * top, generator=g)
+    out = torch.full((n + 1, H), 7.0, device="cuda")
+    ops.moe_combine(y.cuda(), wt.cuda(), place.int().cuda(), out[:n])
+    terms = wt.double()[..., None] * y.double()[place].view(n, top, H)
+    # each of `top` multiply-adds rounds a sum that is at most the terms' sum of sizes
+    assert bool(((out[:n].cpu().double() - terms.sum(1)).abs() <= (top + 1) * 2.0 ** -24 * terms.abs().sum(1)).all()) and bool((out[n:] == 7.0).all())
