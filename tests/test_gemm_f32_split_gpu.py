@@ -1,0 +1,74 @@
+"""float32 products of more than 1,408 columns (csrc/gemm_f32_split.hip): products of bfloat16 parts that add up to the float32 product.
+What rides on the split itself, beyond what tests/test_gemm_f32_gpu.py asks of every float32 product."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# every kernel: groups of 8 rows, streams of 16 and 32 rows of x, x held for both (3, 4, 6, 8 chunks a run), tiles of every kind with rows,
+# weight rows and columns that end within a tile, a chunk and a run
+CASES = [(3, 1030, 1412, "pairs"), (8, 700, 9000, "pairs"), (12, 2070, 1412, "rows16"), (12, 300, 4100, "pairs"), (30, 2040, 1420, "rows16"), (40, 2040, 1500, "rows32"),
+         (7, 2059, 1536, "held_pairs"), (5, 2054, 1800, "held_pairs"), (8, 3000, 3000, "held_pairs"), (2, 2049, 4096, "held_pairs"),
+         (16, 5000, 1532, "held_rows16"), (13, 4098, 2048, "held_rows16"), (100, 2050, 1500, "tile_32_halves"), (500, 1500, 1480, "tile_96_halves"),
+         (449, 2047, 1540, "tile_64_quarters"), (700, 4610, 1412, "tile_64"), (450, 4610, 1500, "tile_32")]
+
+
+def _linear(M, N, K, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(M * 31 + N + seed)
+    return tuple(torch.randn(s, generator=g, device="cuda") for s in ((M, K), (N, K), (N,)))
+
+
+@pytest.mark.parametrize("M,N,K,kernel", CASES)
+def test_as_exact_as_float32_sums_and_without_a_bias(M, N, K, kernel):
+    from zedinfer_amd import ops
+    assert ops.linear_f32_kernel(M, N, K) == kernel
+    x, w, b = _linear(M, N, K)
+    got = ops.linear(x, w, b).double()
+    ref = x.double() @ w.double().t() + b.double()
+    # an instruction adds 32 products to the sum with errors of at most three of the sum's last bits, six instructions to 32 columns in
+    # each of two chains of an eighth of k (rounded up to chunks of 64), then eleven additions: so many times 2^-23 of at most sum |x w| + |b|
+    steps = 2 * 6 * -(-(-(-K // 64)) // 8) + 11
+    bound = steps * 2.0 ** -23 * (x.double().abs() @ w.double().abs().t() + b.double().abs())
+    assert bool(((got - ref).abs() <= bound).all())
+    # the same in the mean: the roundings of one chain's sums times 2^-24 of the result's rms each (the sums grow to it), added as squares
+    err = (got - ref).square().mean().sqrt() / ref.square().mean().sqrt()
+    assert float(err) <= 2.0 ** -24 * steps ** 0.5, float(err)
+    # the instruction rounds small products down: with one sign for both chains the mean error is a fifth of its rms and more
+    assert float((got - ref).mean().abs()) <= float((got - ref).square().mean().sqrt()) * (1 / 16 + 6 / (M * N) ** 0.5)
+    for rows in (slice(M - 1, M), slice(max(0, M - 11), M), slice(max(0, M - 40), M)):
+        assert torch.equal(ops.linear(x[rows].contiguous(), w, b).double(), got[rows])
+
+
+@pytest.mark.parametrize("M,N", [(3, 300), (3, 2100), (12, 4100), (12, 2070), (40, 2040), (100, 2050), (449, 1500), (449, 2047), (700, 4610)])
+def test_values_that_do_not_split(M, N):
+    """Infinities, NaNs and values that round to an infinity in bfloat16 give what the float32 sum gives, in their row and column alone;
+    small and subnormal values keep their last bits."""
+    from zedinfer_amd import ops
+    K = 1500
+    x, w = torch.ones(M, K, device="cuda"), torch.ones(N, K, device="cuda")
+    big = torch.finfo(torch.float32).max
+    x[0, 3], x[1, 1499], x[2, :] = float("inf"), big, 2.0 ** -130
+    w[5, 0], w[6, 7] = float("nan"), float("-inf")
+    y = ops.linear(x, w)
+    cols = [i for i in range(N) if i not in (5, 6)]
+    assert bool((y[0, cols] == float("inf")).all()) and bool(torch.isnan(y[:, 5]).all())
+    assert bool(torch.isnan(y[0, 6])) and bool((y[1:, 6] == float("-inf")).all())
+    assert bool((y[1, cols] == big).all())                      # (the other ones are far below its last bit)
+    assert bool((y[2, cols] == 1500 * 2.0 ** -130).all())
+    if M > 3:
+        assert bool((y[3:][:, cols] == 1500).all())
+    if ops.linear_swiglu_halves_supported(x, torch.cat([w, w])):
+        a = ops.linear_swiglu_halves(x, torch.cat([w, w]))
+        assert torch.equal(a.nan_to_num(), ops.swiglu(y, y).nan_to_num())
+
+
+def test_bits_depend_on_k_alone():
+    """On both sides of the bound on k every number of rows has the same bits, and whole numbers give whole numbers."""
+    from zedinfer_amd import ops
+    for K in (1408, 1412):
+        x, w, b = _linear(300, 2060, K)
+        whole = ops.linear(x, w, b)
+        for m in (1, 8, 9, 16, 17, 33, 130):
+            assert torch.equal(ops.linear(x[:m].contiguous(), w, b), whole[:m])
+    x, w = torch.randint(-8, 9, (40, 2000), device="cuda").float(), torch.randint(-8, 9, (300, 2000), device="cuda").float()
+    assert torch.equal(ops.linear(x, w).double(), x.double() @ w.double().t())

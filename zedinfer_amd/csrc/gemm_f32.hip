@@ -1,5 +1,8 @@
-// out[M,N] = x[M,K] . w[N,K]^T (+ bias[N]), everything float32, on the matrix cores' float32 instruction
-// (v_mfma_f32_16x16x4_f32: float32 products and float32 accumulation, no reduced precision).
+// out[M,N] = x[M,K] . w[N,K]^T (+ bias[N]), everything float32: the entry points, and the products of up to GF_SPLIT_ABOVE columns, on the
+// matrix cores' float32 instruction (v_mfma_f32_16x16x4_f32: float32 products and float32 accumulation, no reduced precision).  Longer k
+// goes to gemm_f32_split.hip, which adds up products of bfloat16 parts at up to 1.5 times the speed and with smaller errors; its start,
+// turning and splitting operands, costs a short k more than it gains (8 and 24 rows, us, here and there: 1,000 x 500 4.7 and 5.2, 5.5 and 6.1;
+// 5,000 x 1,100 9.9 and 9.6, 14.1 and 19.2; 9,000 x 128 5.7 and 6.3, 8.1 and 11.2).  Figures of longer k below are of these kernels too.
 //
 // One order of the sums, the same in every kernel here, so that a row's result does not depend on M, on the tile it
 // falls in or on the rest of the batch: k is cut into GF_PARTS runs of whole chunks of 32 (a function of K alone); within
@@ -21,56 +24,13 @@
 // 4,608 x 3,584 102 and 97.  The scheduling barriers keep the loads ahead of the products: without them the compiler moves a loop's
 // loads to its end and waits for all of them at its head.
 //
-// Measured, weights from memory, against the plain kernel (gemm_generic.hip: a chain of multiply-adds an output, scalar
-// loads), us, launch included: 8 rows 2,048 x 1,536 (N x K) 165 to 6; 1,536 x 8,960 914 to 20; 17,920 x 1,536 212 to 21 (5.2
-// TB/s, gemm_f32_held_kernel); 151,936 x 1,536 761 to 154 (6.0 TB/s; one row 139).  448 rows: 2,048 x 1,536 189 to 30, 1,536 x 8,960
-// 1,050 to 122 (101 TFLOP/s), 17,920 x 1,536 975 to 206 (120 TFLOP/s).  With the activation in its end the gate/up product of 512 rows
-// of 17,920 x 1,536 takes 235 us, of 1,024 452, where the two launches took 258 and 504.
-#include "zi_common.h"
+// Measured, weights from memory, us, launch included: 8 rows of 5,000 x 300 (N x K) 5.0, 1,000 x 500 4.7; 450 rows 22.5 and 10.5; 4,000 rows of
+// 4,000 x 512 160 (102 TFLOP/s).
+#include "zi_gemm_f32.h"
 
-typedef __attribute__((ext_vector_type(4))) float gf_f32x4_t;
-typedef __attribute__((ext_vector_type(4))) unsigned gf_u32x4_t;
-
-#define GF_PARTS 8           // runs of k; the wavefronts of the stream kernel
 #define GF_KB 32             // k of a chunk
+#define GF_HELD_CHUNKS 6      // chunks of a run that a wavefront may have to hold of x
 #define GF_BUFFERS 3         // chunks that the tile kernel holds in LDS, and as many on their way in registers
-#define GF_HELD_CHUNKS 16    // chunks of a run that a wavefront can hold of 8 rows of x beside as many of weights (256 registers)
-#define GF_OUT 0x7fffffff    // an offset past the end of every buffer: the load gives zeros and fetches nothing
-
-union gf_pack {
-    gf_u32x4_t u;
-    gf_f32x4_t f;
-};
-
-// Rows base .. base + rows - 1 of a row-major matrix as a buffer whose range ends with the last row's K values.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t gf_rows(const float* base, int64_t ld, int rows, int K) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, (int)(((int64_t)(rows - 1) * ld + K) * 4), 0x00020000);
-}
-
-template <int AUX>
-__device__ __forceinline__ gf_f32x4_t gf_load(__amdgpu_buffer_rsrc_t rows, int offset) {
-    gf_pack p;
-    p.u = __builtin_amdgcn_raw_buffer_load_b128(rows, offset, 0, AUX);
-    return p.f;
-}
-
-// Four outputs of one row of x, columns n .. n + 3.
-__device__ __forceinline__ void gf_store4(float* __restrict__ out, const float* __restrict__ bias, gf_f32x4_t s, int n, int N, int vec_out) {
-    if (bias) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s[e] += n + e < N ? bias[n + e] : 0.f;
-    }
-    if (vec_out && n + 3 < N) {
-        *reinterpret_cast<gf_f32x4_t*>(out + n) = s;
-    } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (n + e < N) out[n + e] = s[e];
-    }
-}
-
-// up * silu(gate), the arithmetic of the activation's own kernel (elementwise.hip).
-__device__ __forceinline__ float gf_gate(float gate, float up) { return up * (gate / (1.f + expf(-gate))); }
 
 // PAIR: 8 weight rows and up to 8 rows of x; else 16 weight rows and up to 16 * MT rows of x a workgroup.  RING chunks are
 // on their way while one is worked on.
@@ -441,9 +401,6 @@ bool zi_gemm_f32_takes(const void* x, const void* w, int N, int K, int64_t ldx, 
            N <= (1 << 25);
 }
 
-// The kernels a product can take; all give the same bits.
-enum gf_kernel { GF_PAIRS, GF_ROWS16, GF_ROWS32, GF_HELD_PAIRS, GF_HELD_ROWS16, GF_TILE_64, GF_TILE_32, GF_TILE_32_HALVES, GF_TILE_96_HALVES };
-
 // Which kernel M rows of x and N weight rows take is a matter of filling the compute units only.  Up to 16 rows a stream of the
 // weights, 8 or 16 of them a workgroup (one row of a 151,936-row head 190 in pairs, 233 us without), with x held in registers once
 // there are more such groups than units and k is not too long for it (see there).  9 to 16 rows go twice over groups of 8 weight rows
@@ -465,11 +422,13 @@ enum gf_kernel { GF_PAIRS, GF_ROWS16, GF_ROWS32, GF_HELD_PAIRS, GF_HELD_ROWS16, 
 // 7.7 and 7.9).  Up to K = 64 a workgroup is little more than its start, so the
 // larger tiles (1,024 rows, 9,000 x 64: 20.4 against 22.8, in halves 59), after 32 rows a workgroup up to two a unit (320 rows, 256 x 32:
 // 3.3 against 3.6 us).
-static gf_kernel gf_kernel_for(int M, int64_t N, int chunks, int per) {
+static gf_kernel gf_kernel_for(int M, int64_t N, int K) {
+    if (K > GF_SPLIT_ABOVE) return zi_gemm_f32_split_kernel(M, N, K);
+    const int chunks = (K + GF_KB - 1) / GF_KB;
     const int64_t cus = zi_compute_units(), n16 = (N + 15) / 16, m32 = (M + 31) / 32;
     const int64_t t32 = m32 * ((N + 63) / 64), t96 = m32 * ((N + 95) / 96), t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
-    if (M <= 8) return (N + 7) / 8 > cus && per <= GF_HELD_CHUNKS ? GF_HELD_PAIRS : GF_PAIRS;
-    if (M <= 16 && n16 > cus && per <= GF_HELD_CHUNKS / 2) return GF_HELD_ROWS16;
+    if (M <= 8) return (N + 7) / 8 > cus ? GF_HELD_PAIRS : GF_PAIRS;
+    if (M <= 16 && n16 > cus) return GF_HELD_ROWS16;
     if (M <= 16) return (N + 7) / 8 * 2 <= cus ? GF_PAIRS : GF_ROWS16;
     if (n16 * ((M + 15) / 16) <= cus) return GF_ROWS16;
     if (M <= 32 || n16 * m32 <= (chunks <= 2 ? 2 : 1) * cus) return GF_ROWS32;
@@ -483,13 +442,15 @@ static gf_kernel gf_kernel_for(int M, int64_t N, int chunks, int per) {
 
 // (for tests: the kernel by its place in the list above)
 extern "C" int zi_gemm_f32_kernel(int M, int N, int K) {
-    const int chunks = (K + GF_KB - 1) / GF_KB;
-    return gf_kernel_for(M, N, chunks, (chunks + GF_PARTS - 1) / GF_PARTS);
+    return gf_kernel_for(M, N, K);
 }
+
+static_assert((GF_SPLIT_ABOVE + GF_KB - 1) / GF_KB <= GF_PARTS * GF_HELD_CHUNKS, "the longest k's runs fit the kernels that hold x");
 
 template <bool GATED>
 static int gf_launch(float* out, const float* x, const float* w, const float* bias, int M, int N, int K, int64_t ldx, int64_t ldw,
                      int64_t ldo, hipStream_t stream) {
+    if (K > GF_SPLIT_ABOVE) return zi_gemm_f32_split_launch(GATED, out, x, w, bias, M, N, K, ldx, ldw, ldo, stream);
     const int chunks = (K + GF_KB - 1) / GF_KB, per = (chunks + GF_PARTS - 1) / GF_PARTS;
     const int vec_out = ldo % 4 == 0 && (uintptr_t)out % 16 == 0;
 #define ZI_GF_STREAM(MT, PAIR, RING)                                                                                                     \
@@ -514,20 +475,16 @@ static int gf_launch(float* out, const float* x, const float* w, const float* bi
                                                                                                    K, ldx, ldw, ldo, per, vec_out, mt, tiles);  \
         }                                                                                                                                 \
     } while (0)
-    switch (gf_kernel_for(M, (int64_t)N * (GATED ? 2 : 1), chunks, per)) {
+    switch (gf_kernel_for(M, (int64_t)N * (GATED ? 2 : 1), K)) {
         case GF_HELD_PAIRS:
             if (per <= 2) ZI_GF_HELD(true, 2);
             else if (per <= 4) ZI_GF_HELD(true, 4);
-            else if (per <= 6) ZI_GF_HELD(true, 6);
-            else if (per <= 8) ZI_GF_HELD(true, 8);
-            else if (per <= 12) ZI_GF_HELD(true, 12);
-            else ZI_GF_HELD(true, 16);
+            else ZI_GF_HELD(true, 6);
             break;
         case GF_HELD_ROWS16:
             if (per <= 2) ZI_GF_HELD(false, 2);
             else if (per <= 4) ZI_GF_HELD(false, 4);
-            else if (per <= 6) ZI_GF_HELD(false, 6);
-            else ZI_GF_HELD(false, 8);
+            else ZI_GF_HELD(false, 6);
             break;
         case GF_TILE_64:
             if (chunks <= 2) ZI_GF_TILE(64, 2, 1, true);
@@ -539,7 +496,7 @@ static int gf_launch(float* out, const float* x, const float* w, const float* bi
             if constexpr (GATED) {
                 return zi_fail("gemm_f32: no gated kernel for %d rows of %d x %d", M, N, K);      // (zi_gemm_f32_swiglu_takes says so)
             } else {
-                switch (gf_kernel_for(M, N, chunks, per)) {
+                switch (gf_kernel_for(M, N, K)) {
                     case GF_PAIRS: ZI_GF_STREAM(1, true, 6); break;
                     case GF_ROWS16: ZI_GF_STREAM(1, false, 4); break;
                     case GF_ROWS32: ZI_GF_STREAM(2, false, 3); break;
@@ -564,9 +521,8 @@ int zi_gemm_f32_launch(float* out, const float* x, const float* w, const float* 
 extern "C" int zi_gemm_f32_swiglu_takes(const void* x, const void* w, int M, int inter, int K, int64_t ldx, int64_t ldw) {
     if (M < 1 || M > 65535 * 64 || inter < 1 || K < 1 || inter > (1 << 24) || ldx < K || ldw < K || !zi_gemm_f32_takes(x, w, 2 * inter, K, ldx, ldw)) return 0;
     if (((int64_t)inter + 64) * ldw * 4 >= (1ll << 31) - 64) return 0;
-    const int chunks = (K + GF_KB - 1) / GF_KB, per = (chunks + GF_PARTS - 1) / GF_PARTS;
-    const gf_kernel k = gf_kernel_for(M, 2ll * inter, chunks, per);
-    return k == GF_HELD_PAIRS || k == GF_HELD_ROWS16 || k == GF_TILE_64 || k == GF_TILE_32 || k == GF_TILE_32_HALVES;
+    const gf_kernel k = gf_kernel_for(M, 2ll * inter, K);
+    return k == GF_HELD_PAIRS || k == GF_HELD_ROWS16 || k == GF_TILE_64 || k == GF_TILE_32 || k == GF_TILE_32_HALVES || k == GF_TILE_64_QUARTERS;
 }
 
 // out[M, inter] = up * silu(gate), gate and up the products of x with the first and the last inter rows of w: the bits of the product

@@ -1,0 +1,680 @@
+// out[M,N] = x[M,K] . w[N,K]^T (+ bias[N]), everything float32 and K above GF_SPLIT_ABOVE, on the matrix cores' bfloat16 instruction
+// (v_mfma_f32_16x16x32_bf16, sixteen times the multiply-adds a cycle of the float32 one).
+//
+// A float32 value is the sum of three bfloat16 ones, exactly: itself rounded, what is left rounded, and what is left of that (8 + 8 + 8 bits).
+// Of the nine products of two values' parts the six largest are added; the other three lie below 2^-26 of the product.  Weights and x stay
+// float32 in memory and are split on their way into the matrix cores; sums are float32.  A value whose first part rounds to an infinity,
+// and infinities and NaNs themselves, leave parts that are no numbers, so a sum that is not finite is made again from the float32 operands
+// (gf_finite).  Small and subnormal values keep their bits: the instruction takes subnormal parts.
+//
+// The instruction cuts off what lies more than some three bits below its largest term's last bit, downwards whatever the sign, so sums come
+// out low, by a quarter of their rounding errors at 8,960 columns, every output alike; over a model's layers that adds up.  So one of the two
+// chains below is summed with x negated and subtracted: the two errors cancel in the mean.  Error against 64 bits, 2-norm over 2-norm,
+// of the float32 instruction's kernels, of these without the change of sign, of these: 1,536 columns 1.86e-7, 1.42e-7, 1.39e-7; 8,960
+// columns 4.3e-7, 3.7e-7, 3.6e-7; the logits of a 28-layer model 3.7e-7, 4.5e-7, 3.3e-7.
+//
+// One order of the sums, the same in every kernel here, so that a row's result does not depend on M, on the tile it falls in or on the rest
+// of the batch: k is cut into GF_PARTS runs of whole chunks of 64 (a function of K alone); within a run the first and the second 32 of every
+// chunk are two chains, each 32 an instruction for every product of parts, whose lane group g holds k = 4 g .. 4 g + 3 and 16 more; a run's
+// sum is first - second chain; the sums of each half of the runs are added in rising order, then the two halves, then the bias.
+//
+// What bounds it: few rows the one pass over the weights; many rows, by counters at 2,048 rows of 4,096 x 4,096, the vector instructions
+// (57 % of the cycles, eleven for every two values split) and the matrix cores (51 %), which mostly take turns, beside LDS (43 %).
+//
+// Measured, weights from memory, against the float32 instruction's kernels, us, launch included (N x K): 8 rows 2,048 x 1,536 6.9 to 6.7, 1,536 x
+// 8,960 21.3 to 19.0, 17,920 x 1,536 with the activation 23.2 to 21.7; 24 rows 1,536 x 8,960 35.6 to 25.8, 17,920 x 1,536 46.7 to 38.0; 64 rows
+// 1,536 x 8,960 53.5 to 40.6; 512 rows 2,048 x 1,536 32.4 to 28.3, 1,536 x 8,960 136 to 109 (129 TFLOP/s), 17,920 x 1,536 with the activation 232
+// to 184 (153 TFLOP/s); 2,048 rows of 4,608 x 3,584 538 to 406 (166 TFLOP/s; the float32 instruction in a large library product: 152).  Slower: one
+// row of 2,048 x 1,536 5.9 to 6.2, 9 rows of 17,920 x 1,536 with the activation 23.9 to 25.4.
+#include "zi_gemm_f32.h"
+
+#define GF_KB 64             // k of a chunk
+#define GF_HELD_CHUNKS 8     // chunks of a run that a wavefront can hold of 8 rows of x beside as many of weights (256 registers)
+
+// The three bfloat16 parts of eight values, largest first.
+struct gf_parts {
+    gf_pack p[3];
+};
+
+__device__ __forceinline__ gf_parts gf_split(gf_f32x4_t a, gf_f32x4_t b) {
+    gf_parts s;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float lo = i < 2 ? a[2 * i] : b[2 * i - 4], hi = i < 2 ? a[2 * i + 1] : b[2 * i - 3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            const uint32_t u = zi_pack_bf16x2(lo, hi);
+            s.p[p].u[i] = u;
+            if (p < 2) {
+                lo -= __uint_as_float(u << 16);             // exactly: what is left fits a float32
+                hi -= __uint_as_float(u & 0xffff0000u);
+            }
+        }
+    }
+    return s;
+}
+
+enum gf_sign { GF_PLUS, GF_MINUS, GF_MINUS_SECOND };
+
+// A block of 16 lines of 128 bytes, loaded as whole lines (lane l, load i: piece l % 8 of line 8 i + l / 8), as the matrix cores' operand:
+// lane (r, g) gets pieces g and 4 + g of line r, split.  Loads in the operand's own layout would take a line's pieces by lanes 16 apart,
+// which the vector cache serves one lane at a time: 52 instead of 16 of its cycles for an instruction's 1 KB, 16 bytes a clock and unit.
+// SIGN: the values, their negatives, or (of blocks that hold both chains) the negatives of the second chain's lines.
+// `block` is 2 KB of LDS of this wavefront alone (piece c of line q at place c xor (q / 2 mod 8), free of bank conflicts both ways); a
+// wavefront's LDS accesses are in order, so there is nothing to wait for between one block and the next.
+template <gf_sign SIGN>
+__device__ __forceinline__ gf_parts gf_turn(gf_f32x4_t* block, gf_f32x4_t line0, gf_f32x4_t line8, int lane) {
+    const int r = lane & 15, g = lane >> 4, q = lane >> 3, c = lane & 7;
+    block[q * 8 + (c ^ (q >> 1))] = line0;
+    block[(8 + q) * 8 + (c ^ (4 + (q >> 1)))] = line8;
+    gf_f32x4_t a = block[r * 8 + (g ^ (r >> 1))], b = block[r * 8 + ((4 + g) ^ (r >> 1))];
+    if (SIGN == GF_MINUS) {
+        a = -a;
+        b = -b;
+    } else if (SIGN == GF_MINUS_SECOND) {
+        gf_pack p, o;
+        p.f = a;
+        o.f = b;
+        p.u ^= (unsigned)(lane & 8) << 28;
+        o.u ^= (unsigned)(lane & 8) << 28;
+        a = p.f;
+        b = o.f;
+    }
+    return gf_split(a, b);
+}
+
+// A block of x of chain h, or (PAIR) of both chains; the second chain's negated (see the top).
+template <bool PAIR>
+__device__ __forceinline__ gf_parts gf_turn_of_chain(int h, gf_f32x4_t* block, gf_f32x4_t line0, gf_f32x4_t line8, int lane) {
+    if (PAIR) return gf_turn<GF_MINUS_SECOND>(block, line0, line8, lane);
+    return h ? gf_turn<GF_MINUS>(block, line0, line8, lane) : gf_turn<GF_PLUS>(block, line0, line8, lane);
+}
+
+// acc += w . x over the 32 k of an instruction: the six products of parts that reach float32's last bits, the smallest first.
+__device__ __forceinline__ gf_f32x4_t gf_multiply(const gf_parts& w, const gf_parts& x, gf_f32x4_t acc) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.p[2].b, x.p[0].b, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.p[0].b, x.p[2].b, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.p[1].b, x.p[1].b, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.p[1].b, x.p[0].b, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.p[0].b, x.p[1].b, acc, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.p[0].b, x.p[0].b, acc, 0, 0, 0);
+}
+
+// The sum as it is if it is finite.  Else an operand was an infinity, a NaN or a value whose first part rounds to an infinity, whose other
+// parts are no numbers, or the sum left the range: the same sum again from the float32 operands, one k after the other.
+__device__ __forceinline__ float gf_finite(float sum, const float* __restrict__ x_row, const float* __restrict__ w_row, int K) {
+    if ((__float_as_uint(sum) & 0x7f800000u) != 0x7f800000u) return sum;
+    float s = 0.f;
+    for (int k = 0; k < K; k += 4) {
+        const gf_f32x4_t a = *reinterpret_cast<const gf_f32x4_t*>(x_row + k), b = *reinterpret_cast<const gf_f32x4_t*>(w_row + k);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s = fmaf(a[e], b[e], s);
+    }
+    return s;
+}
+
+// PAIR: 8 weight rows and up to 8 rows of x; else 16 weight rows and up to 16 * MT rows of x a workgroup.  RING chunks are
+// on their way while one is worked on.
+template <int MT, bool PAIR, int RING>
+__global__ void __launch_bounds__(GF_PARTS* ZI_WAVE, 4)
+gemm_f32_split_stream_kernel(float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,
+                       const float* __restrict__ bias, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int per, int vec_out) {
+    constexpr int NR = PAIR ? 8 : 16, MR = PAIR ? 8 : 16 * MT, H = PAIR ? 1 : 2;
+    __shared__ __attribute__((aligned(16))) gf_f32x4_t part[GF_PARTS][MT][ZI_WAVE];
+    const int lane = threadIdx.x & (ZI_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / ZI_WAVE);
+    const int r = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * NR, m0 = blockIdx.y * MR;
+    const int rows_w = N - n0 < NR ? N - n0 : NR, rows_x = M - m0 < MR ? M - m0 : MR;
+    const __amdgpu_buffer_rsrc_t wb = gf_rows(w + (int64_t)n0 * ldw, ldw, rows_w, K), xb = gf_rows(x + (int64_t)m0 * ldx, ldx, rows_x, K);
+    __shared__ __attribute__((aligned(16))) gf_f32x4_t turn[GF_PARTS][1 + MT][128];
+    // a block of 16 lines is the rows' lines of one chain, or (PAIR) both chains' lines of 8 rows
+    constexpr int RB = PAIR ? 1 : 2;               // loads of different rows a block
+    const int k_lane = (lane & 7) * 16;
+    int w_row[RB], x_row[MT][RB];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+        const int row = i * 8 + (lane >> 3);
+        w_row[i] = row < rows_w ? (int)(row * ldw * 4) : GF_OUT;
+#pragma unroll
+        for (int t = 0; t < MT; ++t) x_row[t][i] = t * 16 + row < rows_x ? (int)((t * 16 + row) * ldx * 4) : GF_OUT;
+    }
+    const int chunks = (K + GF_KB - 1) / GF_KB;
+    const int c0 = wave * per, c1 = c0 + per < chunks ? c0 + per : chunks;
+
+    gf_f32x4_t wr[RING][H][2], xr[RING][H][MT][2];
+    auto fetch = [&](const int slot, int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int h = 0; h < H; ++h)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int k = c * (GF_KB * 4) + (PAIR ? i : h) * 128 + k_lane;
+                const bool in = c < c1 && k < K * 4;
+#pragma unroll
+                for (int t = 0; t < MT; ++t) xr[slot][h][t][i] = gf_load<0>(xb, in && x_row[t][i % RB] != GF_OUT ? x_row[t][i % RB] + k : GF_OUT);
+                // a weight of up to 8 rows of x is read once by one workgroup: past L2
+                wr[slot][h][i] = gf_load<PAIR ? 2 : 0>(wb, in && w_row[i % RB] != GF_OUT ? w_row[i % RB] + k : GF_OUT);
+            }
+    };
+    gf_f32x4_t acc[H][MT];
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[h][t] = gf_f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < RING; ++s) {
+        fetch(s, c0 + s);
+        __builtin_amdgcn_sched_barrier(0);         // in this order: the loop waits for the oldest only
+    }
+    for (int c = c0; c < c1; c += RING) {
+#pragma unroll
+        for (int s = 0; s < RING; ++s) {
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+                const gf_parts ws = gf_turn<GF_PLUS>(turn[wave][0], wr[s][h][0], wr[s][h][1], lane);
+#pragma unroll
+                for (int t = 0; t < MT; ++t)
+                    acc[h][t] = gf_multiply(ws, gf_turn_of_chain<PAIR>(h, turn[wave][1 + t], xr[s][h][t][0], xr[s][h][t][1], lane), acc[h][t]);
+            }
+            __builtin_amdgcn_sched_barrier(0);     // the loads stay this far ahead of their use
+            fetch(s, c + s + RING);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    // lane (r, g) holds rows 4 g .. 4 g + 3 of column r; PAIR: the first chain in the quadrant of rows and columns 0 .. 7, the
+    // second in the one of 8 .. 15 (the others mix the halves and are dropped)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        gf_f32x4_t s = acc[0][t];
+        if (PAIR) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] -= __shfl(acc[0][t][e], (lane + 40) & 63, ZI_WAVE);
+        } else {
+            s -= acc[H - 1][t];
+        }
+        part[wave][t][lane] = s;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < MT * ZI_WAVE; i += GF_PARTS * ZI_WAVE) {
+        const int t = i / ZI_WAVE, l = i % ZI_WAVE, m = t * 16 + (l & 15), n = (l >> 4) * 4;
+        gf_f32x4_t s = part[0][t][l], s2 = part[GF_PARTS / 2][t][l];
+#pragma unroll
+        for (int p = 1; p < GF_PARTS / 2; ++p) {
+            s += part[p][t][l];
+            s2 += part[GF_PARTS / 2 + p][t][l];
+        }
+        s += s2;
+        if (m < rows_x && n < rows_w) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (n + e < rows_w) s[e] = gf_finite(s[e], x + (m0 + m) * ldx, w + (int64_t)(n0 + n + e) * ldw, K);
+            gf_store4(out + (int64_t)(m0 + m) * ldo, bias, s, n0 + n, N, vec_out);
+        }
+    }
+}
+
+// The same for up to 16 rows of x and more groups of weight rows than there are compute units: a workgroup keeps its wavefronts' runs
+// of x in registers, split into their parts once (PER chunks a wavefront, at most), and walks over groups of 8 (PAIR) or 16 weight rows,
+// gridDim.x apart.  As soon as a chunk of weights has been used, its registers are filled with the same chunk of the next group: PER
+// chunks are always on their way, x passes the loads once a workgroup instead of once a group, as many bytes again as the weights' for 8
+// rows, and a workgroup's start and end come once.  The eight runs' sums meet in one of two LDS buffers, so a group costs one barrier,
+// which does not wait for loads; the wavefronts take the adding and storing in turn.  GATED: a group is as many gate rows as up rows (row
+// n and row N + n of w) and the outputs are up * silu(gate).
+//
+// Bound by the stream of the weights: 151,936 x 1,536 at 8 rows 161 us (5.8 TB/s).  Two workgroups a unit while a lane has registers for that
+// (128): with 4 chunks of x they spill, and one is faster (5,000 x 2,048 with the activation, one row: 17.4 against 20.8 us).
+template <bool PAIR, int PER, bool GATED>
+__global__ void __launch_bounds__(GF_PARTS* ZI_WAVE, (PAIR ? 1 : 2) * PER <= 3 ? 4 : 2)
+gemm_f32_split_held_kernel(float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
+                     int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int per, int vec_out, int groups) {
+    constexpr int NR = PAIR ? 8 : 16, NC = GATED ? NR / 2 : NR, H = PAIR ? 1 : 2;
+    __shared__ __attribute__((aligned(16))) gf_f32x4_t part[2][GF_PARTS][ZI_WAVE];
+    const int lane = threadIdx.x & (ZI_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / ZI_WAVE);
+    __shared__ __attribute__((aligned(16))) gf_f32x4_t turn[GF_PARTS][2][128];
+    constexpr int RB = PAIR ? 1 : 2;               // as above
+    const int r = lane & 15, g = lane >> 4;
+    const int chunks = (K + GF_KB - 1) / GF_KB, c0 = wave * per;
+    const int mine = chunks - c0 < per ? chunks - c0 : per;       // chunks of this wavefront's run (none or fewer at the end of k)
+    const int k0 = c0 * (GF_KB * 4) + (lane & 7) * 16;            // the first byte of a row that this lane loads
+    const __amdgpu_buffer_rsrc_t xb = gf_rows(x, ldx, M, K);
+    int x_row[RB], w_row[RB];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+        const int row = i * 8 + (lane >> 3);
+        x_row[i] = row < M ? (int)(row * ldx * 4) : GF_OUT;
+        w_row[i] = (int)((GATED && row >= NC ? N + row - NC : row) * ldw * 4);
+    }
+    // the weight rows of a group: what lies past the last one gives zeros (or, of a gate row past the last, an output that is not stored)
+    auto weights = [&](int group) {
+        const int64_t n0 = (int64_t)group * NC;
+        const int rows = group >= groups ? 0 : (GATED ? N : 0) + (int)(N - n0 < NC ? N - n0 : NC);
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(w + (rows ? n0 * ldw : 0)), 0,
+                                                 rows ? (int)(((int64_t)(rows - 1) * ldw + K) * 4) : 0, 0x00020000);
+    };
+    auto place = [&](int s, int h, int i) { return s * (GF_KB * 4) + (PAIR ? i : h) * 128; };
+    auto in = [&](int s, int h, int i) { return s < mine && k0 + place(s, h, i) < K * 4; };
+    gf_f32x4_t wr[PER][H][2];
+    gf_parts xs[PER][H];
+    __amdgpu_buffer_rsrc_t wb = weights(blockIdx.x);
+    auto fetch = [&](const int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int h = 0; h < H; ++h)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) wr[s][h][i] = gf_load<2>(wb, in(s, h, i) ? w_row[i % RB] + k0 + place(s, h, i) : GF_OUT);
+    };
+    {
+        gf_f32x4_t xr[PER][H][2];
+#pragma unroll
+        for (int s = 0; s < PER; ++s)
+#pragma unroll
+            for (int h = 0; h < H; ++h)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    xr[s][h][i] = gf_load<0>(xb, in(s, h, i) && x_row[i % RB] != GF_OUT ? x_row[i % RB] + k0 + place(s, h, i) : GF_OUT);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < PER; ++s) {
+            fetch(s);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int s = 0; s < PER; ++s)
+#pragma unroll
+            for (int h = 0; h < H; ++h) xs[s][h] = gf_turn_of_chain<PAIR>(h, turn[wave][(s * H + h) & 1], xr[s][h][0], xr[s][h][1], lane);
+    }
+    int b = 0, whose = 0;
+    for (int group = blockIdx.x; group < groups; group += gridDim.x, b ^= 1, whose = (whose + 1) % GF_PARTS) {
+        wb = weights(group + (int)gridDim.x);
+        gf_f32x4_t acc[H];
+#pragma unroll
+        for (int h = 0; h < H; ++h) acc[h] = gf_f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < PER; ++s) {
+#pragma unroll
+            for (int h = 0; h < H; ++h) acc[h] = gf_multiply(gf_turn<GF_PLUS>(turn[wave][(s * H + h) & 1], wr[s][h][0], wr[s][h][1], lane), xs[s][h], acc[h]);
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(s);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        gf_f32x4_t sum = acc[0];
+        if (PAIR) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum[e] -= __shfl(acc[0][e], (lane + 40) & 63, ZI_WAVE);
+        } else {
+            sum -= acc[H - 1];
+        }
+        part[b][wave][lane] = sum;
+        // all sums are in LDS (and the buffer's reader of two groups ago is past the barrier of the last one); loads travel on
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        if (wave != whose) continue;
+        gf_f32x4_t s = part[b][0][lane], s2 = part[b][GF_PARTS / 2][lane];
+#pragma unroll
+        for (int p = 1; p < GF_PARTS / 2; ++p) {
+            s += part[b][p][lane];
+            s2 += part[b][GF_PARTS / 2 + p][lane];
+        }
+        s += s2;
+        const int64_t n = (int64_t)group * NC + g * 4;
+        if (r < M && g * 4 < NR) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {       // sum e of this lane is weight row g * 4 + e of the group
+                const int of = g * 4 + e, up = GATED && of >= NC;
+                const int64_t at = (int64_t)group * NC + (up ? of - NC : of);
+                if (at < N) s[e] = gf_finite(s[e], x + r * ldx, w + (at + (up ? N : 0)) * ldw, K);
+            }
+        }
+        if (GATED) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] = gf_gate(s[e], __shfl(s[e], lane + (PAIR ? 16 : 32), ZI_WAVE));
+        }
+        if (r < M && g * 4 < NC && n < N) gf_store4(out + (int64_t)r * ldo, bias, s, (int)n, N, vec_out);
+    }
+}
+
+// 16 MT rows of x by 16 NT WAVES weight rows a workgroup, 16 NT weight rows a wavefront; GROUPS (1 or 4) groups of WAVES wavefronts,
+// each over as many eighths of k.  A step is half a chunk, 32 k, one of the two chains.  A wavefront's weight rows are its own: they go
+// from memory into its registers, DEPTH steps ahead, and are split there.  x, which all wavefronts of a group share, is split by the
+// threads that loaded it and goes through LDS as its parts, two buffers, one barrier a step that does not wait for loads.
+// GATED (NT even): of a wavefront's blocks of 16 weight rows the even ones are gate rows and the odd ones the up rows of the same outputs
+// (rows n and N + n of w), and half as many outputs, up * silu(gate), are what the tile leaves.
+// With both operands loaded in the matrix cores' layout (see gf_turn) 512 rows of 1,536 x 8,960 took 126 us and now 109, 256 of 17,920 x 1,536
+// 136 and 120; with two groups of wavefronts instead of four, and one wavefront a SIMD, 160.  Tiles of 128 x 128 with one wavefront a SIMD
+// are no faster (2,048 rows of 4,096 x 4,096 406 against 403 us), nor is one more vector instruction less a pair by v_dot2 (the matrix
+// cores do not run beside it).
+template <int MT, int NT, int WAVES, int GROUPS, bool GATED>
+__global__ void __launch_bounds__(ZI_WAVE* WAVES* GROUPS, GROUPS > 1 ? WAVES * GROUPS / 4 : MT * NT <= 4 ? 3 : 2)
+gemm_f32_split_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,
+                     const float* __restrict__ bias, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int per, int vec_out,
+                     int m_tiles, int tiles) {
+    static_assert(!GATED || NT % 2 == 0, "as many gate as up blocks a wavefront");
+    constexpr int TM = 16 * MT, TN = 16 * NT * WAVES, NC = GATED ? TN / 2 : TN, NW = NC / WAVES;     // NW outputs a row and wavefront
+    constexpr int THREADS = ZI_WAVE * WAVES, PIECES = TM * 4, XP = (PIECES + THREADS - 1) / THREADS;
+    constexpr int DEPTH = GROUPS == 1 ? 2 : 1, RUNS = GF_PARTS / GROUPS, SUMS = GROUPS == 1 ? 1 : RUNS;
+    constexpr bool TOGETHER = GROUPS == 1 && MT * NT > 4;     // two wavefronts a SIMD
+    constexpr int BLOCKS = WAVES * MT * NT;                  // 16 x 16 blocks of the tile
+    constexpr int X_BYTES = GROUPS * 2 * 3 * PIECES * 16, SUM_BYTES = GROUPS == 1 ? 0 : GF_PARTS * BLOCKS * ZI_WAVE * 16, FIRST_BYTES = GROUPS == 1 ? BLOCKS * ZI_WAVE * 16 : 0, TURN_BYTES = GROUPS * WAVES * NT * 2048;
+    __shared__ __attribute__((aligned(16))) gf_u32x4_t lds_all[(GROUPS == 1 || X_BYTES + TURN_BYTES > SUM_BYTES ? X_BYTES + TURN_BYTES + FIRST_BYTES : SUM_BYTES) / 16];
+    gf_u32x4_t(*lds)[2][3][PIECES] = reinterpret_cast<gf_u32x4_t(*)[2][3][PIECES]>(lds_all);
+    gf_f32x4_t* first = reinterpret_cast<gf_f32x4_t*>(lds_all) + (X_BYTES + TURN_BYTES) / 16 + (int)threadIdx.x;      // one group: sums of the first half of the runs
+    // the tiles that share weight rows follow each other on one XCD (workgroup i runs on XCD i mod 8)
+    const int per_xcd = (tiles + 7) / 8, tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if (tile >= tiles) return;
+    const int m0 = (tile % m_tiles) * TM, n0 = (tile / m_tiles) * NC;
+    const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x / ZI_WAVE), group = wave_all / WAVES, wave = wave_all % WAVES;
+    const int lane = threadIdx.x & (ZI_WAVE - 1), tid = wave * ZI_WAVE + lane;
+    const int r = lane & 15, g = lane >> 4;
+    const int rows_w = N - n0 < NC ? N - n0 : NC, rows_x = M - m0 < TM ? M - m0 : TM;
+    const __amdgpu_buffer_rsrc_t wb = gf_rows(w + (int64_t)n0 * ldw, ldw, (GATED ? N : 0) + rows_w, K), xb = gf_rows(x + (int64_t)m0 * ldx, ldx, rows_x, K);
+    // a thread's pieces of x: the eight values of lane group i % 4 of row i / 4, i = tid, tid + THREADS, ...; piece c of row q lies at
+    // place c xor (-(q / 4) mod 4), which keeps the operand reads free of bank conflicts (a read of 16 bytes a lane serves lanes 0 to 3, 12 to
+    // 15 and 20 to 27 in one turn)
+    int x_row[XP], x_place[XP], w_row[NT][2];
+    const int x_lane = (tid & 3) * 16, w_lane = (lane & 7) * 16;
+    gf_f32x4_t* turn = reinterpret_cast<gf_f32x4_t*>(lds_all) + X_BYTES / 16 + wave_all * NT * 128;
+#pragma unroll
+    for (int p = 0; p < XP; ++p) {
+        const int i = tid + p * THREADS, q = i >> 2;
+        x_row[p] = q < rows_x && i < PIECES ? (int)(q * ldx * 4) + x_lane : GF_OUT;
+        x_place[p] = q * 4 + ((i ^ -(q >> 2)) & 3);
+    }
+#pragma unroll
+    for (int u = 0; u < NT; ++u)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int q = wave * NW + (GATED ? u / 2 : u) * 16 + i * 8 + (lane >> 3);
+            w_row[u][i] = q < rows_w ? (int)((q + (GATED && (u & 1) ? N : 0)) * ldw * 4) + w_lane : GF_OUT;
+        }
+    const int chunks = (K + GF_KB - 1) / GF_KB, mine = per * RUNS;
+    const int c0 = group * mine, c1 = GROUPS > 1 && c0 + mine < chunks ? c0 + mine : chunks;
+    const int steps = GROUPS > 1 ? mine : chunks;      // chunks, the same number for all groups: they share the barriers
+    gf_f32x4_t xr[DEPTH][XP][2], wr[DEPTH][NT][2];
+    // (the step's place along k is the loads' scalar offset; bytes of a row from there on, none past the group's last chunk)
+    auto left = [&](const int h, int c) { return c < c1 ? K * 4 - c * (GF_KB * 4) - h * 128 : 0; };
+    auto fetch_x = [&](const int h, int c) __attribute__((always_inline)) {
+        const int rest = left(h, c);
+#pragma unroll
+        for (int p = 0; p < XP; ++p)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) xr[h % DEPTH][p][q] = gf_load<0>(xb, x_lane + q * 64 < rest ? x_row[p] : GF_OUT, c * (GF_KB * 4) + h * 128 + q * 64);
+    };
+    auto fetch_w = [&](const int h, int c) __attribute__((always_inline)) {
+        const int rest = left(h, c);
+#pragma unroll
+        for (int u = 0; u < NT; ++u)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) wr[h % DEPTH][u][i] = gf_load<0>(wb, w_lane < rest ? w_row[u][i] : GF_OUT, c * (GF_KB * 4) + h * 128);
+    };
+    auto stash = [&](const int h) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < XP; ++p) {
+            const gf_parts s = h ? gf_split(-xr[h % DEPTH][p][0], -xr[h % DEPTH][p][1]) : gf_split(xr[h % DEPTH][p][0], xr[h % DEPTH][p][1]);
+            if (PIECES % THREADS == 0 || tid + p * THREADS < PIECES) {
+#pragma unroll
+                for (int i = 0; i < 3; ++i) lds[group][h][i][x_place[p]] = s.p[i].u;
+            }
+        }
+    };
+    const gf_f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+    gf_f32x4_t acc[2][MT][NT], sum[SUMS][MT][NT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+            acc[0][t][u] = acc[1][t][u] = zero;
+#pragma unroll
+            for (int i = 0; i < SUMS; ++i) sum[i][t][u] = zero;
+        }
+    int in_part = 0, parts = 0;
+    const int read_at = r * 4 + ((g ^ -(r >> 2)) & 3);
+    // Half h of chunk c: its weights' parts lie in ws[h] and its x in buffer h.  While it is multiplied the next half's operands are split, one
+    // vector instruction after the other in the time that the matrix cores take, and those of DEPTH halves later are asked for.
+    gf_parts ws[2][NT];
+    auto step = [&](const int h, int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < NT; ++u) ws[h ^ 1][u] = gf_turn<GF_PLUS>(turn + u * 128, wr[(h ^ 1) % DEPTH][u][0], wr[(h ^ 1) % DEPTH][u][1], lane);
+        if (DEPTH == 2) fetch_w(h ^ 1, h ? c + 2 : c + 1);
+        else fetch_w(h, c + 1);
+        stash(h ^ 1);
+        if (DEPTH == 2) fetch_x(h ^ 1, h ? c + 2 : c + 1);
+        else fetch_x(h, c + 1);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            gf_parts xs;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) xs.p[i].u = lds[group][h][i][t * 64 + read_at];
+#pragma unroll
+            for (int u = 0; u < NT; ++u) acc[h][t][u] = gf_multiply(ws[h][u], xs, acc[h][t][u]);
+        }
+        // a product, a few vector instructions, and so on
+        __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+#pragma unroll
+        for (int i = 0; i < 6 * MT * NT; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, TOGETHER ? 4 : 3, 0);
+            if (i % (6 * NT) == 0 && i / (6 * NT) + 2 < MT) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+        }
+        if (TOGETHER) {
+            // (the splitting done here: left to itself the compiler moves it past the barrier, where no product is under way)
+#pragma unroll
+            for (int u = 0; u < NT; ++u)
+#pragma unroll
+                for (int i = 0; i < 3; ++i) asm volatile("" : "+v"(ws[h ^ 1][u].p[i].u));
+        }
+        // x of the next half is in LDS, this half's has been read; loads travel on
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    fetch_x(0, c0);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_w(0, c0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (DEPTH == 2) {
+        fetch_x(1, c0);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_w(1, c0);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    stash(0);
+    if (DEPTH == 2) fetch_x(0, c0 + 1);
+    else fetch_x(1, c0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < NT; ++u) ws[0][u] = gf_turn<GF_PLUS>(turn + u * 128, wr[0][u][0], wr[0][u][1], lane);
+    if (DEPTH == 2) fetch_w(0, c0 + 1);
+    else fetch_w(1, c0);
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();
+    for (int c = 0; c < steps; ++c) {
+        step(0, c0 + c);
+        step(1, c0 + c);
+        if (++in_part == per) {           // a run of k ends
+            in_part = 0;
+            ++parts;
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+                for (int u = 0; u < NT; ++u) {
+                    // one group: the sum of the runs of a half; else a sum for each of the group's runs
+                    const gf_f32x4_t run = acc[0][t][u] - acc[1][t][u];
+                    acc[0][t][u] = acc[1][t][u] = zero;
+                    if (GROUPS == 1) {
+                        sum[0][t][u] += run;
+                        if (parts == GF_PARTS / 2) {
+                            first[(t * NT + u) * THREADS] = sum[0][t][u];
+                            sum[0][t][u] = zero;
+                        }
+                    } else if (parts == 1) {
+                        sum[0][t][u] = run;
+                    } else {
+                        sum[SUMS - 1][t][u] = run;
+                    }
+                }
+        }
+    }
+    auto finish = [&](gf_f32x4_t* s, int t, int u0, int of, int l) __attribute__((always_inline)) {
+        // the sums of a wavefront's block (t, u0), or of its gate and up blocks: checked, activated, stored
+        const int m = m0 + t * 16 + (l & 15), n = n0 + of * NW + (GATED ? u0 / 2 : u0) * 16 + (l >> 4) * 4;
+        if (m >= M || n >= N) return;
+#pragma unroll
+        for (int i = 0; i < (GATED ? 2 : 1); ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (n + e < N) s[i][e] = gf_finite(s[i][e], x + m * ldx, w + ((int64_t)n + e + (i ? N : 0)) * ldw, K);
+        if (GATED) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[0][e] = gf_gate(s[0][e], s[GATED][e]);
+        }
+        gf_store4(out + (int64_t)m * ldo, GATED ? nullptr : bias, s[0], n, N, vec_out);
+    };
+    constexpr int STEP = GATED ? 2 : 1;
+    if (GROUPS == 1) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int u = 0; u < NT; u += STEP) {
+                gf_f32x4_t s[STEP];
+#pragma unroll
+                for (int i = 0; i < STEP; ++i)          // (acc: zeros where the last run ended)
+                {
+                    s[i] = sum[0][t][u + i] + (acc[0][t][u + i] - acc[1][t][u + i]);
+                    if (parts >= GF_PARTS / 2) s[i] = first[(t * NT + u + i) * THREADS] + s[i];
+                }
+                finish(s, t, u, wave, lane);
+            }
+        return;
+    }
+    // the runs' sums meet in LDS (past the last barrier nobody reads x there)
+    gf_f32x4_t* part = reinterpret_cast<gf_f32x4_t*>(lds_all);
+#pragma unroll
+    for (int i = 0; i < RUNS; ++i)
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int u = 0; u < NT; ++u)
+                part[(((group * RUNS + i) * WAVES + wave) * MT * NT + t * NT + u) * ZI_WAVE + lane] =
+                    sum[i % SUMS][t][u];
+    __syncthreads();
+    for (int b = wave_all; b < BLOCKS / STEP; b += WAVES * GROUPS) {
+        gf_f32x4_t s[STEP];
+#pragma unroll
+        for (int i = 0; i < STEP; ++i) {
+            const gf_f32x4_t* at = part + (b * STEP + i) * ZI_WAVE + lane;
+            s[i] = at[0];
+            gf_f32x4_t s2 = at[GF_PARTS / 2 * BLOCKS * ZI_WAVE];
+#pragma unroll
+            for (int p = 1; p < GF_PARTS / 2; ++p) {
+                s[i] += at[p * BLOCKS * ZI_WAVE];
+                s2 += at[(GF_PARTS / 2 + p) * BLOCKS * ZI_WAVE];
+            }
+            s[i] += s2;
+        }
+        const int of = b * STEP / (MT * NT), tu = b * STEP % (MT * NT);
+        finish(s, tu / NT, tu % NT, of, lane);
+    }
+}
+
+// Which kernel M rows of x and N weight rows take is a matter of filling the compute units only.
+// Up to 8 rows a stream of the weights in groups of 8, up to 16 in groups of 16 unless two passes over groups of 8 are one round (1,024 weight
+// rows); x is held in registers once there are more groups than units.  Beyond, groups of 16 weight rows with 16 or 32 rows of x while those are
+// one round of workgroups, 32 up to 32 rows.  Then tiles: the least of what each kind takes, rounds of workgroups times (a start + a time a chunk), us,
+// fitted to runs alone at 8 to 296 chunks: 32 x 64 in four groups 3.7 + 0.59 (1,536 x 8,960 at 256 rows 84, 2,048 x 1,536 at 128 18), 32 x 96 4.3 + 0.7
+// (512 rows 105, 1,536 x 1,536 23), 64 x 64 5.5 + 0.86 (2,048 x 1,536 at 512 rows 27); with one group, where several workgroups share a unit,
+// 32 x 128 1.39, 2.0 and 2.8 for one, two and three of them and 64 x 128 1.6 and 2.72 for one and two.  32 x 96 only for less than two rounds
+// (from there on 32 x 64 was kept, which at 1,024 rows of 1,536 x 8,960 costs 255 against 205 us), and a larger tile has to be that much faster to be worth its idle units:
+// the fit is no better than some per cent.  (256 rows of 17,920 x 1,536: 32 x 128 120 us, 64 x 128 116; 320 rows 157 and 118.)
+gf_kernel zi_gemm_f32_split_kernel(int M, int64_t N, int K) {
+    const int64_t cus = zi_compute_units(), n16 = (N + 15) / 16, m16 = (M + 15) / 16, m32 = (M + 31) / 32, m64 = (M + 63) / 64;
+    const int chunks = (K + GF_KB - 1) / GF_KB, per = (chunks + GF_PARTS - 1) / GF_PARTS;
+    if (M <= 8) return (N + 7) / 8 > cus && per <= GF_HELD_CHUNKS ? GF_HELD_PAIRS : GF_PAIRS;
+    if (M <= 16 && n16 > cus && per <= GF_HELD_CHUNKS / 2) return GF_HELD_ROWS16;
+    if (M <= 16) return (N + 7) / 8 * 2 <= cus ? GF_PAIRS : GF_ROWS16;
+    if (n16 * m16 <= cus) return GF_ROWS16;
+    if (M <= 32 || n16 * m32 <= cus) return GF_ROWS32;
+    const int64_t n64 = (N + 63) / 64, n96 = (N + 95) / 96, n128 = (N + 127) / 128;
+    auto shared = [&](int64_t tiles, float start, float chunk) { return (float)((tiles + cus - 1) / cus) * (start + chunk * chunks); };
+    auto rounds = [&](int64_t tiles, int places, float one, float two, float all) {      // `places` workgroups a unit at a time
+        const int64_t full = tiles / (places * cus), rest = tiles % (places * cus);
+        return (float)chunks * ((float)full * all + (rest == 0 ? 0.f : rest <= cus ? one : rest <= 2 * cus ? two : all));
+    };
+    gf_kernel best = GF_TILE_32_HALVES;
+    float us = shared(m32 * n64, 3.7f, 0.59f);
+    auto consider = [&](gf_kernel kernel, float takes, float unless) {
+        if (takes < unless * us) {
+            best = kernel;
+            us = takes;
+        }
+    };
+    if (m32 * n96 < 2 * cus) consider(GF_TILE_96_HALVES, shared(m32 * n96, 4.3f, 0.7f), 1.f);
+    consider(GF_TILE_32, 6.f + rounds(m32 * n128, 3, 1.39f, 2.f, 2.8f), 1.f);
+    consider(GF_TILE_64_QUARTERS, shared(m64 * n64, 5.5f, 0.86f), 0.96f);
+    consider(GF_TILE_64, 8.5f + rounds(m64 * n128, 2, 1.6f, 2.72f, 2.72f), 0.88f);
+    return best;
+}
+
+template <bool GATED>
+static int gs_launch(float* out, const float* x, const float* w, const float* bias, int M, int N, int K, int64_t ldx, int64_t ldw,
+                     int64_t ldo, hipStream_t stream) {
+    const int chunks = (K + GF_KB - 1) / GF_KB, per = (chunks + GF_PARTS - 1) / GF_PARTS;
+    const int vec_out = ldo % 4 == 0 && (uintptr_t)out % 16 == 0;
+#define ZI_GF_STREAM(MT, PAIR, RING)                                                                                                     \
+    gemm_f32_split_stream_kernel<MT, PAIR, RING><<<dim3((N + (PAIR ? 7 : 15)) / (PAIR ? 8 : 16), (M + (PAIR ? 8 : 16 * MT) - 1) / (PAIR ? 8 : 16 * MT)), \
+                                             GF_PARTS * ZI_WAVE, 0, stream>>>(out, x, w, bias, M, N, K, ldx, ldw, ldo, per, vec_out)
+    // two workgroups a unit while a lane has registers for that (128), else one
+#define ZI_GF_HELD(PAIR, PER)                                                                                                            \
+    do {                                                                                                                                 \
+        const int nc = (PAIR ? 8 : 16) / (GATED ? 2 : 1), groups = (N + nc - 1) / nc;                                                        \
+        const int places = zi_compute_units() * ((PAIR ? 1 : 2) * PER <= 3 ? 2 : 1);                                                         \
+        gemm_f32_split_held_kernel<PAIR, PER, GATED><<<groups < places ? groups : places, GF_PARTS * ZI_WAVE, 0, stream>>>(                         \
+            out, x, w, bias, M, N, K, ldx, ldw, ldo, per, vec_out, groups);                                                               \
+    } while (0)
+    // (rows in as many launches as 2^32 threads of one make necessary: a row's result does not depend on them)
+#define ZI_GF_TILE(MT, NT, WAVES, G)                                                                                                       \
+    do {                                                                                                                                  \
+        const int tm = 16 * MT, nc = 16 * NT * WAVES / (GATED ? 2 : 1);                                                                      \
+        const int64_t nt = (N + nc - 1) / nc, most = ((1ll << 31) / (ZI_WAVE * WAVES * G)) / nt * tm;                                        \
+        for (int64_t m = 0; m < M; m += most) {                                                                                           \
+            const int rows = (int)(M - m < most ? M - m : most), mt = (rows + tm - 1) / tm, tiles = (int)(mt * nt);                          \
+            gemm_f32_split_tile_kernel<MT, NT, WAVES, G, GATED><<<(tiles + 7) / 8 * 8, ZI_WAVE * WAVES * G, 0, stream>>>(                          \
+                out + m * ldo, x + m * ldx, w, bias, rows, N, K, ldx, ldw, ldo, per, vec_out, mt, tiles);                                  \
+        }                                                                                                                                 \
+    } while (0)
+    switch (zi_gemm_f32_split_kernel(M, (int64_t)N * (GATED ? 2 : 1), K)) {
+        case GF_HELD_PAIRS:
+            if (per <= 3) ZI_GF_HELD(true, 3);
+            else if (per <= 4) ZI_GF_HELD(true, 4);
+            else if (per <= 6) ZI_GF_HELD(true, 6);
+            else ZI_GF_HELD(true, 8);
+            break;
+        case GF_HELD_ROWS16:
+            if (per <= 3) ZI_GF_HELD(false, 3);
+            else ZI_GF_HELD(false, 4);
+            break;
+        case GF_TILE_64: ZI_GF_TILE(4, 2, 4, 1); break;
+        case GF_TILE_32: ZI_GF_TILE(2, 2, 4, 1); break;
+        case GF_TILE_32_HALVES: ZI_GF_TILE(2, 2, 2, 4); break;
+        case GF_TILE_64_QUARTERS: ZI_GF_TILE(4, 2, 2, 4); break;
+        default:
+            if constexpr (GATED) {
+                return zi_fail("gemm_f32: no gated kernel for %d rows of %d x %d", M, N, K);      // (zi_gemm_f32_swiglu_takes says so)
+            } else {
+                switch (zi_gemm_f32_split_kernel(M, N, K)) {
+                    case GF_PAIRS: ZI_GF_STREAM(1, true, 3); break;
+                    case GF_ROWS16: ZI_GF_STREAM(1, false, 2); break;
+                    case GF_ROWS32: ZI_GF_STREAM(2, false, 1); break;
+                    default: ZI_GF_TILE(2, 2, 3, 4); break;
+                }
+            }
+    }
+#undef ZI_GF_STREAM
+#undef ZI_GF_HELD
+#undef ZI_GF_TILE
+    return zi_check_launch("gemm_f32_split");
+}
+
+int zi_gemm_f32_split_launch(bool gated, float* out, const float* x, const float* w, const float* bias, int M, int N, int K, int64_t ldx,
+                             int64_t ldw, int64_t ldo, hipStream_t stream) {
+    return gated ? gs_launch<true>(out, x, w, nullptr, M, N, K, ldx, ldw, ldo, stream) : gs_launch<false>(out, x, w, bias, M, N, K, ldx, ldw, ldo, stream);
+}

@@ -1161,7 +1161,7 @@ def linear_swiglu_many(x: torch.Tensor, weight: torch.Tensor, out: Optional[torc
     return _swiglu_epilogue("linear_swiglu_many", x, weight, out)
 
 
-F32_KERNELS = ("pairs", "rows16", "rows32", "held_pairs", "held_rows16", "tile_64", "tile_32", "tile_32_halves", "tile_96_halves")
+F32_KERNELS = ("pairs", "rows16", "rows32", "held_pairs", "held_rows16", "tile_64", "tile_32", "tile_32_halves", "tile_96_halves", "tile_64_quarters")
 
 
 def linear_f32_kernel(M: int, N: int, K: int) -> str:
