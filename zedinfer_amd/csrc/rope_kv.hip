@@ -75,7 +75,14 @@ __global__ void rope_kv_store_kernel(T* __restrict__ q, const T* __restrict__ k,
 // tokens' slots are eight consecutive slots of one page that start at a multiple of eight (the usual case
 // inside a prompt), a thread writes the eight tokens' values of one dim as one 16-byte run of the
 // transposed value cache, else value by value.  half = rot / 2 must be a multiple of 8 (or 0).
+// Bound by a workgroup's trips one after the other (angles and values, queries, keys, the value run) while few workgroups are on the
+// chip, 4 to 6 bytes a clock and unit.  So up to two tiles a unit (4,096 tokens) a tile's work is four workgroups', two for the queries, one
+// for the keys, one for the values: us, one to four, 1,024 / 2,112 / 4,096 tokens, rows from memory: 12 heads of 128 on 2
+// key/value heads 8.7 to 5.9, 9.6 to 7.2, 10.4 to 9.4; 28 on 4 14.2 to 9.6, 15.7 to 11.7, 23.1 to 19.5; 40 on 8 22.5 to 15.5, 31.7 to 22.3, 36.7 to 33.3
+// (3.3 TB/s read and written), from the last-level cache 0.71 to 0.96 of the one's time; 8,192 tokens 19.1 and 17.5, but 21.6 and 22.3 for 16 heads on 4 that turn half.  Five to eight workgroups are
+// no faster, nor is one that asks for four pieces of everything at once (2,112 tokens 9.6 to 11.3).
 #define RKT_TOKENS 8
+#define RKT_SHARES 4
 __global__ void __launch_bounds__(256)
 rope_kv_store_tile_kernel(zi_bf16* __restrict__ q, const zi_bf16* __restrict__ k, const zi_bf16* __restrict__ v,
                           int64_t ldq, int64_t ldk, int64_t ldv, const int32_t* __restrict__ slots,
@@ -87,13 +94,18 @@ rope_kv_store_tile_kernel(zi_bf16* __restrict__ q, const zi_bf16* __restrict__ k
     uint16_t* vt = reinterpret_cast<uint16_t*>(rkt_lds + (size_t)RKT_TOKENS * rot * sizeof(float));   // [token][kvd]
     const int t0 = blockIdx.x * RKT_TOKENS, tid = threadIdx.x;
     const int nt = (n - t0 < RKT_TOKENS) ? n - t0 : RKT_TOKENS;
-    for (int i = tid; i < nt * half; i += 256) {
-        const int tt = i / half, jj = i % half;
-        const float2 e = table[(int64_t)(t0 + tt) * half + jj];
-        cs[tt * rot + jj] = e.x;
-        cs[tt * rot + half + jj] = e.y;
+    // this workgroup's share: all (gridDim.y 1), or the values (the last), the keys (the one before) or a part of the queries
+    const int share = blockIdx.y, shares = gridDim.y, q_shares = shares == 1 ? 1 : write_kv ? shares - 2 : shares;
+    const bool values = write_kv && share == shares - 1, keys = write_kv && (shares == 1 || share == shares - 2);
+    if (shares == 1 || !values) {
+        for (int i = tid; i < nt * half; i += 256) {
+            const int tt = i / half, jj = i % half;
+            const float2 e = table[(int64_t)(t0 + tt) * half + jj];
+            cs[tt * rot + jj] = e.x;
+            cs[tt * rot + half + jj] = e.y;
+        }
     }
-    if (write_kv)
+    if (values)
         for (int i = tid; i < nt * (kvd / 8); i += 256) {
             const int tt = i / (kvd / 8), c8 = i % (kvd / 8);
             *reinterpret_cast<uint4*>(vt + tt * kvd + c8 * 8) =
@@ -112,7 +124,7 @@ rope_kv_store_tile_kernel(zi_bf16* __restrict__ q, const zi_bf16* __restrict__ k
     };
     // queries, in place: (token, head, eight dims of the first half and their partners)
     const int hp = half / 8;
-    for (int i = tid; i < nt * nh * hp; i += 256) {
+    for (int i = share < q_shares ? tid + share * 256 : nt * nh * hp; i < nt * nh * hp; i += 256 * q_shares) {
         const int tt = i / (nh * hp), rem = i % (nh * hp), h = rem / hp, j0 = (rem % hp) * 8;
         zi_bf16* base = q + (int64_t)(t0 + tt) * ldq + (int64_t)h * d + j0;
         float a[8], b[8], lo[8], hi[8];
@@ -128,10 +140,9 @@ rope_kv_store_tile_kernel(zi_bf16* __restrict__ q, const zi_bf16* __restrict__ k
         *reinterpret_cast<uint4*>(base) = pack(lo);
         *reinterpret_cast<uint4*>(base + half) = pack(hi);
     }
-    if (!write_kv) return;
     // keys into the cache: (token, kv head, eight dims)
     const int dp = d / 8;
-    for (int i = tid; i < nt * nkv * dp; i += 256) {
+    for (int i = keys ? tid : nt * nkv * dp; i < nt * nkv * dp; i += 256) {
         const int tt = i / (nkv * dp), rem = i % (nkv * dp), h = rem / dp, j0 = (rem % dp) * 8;
         const ZiSlotPlace place = zi_slot_place(slots[t0 + tt], cache_slots, page_size);
         if (!place.ok) continue;     // the host checks the range; never write outside the pool
@@ -155,6 +166,7 @@ rope_kv_store_tile_kernel(zi_bf16* __restrict__ q, const zi_bf16* __restrict__ k
         }
         *reinterpret_cast<uint4*>(kcache + zi_key_offset(page, h, off, nkv, page_size, d) + j0) = pack(o8);
     }
+    if (!values) return;
     // values: transposed.  Eight tokens in eight consecutive slots from a multiple of eight: one run per dim.
     bool run = nt == RKT_TOKENS;
     const int s0 = slots[t0];
@@ -185,8 +197,8 @@ rope_kv_store_tile_kernel(zi_bf16* __restrict__ q, const zi_bf16* __restrict__ k
 }
 
 // From this many tokens on, the tile kernel (bfloat16, 16-byte pieces).  Below, a workgroup a token is
-// faster (256 tokens with scattered slots, a large decode batch: 4.2 against 8.3 us; the two meet at 1,024
-// tokens in one run of slots, and 2,048 take 7.0 against 8.8 us).
+// faster (us, against the tile kernel in four shares, slots in a run and scattered: 256 tokens of 28 heads on 4 7.8 against 8.5 and 10.4, 960
+// 10.7 against 9.5 and 12.6, of 40 heads on 8 14.8 against 15.5 and 20.4).
 #define ROPE_MANY_TOKENS 1024
 
 extern "C" int zi_rope_kv_store(void* q, const void* k, const void* v, int dt, int n, int64_t ldq, int64_t ldk,
@@ -213,7 +225,8 @@ extern "C" int zi_rope_kv_store(void* q, const void* k, const void* v, int dt, i
                                        ((uintptr_t)vcache % 16) == 0 && ldk % 8 == 0 && ldv % 8 == 0 && page_size % 8 == 0));
         const size_t lds = (size_t)RKT_TOKENS * rot * sizeof(float) + (write_kv ? (size_t)RKT_TOKENS * nkv * d * 2 : 0);
         if (dt == ZI_BF16 && n >= ROPE_MANY_TOKENS && al && lds <= 48 * 1024) {
-            rope_kv_store_tile_kernel<<<(n + RKT_TOKENS - 1) / RKT_TOKENS, 256, lds, stream>>>(
+            const int tiles = (n + RKT_TOKENS - 1) / RKT_TOKENS;
+            rope_kv_store_tile_kernel<<<dim3(tiles, tiles <= 2 * zi_compute_units() ? RKT_SHARES : 1), 256, lds, stream>>>(
                 (zi_bf16*)q, (const zi_bf16*)k, (const zi_bf16*)v, ldq, ldk, ldv, slots, tb, (zi_bf16*)kcache,
                 (zi_bf16*)vcache, n, nh, nkv, d, rot, page_size, write_kv, cache_slots);
             return zi_check_launch("rope_kv_store");
