@@ -400,9 +400,14 @@ extern "C" int zi_latent_attention_cores(void* out, int out_dt, float* partial, 
 // it is loaded) or bfloat16 with row stride ldx and head stride xs, out float32 or bfloat16 with row stride ldo and head stride
 // os.  It carries the queries through W_uk (w = W_uk of the head, transposed at load) and the attended latents through W_uv.
 // GATED: out *= sigmoid(gate[t][h * N + i]), the gate bfloat16 or the sum of `splits` float32 terms.
-// Operands straight from memory.  Many tokens: a wavefront owns 32 tokens x 64 outputs (every operand serves several
-// products), the four wavefronts of a workgroup take neighbouring tokens of one head.  Few: 16 x 16, k dealt over the
-// four wavefronts in runs of 32 and added up in their order.
+// Few tokens: 16 x 16 a workgroup, operands straight from memory, k dealt over the four wavefronts in runs of 32 and added up in their
+// order.  Many: 64 tokens x 128 outputs, a wavefront 32 x 64.  Bound by memory (x once, the results), and before by the vector cache:
+// operands loaded as the product wants them lie in a row apiece, 9 to 10 accesses a line of 128 bytes.  So a step's rows of 128 bytes are
+// loaded whole, two steps on their way in registers, and turn in LDS in places that neither side's lanes share a bank in; the results
+// turn there too and leave as runs of 256 bytes.  us, before and after: 12 heads, 512 outputs of k 128, 2,000 tokens 24.9 to 12.9 (3 TB/s with
+// x once), 128 of 512 26.1 to 14.3; 8,000 tokens 81.5 to 38.6 and 80.8 to 30.9; 128 tokens 6.2 to 4.7 and 13.7 to 8.6; 64 heads, 2,000
+// tokens 108.8 to 54.9 and 90.7 to 42.4; float32 x 18.3 to 12.6 at 1,000 tokens; with a gate 35.4 to 21.8 at 2,048.  One step on its way instead of two: 128 tokens 5.0 and
+// 9.8.  Two workgroups a unit instead of three: 8,000 tokens 43.5 and 38.7.  Slower: a k of 8 with 33 outputs, 4.2 to 5.5.
 struct LaGate {
     const void* g;
     int f32, splits;
@@ -492,67 +497,119 @@ headwise_linear_few_kernel(TO* __restrict__ out, int64_t ldo, int os, const TX* 
     la_store4(out + t * ldo + (int64_t)h * os + n0 + 4 * j, acc, N - n0 - 4 * j);
 }
 
+#define LA_HT 64       // tokens
+#define LA_HN 128      // outputs
+#define LA_HK 64       // k a step: rows of 128 bytes
+#define LA_HROW (LA_HN + 4)
 template <typename TX, typename TO, bool GATED>
-__global__ void __launch_bounds__(4 * ZI_WAVE)
+__global__ void __launch_bounds__(4 * ZI_WAVE, GATED ? 2 : 3)      // (the gate's terms take registers)
 headwise_linear_many_kernel(TO* __restrict__ out, int64_t ldo, int os, const TX* __restrict__ x, int64_t ldx, int xs,
                             const zi_bf16* __restrict__ w, int n, int N, int K, LaGate gt) {
-    constexpr int TM = 2, TN = 4;      // tiles of 16 tokens and of 16 outputs
-    const int lane = threadIdx.x % ZI_WAVE, wave = threadIdx.x / ZI_WAVE, r = lane % 16, j = lane / 16;
-    const int t0 = (blockIdx.x * 4 + wave) * (16 * TM), h = blockIdx.y, n0 = blockIdx.z * (16 * TN);
-    if (t0 >= n) return;
-    const zi_bf16* wrow[TN];
-    const TX* xrow[TM];
+    constexpr int TM = 2, TN = 4;                       // a wavefront's tiles of 16 tokens and of 16 outputs
+    constexpr int PX = LA_HT / 32, PW = LA_HN / 32;     // a thread's pieces of 16 bytes a step
+    constexpr int STEP = (LA_HT + LA_HN) * 8;           // pieces a step
+    __shared__ la_u32x4_t lds[2 * STEP];
+    static_assert(LA_HT * LA_HROW * sizeof(float) <= sizeof(lds), "the results turn in the operands' place");
+    const int tid = threadIdx.x, lane = tid % ZI_WAVE, wave = tid / ZI_WAVE, r = lane % 16, j = lane / 16;
+    const int t0 = blockIdx.x * LA_HT, h = blockIdx.y, n0 = blockIdx.z * LA_HN;
+    const int q = tid / 8, c8 = tid % 8;                // rows q, q + 32, ..; (q + 32 i) / 2 keeps its last three bits
+    const int at = q * 8 + (c8 ^ (q / 2 & 7));
+    const TX* xr[PX];
+    const zi_bf16* wr[PW];
 #pragma unroll
-    for (int c = 0; c < TN; ++c) {
-        const int i = n0 + c * 16 + r;
-        wrow[c] = w + ((int64_t)h * N + (i < N ? i : N - 1)) * K;
+    for (int i = 0; i < PX; ++i) {
+        const int t = t0 + q + 32 * i;
+        xr[i] = x + (int64_t)(t < n ? t : n - 1) * ldx + (int64_t)h * xs;
     }
 #pragma unroll
-    for (int c = 0; c < TM; ++c) {
-        const int t = t0 + c * 16 + r;
-        xrow[c] = x + (int64_t)(t < n ? t : n - 1) * ldx + (int64_t)h * xs;
+    for (int i = 0; i < PW; ++i) {
+        const int o = n0 + q + 32 * i;
+        wr[i] = w + ((int64_t)h * N + (o < N ? o : N - 1)) * K;
     }
+    struct Pieces { la_pack x[PX], w[PW]; };
+    auto load = [&](Pieces& to, int k0) {
+        const int k = k0 + 8 * c8, kc = k < K ? k : 0;      // K is a multiple of 8
+        const unsigned mask = 0u - (unsigned)(k < K);
+#pragma unroll
+        for (int i = 0; i < PX; ++i) to.x[i] = la_load8(xr[i] + kc);
+#pragma unroll
+        for (int i = 0; i < PW; ++i) to.w[i] = la_load8(wr[i] + kc);
+#pragma unroll
+        for (int i = 0; i < PX; ++i) to.x[i].u &= mask;
+#pragma unroll
+        for (int i = 0; i < PW; ++i) to.w[i].u &= mask;
+    };
+    auto stash = [&](const Pieces& p, la_u32x4_t* to) {
+#pragma unroll
+        for (int i = 0; i < PX; ++i) to[at + 32 * 8 * i] = p.x[i].u;
+#pragma unroll
+        for (int i = 0; i < PW; ++i) to[LA_HT * 8 + at + 32 * 8 * i] = p.w[i].u;
+    };
+    const int tw = (wave % 2) * (16 * TM), ow = (wave / 2) * (16 * TN);
     la_f32x4_t acc[TM][TN];
 #pragma unroll
     for (int a = 0; a < TM; ++a)
 #pragma unroll
         for (int c = 0; c < TN; ++c) acc[a][c] = (la_f32x4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-    for (int k0 = 0; k0 < K; k0 += 32) {
-        const int k = k0 + 8 * j, kc = k < K ? k : 0;
-        const unsigned mask = 0u - (unsigned)(k < K);
-        la_pack a[TN], b[TM];
+    // one step on its way in registers, one on its way to memory's answer, one in LDS
+    auto step = [&](int k0, Pieces& mine, const Pieces& next, int buf) {
+        __syncthreads();
+        if (k0 + 2 * LA_HK < K) load(mine, k0 + 2 * LA_HK);
+        const la_u32x4_t *lx = lds + buf * STEP + (tw + r) * 8, *lw = lds + buf * STEP + (LA_HT + ow + r) * 8;
 #pragma unroll
-        for (int c = 0; c < TN; ++c) a[c] = la_load8(wrow[c] + kc);
+        for (int s = 0; s < LA_HK / 32; ++s) {
+            const int place = (4 * s + j) ^ (r / 2 & 7);
+            la_pack a[TN], b[TM];
 #pragma unroll
-        for (int c = 0; c < TM; ++c) b[c] = la_load8(xrow[c] + kc);
+            for (int c = 0; c < TN; ++c) a[c].u = lw[c * 16 * 8 + place];
 #pragma unroll
-        for (int c = 0; c < TN; ++c) a[c].u &= mask;
+            for (int c = 0; c < TM; ++c) b[c].u = lx[c * 16 * 8 + place];
 #pragma unroll
-        for (int c = 0; c < TM; ++c) b[c].u &= mask;
+            for (int m = 0; m < TM; ++m)
 #pragma unroll
-        for (int m = 0; m < TM; ++m)
-#pragma unroll
-            for (int c = 0; c < TN; ++c) acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[c].b, b[m].b, acc[m][c], 0, 0, 0);
+                for (int c = 0; c < TN; ++c) acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[c].b, b[m].b, acc[m][c], 0, 0, 0);
+        }
+        if (k0 + LA_HK < K) stash(next, lds + (buf ^ 1) * STEP);      // read for the last time before this step's barrier
+    };
+    Pieces even, odd;
+    load(even, 0);
+    if (LA_HK < K) load(odd, LA_HK);
+    stash(even, lds);
+    for (int k0 = 0; k0 < K; k0 += 2 * LA_HK) {
+        step(k0, even, odd, 0);
+        if (k0 + LA_HK < K) step(k0 + LA_HK, odd, even, 1);
     }
+    __syncthreads();
+    float* turned = reinterpret_cast<float*>(lds);      // [token][output]
 #pragma unroll
-    for (int m = 0; m < TM; ++m) {
-        const int t = t0 + m * 16 + r;
-        if (t >= n) continue;
+    for (int m = 0; m < TM; ++m)
 #pragma unroll
-        for (int c = 0; c < TN; ++c) {
-            const int i = n0 + c * 16 + 4 * j;
-            if (i >= N) continue;
-            if constexpr (GATED) la_gate4(acc[m][c], la_gates(gt, t, h, i, N));
-            TO* dst = out + (int64_t)t * ldo + (int64_t)h * os + i;
-            if (sizeof(TO) == 2 && i + 3 < N && ((uintptr_t)dst % 8) == 0) {
-                uint2 p;
-                p.x = zi_pack_bf16x2(acc[m][c][0], acc[m][c][1]);
-                p.y = zi_pack_bf16x2(acc[m][c][2], acc[m][c][3]);
-                *reinterpret_cast<uint2*>(dst) = p;
-            } else {
-                la_store4(dst, acc[m][c], N - i);
-            }
+        for (int c = 0; c < TN; ++c)
+            *reinterpret_cast<la_f32x4_t*>(turned + (tw + m * 16 + r) * LA_HROW + ow + c * 16 + 4 * j) = acc[m][c];
+    __syncthreads();
+    for (int p = tid; p < LA_HT * (LA_HN / 8); p += 4 * ZI_WAVE) {
+        const int row = p / (LA_HN / 8), o = p % (LA_HN / 8) * 8, t = t0 + row, i = n0 + o;
+        if (t >= n || i >= N) continue;
+        la_f32x4_t lo = *reinterpret_cast<const la_f32x4_t*>(turned + row * LA_HROW + o);
+        la_f32x4_t hi = *reinterpret_cast<const la_f32x4_t*>(turned + row * LA_HROW + o + 4);
+        if constexpr (GATED) {
+            la_gate4(lo, la_gates(gt, t, h, i, N));
+            la_gate4(hi, la_gates(gt, t, h, i + 4, N));
+        }
+        TO* dst = out + (int64_t)t * ldo + (int64_t)h * os + i;
+        if (sizeof(TO) == 2 && i + 7 < N && ((uintptr_t)dst % 16) == 0) {
+            la_pack b;
+            b.w[0] = zi_pack_bf16x2(lo[0], lo[1]);
+            b.w[1] = zi_pack_bf16x2(lo[2], lo[3]);
+            b.w[2] = zi_pack_bf16x2(hi[0], hi[1]);
+            b.w[3] = zi_pack_bf16x2(hi[2], hi[3]);
+            *reinterpret_cast<la_u32x4_t*>(dst) = b.u;
+        } else if (sizeof(TO) == 4 && i + 7 < N && ((uintptr_t)dst % 16) == 0) {
+            reinterpret_cast<la_f32x4_t*>(dst)[0] = lo;
+            reinterpret_cast<la_f32x4_t*>(dst)[1] = hi;
+        } else {
+            la_store4(dst, lo, N - i);
+            la_store4(dst + 4, hi, N - i - 4);
         }
     }
 }
@@ -576,7 +633,7 @@ extern "C" int zi_headwise_linear_gated(void* out, int out_dt, int64_t ldo, int 
                "headwise_linear: bad gate");
     if (n == 0) return 0;
     const bool many = n >= LA_MANY_TOKENS;
-    const dim3 grid(many ? (n + 127) / 128 : (n + 15) / 16, heads, many ? (N + 63) / 64 : (N + 15) / 16);
+    const dim3 grid(many ? (n + LA_HT - 1) / LA_HT : (n + 15) / 16, heads, many ? (N + LA_HN - 1) / LA_HN : (N + 15) / 16);
     const LaGate gt = {gate, g_dt == ZI_F32, g_splits, ld_gate, g_stride};
 #define ZI_HW(KERNEL, GATED) KERNEL<TX, TO, GATED><<<grid, 4 * ZI_WAVE, 0, stream>>>((TO*)out, ldo, os, (const TX*)x, ldx, xs, (const zi_bf16*)w, n, N, K, gt)
     ZI_DISPATCH_DTYPE(x_dt, TX, ZI_DISPATCH_DTYPE(out_dt, TO, {
