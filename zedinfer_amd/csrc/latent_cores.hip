@@ -20,6 +20,13 @@
 // (Staged through registers, with a transposed copy of the latents written by 2-byte stores, the same walk took 381 us
 // for the 2,048 tokens of a layer with 12 heads, rank 512 and a window of 1,024 keys.)
 //
+// Bound by LDS (68 KB a wavefront and block of rank 512 in about 540 cycles) and, where the tiles are no two for every unit, by the
+// units with one.  A wavefront's turn was 11,000 cycles: a read's wait for each of 68 products, a branch for each tile of the second,
+// and the loads of the next block waited for as soon as they were issued, together with a page number asked for behind them.  us, then
+// and now, rank 512, rot 64, window 1,024: 2,000 tokens of 12 heads 178 to 121, without a window 295 to 193; 2,048 of 28 heads
+// behind 3,000 cached 338 to 241; 31 decoded beside 700 prompt tokens 158 to 101; 32 decoded of 12 heads 25.5 to 23.6; rank 256, 16 heads,
+// 2,048 tokens 104 to 83, rank 128 67 to 59.
+//
 // A tile's keys can be cut into chunks over blockIdx.y (decoded tokens: few rows, many keys); the chunks leave
 // (maximum, sum, unnormalised O) per row and a second kernel merges them.  The cut is a launch parameter that
 // depends on the window and the head count only.  Which tile a workgroup owns it finds itself from the step's
@@ -53,6 +60,26 @@ __device__ __forceinline__ la_s16x4_t la_read_transposed(const char* at) {
     return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) la_s16x4_t*)at);
 }
 
+// COUNT products, the operands of BATCH of them read from LDS together: left to itself, with nearly all registers taken, the compiler
+// reads one, waits for it and makes its product, and a read's wait is ten times the product.  (Four are what the registers have room for
+// at rank 512.)
+template <int BATCH, int COUNT, typename Read, typename Make>
+__device__ __forceinline__ void la_products(Read read, Make make) {
+    static_assert(COUNT % BATCH == 0, "whole batches");
+#pragma unroll
+    for (int b = 0; b < COUNT; b += BATCH) {
+        la_pack a[BATCH];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) a[i] = read(b + i);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) make(b + i, a[i]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
+#define LA_BATCH 4
+
 // SPLIT: all WAVES wavefronts share one tile of 16 rows (decoded tokens): they stage together, each makes the
 // scores again (cheap) and every WAVES-th tile of 16 latent dims of the second product.
 template <int WAVES, int NT, int KS, bool SPLIT>      // rank <= 16 NT, rank + rot <= 32 KS
@@ -69,7 +96,7 @@ latent_attention_cores_kernel(void* __restrict__ out, int out_f32, float* __rest
     static_assert(P % 8 == 0 && (P * 16) % 256 == 128 && KI * WAVES * ZI_WAVE == LA_BK * P, "whole loads, rows half the banks apart");
     __shared__ __attribute__((aligned(16))) la_u32x4_t buf_a[LA_BK * P];
     __shared__ __attribute__((aligned(16))) la_u32x4_t buf_b[LA_BK * P];
-    const int lane = threadIdx.x % ZI_WAVE, wave = threadIdx.x / ZI_WAVE, r = lane % 16, j = lane / 16;
+    const int lane = threadIdx.x % ZI_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / ZI_WAVE), r = lane % 16, j = lane / 16;
     // the entry whose tiles this one is among: 64 entries at a time, a lane each, their tiles summed up over the lanes
     int tile = blockIdx.x, e = entries;
     for (int e0 = 0; e0 < entries; e0 += ZI_WAVE) {
@@ -140,12 +167,15 @@ latent_attention_cores_kernel(void* __restrict__ out, int out_f32, float* __rest
 #pragma unroll
     for (int t = 0; t < OT; ++t) o[t] = (la_f32x4_t){0.f, 0.f, 0.f, 0.f};
 
-    // the place in the pool of key kb + lane % 32, or -1: past the end, or a page that is not held
-    auto places = [&](int kb) {
+    // the page of key kb + lane % 32, and from it its place in the pool, or -1: past the end, or a page that is not held.  Asked for
+    // in one turn and used in the next: to wait for it is to wait for the loads into LDS that were issued before it.
+    auto ask = [&](int kb) {
+        const int kp = kb + (lane & (LA_BK - 1)), pi = (kp <= k_hi ? kp : k_hi) / page_size;
+        return bt[pi < max_pages ? pi : max_pages - 1];
+    };
+    auto places = [&](int kb, int page) {
         const int kp = kb + (lane & (LA_BK - 1)), kc = kp <= k_hi ? kp : k_hi;
-        const int pi = kc / page_size;
-        const int page = bt[pi < max_pages ? pi : max_pages - 1];
-        return (kp <= k_hi && (unsigned)page < (unsigned)num_pages) ? page * page_size + kc % page_size : -1;
+        return (kp <= k_hi) & ((unsigned)page < (unsigned)num_pages) ? page * page_size + kc % page_size : -1;
     };
     auto issue = [&](int slots, la_u32x4_t* dst) {
         int ln = lane;      // (what a lane loads is worked out anew every block: kept, it takes the registers of the sums)
@@ -154,8 +184,9 @@ latent_attention_cores_kernel(void* __restrict__ out, int out_f32, float* __rest
         for (int i = 0; i < KI; ++i) {
             const int L = (wave * KI + i) * ZI_WAVE + ln, key = L / P, d = ((L % P) ^ la_swizzle(key)) * 8;
             const int slot = __shfl(slots, key, ZI_WAVE);
-            const zi_bf16* src = d < rank ? c_cache + (int64_t)slot * rank + d : kr_cache + (int64_t)slot * rot + (d - rank);
-            if (slot < 0 || d >= qw) src = reinterpret_cast<const zi_bf16*>(la_zero16);
+            const bool latent = d < rank;
+            const zi_bf16* src = (latent ? c_cache : kr_cache) + ((int64_t)slot * (latent ? rank : rot) + (latent ? d : d - rank));
+            if ((slot < 0) | (d >= qw)) src = reinterpret_cast<const zi_bf16*>(la_zero16);
             __builtin_amdgcn_global_load_lds(src, dst + (wave * KI + i) * ZI_WAVE, 16, 0, 0);
         }
     };
@@ -171,16 +202,15 @@ latent_attention_cores_kernel(void* __restrict__ out, int out_f32, float* __rest
     auto work = [&](int kb, const la_u32x4_t* buf) {
         const char* base = reinterpret_cast<const char*>(buf);
         la_f32x4_t s[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            s[h] = (la_f32x4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
+        s[0] = s[1] = (la_f32x4_t){0.f, 0.f, 0.f, 0.f};
+        la_products<LA_BATCH, 2 * KS>(
+            [&](int i) {
+                const int ks = i / 2, h = i % 2;
                 la_pack a;
                 a.u = *reinterpret_cast<const la_u32x4_t*>(base + ((ks & 1) ? s_odd : s_even) + h * (16 * P * 16) + (ks / 2) * 128);
-                s[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.b, q[ks].b, s[h], 0, 0, 0);
-            }
-        }
+                return a;
+            },
+            [&](int i, const la_pack& a) { s[i % 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.b, q[i / 2].b, s[i % 2], 0, 0, 0); });
         // lane (r, j) holds, of row r, the keys kb + 16 h + 4 j + x; in base-2 units from here on
         float mb = LA_EMPTY;
         const bool whole = kb >= all_lo && kb + LA_BK - 1 <= all_hi && kb + LA_BK - 1 <= k_hi;
@@ -216,46 +246,44 @@ latent_attention_cores_kernel(void* __restrict__ out, int out_f32, float* __rest
 #pragma unroll
             for (int tq = 0; tq < OT; ++tq) o[tq] *= corr;
         }
+        // groups of tiles, each either whole or left out: what lies behind the rank is staged too, and is not stored
+        constexpr int G = OT < 16 ? OT : 16;
 #pragma unroll
-        for (int tq = 0; tq < OT; ++tq) {
-            if (SPLIT) {
-                const int t = tq * WAVES + wave;
-                if (t * 16 < rank) {
-                    const char* at = base + (vrow * P + ((t * 2 + ((r & 3) >> 1)) ^ vsw)) * 16 + (r & 1) * 8;
+        for (int g = 0; g < OT; g += G) {
+            if (g * (SPLIT ? WAVES : 1) * 16 >= rank) break;
+            la_products<(G < LA_BATCH ? G : LA_BATCH), G>(
+                [&](int i) {
+                    const int tq = g + i, t = tq * WAVES + wave;
+                    const char* at = SPLIT ? base + (vrow * P + ((t * 2 + ((r & 3) >> 1)) ^ vsw)) * 16 + (r & 1) * 8
+                                           : base + v_at[tq & 3] + (tq / 4) * 128;
                     la_pack a;
                     a.h[0] = la_read_transposed(at);
                     a.h[1] = la_read_transposed(at + 16 * P * 16);
-                    o[tq] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.b, pb.b, o[tq], 0, 0, 0);
-                }
-            } else if (tq * 16 < rank) {
-                const char* at = base + v_at[tq & 3] + (tq / 4) * 128;
-                la_pack a;
-                a.h[0] = la_read_transposed(at);
-                a.h[1] = la_read_transposed(at + 16 * P * 16);
-                o[tq] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.b, pb.b, o[tq], 0, 0, 0);
-            }
+                    return a;
+                },
+                [&](int i, const la_pack& a) { o[g + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.b, pb.b, o[g + i], 0, 0, 0); });
         }
     };
     // Two blocks a turn, buffer a then b.  At each barrier the block about to be worked on has arrived (the compiler
     // waits for all loads into LDS before a barrier) and everyone has finished with the other buffer.
     if (k_lo <= k_hi) {
-        issue(places(k_lo), buf_a);
-        int next = places(k_lo + LA_BK);
-        int kb = k_lo;
+        issue(places(k_lo, ask(k_lo)), buf_a);
+        int page = ask(k_lo + LA_BK), kb = k_lo;
+        auto ahead = [&](la_u32x4_t* dst) {
+            asm volatile("" : "+v"(page));      // (here, behind the barrier)
+            if (kb + LA_BK > k_hi) return;
+            const int slots = places(kb + LA_BK, page);
+            page = ask(kb + 2 * LA_BK);
+            issue(slots, dst);
+        };
         while (true) {
             __syncthreads();
-            if (kb + LA_BK <= k_hi) {
-                issue(next, buf_b);
-                next = places(kb + 2 * LA_BK);
-            }
+            ahead(buf_b);
             work(kb, buf_a);
             if (kb + LA_BK > k_hi) break;
             kb += LA_BK;
             __syncthreads();
-            if (kb + LA_BK <= k_hi) {
-                issue(next, buf_a);
-                next = places(kb + 2 * LA_BK);
-            }
+            ahead(buf_a);
             work(kb, buf_b);
             if (kb + LA_BK > k_hi) break;
             kb += LA_BK;
