@@ -479,6 +479,8 @@ __device__ __attribute__((aligned(16))) const unsigned pf_zero16[4] = {0u, 0u, 0
 // does not change.  For that the values' tile holds 16 keys after 16 keys, of each every dim's two pieces (swapped for dims 8 to 15 of 16,
 // so that sixteen lanes' reads touch every bank once), as pages of 16 hold them: an instruction takes 1 KB in one run.  us a layer, the
 // same bits: 2,048 tokens of 12 heads 45.0 to 41.2, 2,048 of 28 heads 72.9 to 69.8, 1,163 tokens after 2,048 of 28 heads 113.9 to 104.2.
+// (With the two buffers in one array the compiler could not tell them apart and waited for the next block's loads before it read this
+// one's: 2,048 tokens of 12 heads 41.2, in arrays of their own 40.5.)
 template <int D, int QW, int KH, bool LOGB, int MAPS, bool PAGED>
 __global__ void __launch_bounds__(4 * KH * ZI_WAVE, KH == 1 ? 2 : 1)
 attention_prefill_dma_kernel(zi_bf16* __restrict__ out, int64_t ldo, const zi_bf16* __restrict__ q, int64_t ldq,
@@ -507,12 +509,8 @@ attention_prefill_dma_kernel(zi_bf16* __restrict__ out, int64_t ldo, const zi_bf
     constexpr int THREADS = WAVES * ZI_WAVE;
     constexpr int KI = KCH / THREADS, VI = VCH / THREADS;   // load instructions a wavefront issues per tile
     constexpr int KSW = 16 / KC;                     // key rows that share 256 bytes of LDS (and one swizzle)
-    __shared__ __attribute__((aligned(16))) uint4 k_ab[2 * KCH];
-    __shared__ __attribute__((aligned(16))) uint4 v_ab[2 * VCH];
-    uint4* const k_a = k_ab;
-    uint4* const k_b = k_ab + KCH;
-    uint4* const v_a = v_ab;
-    uint4* const v_b = v_ab + VCH;
+    // (arrays of their own, so that the compiler can tell a buffer that is read from one that loads are on their way to)
+    __shared__ __attribute__((aligned(16))) uint4 k_a[KCH], k_b[KCH], v_a[VCH], v_b[VCH];
     __shared__ int32_t bt_lds[ZI_PF_CHUNK_LONG / 8 + 8];     // the pages of this workgroup's keys (page size >= 8)
 
     const int tile = blockIdx.x / nh, h = blockIdx.x % nh;
@@ -784,19 +782,18 @@ attention_prefill_dma_kernel(zi_bf16* __restrict__ out, int64_t ldo, const zi_bf
         }
         }
     };
-    // Two blocks a turn, buffer a then b.  At each barrier the block about to be worked on has arrived
-    // (the compiler waits for all loads into LDS before a barrier) and everyone has finished with the
-    // other buffer, so the block after it is requested into that one at once.
+    // Two blocks a turn, buffer a then b.  At each barrier the block about to be worked on has arrived and everyone has finished with
+    // the other buffer, so the block after it is requested into that one at once.
     issue(kb_begin, k_a, v_a);
     int kb0 = kb_begin;
     while (true) {
-        __syncthreads();
+        zi_barrier_loaded();
         if (kb0 + BS <= khi) issue(kb0 + BS, k_b, v_b);
         clean(kb0, v_a);
         work(kb0, k_a, v_a);
         if (kb0 + BS > khi) break;
         kb0 += BS;
-        __syncthreads();
+        zi_barrier_loaded();
         if (kb0 + BS <= khi) issue(kb0 + BS, k_a, v_a);
         clean(kb0, v_b);
         work(kb0, k_b, v_b);
@@ -815,13 +812,15 @@ attention_prefill_dma_kernel(zi_bf16* __restrict__ out, int64_t ldo, const zi_bf
         // the two wavefronts of a query group merge their (maximum, sum, output) through LDS; nobody reads
         // the tiles any more
         // (the tiles of keys are the smaller ones where a key row holds several maps)
-        float* mo = reinterpret_cast<float*>(MAPS == 1 ? k_ab : v_ab);      // [qs][QW][DT][64][4]: within two tiles
-        float* ml = reinterpret_cast<float*>(MAPS == 1 ? v_ab : k_ab);      // [qs][QW][64][2]
-        static_assert(sizeof(float) * 4 * QW * DT * ZI_WAVE * 4 <= sizeof(uint4) * 2 * (MAPS == 1 ? KCH : VCH), "the tiles hold the merge");
+        // sub-tile u's outputs [qs][DT][64][4] in a tile
+        auto mo = [&](int u) { return reinterpret_cast<float*>(MAPS == 1 ? (u ? k_b : k_a) : (u ? v_b : v_a)) + qs * (DT * ZI_WAVE * 4); };
+        float* ml = reinterpret_cast<float*>(MAPS == 1 ? v_a : k_a);      // [qs][QW][64][2]
+        static_assert(sizeof(float) * 4 * DT * ZI_WAVE * 4 <= sizeof(uint4) * (MAPS == 1 ? KCH : VCH) &&
+                      sizeof(float) * 4 * QW * ZI_WAVE * 2 <= sizeof(uint4) * (MAPS == 1 ? VCH : KCH), "the tiles hold the merge");
         if (kh > 0) {
 #pragma unroll
             for (int u = 0; u < QW; ++u) {
-                float* dst = mo + (qs * QW + u) * (DT * ZI_WAVE * 4);
+                float* dst = mo(u);
 #pragma unroll
                 for (int dd = 0; dd < DT; ++dd) *reinterpret_cast<pf_f32x4_t*>(dst + (dd * ZI_WAVE + lane) * 4) = o[u][dd];
                 ml[((qs * QW + u) * ZI_WAVE + lane) * 2] = m[u];
@@ -832,7 +831,7 @@ attention_prefill_dma_kernel(zi_bf16* __restrict__ out, int64_t ldo, const zi_bf
         if (kh > 0) return;
 #pragma unroll
         for (int u = 0; u < QW; ++u) {
-            const float* src = mo + (qs * QW + u) * (DT * ZI_WAVE * 4);
+            const float* src = mo(u);
             const float m2 = ml[((qs * QW + u) * ZI_WAVE + lane) * 2];
             const float l2 = ml[((qs * QW + u) * ZI_WAVE + lane) * 2 + 1];
             const float mm = fmaxf(m[u], m2);

@@ -264,8 +264,8 @@ latent_attention_cores_kernel(void* __restrict__ out, int out_f32, float* __rest
                 [&](int i, const la_pack& a) { o[g + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.b, pb.b, o[g + i], 0, 0, 0); });
         }
     };
-    // Two blocks a turn, buffer a then b.  At each barrier the block about to be worked on has arrived (the compiler
-    // waits for all loads into LDS before a barrier) and everyone has finished with the other buffer.
+    // Two blocks a turn, buffer a then b.  At each barrier the block about to be worked on has arrived and everyone has finished with
+    // the other buffer.
     if (k_lo <= k_hi) {
         issue(places(k_lo, ask(k_lo)), buf_a);
         int page = ask(k_lo + LA_BK), kb = k_lo;
@@ -277,12 +277,12 @@ latent_attention_cores_kernel(void* __restrict__ out, int out_f32, float* __rest
             issue(slots, dst);
         };
         while (true) {
-            __syncthreads();
+            zi_barrier_loaded();
             ahead(buf_b);
             work(kb, buf_a);
             if (kb + LA_BK > k_hi) break;
             kb += LA_BK;
-            __syncthreads();
+            zi_barrier_loaded();
             ahead(buf_a);
             work(kb, buf_b);
             if (kb + LA_BK > k_hi) break;
