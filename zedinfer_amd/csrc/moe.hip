@@ -327,6 +327,11 @@ union moe_pack {
 
 #define MOE_KB 64
 #define MOE_XCDS 8
+// Turns through the buffers in a row.  The compiler waits for all loads at the first read in a loop's body, also for those that were asked
+// for a moment ago: once in this many turns.  us, the two products of 32 experts' prompt tiles, waiting in every turn, every second and
+// every fourth (32 experts of 1,536 x 1,536, 8,000 pairs 91 and 80, 85 and 73, 82 and 72; 73 tiles of 3,584 x 2,560
+// 249 and 262, 230 and 250, 223 and 247; 32 pairs of these 108 and 100, 102 and 96, 100 and 95); eight turns are no faster
+#define MOE_TURNS 4
 // the longest row of weights whose tile of rows a buffer's 31-bit offsets reach
 #define MOE_MAX_K (1 << 21)
 
@@ -390,7 +395,8 @@ moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restr
         w_at[i] = (q < rows_w ? q * K + wpiece[i] : rows_w * K) * 2;
     }
     const int steps = (K + MOE_KB - 1) / MOE_KB;
-    // (columns past K, a multiple of 8: the tokens' are the row's first again, the weights' the next row's or zeros; both masked)
+    // (columns past K, a multiple of 8: the tokens' are the row's first again, the weights' the next row's or zeros; both masked, or, in
+    // the steps past the last that are asked for too, not read)
     auto issue = [&](moe_u32x4_t* buf, int t) {
         const int k0 = t * MOE_KB;
         const bool whole = k0 + MOE_KB <= K;
@@ -409,16 +415,13 @@ moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restr
         for (int c = 0; c < CT; ++c) acc[t][c] = (moe_f32x4_t){0.f, 0.f, 0.f, 0.f};
     const int sw = (r >> 1) & 7;
     auto step = [&](const moe_u32x4_t* buf, moe_u32x4_t* free, int t) __attribute__((always_inline)) {
-        if (t >= steps) return;
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
-        const int after = steps - 1 - t;       // steps whose loads may still be on their way
-        if (after >= ST - 2) moe_wait<(ST - 2) * PW>();
-        else moe_wait<0>();
+        moe_wait<(ST - 2) * PW>();             // the newest steps' loads may still be on their way
         __builtin_amdgcn_s_barrier();          // all wavefronts' loads of the step are there, and all are done with `free`
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
-        if (t + ST - 1 < steps) issue(free, t + ST - 1);
+        issue(free, t + ST - 1);
         __builtin_amdgcn_sched_barrier(0);
         const int left = K - t * MOE_KB;
 #pragma unroll
@@ -445,18 +448,22 @@ moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restr
     };
     issue(s0, 0);
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (ST > 2) if (steps > 1) issue(s1, 1);
+    if constexpr (ST > 2) issue(s1, 1);
     __builtin_amdgcn_sched_barrier(0);
-    for (int t = 0; t < steps; t += ST) {
-        if constexpr (ST == 2) {
-            step(s0, s1, t);
-            step(s1, s0, t + 1);
-        } else {
-            step(s0, s2, t);
-            step(s1, s0, t + 1);
-            step(s2, s1, t + 2);
+    for (int t = 0, left = 1; left;) {
+#pragma unroll
+        for (int turn = 0; turn < MOE_TURNS; ++turn) {
+            step(s0, ST == 2 ? s1 : s2, t);
+            if (!(left = ++t < steps)) break;
+            step(s1, s0, t);
+            if (!(left = ++t < steps)) break;
+            if constexpr (ST > 2) {
+                step(s2, s1, t);
+                if (!(left = ++t < steps)) break;
+            }
         }
     }
+    moe_wait<0>();
     // a lane holds four consecutive columns of a row: one store of 16 (float32) or 8 bytes (bfloat16) where the rows
     // allow it
     const bool whole = ldo % 4 == 0 && ((uintptr_t)out % 16) == 0;
