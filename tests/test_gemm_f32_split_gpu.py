@@ -39,6 +39,36 @@ def test_as_exact_as_float32_sums_and_without_a_bias(M, N, K, kernel):
         assert torch.equal(ops.linear(x[rows].contiguous(), w, b).double(), got[rows])
 
 
+def _mean_bound(K):
+    """The mean of the error, 2-norm over 2-norm: the roundings of one chain's sums times 2^-24 of the result's rms each, added as squares."""
+    return 2.0 ** -24 * (2 * 6 * -(-(-(-K // 64)) // 8) + 11) ** 0.5
+
+
+def _error(x, w):
+    from zedinfer_amd import ops
+    got, ref = ops.linear(x, w).double(), x.double() @ w.double().t()
+    return float(((got - ref).square().sum(1) / ref.square().sum(1)).max().sqrt()) if ref.numel() else 0.0
+
+
+@pytest.mark.parametrize("M,N,K,kernel", CASES)
+def test_sums_made_again_from_the_operands(M, N, K, kernel):
+    """A row whose values all round to an infinity in bfloat16 is as exact as any other; a row with a NaN is NaNs, all of it; neither touches the others."""
+    from zedinfer_amd import ops
+    assert ops.linear_f32_kernel(M, N, K) == kernel
+    x, w, _ = _linear(M, N, K)
+    w *= 2.0 ** -110
+    y = ops.linear(x, w)
+    x[0] = torch.where(x[0] < 0, -3.4e38, 3.4e38)
+    assert _error(x[:1], w) <= _mean_bound(K)
+    x[M - 1, K - 1] = float("nan")
+    got = ops.linear(x, w)
+    ref = x[:1].double() @ w.double().t()
+    assert float((got[:1] - ref).norm() / ref.norm()) <= _mean_bound(K)
+    assert bool(torch.isnan(got[M - 1]).all()) and torch.equal(got[1:M - 1], y[1:M - 1])
+    if N % 2 == 0 and ops.linear_swiglu_halves_supported(x, w):
+        assert torch.equal(ops.linear_swiglu_halves(x, w)[:M - 1], ops.swiglu(got[:, :N // 2], got[:, N // 2:])[:M - 1])
+
+
 @pytest.mark.parametrize("M,N", [(3, 300), (3, 2100), (12, 4100), (12, 2070), (40, 2040), (100, 2050), (449, 1500), (449, 2047), (700, 4610)])
 def test_values_that_do_not_split(M, N):
     """Infinities, NaNs and values that round to an infinity in bfloat16 give what the float32 sum gives, in their row and column alone;

@@ -100,17 +100,55 @@ __device__ __forceinline__ gf_f32x4_t gf_multiply(const gf_parts& w, const gf_pa
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.p[0].b, x.p[0].b, acc, 0, 0, 0);
 }
 
-// The sum as it is if it is finite.  Else an operand was an infinity, a NaN or a value whose first part rounds to an infinity, whose other
-// parts are no numbers, or the sum left the range: the same sum again from the float32 operands, one k after the other.
-__device__ __forceinline__ float gf_finite(float sum, const float* __restrict__ x_row, const float* __restrict__ w_row, int K) {
-    if ((__float_as_uint(sum) & 0x7f800000u) != 0x7f800000u) return sum;
-    float s = 0.f;
-    for (int k = 0; k < K; k += 4) {
-        const gf_f32x4_t a = *reinterpret_cast<const gf_f32x4_t*>(x_row + k), b = *reinterpret_cast<const gf_f32x4_t*>(w_row + k);
+// Four sums of a lane, of row `row` of x and of rows w_row(e) of w, as they are if they are finite.  Else an operand was an infinity, a NaN or a
+// value whose first part rounds to an infinity, whose other parts are no numbers, or the sum left the range: the same sum again from the
+// float32 operands, by the whole wavefront (all its lanes come here together; mine(e): sum e is an output), so that a lane has K / 64
+// multiply-adds one after the other and the sum is at least as exact.  A row of x with a NaN, what a request whose values ran away
+// brings to every product, has NaNs only: it is remembered in nan_rows and its other outputs cost nothing; a weight row with one gives
+// them to all rows in hand.
+// (One such row among 8, us, every lane for itself, now, and without such a row: 17,920 x 1,536 with the activation 1,178, 32 and 21; 1,536 x 8,960 1,053, 23 and
+// 17; 151,936 x 1,536 9,085, 185 and 159.  A weight row with one, 450 rows of 1,536 x 8,960: 376, 114 and 107.)
+template <typename Mine, typename Row>
+__device__ __forceinline__ void gf_finite(gf_f32x4_t& s, int row, Mine mine, Row w_row, const float* x, int64_t ldx, const float* w, int64_t ldw, int K,
+                                          uint64_t& nan_rows) {
+    const float no_number = __uint_as_float(0x7fc00000u);
+    if (__ballot(s[0] * 0.f + s[1] * 0.f + s[2] * 0.f + s[3] * 0.f != 0.f) == 0) return;      // (0 times what is not finite is a NaN)
+    const int lane = threadIdx.x & (ZI_WAVE - 1);
+#pragma unroll 1
+    for (int e = 0; e < 4; ++e) {
+        float sum = e == 0 ? s[0] : e == 1 ? s[1] : e == 2 ? s[2] : s[3];
+        const int row_w = w_row(e);
+        uint64_t todo = __ballot(mine(e) && (__float_as_uint(sum) & 0x7f800000u) == 0x7f800000u);
+        while (todo) {
+            const int of = __builtin_ctzll(todo), of_x = __builtin_amdgcn_readlane(row, of), of_w = __builtin_amdgcn_readlane(row_w, of);
+            todo &= todo - 1;
+            float again = no_number;
+            if (!(nan_rows >> of_x & 1)) {
+                const float *a = x + of_x * ldx, *b = w + of_w * ldw;
+                bool nan_x = false, nan_w = false;
+                again = 0.f;
+#pragma unroll 1
+                for (int k = lane * 4; k < K; k += ZI_WAVE * 4) {
+                    const gf_f32x4_t u = *reinterpret_cast<const gf_f32x4_t*>(a + k), v = *reinterpret_cast<const gf_f32x4_t*>(b + k);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s = fmaf(a[e], b[e], s);
+                    for (int i = 0; i < 4; ++i) {
+                        again = fmaf(u[i], v[i], again);
+                        nan_x |= u[i] != u[i];
+                        nan_w |= v[i] != v[i];
+                    }
+                }
+                again = zi_wave_sum(again);
+                if (__ballot(nan_x)) nan_rows |= 1ull << of_x;
+                if (__ballot(nan_w)) {
+                    todo &= ~__ballot(row_w == of_w);
+                    if (row_w == of_w) sum = no_number;
+                }
+            }
+            if (lane == of) sum = again;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[i] = i == e ? sum : s[i];
     }
-    return s;
 }
 
 // PAIR: 8 weight rows and up to 8 rows of x; else 16 weight rows and up to 16 * MT rows of x a workgroup.  RING chunks are
@@ -194,21 +232,18 @@ gemm_f32_split_stream_kernel(float* __restrict__ out, const float* __restrict__ 
         part[wave][t][lane] = s;
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < MT * ZI_WAVE; i += GF_PARTS * ZI_WAVE) {
-        const int t = i / ZI_WAVE, l = i % ZI_WAVE, m = t * 16 + (l & 15), n = (l >> 4) * 4;
-        gf_f32x4_t s = part[0][t][l], s2 = part[GF_PARTS / 2][t][l];
+    uint64_t nan_rows = 0;
+    for (int t = wave; t < MT; t += GF_PARTS) {
+        const int m = t * 16 + r, n = g * 4;
+        gf_f32x4_t s = part[0][t][lane], s2 = part[GF_PARTS / 2][t][lane];
 #pragma unroll
         for (int p = 1; p < GF_PARTS / 2; ++p) {
-            s += part[p][t][l];
-            s2 += part[GF_PARTS / 2 + p][t][l];
+            s += part[p][t][lane];
+            s2 += part[GF_PARTS / 2 + p][t][lane];
         }
         s += s2;
-        if (m < rows_x && n < rows_w) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (n + e < rows_w) s[e] = gf_finite(s[e], x + (m0 + m) * ldx, w + (int64_t)(n0 + n + e) * ldw, K);
-            gf_store4(out + (int64_t)(m0 + m) * ldo, bias, s, n0 + n, N, vec_out);
-        }
+        gf_finite(s, m, [&](int e) { return m < rows_x && n + e < rows_w; }, [&](int e) { return n0 + n + e; }, x + m0 * ldx, ldx, w, ldw, K, nan_rows);
+        if (m < rows_x && n < rows_w) gf_store4(out + (int64_t)(m0 + m) * ldo, bias, s, n0 + n, N, vec_out);
     }
 }
 
@@ -282,6 +317,7 @@ gemm_f32_split_held_kernel(float* __restrict__ out, const float* __restrict__ x,
             for (int h = 0; h < H; ++h) xs[s][h] = gf_turn_of_chain<PAIR>(h, turn[wave][(s * H + h) & 1], xr[s][h][0], xr[s][h][1], lane);
     }
     int b = 0, whose = 0;
+    uint64_t nan_rows = 0;
     for (int group = blockIdx.x; group < groups; group += gridDim.x, b ^= 1, whose = (whose + 1) % GF_PARTS) {
         wb = weights(group + (int)gridDim.x);
         gf_f32x4_t acc[H];
@@ -316,14 +352,10 @@ gemm_f32_split_held_kernel(float* __restrict__ out, const float* __restrict__ x,
         }
         s += s2;
         const int64_t n = (int64_t)group * NC + g * 4;
-        if (r < M && g * 4 < NR) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {       // sum e of this lane is weight row g * 4 + e of the group
-                const int of = g * 4 + e, up = GATED && of >= NC;
-                const int64_t at = (int64_t)group * NC + (up ? of - NC : of);
-                if (at < N) s[e] = gf_finite(s[e], x + r * ldx, w + (at + (up ? N : 0)) * ldw, K);
-            }
-        }
+        // sum e of this lane is weight row g * 4 + e of the group, a gate row or, from NC on, an up row
+        auto output = [&](int e) { return group * NC + (GATED && g * 4 + e >= NC ? g * 4 + e - NC : g * 4 + e); };
+        gf_finite(s, r, [&](int e) { return r < M && g * 4 + e < NR && output(e) < N; }, [&](int e) { return output(e) + (GATED && g * 4 + e >= NC ? N : 0); },
+                  x, ldx, w, ldw, K, nan_rows);
         if (GATED) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) s[e] = gf_gate(s[e], __shfl(s[e], lane + (PAIR ? 16 : 32), ZI_WAVE));
@@ -514,36 +546,41 @@ gemm_f32_split_tile_kernel(float* __restrict__ out, const float* __restrict__ x,
                 }
         }
     }
-    auto finish = [&](gf_f32x4_t* s, int t, int u0, int of, int l) __attribute__((always_inline)) {
+    constexpr int STEP = GATED ? 2 : 1;
+    uint64_t nan_rows = 0;
+    auto finish = [&](gf_f32x4_t* s, int t, int u0, int of) __attribute__((always_inline)) {
         // the sums of a wavefront's block (t, u0), or of its gate and up blocks: checked, activated, stored
+        int l = lane;
+        asm volatile("" : "+v"(l));        // (what is worked out of it is worked out here: kept, it takes the loop's registers)
         const int m = m0 + t * 16 + (l & 15), n = n0 + of * NW + (GATED ? u0 / 2 : u0) * 16 + (l >> 4) * 4;
+#pragma unroll
+        for (int i = 0; i < STEP; ++i)
+            gf_finite(s[i], t * 16 + (l & 15), [&](int e) { return m < M && n + e < N; }, [&](int e) { return n + e + (i ? N : 0); }, x + m0 * ldx, ldx, w, ldw, K,
+                      nan_rows);
         if (m >= M || n >= N) return;
-#pragma unroll
-        for (int i = 0; i < (GATED ? 2 : 1); ++i)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (n + e < N) s[i][e] = gf_finite(s[i][e], x + m * ldx, w + ((int64_t)n + e + (i ? N : 0)) * ldw, K);
         if (GATED) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) s[0][e] = gf_gate(s[0][e], s[GATED][e]);
         }
         gf_store4(out + (int64_t)m * ldo, GATED ? nullptr : bias, s[0], n, N, vec_out);
     };
-    constexpr int STEP = GATED ? 2 : 1;
     if (GROUPS == 1) {
+        // (through this thread's own places in LDS, so that what checks and stores them is there once and takes no registers from the loop above)
 #pragma unroll
         for (int t = 0; t < MT; ++t)
 #pragma unroll
-            for (int u = 0; u < NT; u += STEP) {
-                gf_f32x4_t s[STEP];
-#pragma unroll
-                for (int i = 0; i < STEP; ++i)          // (acc: zeros where the last run ended)
-                {
-                    s[i] = sum[0][t][u + i] + (acc[0][t][u + i] - acc[1][t][u + i]);
-                    if (parts >= GF_PARTS / 2) s[i] = first[(t * NT + u + i) * THREADS] + s[i];
-                }
-                finish(s, t, u, wave, lane);
+            for (int u = 0; u < NT; ++u) {          // (acc: zeros where the last run ended)
+                gf_f32x4_t& at = first[(t * NT + u) * THREADS];
+                const gf_f32x4_t s = sum[0][t][u] + (acc[0][t][u] - acc[1][t][u]);
+                at = parts >= GF_PARTS / 2 ? at + s : s;
             }
+#pragma unroll 1
+        for (int b = 0; b < MT * NT; b += STEP) {
+            gf_f32x4_t s[STEP];
+#pragma unroll
+            for (int i = 0; i < STEP; ++i) s[i] = first[(b + i) * THREADS];
+            finish(s, b / NT, b % NT, wave);
+        }
         return;
     }
     // the runs' sums meet in LDS (past the last barrier nobody reads x there)
@@ -572,7 +609,7 @@ gemm_f32_split_tile_kernel(float* __restrict__ out, const float* __restrict__ x,
             s[i] += s2;
         }
         const int of = b * STEP / (MT * NT), tu = b * STEP % (MT * NT);
-        finish(s, tu / NT, tu % NT, of, lane);
+        finish(s, tu / NT, tu % NT, of);
     }
 }
 
