@@ -69,10 +69,25 @@ def test_sums_made_again_from_the_operands(M, N, K, kernel):
         assert torch.equal(ops.linear_swiglu_halves(x, w)[:M - 1], ops.swiglu(got[:, :N // 2], got[:, N // 2:])[:M - 1])
 
 
+@pytest.mark.parametrize("M,N,K,kernel", CASES)
+def test_small_and_large_values_keep_their_last_bits(M, N, K, kernel):
+    """Values of any mantissa over float32's whole range, on either side: as exact as values around one."""
+    from zedinfer_amd import ops
+    assert ops.linear_f32_kernel(M, N, K) == kernel
+    x, w, _ = _linear(M, N, K)
+    for e in (-60, -90, -104, -112, -120, -126, -132, -138, -145):       # (from -126 on subnormal: the reference multiplies what is left of them)
+        other = 2.0 ** min(-e - 20, 121)
+        small = x * 2.0 ** e if e > -140 else torch.where(x.abs() < 1, torch.ones_like(x), x.round()) * 2.0 ** e
+        assert _error(small, w * other) <= _mean_bound(K), e
+        small = w * 2.0 ** e if e > -140 else torch.where(w.abs() < 1, torch.ones_like(w), w.round()) * 2.0 ** e
+        assert _error(x * other, small) <= _mean_bound(K), e
+    for e in (70, 104, 125):
+        assert _error(x * 2.0 ** (e - 3), w * 2.0 ** (-e)) <= _mean_bound(K) and _error(x * 2.0 ** (1 - e), w * 2.0 ** (e - 3)) <= _mean_bound(K), e
+
+
 @pytest.mark.parametrize("M,N", [(3, 300), (3, 2100), (12, 4100), (12, 2070), (40, 2040), (100, 2050), (449, 1500), (449, 2047), (700, 4610)])
 def test_values_that_do_not_split(M, N):
-    """Infinities, NaNs and values that round to an infinity in bfloat16 give what the float32 sum gives, in their row and column alone;
-    small and subnormal values keep their last bits."""
+    """Infinities, NaNs and values that round to an infinity in bfloat16 give what the float32 sum gives, in their row and column alone."""
     from zedinfer_amd import ops
     K = 1500
     x, w = torch.ones(M, K, device="cuda"), torch.ones(N, K, device="cuda")
