@@ -39,6 +39,18 @@ def test_as_exact_as_float32_sums_and_without_a_bias(M, N, K, kernel):
         assert torch.equal(ops.linear(x[rows].contiguous(), w, b).double(), got[rows])
 
 
+@pytest.mark.parametrize("half", [0, 1])
+@pytest.mark.parametrize("M,N,K,kernel", CASES)
+def test_no_bias_where_one_half_of_every_chunk_is_empty(M, N, K, kernel, half):
+    """The two chains change places from run to run, so the instruction's rounding down cancels in them too: test_as_exact_...'s bound on the mean."""
+    from zedinfer_amd import ops
+    assert ops.linear_f32_kernel(M, N, K) == kernel
+    x, w, _ = _linear(M, N, K)
+    x *= torch.arange(K, device="cuda") // 32 % 2 == half
+    err = ops.linear(x, w).double() - x.double() @ w.double().t()
+    assert float(err.mean().abs()) <= float(err.square().mean().sqrt()) * (1 / 16 + 6 / (M * N) ** 0.5)
+
+
 def _mean_bound(K):
     """The mean of the error, 2-norm over 2-norm: the roundings of one chain's sums times 2^-24 of the result's rms each, added as squares."""
     return 2.0 ** -24 * (2 * 6 * -(-(-(-K // 64)) // 8) + 11) ** 0.5

@@ -5,21 +5,29 @@
 // That needs the last part's last bit, 2^-23 of the value, to be a bfloat16 one: bfloat16 ends at 2^-133, so values below 2^-110 would lose
 // theirs (below 2^-126 0.4 % and more).  Operands are therefore split times 2^24, an exact step that lifts the smallest float32 to 2^-125,
 // where parts are not even subnormal, and finished sums take 2^-48.
-// Of the nine products of two values' parts the six largest are added; the other three lie below 2^-26 of the product.  Weights and x stay
+// Of the nine products of two values' parts the six largest are added; two of the others reach 2^-25 of the product each, the third 2^-34.  Weights and x stay
 // float32 in memory and are split on their way into the matrix cores; sums are float32.  A value that 2^24 takes past the range (2^104 and
 // above), infinities and NaNs leave parts that are no numbers, and sums from 2^80 on leave the range: a sum that is not finite is made again from the
 // float32 operands (gf_finite).
 //
 // The instruction cuts off what lies more than some three bits below its largest term's last bit, downwards whatever the sign, so sums come
 // out low, by a quarter of their rounding errors at 8,960 columns, every output alike; over a model's layers that adds up.  So one of the two
-// chains below is summed with x negated and subtracted: the two errors cancel in the mean.  Error against 64 bits, 2-norm over 2-norm,
-// of the float32 instruction's kernels, of these without the change of sign, of these: 1,536 columns 1.86e-7, 1.42e-7, 1.39e-7; 8,960
-// columns 4.3e-7, 3.7e-7, 3.6e-7; the logits of a 28-layer model 3.7e-7, 4.5e-7, 3.3e-7.
+// chains below is summed with x negated and subtracted, and the two change places from run to run: the errors cancel in the mean, also where
+// x lies in one half of every chunk alone (mean over rms then, changing places or not: 1,536 columns 0.00 and 0.15,
+// 8,960 0.01 and 0.22).
+//
+// Error against 64 bits, 2-norm over 2-norm, of the float32 instruction's kernels and of these: normal values 1.85e-7 and 1.38e-7 at 1,536 columns,
+// 4.3e-7 and 3.6e-7 at 8,960, their absolute values 4.9e-8 and 4.2e-8, 1.0e-7 and 8.0e-8; the logits of a 28-layer model 3.7e-7 and 3.3e-7 (with one
+// sign for all chains 4.5e-7).  These are further off where few products make a sum, a single one 2.5e-8 and 3.4e-8, eight 5.4e-8 and 6.1e-8, and
+// at many columns where half of every chunk is empty, so that one chain adds up what are two there: 1,536 columns 1.37e-7 and 1.35e-7, absolute
+// values 4.4e-8 and 5.0e-8; 8,960 3.06e-7 and 3.56e-7, 7.7e-8 and 1.04e-7.  That is the instruction's cutting, not the products left out: with the two
+// of 2^-25 added the figures are the same (a single one 3.4e-8), at 8 to 15 % more time.
 //
 // One order of the sums, the same in every kernel here, so that a row's result does not depend on M, on the tile it falls in or on the rest
 // of the batch: k is cut into GF_PARTS runs of whole chunks of 64 (a function of K alone); within a run the first and the second 32 of every
-// chunk are two chains, each 32 an instruction for every product of parts, whose lane group g holds k = 4 g .. 4 g + 3 and 16 more; a run's
-// sum is first - second chain; the sums of each half of the runs are added in rising order, then the two halves, then the bias.
+// chunk (in runs of odd number the second and the first) are two chains, each 32 an instruction for every product of parts, whose lane group
+// g holds k = 4 g .. 4 g + 3 and 16 more; a run's sum is first - second chain; the sums of each half of the runs are added in rising order,
+// then the two halves, then the bias.
 //
 // What bounds it: few rows the one pass over the weights; many rows, by counters at 2,048 rows of 4,096 x 4,096, the vector instructions
 // (57 % of the cycles, eleven for every two values split) and the matrix cores (51 %), which mostly take turns, beside LDS (43 %).
@@ -32,6 +40,7 @@
 #include "zi_gemm_f32.h"
 
 #define GF_KB 64             // k of a chunk
+static_assert((GF_SPLIT_ABOVE / GF_KB + GF_PARTS) / GF_PARTS > 2, "a run has three chunks and more");
 #define GF_HELD_CHUNKS 8     // chunks of a run that a wavefront can hold of 8 rows of x beside as many of weights (256 registers)
 
 // The three bfloat16 parts of eight values, largest first.
@@ -182,7 +191,7 @@ gemm_f32_split_stream_kernel(float* __restrict__ out, const float* __restrict__ 
         for (int h = 0; h < H; ++h)
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                const int k = c * (GF_KB * 4) + (PAIR ? i : h) * 128 + k_lane;
+                const int k = c * (GF_KB * 4) + ((PAIR ? i : h) ^ (wave & 1)) * 128 + k_lane;      // (see the top: the chains change places)
                 const bool in = c < c1 && k < K * 4;
 #pragma unroll
                 for (int t = 0; t < MT; ++t) xr[slot][h][t][i] = gf_load<0>(xb, in && x_row[t][i % RB] != GF_OUT ? x_row[t][i % RB] + k : GF_OUT);
@@ -282,7 +291,7 @@ gemm_f32_split_held_kernel(float* __restrict__ out, const float* __restrict__ x,
         return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(w + (rows ? n0 * ldw : 0)), 0,
                                                  rows ? (int)(((int64_t)(rows - 1) * ldw + K) * 4) : 0, 0x00020000);
     };
-    auto place = [&](int s, int h, int i) { return s * (GF_KB * 4) + (PAIR ? i : h) * 128; };
+    auto place = [&](int s, int h, int i) { return s * (GF_KB * 4) + ((PAIR ? i : h) ^ (wave & 1)) * 128; };      // (the chains change places)
     auto in = [&](int s, int h, int i) { return s < mine && k0 + place(s, h, i) < K * 4; };
     gf_f32x4_t wr[PER][H][2];
     gf_parts xs[PER][H];
@@ -419,20 +428,23 @@ gemm_f32_split_tile_kernel(float* __restrict__ out, const float* __restrict__ x,
     const int steps = GROUPS > 1 ? mine : chunks;      // chunks, the same number for all groups: they share the barriers
     gf_f32x4_t xr[DEPTH][XP][2], wr[DEPTH][NT][2];
     // (the step's place along k is the loads' scalar offset; bytes of a row from there on, none past the group's last chunk)
-    auto left = [&](const int h, int c) { return c < c1 ? K * 4 - c * (GF_KB * 4) - h * 128 : 0; };
-    auto fetch_x = [&](const int h, int c) __attribute__((always_inline)) {
-        const int rest = left(h, c);
+    auto left = [&](int at, int c) { return c < c1 ? K * 4 - at : 0; };
+    int in_part = 0, parts = 0;      // the chunk's place in its run, runs done (a group's first run is of even number)
+    // the chain of half h of the chunk `ahead` (at most 2, a run has 3 and more) after this one: the halves change places from run to run
+    auto place = [&](const int h, int c, int ahead) { return c * (GF_KB * 4) + (h ^ ((parts + (in_part + ahead >= per)) & 1)) * 128; };
+    auto fetch_x = [&](const int h, int c, int ahead) __attribute__((always_inline)) {
+        const int at = place(h, c, ahead), rest = left(at, c);
 #pragma unroll
         for (int p = 0; p < XP; ++p)
 #pragma unroll
-            for (int q = 0; q < 2; ++q) xr[h % DEPTH][p][q] = gf_load<0>(xb, x_lane + q * 64 < rest ? x_row[p] : GF_OUT, c * (GF_KB * 4) + h * 128 + q * 64);
+            for (int q = 0; q < 2; ++q) xr[h % DEPTH][p][q] = gf_load<0>(xb, x_lane + q * 64 < rest ? x_row[p] : GF_OUT, at + q * 64);
     };
-    auto fetch_w = [&](const int h, int c) __attribute__((always_inline)) {
-        const int rest = left(h, c);
+    auto fetch_w = [&](const int h, int c, int ahead) __attribute__((always_inline)) {
+        const int at = place(h, c, ahead), rest = left(at, c);
 #pragma unroll
         for (int u = 0; u < NT; ++u)
 #pragma unroll
-            for (int i = 0; i < 2; ++i) wr[h % DEPTH][u][i] = gf_load<0>(wb, w_lane < rest ? w_row[u][i] : GF_OUT, c * (GF_KB * 4) + h * 128);
+            for (int i = 0; i < 2; ++i) wr[h % DEPTH][u][i] = gf_load<0>(wb, w_lane < rest ? w_row[u][i] : GF_OUT, at);
     };
     auto stash = [&](const int h) __attribute__((always_inline)) {
 #pragma unroll
@@ -454,7 +466,6 @@ gemm_f32_split_tile_kernel(float* __restrict__ out, const float* __restrict__ x,
 #pragma unroll
             for (int i = 0; i < SUMS; ++i) sum[i][t][u] = zero;
         }
-    int in_part = 0, parts = 0;
     const int read_at = r * 4 + ((g ^ -(r >> 2)) & 3);
     // Half h of chunk c: its weights' parts lie in ws[h] and its x in buffer h.  While it is multiplied the next half's operands are split, one
     // vector instruction after the other in the time that the matrix cores take, and those of DEPTH halves later are asked for.
@@ -462,11 +473,11 @@ gemm_f32_split_tile_kernel(float* __restrict__ out, const float* __restrict__ x,
     auto step = [&](const int h, int c) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < NT; ++u) ws[h ^ 1][u] = gf_turn<GF_PLUS>(turn + u * 128, wr[(h ^ 1) % DEPTH][u][0], wr[(h ^ 1) % DEPTH][u][1], lane);
-        if (DEPTH == 2) fetch_w(h ^ 1, h ? c + 2 : c + 1);
-        else fetch_w(h, c + 1);
+        if (DEPTH == 2) fetch_w(h ^ 1, h ? c + 2 : c + 1, h ? 2 : 1);
+        else fetch_w(h, c + 1, 1);
         stash(h ^ 1);
-        if (DEPTH == 2) fetch_x(h ^ 1, h ? c + 2 : c + 1);
-        else fetch_x(h, c + 1);
+        if (DEPTH == 2) fetch_x(h ^ 1, h ? c + 2 : c + 1, h ? 2 : 1);
+        else fetch_x(h, c + 1, 1);
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
             gf_parts xs;
@@ -496,24 +507,24 @@ gemm_f32_split_tile_kernel(float* __restrict__ out, const float* __restrict__ x,
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
         __builtin_amdgcn_sched_barrier(0);
     };
-    fetch_x(0, c0);
+    fetch_x(0, c0, 0);
     __builtin_amdgcn_sched_barrier(0);
-    fetch_w(0, c0);
+    fetch_w(0, c0, 0);
     __builtin_amdgcn_sched_barrier(0);
     if (DEPTH == 2) {
-        fetch_x(1, c0);
+        fetch_x(1, c0, 0);
         __builtin_amdgcn_sched_barrier(0);
-        fetch_w(1, c0);
+        fetch_w(1, c0, 0);
         __builtin_amdgcn_sched_barrier(0);
     }
     stash(0);
-    if (DEPTH == 2) fetch_x(0, c0 + 1);
-    else fetch_x(1, c0);
+    if (DEPTH == 2) fetch_x(0, c0 + 1, 1);
+    else fetch_x(1, c0, 0);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < NT; ++u) ws[0][u] = gf_turn<GF_PLUS>(turn + u * 128, wr[0][u][0], wr[0][u][1], lane);
-    if (DEPTH == 2) fetch_w(0, c0 + 1);
-    else fetch_w(1, c0);
+    if (DEPTH == 2) fetch_w(0, c0 + 1, 1);
+    else fetch_w(1, c0, 0);
     __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
     for (int c = 0; c < steps; ++c) {
