@@ -119,6 +119,19 @@ def test_values_that_do_not_split(M, N):
         assert torch.equal(a.nan_to_num(), ops.swiglu(y, y).nan_to_num())
 
 
+@pytest.mark.parametrize("M,I,K", [(100, 3001, 1500), (129, 4097, 1500), (64, 8960, 1536), (330, 1537, 1412), (600, 1000, 2052)])
+def test_tiles_of_32_by_96_take_the_activation(M, I, K):
+    """The bits of the product and the activation one after the other; gate and up rows that end within a tile."""
+    from zedinfer_amd import ops
+    assert ops.linear_f32_kernel(M, 2 * I, K) == "tile_96_halves"
+    x, w, _ = _linear(M, 2 * I, K)
+    assert ops.linear_swiglu_halves_supported(x, w)
+    two = ops.linear(x, w)
+    wide = torch.zeros((M, I + 6), device="cuda")
+    ops.linear_swiglu_halves(x, w, out=wide[:, 3:I + 3])
+    assert torch.equal(wide[:, 3:I + 3], ops.swiglu(two[:, :I], two[:, I:])) and not wide[:, :3].any() and not wide[:, I + 3:].any()
+
+
 def test_bits_depend_on_k_alone():
     """On both sides of the bound on k every number of rows has the same bits, and whole numbers give whole numbers."""
     from zedinfer_amd import ops

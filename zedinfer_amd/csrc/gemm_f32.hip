@@ -522,6 +522,7 @@ extern "C" int zi_gemm_f32_swiglu_takes(const void* x, const void* w, int M, int
     if (M < 1 || M > 65535 * 64 || inter < 1 || K < 1 || inter > (1 << 24) || ldx < K || ldw < K || !zi_gemm_f32_takes(x, w, 2 * inter, K, ldx, ldw)) return 0;
     if (((int64_t)inter + 64) * ldw * 4 >= (1ll << 31) - 64) return 0;
     const gf_kernel k = gf_kernel_for(M, 2ll * inter, K);
+    if (k == GF_TILE_96_HALVES) return K > GF_SPLIT_ABOVE;      // (three blocks of weight rows a wavefront here, two there)
     return k == GF_HELD_PAIRS || k == GF_HELD_ROWS16 || k == GF_TILE_64 || k == GF_TILE_32 || k == GF_TILE_32_HALVES || k == GF_TILE_64_QUARTERS;
 }
 

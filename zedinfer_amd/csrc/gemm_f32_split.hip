@@ -701,6 +701,7 @@ static int gs_launch(float* out, const float* x, const float* w, const float* bi
         case GF_TILE_32: ZI_GF_TILE(2, 2, 4, 1); break;
         case GF_TILE_32_HALVES: ZI_GF_TILE(2, 2, 2, 4); break;
         case GF_TILE_64_QUARTERS: ZI_GF_TILE(4, 2, 2, 4); break;
+        case GF_TILE_96_HALVES: ZI_GF_TILE(2, 2, 3, 4); break;
         default:
             if constexpr (GATED) {
                 return zi_fail("gemm_f32: no gated kernel for %d rows of %d x %d", M, N, K);      // (zi_gemm_f32_swiglu_takes says so)
@@ -708,8 +709,7 @@ static int gs_launch(float* out, const float* x, const float* w, const float* bi
                 switch (zi_gemm_f32_split_kernel(M, N, K)) {
                     case GF_PAIRS: ZI_GF_STREAM(1, true, 3); break;
                     case GF_ROWS16: ZI_GF_STREAM(1, false, 2); break;
-                    case GF_ROWS32: ZI_GF_STREAM(2, false, 1); break;
-                    default: ZI_GF_TILE(2, 2, 3, 4); break;
+                    default: ZI_GF_STREAM(2, false, 1); break;
                 }
             }
     }
