@@ -142,10 +142,12 @@ def test_which_products_of_9_to_16_rows_go_twice_over_groups_of_8(N, K, kernel):
 
 
 @pytest.mark.parametrize("M,N,K,kernel", [(4000, 4000, 64, "tile_64"), (4000, 4000, 65, "tile_32"), (4000, 4000, 128, "tile_32"), (512, 17920, 320, "tile_32"),
-                                          (1024, 9728, 384, "tile_64"), (1024, 9728, 388, "tile_32"), (1024, 9728, 512, "tile_32"), (1024, 9728, 516, "tile_64"), (256, 17920, 1536, "tile_32"),
+                                          (1024, 9728, 384, "tile_64"), (1024, 9728, 388, "tile_32"), (1024, 9728, 512, "tile_32"), (1024, 9728, 516, "tile_64"), (256, 17920, 1536, "tile_64"),
                                           (128, 6144, 192, "tile_32"), (128, 6144, 193, "tile_96_halves"), (128, 2000, 192, "tile_32_halves"),
-                                          (448, 1536, 8960, "tile_96_halves"), (1024, 1536, 8960, "tile_32_halves")])
+                                          (448, 1536, 8960, "tile_96_halves"), (1024, 1536, 8960, "tile_96_halves"),
+                                          (992, 1536, 8960, "tile_96_halves"), (1024, 1536, 1536, "tile_96_halves"), (1500, 1536, 8960, "tile_96_halves"), (450, 4608, 3584, "tile_96_halves"),
+                                          (2048, 3584, 18944, "tile_64"), (80, 17920, 1536, "tile_32"), (512, 2048, 1536, "tile_64_quarters"), (256, 1536, 8960, "tile_32_halves")])
 def test_which_tiles_a_product_takes(M, N, K, kernel):
-    """The large tiles, which work a multiple of three chunks of 32, only where k is long."""
+    """The large tiles of the float32 instruction, which work a multiple of three chunks of 32, only where k is long; of more than 1,408 columns the fastest by measurement."""
     from zedinfer_amd import ops
     assert ops.linear_f32_kernel(M, N, K) == kernel

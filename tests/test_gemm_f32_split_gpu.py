@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 CASES = [(3, 1030, 1412, "pairs"), (8, 700, 9000, "pairs"), (12, 2070, 1412, "rows16"), (12, 300, 4100, "pairs"), (30, 2040, 1420, "rows16"), (40, 2040, 1500, "rows32"),
          (7, 2059, 1536, "held_pairs"), (5, 2054, 1800, "held_pairs"), (8, 3000, 3000, "held_pairs"), (2, 2049, 4096, "held_pairs"),
          (16, 5000, 1532, "held_rows16"), (13, 4098, 2048, "held_rows16"), (100, 2050, 1500, "tile_32_halves"), (500, 1500, 1480, "tile_96_halves"),
-         (449, 2047, 1540, "tile_64_quarters"), (700, 4610, 1412, "tile_64"), (450, 4610, 1500, "tile_32")]
+         (449, 2047, 1540, "tile_64_quarters"), (700, 4610, 1412, "tile_64"), (450, 4610, 1500, "tile_96_halves"), (449, 8194, 1500, "tile_32")]
 
 
 def _linear(M, N, K, seed=0):

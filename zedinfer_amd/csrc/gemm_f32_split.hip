@@ -624,12 +624,13 @@ gemm_f32_split_tile_kernel(float* __restrict__ out, const float* __restrict__ x,
 // Which kernel M rows of x and N weight rows take is a matter of filling the compute units only.
 // Up to 8 rows a stream of the weights in groups of 8, up to 16 in groups of 16 unless two passes over groups of 8 are one round (1,024 weight
 // rows); x is held in registers once there are more groups than units.  Beyond, groups of 16 weight rows with 16 or 32 rows of x while those are
-// one round of workgroups, 32 up to 32 rows.  Then tiles: the least of what each kind takes, rounds of workgroups times (a start + a time a chunk), us,
-// fitted to runs alone at 8 to 296 chunks: 32 x 64 in four groups 3.7 + 0.59 (1,536 x 8,960 at 256 rows 84, 2,048 x 1,536 at 128 18), 32 x 96 4.3 + 0.7
-// (512 rows 105, 1,536 x 1,536 23), 64 x 64 5.5 + 0.86 (2,048 x 1,536 at 512 rows 27); with one group, where several workgroups share a unit,
-// 32 x 128 1.39, 2.0 and 2.8 for one, two and three of them and 64 x 128 1.6 and 2.72 for one and two.  32 x 96 only for less than two rounds
-// (from there on 32 x 64 was kept, which at 1,024 rows of 1,536 x 8,960 costs 255 against 205 us), and a larger tile has to be that much faster to be worth its idle units:
-// the fit is no better than some per cent.  (256 rows of 17,920 x 1,536: 32 x 128 120 us, 64 x 128 116; 320 rows 157 and 118.)
+// one round of workgroups, 32 up to 32 rows.  Then the tiles that take the least: rounds of workgroups times (a start + a time a chunk), us, or,
+// with one group of wavefronts, where several workgroups share a unit, a start and a time a chunk for one, two and three of them, both fitted to 255
+// products alone of 33 to 3,200 rows, 400 to 24,000 weight rows and 23 to 296 chunks.  The choice takes 0.8 % more than the best of the five in the
+// mean, over 5 % in 12 of the 255 and at most 20 % (few rows and more weights than stream in that time: 115 rows of 9,988 x 2,148 82 us
+// in tiles of 32 x 96, 68 in 64 x 128).  Chosen and next, us: 450 rows of 4,608 x 3,584 32 x 96 135, 64 x 64 159; 1,024 of 1,536 x 8,960 32 x 96 222, 64 x 128 237,
+// 32 x 64 269; 2,048 of 4,608 x 3,584 64 x 128 430, 32 x 128 496; 256 of 17,920 x 1,536 with the activation 64 x 128 121, 32 x 128 130, 80 rows of it 32 x 128 62, 32 x 64 73;
+// 512 of 2,048 x 1,536 64 x 64 28, 32 x 64 36; 256 of 1,536 x 8,960 32 x 64 92, 32 x 96 107.
 gf_kernel zi_gemm_f32_split_kernel(int M, int64_t N, int K) {
     const int64_t cus = zi_compute_units(), n16 = (N + 15) / 16, m16 = (M + 15) / 16, m32 = (M + 31) / 32, m64 = (M + 63) / 64;
     const int chunks = (K + GF_KB - 1) / GF_KB, per = (chunks + GF_PARTS - 1) / GF_PARTS;
@@ -640,22 +641,22 @@ gf_kernel zi_gemm_f32_split_kernel(int M, int64_t N, int K) {
     if (M <= 32 || n16 * m32 <= cus) return GF_ROWS32;
     const int64_t n64 = (N + 63) / 64, n96 = (N + 95) / 96, n128 = (N + 127) / 128;
     auto shared = [&](int64_t tiles, float start, float chunk) { return (float)((tiles + cus - 1) / cus) * (start + chunk * chunks); };
-    auto rounds = [&](int64_t tiles, int places, float one, float two, float all) {      // `places` workgroups a unit at a time
+    auto rounds = [&](int64_t tiles, int places, float start, float one, float two, float all) {      // `places` workgroups a unit at a time
         const int64_t full = tiles / (places * cus), rest = tiles % (places * cus);
-        return (float)chunks * ((float)full * all + (rest == 0 ? 0.f : rest <= cus ? one : rest <= 2 * cus ? two : all));
+        return start + (float)chunks * ((float)full * all + (rest == 0 ? 0.f : rest <= cus ? one : rest <= 2 * cus ? two : all));
     };
     gf_kernel best = GF_TILE_32_HALVES;
-    float us = shared(m32 * n64, 3.7f, 0.59f);
-    auto consider = [&](gf_kernel kernel, float takes, float unless) {
-        if (takes < unless * us) {
+    float us = shared(m32 * n64, 3.82f, 0.63f);
+    auto consider = [&](gf_kernel kernel, float takes) {
+        if (takes < us) {
             best = kernel;
             us = takes;
         }
     };
-    if (m32 * n96 < 2 * cus) consider(GF_TILE_96_HALVES, shared(m32 * n96, 4.3f, 0.7f), 1.f);
-    consider(GF_TILE_32, 6.f + rounds(m32 * n128, 3, 1.39f, 2.f, 2.8f), 1.f);
-    consider(GF_TILE_64_QUARTERS, shared(m64 * n64, 5.5f, 0.86f), 0.96f);
-    consider(GF_TILE_64, 8.5f + rounds(m64 * n128, 2, 1.6f, 2.72f, 2.72f), 0.88f);
+    consider(GF_TILE_96_HALVES, shared(m32 * n96, 4.68f, 0.788f));
+    consider(GF_TILE_64_QUARTERS, shared(m64 * n64, 5.73f, 0.938f));
+    consider(GF_TILE_32, rounds(m32 * n128, 3, 7.39f, 1.52f, 2.19f, 2.89f));
+    consider(GF_TILE_64, rounds(m64 * n128, 2, 8.83f, 1.65f, 2.94f, 2.94f));
     return best;
 }
 
