@@ -6,7 +6,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("rows", [16, 32, 64, 128])
-@pytest.mark.parametrize("K", [8, 64, 72, 128, 192, 256, 264, 512, 576, 704, 768, 776, 1536, 1600])
+@pytest.mark.parametrize("K", [8, 64, 72, 128, 192, 256, 264, 320, 376, 384, 392, 448, 504, 512, 520, 576, 640, 704, 768, 776, 832, 896, 960, 1152, 1160, 1536, 1600])
 def test_whole_numbers_come_out_exact(rows, K):
     """|sum| <= 1,600 * 9: exact in float32 in any order.  What lies behind the weights and beside the tokens is no number."""
     from zedinfer_amd import ops

@@ -328,10 +328,15 @@ union moe_pack {
 #define MOE_KB 64
 #define MOE_XCDS 8
 // Turns through the buffers in a row.  The compiler waits for all loads at the first read in a loop's body, also for those that were asked
-// for a moment ago: once in this many turns.  us, the two products of 32 experts' prompt tiles, waiting in every turn, every second and
-// every fourth (32 experts of 1,536 x 1,536, 8,000 pairs 91 and 80, 85 and 73, 82 and 72; 73 tiles of 3,584 x 2,560
-// 249 and 262, 230 and 250, 223 and 247; 32 pairs of these 108 and 100, 102 and 96, 100 and 95); eight turns are no faster
-#define MOE_TURNS 4
+// for a moment ago: once in TURNS turns.  More turns are more instructions, which every compute unit fetches once a launch, and with more
+// than one a tile asks for ST - 1 steps past its last.  Time over that of one turn, of two and four turns, geometric means over 2 to 3
+// numbers of pairs of five sets of experts (8 to 64, 512 to 4,096 columns), by columns of K:
+//   tiles of 16 rows   64: 1.04, 1.05    256: 1.01, 1.00    384: 0.98, 0.98    640: 0.98, 0.96    1,536: 0.96, 0.94    3,584: 0.95, 0.94
+//   of 32              64: 1.08, 1.16    384: 0.99, 1.07    512: 1.00, 1.06    640: 0.99, 1.04    1,536: 0.95, 1.01    3,584: 0.95, 1.00
+//   of 128             64: 1.04, 1.08    384: 0.99, 1.02    512: 1.00, 1.01    640: 0.98, 0.99    1,536: 0.94, 0.94    3,584: 0.94, 0.94
+// Tiles of 64 rows have two buffers and wait for every load in every step: four turns 1.02 to 1.06.  So 16 rows take four from 384
+// columns on, 32 and 128 two beyond 512.  (Slower there: 8 experts of 4,096 columns at 12 rows, four turns 1.03 to 1.05.)
+static int moe_turns(int tile_rows, int K) { return tile_rows == 16 ? (K >= 384 ? 4 : 1) : tile_rows == 64 ? 1 : K > 512 ? 2 : 1; }
 // the longest row of weights whose tile of rows a buffer's 31-bit offsets reach
 #define MOE_MAX_K (1 << 21)
 
@@ -355,8 +360,8 @@ __device__ __forceinline__ void moe_to_lds(__amdgpu_buffer_rsrc_t from, moe_u32x
 #endif
 }
 
-// WR: wavefronts along the rows of a tile, each with RT / WR of its sixteens; four times as many in all.
-template <typename TO, int RT, int CT, int ST, int WR>
+// WR: wavefronts along the rows of a tile, each with RT / WR of its sixteens; four times as many in all.  TURNS: see moe_turns.
+template <typename TO, int RT, int CT, int ST, int WR, int TURNS>
 __global__ void __launch_bounds__(4 * WR * ZI_WAVE)
 moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restrict__ x, int64_t ldx,
                        const zi_bf16* __restrict__ w, const int32_t* __restrict__ plan,
@@ -415,13 +420,15 @@ moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restr
         for (int c = 0; c < CT; ++c) acc[t][c] = (moe_f32x4_t){0.f, 0.f, 0.f, 0.f};
     const int sw = (r >> 1) & 7;
     auto step = [&](const moe_u32x4_t* buf, moe_u32x4_t* free, int t) __attribute__((always_inline)) {
+        if (TURNS == 1 && t >= steps) return;
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
-        moe_wait<(ST - 2) * PW>();             // the newest steps' loads may still be on their way
+        if (TURNS > 1 || steps - 1 - t >= ST - 2) moe_wait<(ST - 2) * PW>();      // the newest steps' loads may still be on their way
+        else moe_wait<0>();
         __builtin_amdgcn_s_barrier();          // all wavefronts' loads of the step are there, and all are done with `free`
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
-        issue(free, t + ST - 1);
+        if (TURNS > 1 || t + ST - 1 < steps) issue(free, t + ST - 1);
         __builtin_amdgcn_sched_barrier(0);
         const int left = K - t * MOE_KB;
 #pragma unroll
@@ -448,22 +455,30 @@ moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restr
     };
     issue(s0, 0);
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (ST > 2) issue(s1, 1);
+    if (ST > 2 && (TURNS > 1 || steps > 1)) issue(s1, 1);
     __builtin_amdgcn_sched_barrier(0);
-    for (int t = 0, left = 1; left;) {
-#pragma unroll
-        for (int turn = 0; turn < MOE_TURNS; ++turn) {
+    if constexpr (TURNS == 1) {
+        for (int t = 0; t < steps; t += ST) {
             step(s0, ST == 2 ? s1 : s2, t);
-            if (!(left = ++t < steps)) break;
-            step(s1, s0, t);
-            if (!(left = ++t < steps)) break;
-            if constexpr (ST > 2) {
-                step(s2, s1, t);
+            step(s1, s0, t + 1);
+            if constexpr (ST > 2) step(s2, s1, t + 2);
+        }
+    } else {
+        for (int t = 0, left = 1; left;) {
+#pragma unroll
+            for (int turn = 0; turn < TURNS; ++turn) {
+                step(s0, ST == 2 ? s1 : s2, t);
                 if (!(left = ++t < steps)) break;
+                step(s1, s0, t);
+                if (!(left = ++t < steps)) break;
+                if constexpr (ST > 2) {
+                    step(s2, s1, t);
+                    if (!(left = ++t < steps)) break;
+                }
             }
         }
+        moe_wait<0>();
     }
-    moe_wait<0>();
     // a lane holds four consecutive columns of a row: one store of 16 (float32) or 8 bytes (bfloat16) where the rows
     // allow it
     const bool whole = ldo % 4 == 0 && ((uintptr_t)out % 16) == 0;
@@ -503,15 +518,19 @@ extern "C" int zi_moe_linear(void* out, int out_dt, int64_t ldo, const void* x, 
     const int wide = cores ? (tile_rows < 64 ? 64 * (tile_rows / 16) : 256) : 64;       // columns of a workgroup
     const int64_t most = ((int64_t)N + wide - 1) / wide * max_tiles + MOE_XCDS;
     if (cores && K <= MOE_MAX_K && most * (tile_rows == 128 ? 512 : 256) < (1LL << 32)) {
-#define ZI_MOE_CORES(RT, CT, ST, WR)                                                                                                   \
-    moe_linear_mfma_kernel<TO, RT, CT, ST, WR><<<dim3((((N + 64 * CT - 1) / (64 * CT)) * (int64_t)max_tiles + MOE_XCDS - 1) / MOE_XCDS * \
-                                             MOE_XCDS), 256 * WR, 0, stream>>>((TO*)out, ldo, (const zi_bf16*)x, ldx,                      \
-                                                                          (const zi_bf16*)w, plan, source, source_div, N, K, act)
+#define ZI_MOE_CORES(RT, CT, ST, WR, TURNS)                                                                                                   \
+    moe_linear_mfma_kernel<TO, RT, CT, ST, WR, TURNS><<<dim3((((N + 64 * CT - 1) / (64 * CT)) * (int64_t)max_tiles + MOE_XCDS - 1) / MOE_XCDS * \
+                                                        MOE_XCDS), 256 * WR, 0, stream>>>((TO*)out, ldo, (const zi_bf16*)x, ldx,                      \
+                                                                                       (const zi_bf16*)w, plan, source, source_div, N, K, act)
         ZI_DISPATCH_DTYPE(out_dt, TO, {
-            if (tile_rows == 16) ZI_MOE_CORES(1, 1, 3, 1);
-            else if (tile_rows == 32) ZI_MOE_CORES(2, 2, 3, 1);
-            else if (tile_rows == 64) ZI_MOE_CORES(4, 4, 2, 1);
-            else ZI_MOE_CORES(8, 4, 3, 2);
+            const int turns = moe_turns(tile_rows, K);
+            if (tile_rows == 16 && turns > 1) ZI_MOE_CORES(1, 1, 3, 1, 4);
+            else if (tile_rows == 16) ZI_MOE_CORES(1, 1, 3, 1, 1);
+            else if (tile_rows == 32 && turns > 1) ZI_MOE_CORES(2, 2, 3, 1, 2);
+            else if (tile_rows == 32) ZI_MOE_CORES(2, 2, 3, 1, 1);
+            else if (tile_rows == 64) ZI_MOE_CORES(4, 4, 2, 1, 1);
+            else if (turns > 1) ZI_MOE_CORES(8, 4, 3, 2, 2);
+            else ZI_MOE_CORES(8, 4, 3, 2, 1);
         });
         return zi_check_launch("moe_linear");
     }
