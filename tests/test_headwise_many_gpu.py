@@ -26,3 +26,22 @@ def test_whole_numbers_come_out_exact(n, vdim, rank, dtype, out_dtype):
     out = ops.latent_value(*args, out=torch.empty((n, heads * vdim), dtype=out_dtype, device=dev), gate=gate.to(dev))
     ref = want * torch.sigmoid(gate.double().sum(0))
     assert (out.double().cpu() - ref).abs().le(ref.abs() * (2.0 ** -8 if out_dtype == torch.bfloat16 else 1e-5)).all()
+
+
+@pytest.mark.parametrize("n", [128, 195])
+@pytest.mark.parametrize("vdim", [8, 16, 31, 32, 33, 48, 64, 65, 96, 130])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_tiles_of_32_and_64_outputs_with_either_gate(n, vdim, dtype):
+    """As above, 32 outputs a tile up to that many, else 64; gates in bfloat16 and as one and five terms."""
+    from zedinfer_amd import ops
+    heads, rank, dev = 5, 72, "cuda"
+    g = torch.Generator().manual_seed(n * vdim)
+    o = torch.randint(-3, 4, (n, heads, rank), generator=g).double()
+    uv = torch.randint(-3, 4, (heads * vdim, rank), generator=g).double()
+    want = torch.einsum("nhr,hvr->nhv", o, uv.view(heads, vdim, rank)).reshape(n, -1)
+    for gate in (torch.randn((n, heads * vdim), generator=g).bfloat16(), torch.randn((1, n, heads * vdim), generator=g),
+                 torch.randn((5, n, heads * vdim), generator=g)):
+        out = ops.latent_value(o.to(dtype).to(dev), uv.bfloat16().to(dev), vdim, torch.empty((n, heads * vdim), dtype=dtype, device=dev), gate=gate.to(dev))
+        ref = want * torch.sigmoid(gate.double() if gate.dim() == 2 else gate.double().sum(0))
+        # (the terms' sum: five roundings of at most 2^-24 of 16; the exponential and the division)
+        assert (out.double().cpu() - ref).abs().le(ref.abs() * (2.0 ** -8 if dtype == torch.bfloat16 else 1e-5)).all()

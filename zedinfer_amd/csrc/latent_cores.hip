@@ -429,13 +429,15 @@ extern "C" int zi_latent_attention_cores(void* out, int out_dt, float* partial, 
 // os.  It carries the queries through W_uk (w = W_uk of the head, transposed at load) and the attended latents through W_uv.
 // GATED: out *= sigmoid(gate[t][h * N + i]), the gate bfloat16 or the sum of `splits` float32 terms.
 // Few tokens: 16 x 16 a workgroup, operands straight from memory, k dealt over the four wavefronts in runs of 32 and added up in their
-// order.  Many: 64 tokens x 128 outputs, a wavefront 32 x 64.  Bound by memory (x once, the results), and before by the vector cache:
-// operands loaded as the product wants them lie in a row apiece, 9 to 10 accesses a line of 128 bytes.  So a step's rows of 128 bytes are
-// loaded whole, two steps on their way in registers, and turn in LDS in places that neither side's lanes share a bank in; the results
-// turn there too and leave as runs of 256 bytes.  us, before and after: 12 heads, 512 outputs of k 128, 2,000 tokens 24.9 to 12.9 (3 TB/s with
-// x once), 128 of 512 26.1 to 14.3; 8,000 tokens 81.5 to 38.6 and 80.8 to 30.9; 128 tokens 6.2 to 4.7 and 13.7 to 8.6; 64 heads, 2,000
-// tokens 108.8 to 54.9 and 90.7 to 42.4; float32 x 18.3 to 12.6 at 1,000 tokens; with a gate 35.4 to 21.8 at 2,048.  One step on its way instead of two: 128 tokens 5.0 and
-// 9.8.  Two workgroups a unit instead of three: 8,000 tokens 43.5 and 38.7.  Slower: a k of 8 with 33 outputs, 4.2 to 5.5.
+// order.  Many: 64 tokens x 32, 64 or 128 outputs (la_tile_outputs), a wavefront 32 x half of these.  Bound by memory (x once, the results), and
+// before by the vector cache: operands loaded as the product wants them lie in a row apiece, 9 to 10 accesses a line of 128 bytes.  So a step's
+// rows of 128 bytes are loaded whole, two steps on their way in registers, and turn in LDS in places that neither side's lanes share a bank in;
+// the results turn there too and leave in runs of whole rows of the tile; a thread asks for all its gates at once.  us, operands straight from
+// memory, tiles of 128 outputs with gates asked for one after the other, now: 12 heads, 512 outputs of k 128, 2,000 tokens 24.5, 12.5, 12.6 (3 TB/s with
+// x once), 8,000 82, 38.5, 38.4; 128 of 512 26.4, 14.2, 12.8 and 84, 31.2, 30.9; 128 tokens 5.9, 4.4, 3.9 and 13.4, 8.3, 6.6; with a gate 34.6, 21.4,
+// 16.6 (2,000 tokens); 64 outputs of 512 14.6, 11.4, 8.7; 16 of 16 with a gate 4.7, 10.0, 4.7; 64 heads, 64 of 64 with a gate, 8,000 tokens 100, 145, 51.
+// One step on its way instead of two: 128 tokens 5.0 and 9.8.  Over 4,780 products 0.68 of the first's time; slower by a tenth or more: gates over 8 or 16
+// outputs of a k of up to 128 at 8,000 tokens (12 heads, 16 of 16, three terms 1.29), 33 outputs of up to 16 (1.18).
 struct LaGate {
     const void* g;
     int f32, splits;
@@ -457,29 +459,28 @@ __device__ __forceinline__ la_pack la_load8(const zi_bf16* p) {
     return b;
 }
 
-// four gates of one token and head, columns n0 .. n0 + 3 (clamped to the head)
+// four gates of one token and head, columns n0 .. n0 + 3 (clamped to the head), stored as T
+template <typename T>
 __device__ __forceinline__ la_f32x4_t la_gates(const LaGate& gt, int64_t t, int h, int n0, int N) {
     const int64_t at = t * gt.ld + (int64_t)h * N;
+    const T* g0 = (const T*)gt.g + at;
     la_f32x4_t g;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int col = n0 + i < N ? n0 + i : N - 1;
-        g[i] = gt.f32 ? ((const float*)gt.g)[at + col] : zi_load((const zi_bf16*)gt.g + at + col);
-    }
-    if (gt.f32) {
+    for (int i = 0; i < 4; ++i) g[i] = zi_load(g0 + (n0 + i < N ? n0 + i : N - 1));
+    if (sizeof(T) == 4) {
         int s = 1;
         for (; s + 3 < gt.splits; s += 4) {      // four terms in flight, added in their order
             la_f32x4_t v[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) v[u][i] = ((const float*)gt.g)[(s + u) * gt.stride + at + (n0 + i < N ? n0 + i : N - 1)];
+                for (int i = 0; i < 4; ++i) v[u][i] = zi_load(g0 + (s + u) * gt.stride + (n0 + i < N ? n0 + i : N - 1));
 #pragma unroll
             for (int u = 0; u < 4; ++u) g += v[u];
         }
         for (; s < gt.splits; ++s)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) g[i] += ((const float*)gt.g)[s * gt.stride + at + (n0 + i < N ? n0 + i : N - 1)];
+            for (int i = 0; i < 4; ++i) g[i] += zi_load(g0 + s * gt.stride + (n0 + i < N ? n0 + i : N - 1));
     }
     return g;
 }
@@ -505,7 +506,7 @@ headwise_linear_few_kernel(TO* __restrict__ out, int64_t ldo, int os, const TX* 
     const int64_t t = t0 + r < n ? t0 + r : n - 1;
     const TX* xrow = x + t * ldx + (int64_t)h * xs;
     la_f32x4_t acc = (la_f32x4_t){0.f, 0.f, 0.f, 0.f}, gate = acc;
-    if (GATED && wave == 0) gate = la_gates(gt, t, h, n0 + 4 * j, N);      // asked for before the product, used after it
+    if (GATED && wave == 0) gate = gt.f32 ? la_gates<float>(gt, t, h, n0 + 4 * j, N) : la_gates<zi_bf16>(gt, t, h, n0 + 4 * j, N);      // asked for before the product, used after it
 #pragma unroll 4
     for (int k0 = wave * 32; k0 < K; k0 += 128) {
         const int k = k0 + 8 * j, kc = k < K ? k : 0;      // K is a multiple of 8
@@ -526,20 +527,18 @@ headwise_linear_few_kernel(TO* __restrict__ out, int64_t ldo, int os, const TX* 
 }
 
 #define LA_HT 64       // tokens
-#define LA_HN 128      // outputs
 #define LA_HK 64       // k a step: rows of 128 bytes
-#define LA_HROW (LA_HN + 4)
-template <typename TX, typename TO, bool GATED>
-__global__ void __launch_bounds__(4 * ZI_WAVE, GATED ? 2 : 3)      // (the gate's terms take registers)
+template <typename TX, typename TO, bool GATED, int TN>
+__global__ void __launch_bounds__(4 * ZI_WAVE, 3)
 headwise_linear_many_kernel(TO* __restrict__ out, int64_t ldo, int os, const TX* __restrict__ x, int64_t ldx, int xs,
                             const zi_bf16* __restrict__ w, int n, int N, int K, LaGate gt) {
-    constexpr int TM = 2, TN = 4;                       // a wavefront's tiles of 16 tokens and of 16 outputs
-    constexpr int PX = LA_HT / 32, PW = LA_HN / 32;     // a thread's pieces of 16 bytes a step
-    constexpr int STEP = (LA_HT + LA_HN) * 8;           // pieces a step
+    constexpr int TM = 2, HN = 32 * TN, HROW = HN + 4;      // a wavefront's tiles of 16 tokens; outputs, a row of results
+    constexpr int PX = LA_HT / 32, PW = HN / 32;     // a thread's pieces of 16 bytes a step
+    constexpr int STEP = (LA_HT + HN) * 8;           // pieces a step
     __shared__ la_u32x4_t lds[2 * STEP];
-    static_assert(LA_HT * LA_HROW * sizeof(float) <= sizeof(lds), "the results turn in the operands' place");
+    static_assert(LA_HT * HROW * sizeof(float) <= sizeof(lds), "the results turn in the operands' place");
     const int tid = threadIdx.x, lane = tid % ZI_WAVE, wave = tid / ZI_WAVE, r = lane % 16, j = lane / 16;
-    const int t0 = blockIdx.x * LA_HT, h = blockIdx.y, n0 = blockIdx.z * LA_HN;
+    const int t0 = blockIdx.x * LA_HT, h = blockIdx.y, n0 = blockIdx.z * HN;
     const int q = tid / 8, c8 = tid % 8;                // rows q, q + 32, ..; (q + 32 i) / 2 keeps its last three bits
     const int at = q * 8 + (c8 ^ (q / 2 & 7));
     const TX* xr[PX];
@@ -607,22 +606,45 @@ headwise_linear_many_kernel(TO* __restrict__ out, int64_t ldo, int os, const TX*
         step(k0, even, odd, 0);
         if (k0 + LA_HK < K) step(k0 + LA_HK, odd, even, 1);
     }
+    // eight outputs' gates for each of this thread's pieces, all asked for at once
+    la_f32x4_t gates[GATED ? TN : 1][2];
+    auto piece = [&](int u, int& row, int& o) {
+        const int p = tid + u * (4 * ZI_WAVE);
+        row = p / (HN / 8);
+        o = p % (HN / 8) * 8;
+        return t0 + row < n && n0 + o < N;
+    };
+    if constexpr (GATED) {
+        auto ask = [&](auto read) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < TN; ++u) {
+                int row, o;
+                if (!piece(u, row, o)) continue;
+                gates[u][0] = read(t0 + row, n0 + o);
+                gates[u][1] = read(t0 + row, n0 + o + 4);
+            }
+        };
+        if (gt.f32) ask([&](int t, int i) { return la_gates<float>(gt, t, h, i, N); });
+        else ask([&](int t, int i) { return la_gates<zi_bf16>(gt, t, h, i, N); });
+    }
     __syncthreads();
     float* turned = reinterpret_cast<float*>(lds);      // [token][output]
 #pragma unroll
     for (int m = 0; m < TM; ++m)
 #pragma unroll
         for (int c = 0; c < TN; ++c)
-            *reinterpret_cast<la_f32x4_t*>(turned + (tw + m * 16 + r) * LA_HROW + ow + c * 16 + 4 * j) = acc[m][c];
+            *reinterpret_cast<la_f32x4_t*>(turned + (tw + m * 16 + r) * HROW + ow + c * 16 + 4 * j) = acc[m][c];
     __syncthreads();
-    for (int p = tid; p < LA_HT * (LA_HN / 8); p += 4 * ZI_WAVE) {
-        const int row = p / (LA_HN / 8), o = p % (LA_HN / 8) * 8, t = t0 + row, i = n0 + o;
-        if (t >= n || i >= N) continue;
-        la_f32x4_t lo = *reinterpret_cast<const la_f32x4_t*>(turned + row * LA_HROW + o);
-        la_f32x4_t hi = *reinterpret_cast<const la_f32x4_t*>(turned + row * LA_HROW + o + 4);
+#pragma unroll
+    for (int u = 0; u < TN; ++u) {
+        int row, o;
+        if (!piece(u, row, o)) continue;
+        const int t = t0 + row, i = n0 + o;
+        la_f32x4_t lo = *reinterpret_cast<const la_f32x4_t*>(turned + row * HROW + o);
+        la_f32x4_t hi = *reinterpret_cast<const la_f32x4_t*>(turned + row * HROW + o + 4);
         if constexpr (GATED) {
-            la_gate4(lo, la_gates(gt, t, h, i, N));
-            la_gate4(hi, la_gates(gt, t, h, i + 4, N));
+            la_gate4(lo, gates[u][0]);
+            la_gate4(hi, gates[u][1]);
         }
         TO* dst = out + (int64_t)t * ldo + (int64_t)h * os + i;
         if (sizeof(TO) == 2 && i + 7 < N && ((uintptr_t)dst % 16) == 0) {
@@ -649,6 +671,22 @@ extern "C" int zi_headwise_linear_supported(int w_dt, int K, int64_t ldx, int xs
 
 #define LA_MANY_TOKENS 128      // from this many tokens on the kernel for many
 
+// Outputs of its tiles: 32 for heads that have no more.  Else 64, and 128 without a gate where the tiles of 128 fill the chip, three
+// workgroups a unit (two and a half of them, eight where half of a head's last tile is empty): x is read once a tile, but a tile's end is one
+// long wait.  Time in tiles of 128 over that in tiles of 64, geometric means by tiles of 128 a unit, 1,087 products of 2 to 64 heads, 65 to 512
+// outputs, a k of 16 to 512, 128 to 12,000 tokens:
+//   up to 1     1.16   x float32 1.15   a bfloat16 gate 1.35   three terms of a gate 1.46
+//   1 to 2.5    1.04             1.01                   1.17                         1.15
+//   2.5 to 6    0.93             0.87                   1.03                         1.06
+//   from 6 on   0.88             0.80                   0.99                         1.08
+// half empty tiles, up to 8 1.03 to 1.15 and 0.99 to 1.13, from there on 0.99 and 0.90.
+static int la_tile_outputs(int n, int heads, int N, bool gated) {
+    if (N <= 32) return 32;
+    if (gated || N <= 64) return 64;
+    const int64_t tiles = (int64_t)((n + LA_HT - 1) / LA_HT) * heads * ((N + 127) / 128);
+    return tiles >= (int64_t)zi_compute_units() * ((N - 1) % 128 < 64 ? 16 : 5) / 2 ? 128 : 64;
+}
+
 extern "C" int zi_headwise_linear_gated(void* out, int out_dt, int64_t ldo, int os, const void* x, int x_dt, int64_t ldx, int xs,
                                         const void* w, int n, int heads, int N, int K, const void* gate, int g_dt,
                                         int64_t ld_gate, int g_splits, int64_t g_stride, hipStream_t stream) {
@@ -661,15 +699,23 @@ extern "C" int zi_headwise_linear_gated(void* out, int out_dt, int64_t ldo, int 
                "headwise_linear: bad gate");
     if (n == 0) return 0;
     const bool many = n >= LA_MANY_TOKENS;
-    const dim3 grid(many ? (n + LA_HT - 1) / LA_HT : (n + 15) / 16, heads, many ? (N + LA_HN - 1) / LA_HN : (N + 15) / 16);
+    const int wide = la_tile_outputs(n, heads, N, gate) / 32;
+    const dim3 grid(many ? (n + LA_HT - 1) / LA_HT : (n + 15) / 16, heads, many ? (N + 32 * wide - 1) / (32 * wide) : (N + 15) / 16);
     const LaGate gt = {gate, g_dt == ZI_F32, g_splits, ld_gate, g_stride};
-#define ZI_HW(KERNEL, GATED) KERNEL<TX, TO, GATED><<<grid, 4 * ZI_WAVE, 0, stream>>>((TO*)out, ldo, os, (const TX*)x, ldx, xs, (const zi_bf16*)w, n, N, K, gt)
+#define ZI_HW(...) __VA_ARGS__<<<grid, 4 * ZI_WAVE, 0, stream>>>((TO*)out, ldo, os, (const TX*)x, ldx, xs, (const zi_bf16*)w, n, N, K, gt)
+#define ZI_HW_MANY(GATED)                                                                 \
+    do {                                                                                  \
+        if (wide == 1) ZI_HW(headwise_linear_many_kernel<TX, TO, GATED, 1>);              \
+        else if (GATED || wide == 2) ZI_HW(headwise_linear_many_kernel<TX, TO, GATED, 2>); \
+        else ZI_HW(headwise_linear_many_kernel<TX, TO, GATED, GATED ? 2 : 4>);            \
+    } while (0)
     ZI_DISPATCH_DTYPE(x_dt, TX, ZI_DISPATCH_DTYPE(out_dt, TO, {
-        if (many && gate) ZI_HW(headwise_linear_many_kernel, true);
-        else if (many) ZI_HW(headwise_linear_many_kernel, false);
-        else if (gate) ZI_HW(headwise_linear_few_kernel, true);
-        else ZI_HW(headwise_linear_few_kernel, false);
+        if (many && gate) ZI_HW_MANY(true);
+        else if (many) ZI_HW_MANY(false);
+        else if (gate) ZI_HW(headwise_linear_few_kernel<TX, TO, true>);
+        else ZI_HW(headwise_linear_few_kernel<TX, TO, false>);
     }));
+#undef ZI_HW_MANY
 #undef ZI_HW
     return zi_check_launch("headwise_linear");
 }
