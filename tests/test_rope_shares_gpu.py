@@ -34,3 +34,23 @@ def test_a_tile_in_one_workgroup_and_in_four(nh, nkv, d, rot, ps, scattered, sto
 
     for one, four in zip(run(n), run(2053)):        # (2,053 and 2,054 tokens: the last tile is not whole)
         assert torch.equal(one, four)
+
+
+@pytest.mark.parametrize("nh,d,rot", [(2, 64, 64), (16, 128, 64), (12, 128, 128), (33, 64, 64)])
+def test_queries_alone_in_one_workgroup_and_in_four(nh, d, rot):
+    """One, two, three and five pieces a thread and tile: shared never, up to a tile a unit, up to two; 8,200 tokens are more, 1,031 fewer
+    than a tile a unit and 3,001 between one and two (of 256)."""
+    from zedinfer_amd import ops
+    n = 8200
+    g = torch.Generator(device="cuda").manual_seed(nh)
+    q, table = torch.randn(n, nh * d, generator=g, device="cuda").bfloat16(), torch.randn(n, rot // 2, 2, generator=g, device="cuda")
+
+    def run(step):
+        x = q.clone()
+        for a in range(0, n, step):
+            b = min(n, a + step)
+            ops.rope_kv_store(x[a:b], None, None, table[a:b], None, None, None, nh, 0, d)
+        return x
+
+    one = run(n)
+    assert torch.equal(one, run(1031)) and torch.equal(one, run(3001))

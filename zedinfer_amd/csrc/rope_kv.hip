@@ -226,7 +226,12 @@ extern "C" int zi_rope_kv_store(void* q, const void* k, const void* v, int dt, i
         const size_t lds = (size_t)RKT_TOKENS * rot * sizeof(float) + (write_kv ? (size_t)RKT_TOKENS * nkv * d * 2 : 0);
         if (dt == ZI_BF16 && n >= ROPE_MANY_TOKENS && al && lds <= 48 * 1024) {
             const int tiles = (n + RKT_TOKENS - 1) / RKT_TOKENS;
-            rope_kv_store_tile_kernel<<<dim3(tiles, tiles <= 2 * zi_compute_units() ? RKT_SHARES : 1), 256, lds, stream>>>(
+            // queries alone: pieces of eight dims and their partners a thread.  One is one trip however it is shared, two and three gain up to
+            // a tile a unit, four and more up to two (four workgroups over one: 1 piece 1.01 to 1.03 and, 4,096 tokens, 1.13; 2 and 3 0.87 to
+            // 0.95, 3,000 tokens 1.00 and 1.04; 4 0.81 to 0.88, 3,000 0.98; 7 0.74 to 0.85, 3,000 0.82, 4,096 1.02)
+            const int pieces = (RKT_TOKENS * nh * (rot / 16) + 255) / 256;
+            const int shared_tiles = (write_kv || pieces >= 4 ? 2 : pieces >= 2 ? 1 : 0) * zi_compute_units();
+            rope_kv_store_tile_kernel<<<dim3(tiles, tiles <= shared_tiles ? RKT_SHARES : 1), 256, lds, stream>>>(
                 (zi_bf16*)q, (const zi_bf16*)k, (const zi_bf16*)v, ldq, ldk, ldv, slots, tb, (zi_bf16*)kcache,
                 (zi_bf16*)vcache, n, nh, nkv, d, rot, page_size, write_kv, cache_slots);
             return zi_check_launch("rope_kv_store");
