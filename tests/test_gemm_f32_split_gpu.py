@@ -142,3 +142,25 @@ def test_bits_depend_on_k_alone():
             assert torch.equal(ops.linear(x[:m].contiguous(), w, b), whole[:m])
     x, w = torch.randint(-8, 9, (40, 2000), device="cuda").float(), torch.randint(-8, 9, (300, 2000), device="cuda").float()
     assert torch.equal(ops.linear(x, w).double(), x.double() @ w.double().t())
+
+
+@pytest.mark.parametrize("N,K", [(700, 9000), (1030, 1412), (300, 4100), (2059, 1536), (2054, 1800), (3000, 3000), (2049, 4096)])
+def test_one_to_eight_rows_alone_and_together(N, K):
+    """Up to two and up to four rows of x are loaded and split by all lanes: the bits of eight rows, in the streams and where x is held (3, 4, 6, 8 chunks)."""
+    from zedinfer_amd import ops
+    x, w, b = _linear(8, N, K)
+    x[5, :40] = 0.0
+    x[6] *= 2.0 ** -140
+    y = ops.linear(x, w, b)
+    halves = N % 2 == 0 and ops.linear_swiglu_halves_supported(x, w)
+    z = ops.linear_swiglu_halves(x, w) if halves else None
+    for rows in range(1, 8):
+        for first in (0, 8 - rows):
+            part = torch.full((rows + 2, K + 4), float("nan"), device="cuda")      # (what lies beside the rows is no number)
+            part[:rows, :K] = x[first:first + rows]
+            assert torch.equal(ops.linear(part[:rows, :K], w, b), y[first:first + rows])
+            if halves and ops.linear_swiglu_halves_supported(part[:rows, :K], w):
+                assert torch.equal(ops.linear_swiglu_halves(part[:rows, :K], w), z[first:first + rows])
+    x[2, K - 1] = float("nan")
+    got = ops.linear(x[2:4].contiguous(), w, b)
+    assert bool(torch.isnan(got[0]).all()) and torch.equal(got[1], y[3])

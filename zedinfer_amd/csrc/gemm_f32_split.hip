@@ -30,13 +30,16 @@
 // then the two halves, then the bias.
 //
 // What bounds it: few rows the one pass over the weights; many rows, by counters at 2,048 rows of 4,096 x 4,096, the vector instructions
-// (57 % of the cycles, eleven for every two values split) and the matrix cores (51 %), which mostly take turns, beside LDS (43 %).
+// (57 % of the cycles, eleven for every two values split, thirteen since they are split times 2^24) and the matrix cores (51 %), which mostly take turns, beside LDS (43 %).
 //
-// Measured, weights from memory, against the float32 instruction's kernels, us, launch included (N x K): 8 rows 2,048 x 1,536 6.9 to 6.7, 1,536 x
-// 8,960 21.3 to 19.0, 17,920 x 1,536 with the activation 23.2 to 21.7; 24 rows 1,536 x 8,960 35.6 to 25.8, 17,920 x 1,536 46.7 to 38.0; 64 rows
-// 1,536 x 8,960 53.5 to 40.6; 512 rows 2,048 x 1,536 32.4 to 28.3, 1,536 x 8,960 136 to 109 (129 TFLOP/s), 17,920 x 1,536 with the activation 232
-// to 184 (153 TFLOP/s); 2,048 rows of 4,608 x 3,584 538 to 406 (166 TFLOP/s; the float32 instruction in a large library product: 152).  Slower: one
-// row of 2,048 x 1,536 5.9 to 6.2, 9 rows of 17,920 x 1,536 with the activation 23.9 to 25.4.
+// Measured, weights from memory, against the float32 instruction's kernels, us, launch included (N x K; act: with the activation):
+//   1 row      2,048 x 1,536 5.1 and 5.1, 1,536 x 8,960 13.2 and 11.8, 17,920 x 1,536 act 19.8 and 20.1, 151,936 x 1,536 135.5 and 140.5
+//   8 rows     5.9 and 5.6, 18.6 and 15.9, 21.2 and 20.4, 156.8 and 155.1
+//   24 rows    9.4 and 8.8, 34.5 and 24.8, 151,936 x 1,536 317 and 248; 64 rows 11.9 and 10.0, 51.8 and 37.3, 297 and 240
+//   450 rows   32.3 and 28.1, 122 and 112 (111 TFLOP/s), 230 and 187 (132)
+//   2,048 rows 116 and 84.7, 473 and 428, 903 and 711 (159), 4,608 x 3,584 534 and 429 (158; the float32 instruction in a large library product: 152)
+// Slower: up to 4 rows of 151,936 x 1,536 2 to 4 %, up to 8 of 37,888 x 3,584 act 1 to 3 %, and, where tiles are one or two rounds of workgroups, 96 to
+// 256 rows of 2,048 x 1,536 1 to 4 %, 48 to 128 of 3,584 x 3,584 0 to 3 %, 200 of 4,608 x 3,584 9 % (69 and 75).
 #include "zi_gemm_f32.h"
 
 #define GF_KB 64             // k of a chunk
@@ -48,26 +51,32 @@ struct gf_parts {
     gf_pack p[3];
 };
 
+typedef unsigned __attribute__((may_alias)) gf_u32_alias_t;
+
 #define GF_UP 0x1p24f        // what operands are multiplied by before they are split (x of the negated chain by its negative), ...
 #define GF_DOWN 0x1p-48f     // ... and sums when they are finished
 
-__device__ __forceinline__ gf_parts gf_split(gf_f32x4_t a, gf_f32x4_t b, float up) {
-    gf_parts s;
-    a *= up;
-    b *= up;
+// The parts of two values, packed, through set(part, both).
+template <typename Set>
+__device__ __forceinline__ void gf_split_two(float lo, float hi, float up, Set set) {
+    lo *= up;
+    hi *= up;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        float lo = i < 2 ? a[2 * i] : b[2 * i - 4], hi = i < 2 ? a[2 * i + 1] : b[2 * i - 3];
-#pragma unroll
-        for (int p = 0; p < 3; ++p) {
-            const uint32_t u = zi_pack_bf16x2(lo, hi);
-            s.p[p].u[i] = u;
-            if (p < 2) {
-                lo -= __uint_as_float(u << 16);             // exactly: what is left fits a float32
-                hi -= __uint_as_float(u & 0xffff0000u);
-            }
+    for (int p = 0; p < 3; ++p) {
+        const uint32_t u = zi_pack_bf16x2(lo, hi);
+        set(p, u);
+        if (p < 2) {
+            lo -= __uint_as_float(u << 16);             // exactly: what is left fits a float32
+            hi -= __uint_as_float(u & 0xffff0000u);
         }
     }
+}
+
+__device__ __forceinline__ gf_parts gf_split(gf_f32x4_t a, gf_f32x4_t b, float up) {
+    gf_parts s;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        gf_split_two(i < 2 ? a[2 * i] : b[2 * i - 4], i < 2 ? a[2 * i + 1] : b[2 * i - 3], up, [&](int p, uint32_t u) { s.p[p].u[i] = u; });
     return s;
 }
 
@@ -94,6 +103,58 @@ __device__ __forceinline__ gf_parts gf_turn_of_chain(int h, gf_f32x4_t* block, g
     if (PAIR) return gf_turn<GF_MINUS_SECOND>(block, line0, line8, lane);
     return h ? gf_turn<GF_MINUS>(block, line0, line8, lane) : gf_turn<GF_PLUS>(block, line0, line8, lane);
 }
+
+// x of up to V rows (V 2 or 4) where a block holds 8: a lane loads and splits V values of a chunk instead of 8, of which most would be
+// rows that are not there (a row of x, us: 1,536 x 8,960 13.1 to 11.7, 2,048 x 1,536 5.5 to 5.15, 3,584 x 18,944 50.2 to 46.2; rows that
+// are held were split for 2 us before the first weights were looked at: 4,608 x 3,584 17.1 to 15.8).  Lane l holds values V c .. V c + V - 1 of the chunk's 64 of row l / (64 / V), c = l mod (64 / V); the parts go
+// through 2 KB of LDS, 64 bytes for a row and chain, into the same operand as gf_turn's; rows past V are one line of zeros.
+template <int V>
+struct gf_few {
+    static constexpr int LANES = ZI_WAVE / V, PART = (2 * V + 1) * 64;      // lanes a row; bytes of one part, the zeros last
+    static_assert(V == 2 || V == 4, "whole pairs, within 2 KB");
+    float up;
+    int put, get;
+    __device__ __forceinline__ gf_few(char* block, int lane, int exchanged) {
+        const int m = lane / LANES, k = lane % LANES * V, chain = (k / 32) ^ exchanged, piece = k % 32 / 4, r = lane & 15, g = lane >> 4;
+        up = chain ? -GF_UP : GF_UP;
+        put = (chain * V + m) * 64 + (piece & 3) * 16 + (piece >> 2) * 8 + (k & 3) * 2;
+        get = (r % 8 < V ? r / 8 * V + r % 8 : 2 * V) * 64 + g * 16;
+        if (lane < 12) *reinterpret_cast<gf_f32x4_t*>(block + lane / 4 * PART + 2 * V * 64 + lane % 4 * 16) = gf_f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    __device__ __forceinline__ gf_parts turn(char* block, const gf_pack& x) const {
+#pragma unroll
+        for (int i = 0; i < V; i += 2)
+            gf_split_two(x.f[i], x.f[i + 1], up, [&](int p, uint32_t u) { *reinterpret_cast<gf_u32_alias_t*>(block + p * PART + put + i * 2) = u; });
+        gf_parts s;
+#pragma unroll
+        for (int p = 0; p < 3; ++p) s.p[p].f = *reinterpret_cast<const gf_f32x4_t*>(block + p * PART + get);
+        return s;
+    }
+    __device__ __forceinline__ static gf_pack load(__amdgpu_buffer_rsrc_t rows, int offset) {
+        gf_pack x;
+        if constexpr (V == 4) {
+            x.f = gf_load<0>(rows, offset);
+        } else {
+            const auto two = __builtin_amdgcn_raw_buffer_load_b64(rows, offset, 0, 0);
+            x.u[0] = two[0];
+            x.u[1] = two[1];
+        }
+        return x;
+    }
+};
+// Where lane l's values lie: `row` bytes into x (GF_OUT: a row that is not there, see fetch), `k` bytes into the chunk.
+struct gf_few_place {
+    int row, k;
+};
+template <int V>
+__device__ __forceinline__ gf_few_place gf_few_at(int lane, int rows_x, int64_t ldx) {
+    const int m = lane / (ZI_WAVE / V), k = lane % (ZI_WAVE / V) * V * 4;
+    return {m < rows_x ? (int)(m * ldx * 4) + k : GF_OUT, k};
+}
+template <>
+struct gf_few<8> {      // (none: blocks of 8 rows)
+    __device__ __forceinline__ gf_few(char*, int, int) {}
+};
 
 // acc += w . x over the 32 k of an instruction: the six products of parts that reach float32's last bits, the smallest first.
 __device__ __forceinline__ gf_f32x4_t gf_multiply(const gf_parts& w, const gf_parts& x, gf_f32x4_t acc) {
@@ -157,9 +218,9 @@ __device__ __forceinline__ void gf_finite(gf_f32x4_t& s, int row, Mine mine, Row
     }
 }
 
-// PAIR: 8 weight rows and up to 8 rows of x; else 16 weight rows and up to 16 * MT rows of x a workgroup.  RING chunks are
-// on their way while one is worked on.
-template <int MT, bool PAIR, int RING>
+// PAIR: 8 weight rows and up to 8 rows of x (XV < 8: up to XV of them, see gf_few); else 16 weight rows and up to 16 * MT rows of x a
+// workgroup.  RING chunks are on their way while one is worked on.
+template <int MT, bool PAIR, int RING, int XV>
 __global__ void __launch_bounds__(GF_PARTS* ZI_WAVE, 4)
 gemm_f32_split_stream_kernel(float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,
                        const float* __restrict__ bias, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int per, int vec_out) {
@@ -184,9 +245,15 @@ gemm_f32_split_stream_kernel(float* __restrict__ out, const float* __restrict__ 
     }
     const int chunks = (K + GF_KB - 1) / GF_KB;
     const int c0 = wave * per, c1 = c0 + per < chunks ? c0 + per : chunks;
+    constexpr bool FEW = PAIR && XV < 8;
+    char* const few_block = reinterpret_cast<char*>(turn[wave][1]);
+    const gf_few<PAIR ? XV : 8> few(few_block, lane, wave & 1);
+    const gf_few_place at_few = gf_few_at<XV>(lane, rows_x, ldx);
 
     gf_f32x4_t wr[RING][H][2], xr[RING][H][MT][2];
+    gf_pack xf[RING];
     auto fetch = [&](const int slot, int c) __attribute__((always_inline)) {
+        if constexpr (FEW) xf[slot] = few.load(xb, c < c1 && c * (GF_KB * 4) + at_few.k < K * 4 && at_few.row != GF_OUT ? at_few.row + c * (GF_KB * 4) : GF_OUT);
 #pragma unroll
         for (int h = 0; h < H; ++h)
 #pragma unroll
@@ -194,7 +261,8 @@ gemm_f32_split_stream_kernel(float* __restrict__ out, const float* __restrict__ 
                 const int k = c * (GF_KB * 4) + ((PAIR ? i : h) ^ (wave & 1)) * 128 + k_lane;      // (see the top: the chains change places)
                 const bool in = c < c1 && k < K * 4;
 #pragma unroll
-                for (int t = 0; t < MT; ++t) xr[slot][h][t][i] = gf_load<0>(xb, in && x_row[t][i % RB] != GF_OUT ? x_row[t][i % RB] + k : GF_OUT);
+                for (int t = 0; t < MT; ++t)
+                    if constexpr (!FEW) xr[slot][h][t][i] = gf_load<0>(xb, in && x_row[t][i % RB] != GF_OUT ? x_row[t][i % RB] + k : GF_OUT);
                 // a weight of up to 8 rows of x is read once by one workgroup: past L2
                 wr[slot][h][i] = gf_load<PAIR ? 2 : 0>(wb, in && w_row[i % RB] != GF_OUT ? w_row[i % RB] + k : GF_OUT);
             }
@@ -216,8 +284,10 @@ gemm_f32_split_stream_kernel(float* __restrict__ out, const float* __restrict__ 
             for (int h = 0; h < H; ++h) {
                 const gf_parts ws = gf_turn<GF_PLUS>(turn[wave][0], wr[s][h][0], wr[s][h][1], lane);
 #pragma unroll
-                for (int t = 0; t < MT; ++t)
-                    acc[h][t] = gf_multiply(ws, gf_turn_of_chain<PAIR>(h, turn[wave][1 + t], xr[s][h][t][0], xr[s][h][t][1], lane), acc[h][t]);
+                for (int t = 0; t < MT; ++t) {
+                    if constexpr (FEW) acc[h][t] = gf_multiply(ws, few.turn(few_block, xf[s]), acc[h][t]);
+                    else acc[h][t] = gf_multiply(ws, gf_turn_of_chain<PAIR>(h, turn[wave][1 + t], xr[s][h][t][0], xr[s][h][t][1], lane), acc[h][t]);
+                }
             }
             __builtin_amdgcn_sched_barrier(0);     // the loads stay this far ahead of their use
             fetch(s, c + s + RING);
@@ -263,7 +333,7 @@ gemm_f32_split_stream_kernel(float* __restrict__ out, const float* __restrict__ 
 //
 // Bound by the stream of the weights: 151,936 x 1,536 at 8 rows 161 us (5.8 TB/s).  Two workgroups a unit while a lane has registers for that
 // (128): with 4 chunks of x they spill, and one is faster (5,000 x 2,048 with the activation, one row: 17.4 against 20.8 us).
-template <bool PAIR, int PER, bool GATED>
+template <bool PAIR, int PER, bool GATED, int XV>
 __global__ void __launch_bounds__(GF_PARTS* ZI_WAVE, (PAIR ? 1 : 2) * PER <= 3 ? 4 : 2)
 gemm_f32_split_held_kernel(float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
                      int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int per, int vec_out, int groups) {
@@ -302,10 +372,19 @@ gemm_f32_split_held_kernel(float* __restrict__ out, const float* __restrict__ x,
 #pragma unroll
             for (int i = 0; i < 2; ++i) wr[s][h][i] = gf_load<2>(wb, in(s, h, i) ? w_row[i % RB] + k0 + place(s, h, i) : GF_OUT);
     };
+    constexpr bool FEW = PAIR && XV < 8;
     {
+        char* const few_block = reinterpret_cast<char*>(turn[wave][0]);
+        const gf_few<PAIR ? XV : 8> few(few_block, lane, wave & 1);
+        const gf_few_place at_few = gf_few_at<XV>(lane, M, ldx);
+        gf_pack xf[PER];
         gf_f32x4_t xr[PER][H][2];
 #pragma unroll
         for (int s = 0; s < PER; ++s)
+            if constexpr (FEW)
+                xf[s] = few.load(xb, s < mine && (c0 + s) * (GF_KB * 4) + at_few.k < K * 4 && at_few.row != GF_OUT ? at_few.row + (c0 + s) * (GF_KB * 4) : GF_OUT);
+#pragma unroll
+        for (int s = 0; s < PER && !FEW; ++s)
 #pragma unroll
             for (int h = 0; h < H; ++h)
 #pragma unroll
@@ -320,7 +399,10 @@ gemm_f32_split_held_kernel(float* __restrict__ out, const float* __restrict__ x,
 #pragma unroll
         for (int s = 0; s < PER; ++s)
 #pragma unroll
-            for (int h = 0; h < H; ++h) xs[s][h] = gf_turn_of_chain<PAIR>(h, turn[wave][(s * H + h) & 1], xr[s][h][0], xr[s][h][1], lane);
+            for (int h = 0; h < H; ++h) {
+                if constexpr (FEW) xs[s][h] = few.turn(few_block, xf[s]);
+                else xs[s][h] = gf_turn_of_chain<PAIR>(h, turn[wave][(s * H + h) & 1], xr[s][h][0], xr[s][h][1], lane);
+            }
     }
     int b = 0, whose = 0;
     uint64_t nan_rows = 0;
@@ -665,15 +747,21 @@ static int gs_launch(float* out, const float* x, const float* w, const float* bi
                      int64_t ldo, hipStream_t stream) {
     const int chunks = (K + GF_KB - 1) / GF_KB, per = (chunks + GF_PARTS - 1) / GF_PARTS;
     const int vec_out = ldo % 4 == 0 && (uintptr_t)out % 16 == 0;
-#define ZI_GF_STREAM(MT, PAIR, RING)                                                                                                     \
-    gemm_f32_split_stream_kernel<MT, PAIR, RING><<<dim3((N + (PAIR ? 7 : 15)) / (PAIR ? 8 : 16), (M + (PAIR ? 8 : 16 * MT) - 1) / (PAIR ? 8 : 16 * MT)), \
+#define ZI_GF_STREAM(MT, PAIR, RING, XV)                                                                                                 \
+    gemm_f32_split_stream_kernel<MT, PAIR, RING, XV><<<dim3((N + (PAIR ? 7 : 15)) / (PAIR ? 8 : 16), (M + (PAIR ? 8 : 16 * MT) - 1) / (PAIR ? 8 : 16 * MT)), \
                                              GF_PARTS * ZI_WAVE, 0, stream>>>(out, x, w, bias, M, N, K, ldx, ldw, ldo, per, vec_out)
     // two workgroups a unit while a lane has registers for that (128), else one
-#define ZI_GF_HELD(PAIR, PER)                                                                                                            \
+#define ZI_GF_HELD_PAIRS(PER)                                                                                                            \
+    do {                                                                                                                                 \
+        if (M <= 2) ZI_GF_HELD(true, PER, 2);                                                                                             \
+        else if (M <= 4) ZI_GF_HELD(true, PER, 4);                                                                                        \
+        else ZI_GF_HELD(true, PER, 8);                                                                                                    \
+    } while (0)
+#define ZI_GF_HELD(PAIR, PER, XV)                                                                                                        \
     do {                                                                                                                                 \
         const int nc = (PAIR ? 8 : 16) / (GATED ? 2 : 1), groups = (N + nc - 1) / nc;                                                        \
         const int places = zi_compute_units() * ((PAIR ? 1 : 2) * PER <= 3 ? 2 : 1);                                                         \
-        gemm_f32_split_held_kernel<PAIR, PER, GATED><<<groups < places ? groups : places, GF_PARTS * ZI_WAVE, 0, stream>>>(                         \
+        gemm_f32_split_held_kernel<PAIR, PER, GATED, XV><<<groups < places ? groups : places, GF_PARTS * ZI_WAVE, 0, stream>>>(                         \
             out, x, w, bias, M, N, K, ldx, ldw, ldo, per, vec_out, groups);                                                               \
     } while (0)
     // (rows in as many launches as 2^32 threads of one make necessary: a row's result does not depend on them)
@@ -689,14 +777,15 @@ static int gs_launch(float* out, const float* x, const float* w, const float* bi
     } while (0)
     switch (zi_gemm_f32_split_kernel(M, (int64_t)N * (GATED ? 2 : 1), K)) {
         case GF_HELD_PAIRS:
-            if (per <= 3) ZI_GF_HELD(true, 3);
-            else if (per <= 4) ZI_GF_HELD(true, 4);
-            else if (per <= 6) ZI_GF_HELD(true, 6);
-            else ZI_GF_HELD(true, 8);
+            if (per <= 3) ZI_GF_HELD_PAIRS(3);
+            else if (per <= 4) ZI_GF_HELD_PAIRS(4);
+            else if (per <= 6) ZI_GF_HELD_PAIRS(6);
+            else if (per <= 7) ZI_GF_HELD_PAIRS(7);
+            else ZI_GF_HELD_PAIRS(8);
             break;
         case GF_HELD_ROWS16:
-            if (per <= 3) ZI_GF_HELD(false, 3);
-            else ZI_GF_HELD(false, 4);
+            if (per <= 3) ZI_GF_HELD(false, 3, 8);
+            else ZI_GF_HELD(false, 4, 8);
             break;
         case GF_TILE_64: ZI_GF_TILE(4, 2, 4, 1); break;
         case GF_TILE_32: ZI_GF_TILE(2, 2, 4, 1); break;
@@ -708,14 +797,19 @@ static int gs_launch(float* out, const float* x, const float* w, const float* bi
                 return zi_fail("gemm_f32: no gated kernel for %d rows of %d x %d", M, N, K);      // (zi_gemm_f32_swiglu_takes says so)
             } else {
                 switch (zi_gemm_f32_split_kernel(M, N, K)) {
-                    case GF_PAIRS: ZI_GF_STREAM(1, true, 3); break;
-                    case GF_ROWS16: ZI_GF_STREAM(1, false, 2); break;
-                    default: ZI_GF_STREAM(2, false, 1); break;
+                    case GF_PAIRS:
+                        if (M <= 2) ZI_GF_STREAM(1, true, 3, 2);
+                        else if (M <= 4) ZI_GF_STREAM(1, true, 3, 4);
+                        else ZI_GF_STREAM(1, true, 3, 8);
+                        break;
+                    case GF_ROWS16: ZI_GF_STREAM(1, false, 2, 8); break;
+                    default: ZI_GF_STREAM(2, false, 1, 8); break;
                 }
             }
     }
 #undef ZI_GF_STREAM
 #undef ZI_GF_HELD
+#undef ZI_GF_HELD_PAIRS
 #undef ZI_GF_TILE
     return zi_check_launch("gemm_f32_split");
 }

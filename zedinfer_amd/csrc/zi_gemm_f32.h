@@ -10,7 +10,15 @@ typedef __attribute__((ext_vector_type(8))) __bf16 gf_bf16x8_t;
 #define GF_OUT 0x7fffffff    // an offset past the end of every buffer: the load gives zeros and fetches nothing
 
 // Products of more columns than this go as products of bfloat16 parts (gemm_f32_split.hip), the others through the float32 instruction
-// (gemm_f32.hip): a rule on k alone, so that a row's bits do not depend on the rows beside it.
+// (gemm_f32.hip): a rule on k alone, so that a row's bits do not depend on the rows beside it.  Time by parts over that of the instruction,
+// ranges over 1,024 to 65,536 weight rows, by columns:
+//                        1,028           1,152           1,408           1,536           2,048
+//   1 and 4 rows         0.96 to 1.15    0.93 to 1.03    0.94 to 1.05    0.96 to 1.05    0.94 to 1.15
+//   8 to 24 rows         0.92 to 1.17    0.80 to 0.99    0.83 to 1.02    0.81 to 1.02    0.78 to 1.06
+//   64 and 200 rows      0.74 to 1.17    0.72 to 1.14    0.74 to 1.02    0.75 to 1.04    0.74 to 1.01
+//   450 and 1,000 rows   0.76 to 1.15    0.74 to 1.15    0.74 to 0.99    0.74 to 0.99    0.74 to 1.01
+// (1 and 4 rows before gf_few, which takes 2 to 10 % off them.)  Three chunks a run are 24; 1,028 columns fill 17 of them, 1,408 22, and a round of
+// tiles is up to 1.15 of the other's time until they are full.
 #define GF_SPLIT_ABOVE 1408
 
 // The kernels a product can take; all of one k give the same bits.
