@@ -80,7 +80,7 @@ extern "C" int zi_gemm_generic(void* out, int out_dt, const void* x, int x_dt, c
     if (M == 0) return 0;
     const dim3 grid((N + GT - 1) / GT, (M + GT - 1) / GT);
     ZI_REQUIRE(grid.y <= 65535, "gemm: M=%d is too large for one launch", M);
-    // all float32 and whole 16-byte pieces a row: the matrix cores' float32 instruction (gemm_f32.hip), whatever M is
+    // all float32 and whole 16-byte pieces a row: the matrix cores (gemm_f32.hip and, for a long k, gemm_f32_split.hip), whatever M is
     if (x_dt == ZI_F32 && w_dt == ZI_F32 && out_dt == ZI_F32 && (!bias || bias_dt == ZI_F32) && zi_gemm_f32_takes(x, w, N, K, ldx, ldw))
         return zi_gemm_f32_launch((float*)out, (const float*)x, (const float*)w, (const float*)bias, M, N, K, ldx, ldw, ldo, stream);
     if (!bias) bias_dt = ZI_F32;
