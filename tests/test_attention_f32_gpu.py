@@ -194,3 +194,34 @@ def test_tokens_one_by_one_give_the_bits_of_tiles(nh, nkv, d, n):
     args = (q, kc, vc, seqs, poss, table, nh, nkv, d, d ** -0.5)
     one = ops.attention(*args, tok_index=index, decoded=True)
     assert torch.equal(one, ops.attention(*args, tok_index=index, decoded=False)) and bool(torch.isfinite(one).all())
+
+
+@pytest.mark.parametrize("nh,nkv,d,ps", [(12, 2, 128, 16), (4, 4, 16, 32), (3, 1, 24, 16), (6, 2, 40, 8)])
+@pytest.mark.parametrize("decoded", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_a_token_that_sees_no_key_has_zeros(nh, nkv, d, ps, decoded, dtype):
+    """What stands behind a step's requests to fill it up: a sequence that holds no page, in the kernel of the matrix cores and in the plain one
+    (head sizes of 24 and 40, bfloat16).  The tokens beside it keep their bits."""
+    from zedinfer_amd import ops
+    g = torch.Generator().manual_seed(nh * d)
+    kc, vc, table, _, _ = paged([40, 7], nkv, d, ps, g)
+    kc, vc = kc.to(dtype), vc.to(dtype)
+    table = torch.cat([table, torch.full_like(table[:1], -1)])
+    q = torch.randn(5, nh * d, generator=g).to(dtype).cuda()
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    seq, pos = i32([0, 1, 2, 0, 2]), i32([39, 6, 0, 21, 0])
+    got = ops.attention(q, kc, vc, seq, pos, table, nh, nkv, d, d ** -0.5, decoded=decoded)
+    assert bool((got[[2, 4]] == 0).all()) and bool(torch.isfinite(got).all())
+    real = [0, 1, 3]
+    assert torch.equal(got[real], ops.attention(q[real].contiguous(), kc, vc, seq[real].contiguous(), pos[real].contiguous(), table, nh, nkv, d, d ** -0.5, decoded=decoded))
+
+
+def test_a_latent_token_that_sees_no_key_has_zeros():
+    from zedinfer_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rank, rot, heads, ps = 40, 8, 3, 16
+    c, kr = (torch.randn(3, ps, n, generator=g, device="cuda") for n in (rank, rot))
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    qa = torch.randn(3, heads, rank + rot, generator=g, device="cuda")
+    out = ops.latent_attention(qa, c, kr, i32([0, 1, 0]), i32([20, 0, 3]), i32([[2, 0], [-1, -1]]), 0.2, 0, torch.empty(3, heads, rank, device="cuda"))
+    assert bool((out[1] == 0).all()) and bool(torch.isfinite(out).all()) and bool((out[[0, 2]] != 0).any())

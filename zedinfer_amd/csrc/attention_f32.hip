@@ -92,6 +92,7 @@ attention_f32_kernel(float* __restrict__ out, const float* __restrict__ q, int64
             for (int i = 0; i < DV; ++i) vr[i] = *reinterpret_cast<const af_f32x4_t*>(v + (int64_t)i * 16 * page_size);
         };
         float m = -INFINITY, l = 0.f;
+        bool any = false;      // this column saw a key
         af_f32x4_t acc[DV];
 #pragma unroll
         for (int i = 0; i < DV; ++i) acc[i] = zero;
@@ -119,6 +120,7 @@ attention_f32_kernel(float* __restrict__ out, const float* __restrict__ q, int64
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 seen[e] = mine && page >= 0 && key + e <= p && key + e >= lo;
+                any |= seen[e];
                 s0[e] = seen[e] ? s0[e] * scale : -INFINITY;
                 top = fmaxf(top, s0[e]);
             }
@@ -185,9 +187,10 @@ attention_f32_kernel(float* __restrict__ out, const float* __restrict__ q, int64
         }
         l += __shfl_xor(l, 16, ZI_WAVE);
         l += __shfl_xor(l, 32, ZI_WAVE);
+        const uint64_t who = __ballot(any);
         if (g == 0) {
             ms[wave][c] = m;
-            ls[wave][c] = l;
+            ls[wave][c] = (who | who >> 16 | who >> 32 | who >> 48) >> c & 1 ? l : -1.f;      // (below zero: saw none)
         }
 #pragma unroll
         for (int i = 0; i < DV; ++i) os[wave][i][lane] = acc[i];
@@ -196,13 +199,17 @@ attention_f32_kernel(float* __restrict__ out, const float* __restrict__ q, int64
 #pragma unroll
         for (int u = 1; u < AF_WAVES; ++u) top = fmaxf(top, ms[u][c]);
         float part[AF_WAVES], total = 0.f;
+        bool none = true;
 #pragma unroll
         for (int u = 0; u < AF_WAVES; ++u) {
+            none &= ls[u][c] < 0.f;
             part[u] = ms[u][c] == -INFINITY ? 0.f : expf(ms[u][c] - top);
             total += ls[u][c] * part[u];
         }
         if (sinks) total += expf(sinks[h] - top);
-        const float inv = 1.f / total;
+        // (a token that sees no key, as one that stands behind a step's requests to fill it up, has zeros, not 0 / 0: sums over it
+        // that are no numbers would be made again in the products that follow)
+        const float inv = none ? 0.f : 1.f / total;
         for (int i = wave; i < DV; i += AF_WAVES) {
             af_f32x4_t o = os[0][i][lane] * part[0];
 #pragma unroll

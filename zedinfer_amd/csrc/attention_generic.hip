@@ -107,7 +107,7 @@ attention_generic_kernel(T* __restrict__ out, const T* __restrict__ q, int64_t l
     T* orow = out + (int64_t)t * ldo + (int64_t)h * d;
     // a sink counts once in the denominator: exp(sink), unscaled, with no key and no value
     if (sinks) l += expf(sinks[h] - m);
-    const float inv = 1.f / l;
+    const float inv = l == 0.f ? 0.f : 1.f / l;      // (zero: it saw no key)
 #pragma unroll
     for (int i = 0; i < ATTN_ACC; ++i) {
         const int x = lane + i * ZI_WAVE;

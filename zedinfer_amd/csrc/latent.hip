@@ -304,7 +304,7 @@ latent_attention_kernel(float* __restrict__ out, const float* __restrict__ qa, c
         __syncthreads();
     }
     float* orow = out + ((int64_t)t * heads + h) * rank;
-    const float inv = 1.f / l;
+    const float inv = l == 0.f ? 0.f : 1.f / l;      // (zero: it saw no key)
 #pragma unroll
     for (int i = 0; i < ACC; ++i) {
         const int x = lane + i * ZI_WAVE;
