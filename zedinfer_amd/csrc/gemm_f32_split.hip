@@ -166,13 +166,14 @@ __device__ __forceinline__ gf_f32x4_t gf_multiply(const gf_parts& w, const gf_pa
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.p[0].b, x.p[0].b, acc, 0, 0, 0);
 }
 
-// Finishes four sums of a lane, of row `row` of x and of rows w_row(e) of w.  One that is not finite (an operand was no number or too large to split,
-// or the sum left the range: see the top) is made again from the float32 operands, by the whole wavefront (all its lanes come here together; mine(e): sum e is an output), so that a lane has K / 64
-// multiply-adds one after the other and the sum is at least as exact.  A row of x with a NaN, what a request whose values ran away
-// brings to every product, has NaNs only: it is remembered in nan_rows and its other outputs cost nothing; a weight row with one gives
-// them to all rows in hand.
-// (One such row among 8, us, every lane for itself, now, and without such a row: 17,920 x 1,536 with the activation 1,178, 32 and 21; 1,536 x 8,960 1,053, 23 and
-// 17; 151,936 x 1,536 9,085, 185 and 159.  A weight row with one, 450 rows of 1,536 x 8,960: 376, 114 and 107.)
+// Finishes four sums of a lane, of row `row` of x and of rows w_row(e) of w.  One that is not finite (an operand was no number or too large
+// to split, or the sum left the range: see the top) is made again from the float32 operands, by the whole wavefront (all its lanes come here
+// together; mine(e): sum e is an output), so that a lane has K / 64 multiply-adds one after the other and the sum is at least as exact.  A
+// row of x with a NaN, what a request whose values ran away brings to every product, has NaNs only: it is looked for first, four loads
+// on their way, and remembered in nan_rows; a weight row with one gives them to all rows in hand.
+// (Rows with a NaN, us, every lane for itself, summed by the wavefront before it is looked for, now, and without such rows.  One among 8:
+// 17,920 x 1,536 with the activation 1,178, 32, 24.6 and 20.2; 1,536 x 8,960 1,053, 23, 18.2 and 15.9; 151,936 x 1,536 9,085, 185, 156 and 156.  Four among 72
+// of 1,536 x 8,960 97.7 and 85.9, 20 among 450 158 and 117.  A weight row with one, 450 rows of 1,536 x 8,960: 376, 114 and, without, 107.)
 template <typename Mine, typename Row>
 __device__ __forceinline__ void gf_finite(gf_f32x4_t& s, int row, Mine mine, Row w_row, const float* x, int64_t ldx, const float* w, int64_t ldw, int K,
                                           uint64_t& nan_rows) {
@@ -185,31 +186,43 @@ __device__ __forceinline__ void gf_finite(gf_f32x4_t& s, int row, Mine mine, Row
     for (int e = 0; e < 4; ++e) {
         float sum = e == 0 ? s[0] : e == 1 ? s[1] : e == 2 ? s[2] : s[3];
         const int row_w = w_row(e);
-        uint64_t todo = __ballot(mine(e) && (__float_as_uint(sum) & 0x7f800000u) == 0x7f800000u);
+        const bool known = nan_rows >> row & 1;
+        if (known) sum = no_number;
+        uint64_t todo = __ballot(mine(e) && !known && (__float_as_uint(sum) & 0x7f800000u) == 0x7f800000u);
         while (todo) {
             const int of = __builtin_ctzll(todo), of_x = __builtin_amdgcn_readlane(row, of), of_w = __builtin_amdgcn_readlane(row_w, of);
             todo &= todo - 1;
-            float again = no_number;
-            if (!(nan_rows >> of_x & 1)) {
-                const float *a = x + of_x * ldx, *b = w + of_w * ldw;
-                bool nan_x = false, nan_w = false;
-                again = 0.f;
-#pragma unroll 1
-                for (int k = lane * 4; k < K; k += ZI_WAVE * 4) {
-                    const gf_f32x4_t u = *reinterpret_cast<const gf_f32x4_t*>(a + k), v = *reinterpret_cast<const gf_f32x4_t*>(b + k);
+            float again = 0.f;
+            const float *a = x + of_x * ldx, *b = w + of_w * ldw;
+            bool nan_x = false, nan_w = false;
+            for (int k0 = lane * 4; k0 < K; k0 += ZI_WAVE * 16) {      // (four loads on their way)
+                gf_f32x4_t u[4];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        again = fmaf(u[i], v[i], again);
-                        nan_x |= u[i] != u[i];
-                        nan_w |= v[i] != v[i];
-                    }
+                for (int i = 0; i < 4; ++i) u[i] = *reinterpret_cast<const gf_f32x4_t*>(a + (k0 + i * ZI_WAVE * 4 < K ? k0 + i * ZI_WAVE * 4 : k0));
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) nan_x |= u[i][j] != u[i][j];
+            }
+            if (__ballot(nan_x)) {
+                nan_rows |= 1ull << of_x;
+                todo &= ~__ballot(row == of_x);
+                if (row == of_x) sum = no_number;
+                continue;
+            }
+#pragma unroll 1
+            for (int k = lane * 4; k < K; k += ZI_WAVE * 4) {
+                const gf_f32x4_t u = *reinterpret_cast<const gf_f32x4_t*>(a + k), v = *reinterpret_cast<const gf_f32x4_t*>(b + k);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    again = fmaf(u[i], v[i], again);
+                    nan_w |= v[i] != v[i];
                 }
-                again = zi_wave_sum(again);
-                if (__ballot(nan_x)) nan_rows |= 1ull << of_x;
-                if (__ballot(nan_w)) {
-                    todo &= ~__ballot(row_w == of_w);
-                    if (row_w == of_w) sum = no_number;
-                }
+            }
+            again = zi_wave_sum(again);
+            if (__ballot(nan_w)) {
+                todo &= ~__ballot(row_w == of_w);
+                if (row_w == of_w) sum = no_number;
             }
             if (lane == of) sum = again;
         }
