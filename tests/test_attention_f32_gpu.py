@@ -225,3 +225,20 @@ def test_a_latent_token_that_sees_no_key_has_zeros():
     qa = torch.randn(3, heads, rank + rot, generator=g, device="cuda")
     out = ops.latent_attention(qa, c, kr, i32([0, 1, 0]), i32([20, 0, 3]), i32([[2, 0], [-1, -1]]), 0.2, 0, torch.empty(3, heads, rank, device="cuda"))
     assert bool((out[1] == 0).all()) and bool(torch.isfinite(out).all()) and bool((out[[0, 2]] != 0).any())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_a_pooled_token_that_sees_no_key_has_zeros(dtype):
+    """... and one whose every score is minus infinity has no number, as a softmax over them has none."""
+    from zedinfer_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(6)
+    nh, nkv, d, ps = 4, 2, 32, 16
+    kc, vc = (torch.randn(3, ps, nkv, d, generator=g, device="cuda").to(dtype) for _ in range(2))
+    q = torch.randn(3, nh * d, generator=g, device="cuda").to(dtype)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    run = lambda: ops.pooled_attention(q, kc, vc, None, None, i32([0, 1, 0]), i32([20, 0, 3]), i32([[2, 0], [-1, -1]]), None, nh, nkv, d, d, 0, 0,  # noqa: E731
+                                       d ** -0.5, torch.empty_like(q)).clone()
+    out = run()
+    assert bool((out[1] == 0).all()) and bool(torch.isfinite(out).all()) and bool((out[[0, 2]] != 0).any())
+    kc[2, :4], q[2] = float("-inf"), q[2].abs() + 1
+    assert bool(torch.isnan(run()[2]).all())

@@ -334,6 +334,7 @@ pooled_attention_kernel(T* __restrict__ out, int64_t ldo, const T* __restrict__ 
     float acc[PA_ACC];
 #pragma unroll
     for (int i = 0; i < PA_ACC; ++i) acc[i] = 0.f;
+    bool any = false;      // this wavefront saw a key
 
     for (int base = wave * ZI_WAVE; base < count; base += PA_WAVES * ZI_WAVE) {
         const int at = base + lane;
@@ -369,6 +370,7 @@ pooled_attention_kernel(T* __restrict__ out, int64_t ldo, const T* __restrict__ 
         const float pj = (valid && m_new > -INFINITY) ? expf(s - m_new) : 0.f;
         const float corr = (m == -INFINITY) ? 0.f : expf(m - m_new);
         l = l * corr + zi_wave_sum(pj);
+        any |= __ballot(valid) != 0;
         ps[wave][lane] = pj;
         vat[wave][lane] = valid ? vrow : -1;
         __builtin_amdgcn_wave_barrier();
@@ -406,20 +408,22 @@ pooled_attention_kernel(T* __restrict__ out, int64_t ldo, const T* __restrict__ 
     }
     if (lane == 0) {
         merged[wave][PA_MAX_D] = m;
-        merged[wave][PA_MAX_D + 1] = l;
+        merged[wave][PA_MAX_D + 1] = any ? l : -1.f;      // (below zero: saw none)
     }
     __syncthreads();
     float mm = -INFINITY;
 #pragma unroll
     for (int w = 0; w < PA_WAVES; ++w) mm = fmaxf(mm, merged[w][PA_MAX_D]);
     float ll = 0.f, f[PA_WAVES];
+    bool none = true;
 #pragma unroll
     for (int w = 0; w < PA_WAVES; ++w) {
+        none &= merged[w][PA_MAX_D + 1] < 0.f;
         const float mw = merged[w][PA_MAX_D];
         f[w] = mw == -INFINITY ? 0.f : expf(mw - mm);
         ll += merged[w][PA_MAX_D + 1] * f[w];
     }
-    const float inv = 1.f / ll;
+    const float inv = none ? 0.f : 1.f / ll;      // (a token that sees no key has zeros)
     __syncthreads();
     for (int x = tid; x < vdim; x += PA_WAVES * ZI_WAVE) {
         float o = 0.f;
