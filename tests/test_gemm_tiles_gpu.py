@@ -1,0 +1,177 @@
+"""Products of many rows in tiles (``csrc/gemm_tiles.hip``) at the edges of every tile, against float64 products of the same bfloat16
+operands.  Sums are float32, of K products each of which is exact: their error is below K 2^-24 of the sum of the products'
+magnitudes (K a few hundred to thousands, errors of both signs: a fiftieth of that bound is allowed here), and bfloat16 results are
+rounded once, by at most 2^-8 of their size (eight bits: half of 2^-7 of the power of two below)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+BF16, F32, SWIGLU, GATED = 0, 1, 2, 3
+# rows and weight rows of the tiles, in the kernel's order
+TILES = [(64, 64), (128, 64), (128, 96), (128, 128), (128, 192), (192, 160), (192, 224), (128, 256), (192, 192), (256, 256)]
+
+
+def rnd(*shape, seed=0, scale=1.0):
+    return (torch.randn(*shape, generator=torch.Generator().manual_seed(seed)) * scale).bfloat16().cuda()
+
+
+def tiles(epi, x, w, N, bias=None, out=None, up_at=0, act=0, splits=1, tile=-1):
+    from zedinfer_amd.ops import _lib
+    from zedinfer_amd.ops.functional import _p, _stream
+    M, K = x.shape
+    if out is None:
+        shape = (splits, M, N) if splits > 1 else (M, N)
+        out = torch.full(shape, float("nan"), dtype=torch.float32 if epi == F32 else torch.bfloat16, device="cuda")
+    _lib.call("zi_gemm_tiles", _p(out), epi, _p(x), _p(w), _p(bias), M, N, K, x.stride(0), w.stride(0),
+              out.stride(-2), up_at, act, splits, tile, _stream())
+    return out
+
+
+def close(got, x, w, epi, bias=None, act=None, up=None):
+    """``act``: what is made of gate and up; ``up``: the up rows."""
+    X = x.double()
+    ref, size = X @ w.double().t(), X.abs() @ w.double().abs().t()
+    bound = size * (x.shape[1] * 2.0 ** -24 / 50) + 2.0 ** -23 * ref.abs()
+    if bias is not None:
+        ref = ref + bias.double()
+        bound = bound + 2.0 ** -23 * ref.abs()
+    if act is not None:
+        u = X @ up.double().t()
+        bound = 1.2 * bound * u.abs() + ref.abs() * (X.abs() @ up.double().abs().t()) * (x.shape[1] * 2.0 ** -24 / 50)      # (slopes of the activations: up to 1.13)
+        ref = act(ref) * u
+        bound = bound + 2.0 ** -20 * ref.abs()
+    if epi != F32:
+        bound = bound + 2.0 ** -8 * (ref.abs() + bound)
+    assert not got.isnan().any()
+    assert bool(((got.double() - ref).abs() <= bound + 1e-30).all()), float(((got.double() - ref).abs() / (bound + 1e-30)).max())
+
+
+def gelu_tanh(z):
+    return torch.nn.functional.gelu(z, approximate="tanh")
+
+
+def test_the_kernels_tiles():
+    from zedinfer_amd import ops
+    assert ops.load().zi_gemm_tiles_count() == len(TILES)
+
+
+@pytest.mark.parametrize("tile", range(len(TILES)))
+@pytest.mark.parametrize("rows,cols,K", [(0, 0, 320), (1, 8, 384), (-1, -8, 704), (17, 24, 640)])
+def test_every_tile_at_its_edges(tile, rows, cols, K):
+    """One tile and a little more or less, and several of them, with and without a bias, into rows of a wider buffer."""
+    bm, bn = TILES[tile]
+    for many in (1, 3):
+        M, N = many * bm + rows, max(8, many * bn + cols)
+        x, w, bias = rnd(M, K, seed=tile), rnd(N, K, seed=tile + 50, scale=0.2), rnd(N, seed=tile + 90)
+        close(tiles(BF16, x, w, N, bias, tile=tile), x, w, BF16, bias)
+        close(tiles(F32, x, w, N, tile=tile), x, w, F32)
+        wide = torch.zeros(M, N + 16, dtype=torch.bfloat16, device="cuda")
+        tiles(BF16, x, w, N, out=wide[:, 8:N + 8], tile=tile)
+        close(wide[:, 8:N + 8], x, w, BF16)
+        assert float(wide[:, :8].abs().max()) == 0 and float(wide[:, N + 8:].abs().max()) == 0
+        apart = rnd(M, K + 24, seed=tile)[:, 8:K + 8]
+        close(tiles(BF16, apart, w, N, tile=tile), apart, w, BF16)
+
+
+@pytest.mark.parametrize("tile", [t for t in range(len(TILES)) if TILES[t][1] // 32 % 2 == 0])
+@pytest.mark.parametrize("rows,cols,K", [(0, 0, 320), (1, 8, 384), (-1, -8, 704)])
+def test_gate_and_up(tile, rows, cols, K):
+    """Gate and up rows in turn and one block after the other, up to rows that no column of the result belongs to."""
+    bm, bn = TILES[tile]
+    M, N = bm + rows, max(8, bn + cols)
+    x, g, u = rnd(M, K, seed=tile), rnd(N, K, seed=tile + 50, scale=0.2), rnd(N, K, seed=tile + 90, scale=0.2)
+    turns = torch.stack([g.view(N // 8, 8, K), u.view(N // 8, 8, K)], dim=1).reshape(2 * N, K).contiguous()
+    close(tiles(SWIGLU, x, turns, N, tile=tile), x, g, SWIGLU, act=torch.nn.functional.silu, up=u)
+    for act, fn in enumerate((torch.nn.functional.silu, gelu_tanh, torch.nn.functional.gelu)):
+        up_at = N + 8 * act
+        halves = torch.full((up_at + N, K), float("nan"), dtype=torch.bfloat16, device="cuda")
+        halves[:N], halves[up_at:] = g, u
+        close(tiles(GATED, x, halves, N, up_at=up_at, act=act, tile=tile), x, g, GATED, act=fn, up=u)
+
+
+def test_large_and_infinite_gates():
+    """up * silu(gate) where the exponential overflows or vanishes, and of what is no number, as the activation's own kernel has it."""
+    from zedinfer_amd import ops
+    K, N = 320, 64
+    gates = torch.tensor([0.0, -0.0, 1e-30, -1e-30, 30.0, -30.0, 87.0, -87.0, 88.8, -88.8, 104.0, -104.0, 3e4, -3e4, 3e38, -3e38, float("inf"),
+                          float("-inf"), float("nan")])
+    x = torch.zeros(300, K, dtype=torch.bfloat16, device="cuda")
+    x[:, 0] = 1.0
+    x[:len(gates), 1] = gates.bfloat16().cuda()
+    turns = torch.zeros(2 * N, K, dtype=torch.bfloat16, device="cuda")
+    turns[torch.arange(2 * N, device="cuda") % 16 < 8, 1] = 1.0      # gates: x[:, 1]
+    turns[torch.arange(2 * N, device="cuda") % 16 >= 8, 0] = 1.5     # ups
+    got = tiles(SWIGLU, x, turns, N)
+    both = torch.zeros(300, 2 * N, dtype=torch.bfloat16, device="cuda")
+    both[:, torch.arange(2 * N, device="cuda") % 16 < 8] = x[:, 1:2]
+    both[:, torch.arange(2 * N, device="cuda") % 16 >= 8] = 1.5
+    # (zeros times what is no number are none either: those rows' ups)
+    both[torch.isinf(x[:, 1]) | torch.isnan(x[:, 1])] = float("nan")
+    want = ops.swiglu(both, interleave=8)
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.isinf(), want.isinf())
+    good = want.isfinite()
+    # (two roundings of nearly the same value; a quotient below 2^-126 is zero, times a gate of up to 89 and 1.5)
+    assert bool(((got - want)[good].float().abs() <= 2.0 ** -7 * want[good].float().abs() + 140 * 2.0 ** -126).all())
+
+
+@pytest.mark.parametrize("M,N,K,splits", [(257, 520, 1536, 2), (512, 1536, 8960, 4), (300, 640, 2560, 8), (1024, 768, 2048, 3), (2048, 1536, 8960, 2)])
+def test_partial_sums(M, N, K, splits):
+    x, w = rnd(M, K, seed=M), rnd(N, K, seed=N, scale=0.1)
+    for tile in range(len(TILES)):
+        sums = tiles(F32, x, w, N, splits=splits, tile=tile)
+        close(sums.sum(0, dtype=torch.float64), x, w, F32)
+
+
+def test_more_tiles_than_workgroups_and_replays():
+    """Workgroups that take several tiles, of which the last are few; the same bits eagerly and from a replayed graph with other work between."""
+    from zedinfer_amd import ops
+    M, N, K = 1600, 4104, 576
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2, scale=0.2)
+    for tile in (0, 3, 8, 9):
+        out = tiles(BF16, x, w, N, tile=tile)
+        close(out, x, w, BF16)
+        again = torch.empty_like(out)
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            tiles(BF16, x, w, N, out=again, tile=tile)
+        for _ in range(3):
+            again.zero_()
+            g.replay()
+            assert torch.equal(out, again)
+            ops.linear(x[:64], w)
+            torch.cuda.synchronize()
+
+
+def test_which_products_take_the_tiles(monkeypatch):
+    """``ops.linear`` of more than 256 rows by the sizes, and what the kernel cannot load by the library as before."""
+    from zedinfer_amd import ops
+    calls, real = [], ops._lib.call
+    monkeypatch.setattr(ops._lib, "call", lambda name, *a: (calls.append(name), real(name, *a))[1])
+
+    def taken(M, N, K, bias=False, **kw):
+        x, w = rnd(M, K, seed=3), rnd(N, K, seed=4, scale=0.1)
+        b = rnd(N, seed=5) if bias else None
+        calls.clear()
+        out = ops.linear(x, w, b, **kw)
+        ref = x.double() @ w.double().t() + (b.double() if bias else 0)
+        assert float((out.double() - ref).norm() / ref.norm()) <= (1e-5 if out.dtype == torch.float32 else 3e-3)
+        return calls == ["zi_gemm_tiles"]
+    assert taken(257, 1536, 1536) and taken(2048, 2048, 1536, bias=True) and taken(640, 1536, 8960, out_dtype=torch.float32)
+    assert not taken(256, 1536, 1536) and not taken(300, 1536, 1528) and not taken(300, 1532, 1536) and not taken(320, 512, 4608)
+    x, w = rnd(300, 1544, seed=6)[:, 4:1540], rnd(1536, 1536, seed=7)      # rows that do not begin at 16 bytes
+    calls.clear()
+    ops.linear(x, w)
+    assert "zi_gemm_tiles" not in calls
+    assert ops.linear_tune(rnd(300, 1536), w) is None
+
+
+def test_what_is_refused():
+    from zedinfer_amd import ops
+    x, w = rnd(300, 640), rnd(640, 640)
+    for bad in (dict(N=644), dict(N=640, splits=3, epi=BF16), dict(N=640, tile=len(TILES)), dict(N=320, epi=SWIGLU, tile=2),
+                dict(N=320, epi=GATED, up_at=312), dict(N=640, splits=4, epi=F32), dict(N=320, epi=GATED, up_at=320, act=3)):
+        with pytest.raises(ops.KernelLibraryError):
+            tiles(bad.pop("epi", BF16), x, w, **bad)
+    with pytest.raises(ops.KernelLibraryError):
+        tiles(BF16, rnd(300, 256), rnd(640, 256), 640)

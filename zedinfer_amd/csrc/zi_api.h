@@ -108,6 +108,9 @@ int zi_gemm_f32_swiglu(float* out, const float* x, const float* w, int M, int in
 int zi_gemm_lt(void* out, int out_dt, const void* x, const void* weight, const void* bias, int transposed, int64_t M,
     int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldo, void* workspace, int64_t workspace_bytes, hipStream_t
     stream);
+// gemm_tiles.hip
+int zi_gemm_tiles(void* out, int epi, const void* x, const void* w, const void* bias, int M, int N, int K, int64_t ldx,
+    int64_t ldw, int64_t ldo, int up_at, int act, int splits, int tile, hipStream_t stream);
 // gemm_skinny.hip
 int zi_gemm_skinny(void* out, int out_dt, int mode, const void* x, const void* w, const void* bias, int M, int N, int
     K, int64_t ldx, int64_t ldw, int64_t ldo, float* workspace, int64_t workspace_floats, hipStream_t stream);
@@ -422,6 +425,7 @@ int zi_sample(int32_t* out, const float* logits, int64_t ld, float* work, int ro
     X(zi_gemm_generic) \
     X(zi_gemm_f32_swiglu) \
     X(zi_gemm_lt) \
+    X(zi_gemm_tiles) \
     X(zi_gemm_skinny) \
     X(zi_reduce_splits) \
     X(zi_rmsnorm) \

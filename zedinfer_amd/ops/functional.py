@@ -922,7 +922,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     """out[M,N] = x[M,K] . weight[N,K]^T + bias[N], accumulated in float32
     (reference: src/backend/ops/linear/op.cpp:57-58).
 
-    bfloat16 inputs with bfloat16 weights and output (or float32 output and more than 64 rows) go
+    bfloat16 inputs with bfloat16 weights and output (or float32 output and more than 64 rows) go, of
+    more than 256 rows, to the tiles of ``csrc/gemm_tiles.hip`` where those were measured to be faster, else
     to the library matrix product, as the reference sends them to its vendor library (reference:
     src/backend/ops/linear/nvidia/linear_cublas.cu:134-231); float32 operands go to the
     matrix cores: up to 1,408 columns to their float32 instruction (products and sums in float32), beyond to the bfloat16 one as
@@ -947,6 +948,10 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
         return out
     bf = torch.bfloat16
     all_bf = x.dtype == bf and weight.dtype == bf and (bias is None or bias.dtype == bf)
+    if all_bf and _tiles_take(x, weight, out, bias, TILES_PLAIN):
+        _lib.call("zi_gemm_tiles", _p(out), int(out.dtype == torch.float32), _p(x), _p(weight), _p(bias), M, N, K, ldx, ldw, ldo,
+                  0, 0, 1, -1, _stream())
+        return out
     if all_bf and out.dtype == torch.float32 and M > SKINNY_MAX_ROWS and bias is None and _library_ok(x, weight, out):
         # float32 output for many rows (logits of a large decode batch or of every place of a prompt): the
         # library's product with float32 results, one pass over the weights instead of one per 64 rows
@@ -988,6 +993,31 @@ def linear_transposed(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch
     return out
 
 
+TILES_PLAIN, TILES_GATES, TILES_SUMS = 0, 1, 2      # what of a product ``zi_gemm_tiles_pays`` is asked about
+TILES_ABOVE = 256                                    # rows up to which it says no
+
+
+def _tiles_operands(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """bfloat16 matrices of more than 256 rows whose rows the tiles' kernel can load."""
+    if x.dim() != 2 or x.shape[0] <= TILES_ABOVE or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 \
+            or weight.dim() != 2 or x.shape[1] != weight.shape[1]:
+        return False
+    return all(t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (x, weight)) \
+        and x.stride(0) <= 1 << 21 and weight.shape[0] * weight.stride(0) < 1 << 30
+
+
+def _tiles_pay(M: int, N: int, K: int, kind: int) -> bool:
+    return bool(_lib.load().zi_gemm_tiles_pays(int(M), int(N), int(K), kind))
+
+
+def _tiles_take(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, bias: Optional[torch.Tensor], kind: int) -> bool:
+    """Whether ``linear`` gives the product to the tiles' kernel: operands and a result it can load and store, and sizes at which it
+    was measured to be faster than the library's product."""
+    return (_tiles_operands(x, weight) and out.stride(1) == 1 and out.data_ptr() % 16 == 0
+            and out.stride(0) % (4 if out.dtype == torch.float32 else 8) == 0 and (bias is None or bias.dtype == torch.bfloat16)
+            and _tiles_pay(x.shape[0], weight.shape[0], x.shape[1], kind))
+
+
 LIBRARY_WORKSPACE_BYTES = 64 << 20     # what an algorithm of the library's product may use beside its operands
 _LIBRARY_WORKSPACES = {}
 
@@ -1014,7 +1044,7 @@ def linear_tune(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
                 out_dtype: Optional[torch.dtype] = None, candidates: Optional[int] = None, rounds: Optional[int] = None):
     """Let the library time its proposals for the product ``linear`` (``linear_transposed``) makes of these operands
     and keep the fastest for every later call of the shape; returns (chosen, proposed, microseconds), or None when
-    the product is not the library's (few rows, float32 operands).  Waits for the device.  ``candidates``: how
+    the product is not the library's (few rows, float32 operands, many rows that the tiles' kernel takes).  Waits for the device.  ``candidates``: how
     many of the proposals are timed (None: the first 16, the first 8 of a product of about 250 us and more);
     ``rounds``: timed runs of each (None: five of a short product, fewer of one that takes long enough for the
     clock: three beyond about 50 us, two beyond 250)."""
@@ -1031,7 +1061,7 @@ def linear_tune(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     if M <= (SKINNY_MAX_ROWS if out_dtype == torch.float32 else FEW_ROWS) or (out_dtype == torch.float32 and bias is not None):
         return None
     out = torch.empty((N, M) if transposed else (M, N), dtype=out_dtype, device=x.device)
-    if not _library_ok(x, weight, out):
+    if not _library_ok(x, weight, out) or (not transposed and _tiles_take(x, weight, out, bias, TILES_PLAIN)):
         return None
     chosen, proposed, us = c_int(0), c_int(0), c_float(0.0)
     _lib.call("zi_gemm_lt_tune", *_library_args(out, x, weight, bias, transposed), int(candidates), int(rounds),
