@@ -175,3 +175,30 @@ def test_what_is_refused():
             tiles(bad.pop("epi", BF16), x, w, **bad)
     with pytest.raises(ops.KernelLibraryError):
         tiles(BF16, rnd(300, 256), rnd(640, 256), 640)
+
+
+@pytest.mark.parametrize("kind,activation", [("swiglu", "silu"), ("gated_mlp", "silu"), ("gated_mlp", "gelu_tanh"), ("gated_mlp", "gelu_erf")])
+@pytest.mark.parametrize("n,H,I", [(257, 640, 1000), (640, 1536, 2048)])
+def test_feed_forwards_of_many_rows(kind, activation, n, H, I, monkeypatch):
+    """Parts whose gate/up product ends in the activation: against float64, and nothing of it is timed or launched apart."""
+    from zedinfer_amd.config.forward_config import PartSpec
+    from zedinfer_amd.ops import _lib
+    from zedinfer_amd.parts import FEED_FORWARDS
+    from zedinfer_amd.parts.base import Runtime
+    w = {"gate": rnd(I, H, seed=1, scale=0.05), "up": rnd(I, H, seed=2, scale=0.05), "down": rnd(H, I, seed=3, scale=0.05)}
+    x, rt = rnd(n, H, seed=4), Runtime("cuda", torch.bfloat16)
+    params = {"hidden_size": H, "intermediate_size": I, "activation": activation}
+    part = FEED_FORWARDS.get(kind)(PartSpec(kind, params, {k: k for k in w}), w, rt)
+    part.tune(n)
+    assert not [k for k in rt.choices if k[0] == "gate_up_transposed" or k[2] > H]
+    calls, real = [], _lib.call
+    monkeypatch.setattr(_lib, "call", lambda name, *a: (calls.append(name), real(name, *a))[1])
+    got = part.forward(x).double()
+    if got.dim() == 3:
+        got = got.sum(0)
+    assert calls[0] == "zi_gemm_tiles" and not {"zi_swiglu", "zi_swiglu_t", "zi_gated_act"} & set(calls)
+    fn = {"silu": torch.nn.functional.silu, "gelu_tanh": gelu_tanh, "gelu_erf": torch.nn.functional.gelu}[activation]
+    X = x.double()
+    ref = (fn(X @ w["gate"].double().t()) * (X @ w["up"].double().t())) @ w["down"].double().t()
+    # the activation and the result are rounded to bfloat16 once each, evenly: 2^-8 / sqrt(3) at most of every value, less of a sum
+    assert float((got - ref).norm() / ref.norm()) <= 2 * 2.0 ** -8 / 3 ** 0.5

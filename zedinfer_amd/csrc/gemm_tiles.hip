@@ -40,6 +40,7 @@ union gt_pack {
 #define GT_F32 1           // float32 results with a bias, or partial sums [split][M][N]
 #define GT_SWIGLU 2        // gate and up rows of the weights alternate in blocks of 8; bfloat16
 #define GT_GATED 3         // the gate rows come first, the up rows from row `up_at` on; an activation by its code; bfloat16
+#define GT_ERF 4           // the same with the error function's GELU (a kernel of its own: the function is 40 instructions)
 
 // Loads but for the newest n have arrived, and every read of LDS.
 template <int n>
@@ -103,13 +104,23 @@ __device__ __forceinline__ void gt_place(const gt_args& g, int unit, int* m, int
     *m = group * GT_GROUP + in - *n * rows;
 }
 
-// up * silu(gate).  exp(-gate) is 2^t (1 + rest): the rounding of t, which the chip's exponential would make large for large gates, is put
+// up * z sigmoid(s).  exp(-s) is 2^t (1 + rest): the rounding of t, which the chip's exponential would make large for large s, is put
 // back; then the chip's reciprocal.  (The library's exponential and quotient are 30 instructions a value, which nothing overlaps with
 // at a tile's end.)
-__device__ __forceinline__ float gt_silu_mul(float gate, float up) {
-    const float t = gate * -1.44269504f, rest = __builtin_fmaf(gate, -1.44269504f, -t) + gate * -1.92596303e-8f;
+__device__ __forceinline__ float gt_sigmoid_mul(float z, float s, float up) {
+    const float t = s * -1.44269504f, rest = __builtin_fmaf(s, -1.44269504f, -t) + s * -1.92596303e-8f;
     const float e = __builtin_amdgcn_exp2f(t);
-    return up * (gate * __builtin_amdgcn_rcpf(1.f + (fabsf(t) < 126.f ? __builtin_fmaf(e, rest * 0.693147182f, e) : e)));      // (beyond, e or rest may be infinite)
+    return up * (z * __builtin_amdgcn_rcpf(1.f + (fabsf(t) < 126.f ? __builtin_fmaf(e, rest * 0.693147182f, e) : e)));      // (beyond, e or rest may be infinite)
+}
+
+// up times the activation of z: SiLU, GELU in its tanh form, which is z sigmoid(2 u), u = sqrt(2 / pi) (z + 0.044715 z^3), or with the
+// error function.
+template <int EPI>
+__device__ __forceinline__ float gt_gate(float z, float up, int act) {
+    if (EPI == GT_ERF) return zi_activation(z, ZI_ACT_GELU_ERF) * up;
+    if (EPI == GT_SWIGLU) return gt_sigmoid_mul(z, z, up);
+    const float u = z * __builtin_fmaf(0.044715f * 2.f * 0.7978845608028654f * z, z, 2.f * 0.7978845608028654f);
+    return gt_sigmoid_mul(z, act == ZI_ACT_GELU_TANH ? u : z, up);
 }
 
 template <int WM, int MW, int NW>
@@ -122,7 +133,7 @@ template <int WM, int MW, int NW, int EPI>
 __global__ void __launch_bounds__(128 * WM, 1) gemm_tiles_kernel(gt_args g) {
     typedef gt_shape<WM, MW, NW> Z;
     constexpr int S = Z::STAGES, WAVES = Z::WAVES, BM = Z::ROWS, BN = Z::WROWS, XI = BM / 8, PW = Z::LOADS / WAVES, PIECES = Z::LOADS * ZI_WAVE;
-    constexpr bool GATES = EPI == GT_SWIGLU || EPI == GT_GATED;
+    constexpr bool GATES = EPI >= GT_SWIGLU, HALVES = EPI >= GT_GATED;
     constexpr int COLS = GATES ? BN / 2 : BN;
     static_assert(XI % WAVES == 0 && Z::LOADS % WAVES == 0 && S >= 2 && (!GATES || NW % 2 == 0), "whole shares, gates and ups in pairs");
     __shared__ __attribute__((aligned(16))) gt_u32x4_t all[PIECES * S];
@@ -139,7 +150,7 @@ __global__ void __launch_bounds__(128 * WM, 1) gemm_tiles_kernel(gt_args g) {
         if (L >= XI) {
             int up;
             const int c = q / (16 * NW) * (GATES ? 8 * NW : 16 * NW) + gt_row_of<NW, GATES>(q % (16 * NW), &up);
-            row = EPI == GT_SWIGLU ? c / 8 * 16 + up * 8 + c % 8 : EPI == GT_GATED ? c + up * g.up_at : c;
+            row = EPI == GT_SWIGLU ? c / 8 * 16 + up * 8 + c % 8 : HALVES ? c + up * g.up_at : c;
         }
         lane_at[i] = (int)(row * (L < XI ? g.ldx : g.ldw) * 2) + ((lane & 7) ^ ((q >> 1) & 7)) * 16;
     }
@@ -147,7 +158,7 @@ __global__ void __launch_bounds__(128 * WM, 1) gemm_tiles_kernel(gt_args g) {
         const zi_bf16 *x, *w;      // of the tile's first rows, at its first column
         int x_bytes, w_bytes, steps;
     };
-    const int last_row = EPI == GT_SWIGLU ? 2 * g.N : EPI == GT_GATED ? g.up_at + g.N : g.N;
+    const int last_row = EPI == GT_SWIGLU ? 2 * g.N : HALVES ? g.up_at + g.N : g.N;
     auto work_of = [&](int round) {
         work f{g.x, g.w, 0, 0, 64};
         const int unit = gt_unit(g, blockIdx.x, round);
@@ -280,8 +291,7 @@ __global__ void __launch_bounds__(128 * WM, 1) gemm_tiles_kernel(gt_args g) {
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const int up = n + 2 * h + 1 < NW ? n + 2 * h + 1 : 0;
-                        if (EPI == GT_SWIGLU) v[h * 4 + e] = gt_silu_mul(acc[n + 2 * h][m][e], acc[up][m][e]);
-                        else if (EPI == GT_GATED) v[h * 4 + e] = zi_activation(acc[n + 2 * h][m][e], g.act) * acc[up][m][e];
+                        if (GATES) v[h * 4 + e] = gt_gate<EPI>(acc[n + 2 * h][m][e], acc[up][m][e], g.act);
                         else v[h * 4 + e] = acc[n + h][m][e] + bias[h * 4 + e];
                     }
                 if (row < g.M && col < g.N) {
@@ -395,6 +405,7 @@ static int gt_launch(gt_args g, int epi, hipStream_t stream) {
     else if (epi == GT_F32) gemm_tiles_kernel<WM, MW, NW, GT_F32><<<grid, 128 * WM, 0, stream>>>(g);
     else if constexpr (NW % 2 == 0) {
         if (epi == GT_SWIGLU) gemm_tiles_kernel<WM, MW, NW, GT_SWIGLU><<<grid, 128 * WM, 0, stream>>>(g);
+        else if (g.act == ZI_ACT_GELU_ERF) gemm_tiles_kernel<WM, MW, NW, GT_ERF><<<grid, 128 * WM, 0, stream>>>(g);
         else gemm_tiles_kernel<WM, MW, NW, GT_GATED><<<grid, 128 * WM, 0, stream>>>(g);
     } else {
         return zi_fail("gemm_tiles: gate and up take a tile of an even number of blocks");

@@ -1018,6 +1018,52 @@ def _tiles_take(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, bias: 
             and _tiles_pay(x.shape[0], weight.shape[0], x.shape[1], kind))
 
 
+def linear_tiles_gates_pay(x: torch.Tensor, weight: torch.Tensor, inter: int) -> bool:
+    """Whether the gate/up product of more than 256 rows with ``inter`` columns each is one that the tiles' kernel takes, the activation
+    in its end, and was measured to make faster than the library's product and the activation's launch."""
+    return int(inter) % 8 == 0 and _tiles_operands(x, weight) and _tiles_pay(x.shape[0], inter, x.shape[1], TILES_GATES)
+
+
+def _gates_out(what: str, x: torch.Tensor, weight: torch.Tensor, inter: int, out: Optional[torch.Tensor]):
+    _gpu(what, x, weight, out)
+    if not linear_tiles_gates_pay(x, weight, inter):
+        raise ValueError(f"{what}: not a product of more than 256 rows that it is for")
+    M = x.shape[0]
+    if out is None:
+        out = torch.empty((M, inter), dtype=torch.bfloat16, device=x.device)
+    ldo, _ = _rows(out, f"{what} out")
+    if tuple(out.shape) != (M, inter) or out.dtype != torch.bfloat16 or ldo % 8 or out.data_ptr() % 16:
+        raise ValueError(f"{what}: out must be bfloat16 [{M}, {inter}], its rows 16-byte aligned")
+    return out, ldo
+
+
+def linear_tiles_swiglu(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """up * silu(gate) of x . weight^T in one kernel for more than 256 rows (``linear_tiles_gates_pay``), for a weight [2I, K]
+    whose rows are 8 gate rows, then the 8 up rows of the same columns, and so on; out [M, I] bfloat16."""
+    inter = weight.shape[0] // 2
+    out, ldo = _gates_out("linear_tiles_swiglu", x, weight, inter, out)
+    _lib.call("zi_gemm_tiles", _p(out), 2, _p(x), _p(weight), c_void_p(0), x.shape[0], inter, x.shape[1], x.stride(0), weight.stride(0),
+              ldo, 0, 0, 1, -1, _stream())
+    return out
+
+
+GATED_ACTIVATIONS = {"silu": 0, "gelu_tanh": 1, "gelu_erf": 2}
+
+
+def linear_tiles_gated(x: torch.Tensor, weight: torch.Tensor, inter: int, up_at: int, activation: str,
+                       out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """activation(gate) * up of x . weight^T in one kernel for more than 256 rows (``linear_tiles_gates_pay``): the first ``inter``
+    rows of the weight are the gates', those from row ``up_at`` on the ups'; out [M, inter] bfloat16."""
+    if activation not in GATED_ACTIVATIONS:
+        raise ValueError(f"linear_tiles_gated: unknown activation {activation!r}")
+    if not inter <= up_at <= weight.shape[0] - inter:
+        raise ValueError("linear_tiles_gated: the up rows must follow the gate rows within the weight")
+    out, ldo = _gates_out("linear_tiles_gated", x, weight, inter, out)
+    _lib.call("zi_gemm_tiles", _p(out), 3, _p(x), _p(weight), c_void_p(0), x.shape[0], int(inter), x.shape[1], x.stride(0),
+              weight.stride(0), ldo, int(up_at), GATED_ACTIVATIONS[activation], 1, -1, _stream())
+    return out
+
+
 LIBRARY_WORKSPACE_BYTES = 64 << 20     # what an algorithm of the library's product may use beside its operands
 _LIBRARY_WORKSPACES = {}
 

@@ -40,7 +40,7 @@ class SwiGLU(FeedForward):
 
     graph_safe = True
     tape_safe = True
-    # For many rows the gate/up product is the library's, and at some sizes it makes the transposed
+    # For many rows the gate/up product is made in tiles that end in the activation (``ops.linear_tiles_swiglu``) or the library's, and at some sizes it makes the transposed
     # result, W . x^T, faster than x . W^T (measured at the 1.5B sizes: 100 against 119 us at 2,048 rows,
     # 31 against 37 at 512, 73 against 67 at 1,024).  The transposed result goes through the activation
     # kernel that turns it back; the two ways differ by rounding.  Which one a step of n rows takes is
@@ -61,6 +61,10 @@ class SwiGLU(FeedForward):
     def _can_transpose(self, n: int) -> bool:
         return (self.interleave == GATE_UP_BLOCK and self.rt.dtype == torch.bfloat16
                 and n >= self.TRANSPOSED_MIN_ROWS and n % 8 == 0)
+
+    def _tiles(self, x: torch.Tensor) -> bool:
+        """Steps of more than 256 rows whose gate/up product is made in tiles that end in the activation."""
+        return self.interleave == GATE_UP_BLOCK and ops.linear_tiles_gates_pay(x, self.gate_up, self.inter)
 
     def _gate_up_straight(self, x: torch.Tensor, act: torch.Tensor) -> None:
         gu = self.rt.buffer("ffn_gate_up", (x.shape[0], 2 * self.inter))
@@ -96,7 +100,7 @@ class SwiGLU(FeedForward):
         x = self.rt.buffer("norm_out", (n, self.hidden))
         act = self.rt.buffer("ffn_act", (n, self.inter))
         self.rt.tune_linear(act, self.down, sums=True)
-        if self.interleave and ops.linear_swiglu_many_pays(x, self.gate_up):
+        if self.interleave and (ops.linear_swiglu_many_pays(x, self.gate_up) or self._tiles(x)):
             return
         # first the library's algorithm, then the way round with it
         if self.gate_up is not None:
@@ -146,6 +150,8 @@ class SwiGLU(FeedForward):
         elif self.interleave == GATE_UP_BLOCK and x.dtype == torch.bfloat16:
             if ops.linear_swiglu_many_pays(x, self.gate_up):
                 ops.linear_swiglu_many(x, self.gate_up, out=act)
+            elif self._tiles(x):
+                ops.linear_tiles_swiglu(x, self.gate_up, out=act)
             else:
                 self._gate_up_many_rows(x, act)
         elif not self.interleave and self.gate_up is not None and ops.linear_swiglu_halves_supported(x, self.gate_up):
@@ -219,18 +225,22 @@ class GatedMLP(FeedForward):
         return ProductRows.step_rows(rows, kind)
 
     def tune(self, num_tokens: int) -> None:
-        n = int(num_tokens)
-        self.rt.tune_linear(self.rt.buffer("norm_out", (n, self.hidden)), self.gate_up)
+        x = self.rt.buffer("norm_out", (int(num_tokens), self.hidden))
+        if not ops.linear_tiles_gates_pay(x, self.gate_up, self.inter):
+            self.rt.tune_linear(x, self.gate_up)
 
     def out_sums(self, rows: int) -> int:
         return ops.linear_out_sums(self.rt.dtype, rows, self.down)
 
     def forward(self, x: torch.Tensor, out=None) -> torch.Tensor:
         n, I = x.shape[0], self.inter
-        gu = self.rt.buffer("ffn_gate_up", (n, self.up_at + I))
-        ops.linear(x, self.gate_up, out=gu)
         act = self.rt.buffer("ffn_act", (n, I))
-        ops.gated_act(gu[:, :I], gu[:, self.up_at:], self.activation, out=act)
+        if ops.linear_tiles_gates_pay(x, self.gate_up, I):
+            ops.linear_tiles_gated(x, self.gate_up, I, self.up_at, self.activation, out=act)
+        else:
+            gu = self.rt.buffer("ffn_gate_up", (n, self.up_at + I))
+            ops.linear(x, self.gate_up, out=gu)
+            ops.gated_act(gu[:, :I], gu[:, self.up_at:], self.activation, out=act)
         if out is None:
             out = self.rt.buffer("ffn_out", (n, self.hidden))
         if out.dim() == 3:
