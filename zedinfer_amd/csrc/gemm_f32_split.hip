@@ -726,7 +726,7 @@ gemm_f32_split_tile_kernel(float* __restrict__ out, const float* __restrict__ x,
 // in tiles of 32 x 96, 68 in 64 x 128).  Chosen and next, us: 450 rows of 4,608 x 3,584 32 x 96 135, 64 x 64 159; 1,024 of 1,536 x 8,960 32 x 96 222, 64 x 128 237,
 // 32 x 64 269; 2,048 of 4,608 x 3,584 64 x 128 430, 32 x 128 496; 256 of 17,920 x 1,536 with the activation 64 x 128 121, 32 x 128 130, 80 rows of it 32 x 128 62, 32 x 64 73;
 // 512 of 2,048 x 1,536 64 x 64 28, 32 x 64 36; 256 of 1,536 x 8,960 32 x 64 92, 32 x 96 107.
-gf_kernel zi_gemm_f32_split_kernel(int M, int64_t N, int K) {
+static gf_kernel gf_choose(int M, int64_t N, int K, float* tiles_us) {      // (tiles_us: set where it is a tile)
     const int64_t cus = zi_compute_units(), n16 = (N + 15) / 16, m16 = (M + 15) / 16, m32 = (M + 31) / 32, m64 = (M + 63) / 64;
     const int chunks = (K + GF_KB - 1) / GF_KB, per = (chunks + GF_PARTS - 1) / GF_PARTS;
     if (M <= 8) return (N + 7) / 8 > cus && per <= GF_HELD_CHUNKS ? GF_HELD_PAIRS : GF_PAIRS;
@@ -752,7 +752,13 @@ gf_kernel zi_gemm_f32_split_kernel(int M, int64_t N, int K) {
     consider(GF_TILE_64_QUARTERS, shared(m64 * n64, 5.73f, 0.938f));
     consider(GF_TILE_32, rounds(m32 * n128, 3, 7.39f, 1.52f, 2.19f, 2.89f));
     consider(GF_TILE_64, rounds(m64 * n128, 2, 8.83f, 1.65f, 2.94f, 2.94f));
+    *tiles_us = us;
     return best;
+}
+
+gf_kernel zi_gemm_f32_split_kernel(int M, int64_t N, int K) {
+    float us;
+    return gf_choose(M, N, K, &us);
 }
 
 template <bool GATED>
@@ -830,4 +836,488 @@ static int gs_launch(float* out, const float* x, const float* w, const float* bi
 int zi_gemm_f32_split_launch(bool gated, float* out, const float* x, const float* w, const float* bias, int M, int N, int K, int64_t ldx,
                              int64_t ldw, int64_t ldo, hipStream_t stream) {
     return gated ? gs_launch<true>(out, x, w, nullptr, M, N, K, ldx, ldw, ldo, stream) : gs_launch<false>(out, x, w, bias, M, N, K, ldx, ldw, ldo, stream);
+}
+
+// ---- many rows ------------------------------------------------------------------------------------------------------------
+// The tiles above split x again in every workgroup of a row of tiles (140 times at 17,920 weight rows) and every weight once for 64 rows of x,
+// thirteen vector instructions for two values that the matrix cores mostly wait for.  Here x is split once, by a launch of its own
+// (gf_parts_kernel), into a workspace that holds the parts as the tiles' LDS does, and a wavefront multiplies each weight that it has split
+// with up to 128 rows.  That takes most of a SIMD's registers, so one wavefront a SIMD has to hide its own waits: parts of x go straight into
+// LDS three steps ahead, weights into registers two steps ahead, and a weight's split, 1.1 to 2.2 vector instructions a product, stands between
+// products of four different sums.  The chains, the runs and their order are the same as everywhere in this file, and so are the bits.
+
+// The parts of x times 2^24, the second chain's negative: [block of 16 rows][chunk][chain][part][a KB as LDS holds it].  Rows past M and
+// columns past K are zeros.  A wavefront a chain.
+__global__ void __launch_bounds__(4 * ZI_WAVE) gf_parts_kernel(gf_u32x4_t* __restrict__ parts, const float* __restrict__ x, int M, int K,
+                                                                     int64_t ldx, int chunks, int per) {
+    const int lane = threadIdx.x & (ZI_WAVE - 1), s = blockIdx.x * 4 + (int)(threadIdx.x / ZI_WAVE), c = s >> 1, h = s & 1;
+    if (c >= chunks) return;
+    const int q = lane >> 2, g = (lane ^ -(q >> 2)) & 3;
+    const int k = c * GF_KB + (h ^ ((c / per) & 1)) * 32 + g * 4;
+    const int64_t row = (int64_t)blockIdx.y * 16 + q;
+    gf_f32x4_t v[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) v[i] = row < M && k + 16 * i < K ? *reinterpret_cast<const gf_f32x4_t*>(x + row * ldx + k + 16 * i) : gf_f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const gf_parts p = gf_split(v[0], v[1], h ? -GF_UP : GF_UP);
+    gf_u32x4_t* to = parts + (((int64_t)blockIdx.y * chunks + c) * 2 + h) * (3 * ZI_WAVE) + lane;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) to[i * ZI_WAVE] = p.p[i].u;
+}
+
+// Loads but for the newest n have arrived, and every read of LDS.
+template <int n>
+__device__ __forceinline__ void gf_wait() {
+    static_assert(n < 64, "the counter has six bits");
+    __builtin_amdgcn_s_waitcnt((n & 15) | (7 << 4) | ((n >> 4) << 14));
+}
+
+#define GF_STAGES 4
+
+// The sums stay in the accumulation registers over the loop: without this the compiler moves all of them to other registers and back.
+#ifdef __HIP_DEVICE_COMPILE__
+#define GF_KEEP(v) asm volatile("" : "+a"(v))
+#else
+#define GF_KEEP(v)
+#endif
+
+struct gf_many_args {
+    float* out;                  // (RUNS: the sums of the runs, [8][M][N], gated [8][M][2 N], the gates' first)
+    const gf_u32x4_t* parts;
+    const float *x, *w, *bias;
+    int M, N, K;
+    int64_t ldx, ldw, ldo;
+    int chunks, per, vec_out, m_tiles, tiles, runs;     // runs: of a workgroup (RUNS), an even number
+    int up_at;                   // (gated: the up rows' place behind the gate rows)
+};
+
+// 16 MT rows of x by 128 weight rows a workgroup of four wavefronts, 32 weight rows a wavefront.  A step is one chain of a chunk, 32 k.
+// GATED as above.  RUNS: blockIdx.y takes `runs` of the eight runs of k and leaves their sums.
+template <int MT, bool GATED, bool RUNS>
+__global__ void __launch_bounds__(4 * ZI_WAVE, 1) gemm_f32_split_many_kernel(gf_many_args a) {
+    constexpr int NT = 2, WAVES = 4, TM = 16 * MT, NC = GATED ? 64 : 128, NW = NC / WAVES;
+    constexpr int LOADS = 3 * MT, PW = (LOADS + WAVES - 1) / WAVES, PIECES = LOADS * ZI_WAVE, STEP_LOADS = PW + 2 * NT;
+    static_assert(MT % 2 == 0 && GF_STAGES * PIECES >= WAVES * MT * NT * ZI_WAVE, "rows in pairs of blocks; the sums fit where x was");
+    // (spare: where loads go that nobody needs)
+    __shared__ __attribute__((aligned(16))) gf_u32x4_t all[GF_STAGES * PIECES], spare[ZI_WAVE];
+    __shared__ __attribute__((aligned(16))) gf_f32x4_t turns[WAVES][NT * 128];
+    const int per_xcd = (a.tiles + 7) / 8, tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if (tile >= a.tiles) return;
+    const int m_tile = tile % a.m_tiles, m0 = m_tile * TM, n0 = tile / a.m_tiles * NC;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / ZI_WAVE), lane = threadIdx.x & (ZI_WAVE - 1), r = lane & 15, g = lane >> 4;
+    const int M = a.M, N = a.N, K = a.K, per = a.per, chunks = a.chunks;
+    const int rows_w = N - n0 < NC ? N - n0 : NC;
+    const __amdgpu_buffer_rsrc_t wb = gf_rows(a.w + (int64_t)n0 * a.ldw, a.ldw, (GATED ? a.up_at : 0) + rows_w, K);
+    const int block_bytes = chunks * 6 * 1024, blocks = (M + 15) / 16 - m_tile * MT;
+    const char* const parts = reinterpret_cast<const char*>(a.parts) + (int64_t)m_tile * MT * block_bytes;
+    const int parts_bytes = (blocks < MT ? blocks : MT) * block_bytes;
+    int x_at[PW], w_row[NT][2];
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {
+        const int L = i * WAVES + wave;
+        x_at[i] = L < LOADS && L / 3 < blocks ? L / 3 * block_bytes + L % 3 * 1024 + lane * 16 : GF_OUT;
+    }
+    const int w_lane = (lane & 7) * 16;
+#pragma unroll
+    for (int u = 0; u < NT; ++u)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int q = wave * NW + (GATED ? 0 : u) * 16 + i * 8 + (lane >> 3);
+            w_row[u][i] = q < rows_w ? (int)((q + (GATED && (u & 1) ? a.up_at : 0)) * a.ldw * 4) + w_lane : GF_OUT;
+        }
+    gf_f32x4_t* const turn = turns[wave];
+    const int c0 = RUNS ? (int)blockIdx.y * a.runs * per : 0, end = RUNS && c0 + a.runs * per < chunks ? c0 + a.runs * per : chunks;
+    int parts_done = 0, in_part = 0;      // runs done (the first is of even number), the chunk's place in its run
+    auto fetch_w = [&](gf_f32x4_t (&to)[NT][2], int h, int c, int ahead) __attribute__((always_inline)) {      // as in the tiles above
+        const int at = c * (GF_KB * 4) + (h ^ ((parts_done + (in_part + ahead >= per)) & 1)) * 128, rest = c < end ? K * 4 - at : 0;
+#pragma unroll
+        for (int u = 0; u < NT; ++u)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) to[u][i] = gf_load<0>(wb, w_lane < rest ? w_row[u][i] : GF_OUT, at);
+    };
+    // (a step's place is in the buffer it is loaded from: the range is sure to be held against the lane's offset alone)
+    auto load_x = [&](__amdgpu_buffer_rsrc_t from, int buf, const int i) __attribute__((always_inline)) {
+        const int L = i * WAVES + wave;
+#ifdef __HIP_DEVICE_COMPILE__       // (the host's pass knows loads of this size for no target)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(from, L < LOADS ? all + buf + L * ZI_WAVE : spare, 16, x_at[i], 0, 0, 0);
+#endif
+    };
+    gf_f32x4_t acc[2][MT][NT], sum[MT][NT], first[MT][NT], wr[2][NT][2];
+    const gf_f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int u = 0; u < NT; ++u) sum[t][u] = first[t][u] = zero;
+    gf_parts ws[2][NT], xs[2][2];         // xs: of a pair of blocks, and of the next pair
+    gf_f32x4_t lines[NT][2];
+    const int read_at = r * 4 + ((g ^ -(r >> 2)) & 3), q8 = lane >> 3, c8 = lane & 7;
+    int cur = 0;      // the step's buffer
+    auto put_w = [&](const gf_f32x4_t (&from)[NT][2], const int u) __attribute__((always_inline)) {       // gf_turn in its pieces
+        turn[u * 128 + q8 * 8 + (c8 ^ (q8 >> 1))] = from[u][0];
+        turn[u * 128 + (8 + q8) * 8 + (c8 ^ (4 + (q8 >> 1)))] = from[u][1];
+    };
+    auto get_w = [&](const int u, const int i) __attribute__((always_inline)) { lines[u][i] = turn[u * 128 + r * 8 + ((4 * i + g) ^ (r >> 1))]; };
+    auto split_w = [&](gf_parts (&to)[NT], const int j) __attribute__((always_inline)) {       // two values of the eight of block j / 4
+        const int u = j / 4, i = j % 4;
+        gf_split_two(lines[u][i / 2][i % 2 * 2], lines[u][i / 2][i % 2 * 2 + 1], GF_UP, [&](int p, uint32_t v) {
+            asm volatile("" ::"v"(v));       // (here, not where it is used)
+            to[u].p[p].u[i] = v;
+        });
+    };
+    auto read_x = [&](gf_parts (&to)[2], int buf, const int t, const int i) __attribute__((always_inline)) {      // operand i of six
+        to[i / 3].p[i % 3].u = all[buf + ((t + i / 3) * 3 + i % 3) * ZI_WAVE + read_at];
+    };
+    // Chain h of chunk c: its weights' parts lie in ws[h], its x in LDS at `cur`, the first two blocks of that in xs of the step's first pair.
+    // Three groups of eight products for every two blocks of rows, two for each of four sums, and beside each group a share of the rest: the next
+    // operands of x, the next step's weights through LDS and split, the loads.  Two vector instructions a product cost nothing, a third as much as
+    // half a product (8.4, 9.0 and 12.6 ns), and left to itself the compiler puts products of one sum behind each other, so the order is given here.
+    constexpr int GROUPS = 3 * MT / 2, LAST = GROUPS - 3;
+    const char* x_next = parts + (int64_t)c0 * 6144;          // the parts of the step that is asked for next, and their buffer's bytes from there on
+    int x_left = parts_bytes - c0 * 6144;
+    auto x_step = [&]() __attribute__((always_inline)) {      // (past the last step: other rows' parts or nothing, never used)
+        const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(x_next), 0, x_left > 0 ? x_left : 0, 0x00020000);
+        x_next += 3072;
+        x_left -= 3072;
+        return xb;
+    };
+    auto step = [&](const int h, int c, const bool fresh) __attribute__((always_inline)) {
+        const int next = cur == (GF_STAGES - 1) * PIECES ? 0 : cur + PIECES;
+        static const int order[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};      // parts of w and x, gf_multiply's order
+        const __amdgpu_buffer_rsrc_t xb = x_step();
+#pragma unroll
+        for (int k = 0; k < GROUPS; ++k) {
+            const int pair = k / 3, in_pair = k % 3, now = (h * (MT / 2) + pair) & 1;
+            if (k == LAST) {
+                __builtin_amdgcn_sched_barrier(0);
+                asm volatile("" ::: "memory");
+                // the next step's x is there, all wavefronts have read this step's
+                gf_wait<2 * (PW + 2 * NT)>();
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            // (reads of LDS spread, of four wavefronts at a time it serves one in 32 cycles; none right in front of the barrier)
+            const int read_from = k < LAST ? cur : next, read_t = k < LAST ? 2 * pair + 2 : 0, reads = pair == MT / 2 - 2 ? 3 : 2;
+#pragma unroll
+            for (int i = 0; i < 6; ++i)
+                if (i / reads == in_pair) read_x(xs[now ^ 1], read_from, read_t, i);
+            if (k == 0) get_w(0, 0), get_w(0, 1);
+            if (k == 2) get_w(1, 0);
+            if (k == 3) get_w(1, 1);
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (k == (MT >= 6 ? 1 + j : 1 + j * 5 / 8)) split_w(ws[h ^ 1], j);
+            if (k == LAST + 1) put_w(wr[h], 0);
+            if (k == LAST + 2) {
+                put_w(wr[h], 1);
+                fetch_w(wr[h], h, c + 2, 2);
+            }
+#pragma unroll
+            for (int i = 0; i < PW; ++i)
+                if (k >= LAST && i % 3 == in_pair) load_x(xb, cur, i);
+#pragma unroll
+            for (int o = 2 * in_pair; o < 2 * in_pair + 2; ++o)
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+#pragma unroll
+                    for (int u = 0; u < NT; ++u)
+                        acc[h][2 * pair + q][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ws[h][u].p[order[o][0]].b, xs[now][q].p[order[o][1]].b,
+                                                                                          fresh && o == 0 ? zero : acc[h][2 * pair + q][u], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x2, MT >= 6 ? 2 : 4, 0);
+                if (i % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x300, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        cur = next;
+    };
+    fetch_w(wr[0], 0, c0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_w(wr[1], 1, c0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < GF_STAGES; ++i) {
+        const __amdgpu_buffer_rsrc_t xb = x_step();
+#pragma unroll
+        for (int k = 0; k < PW; ++k) load_x(xb, i * PIECES, k);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int u = 0; u < NT; ++u) put_w(wr[h], u);
+        if (h == 0) {
+#pragma unroll
+            for (int i = 0; i < 2 * NT; ++i) get_w(i / 2, i % 2);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) split_w(ws[0], j);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_w(wr[h], h, c0 + 1, 1);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    asm volatile("" ::: "memory");
+    gf_wait<(GF_STAGES - 1) * PW + 4 * NT>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 6; ++i) read_x(xs[0], 0, 0, i);
+    for (int c = c0; c < end;) {         // the runs
+        in_part = 0;
+        step(0, c, true);
+        step(1, c, true);
+        ++c;
+        for (in_part = 1; in_part < per && c < end; ++in_part, ++c) {
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+                for (int u = 0; u < NT; ++u) {
+                    GF_KEEP(acc[0][t][u]);
+                    GF_KEEP(acc[1][t][u]);
+                }
+            step(0, c, false);
+            step(1, c, false);
+        }
+        if (!RUNS && parts_done == GF_PARTS / 2) {
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+                for (int u = 0; u < NT; ++u) {
+                    first[t][u] = sum[t][u];
+                    sum[t][u] = zero;
+                }
+        }
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int u = 0; u < NT; ++u) {
+                const gf_f32x4_t run = acc[0][t][u] - acc[1][t][u];
+                if (RUNS) {
+                    const int m = m0 + t * 16 + r, n = n0 + wave * NW + (GATED ? 0 : u) * 16 + g * 4;      // (N a multiple of four)
+                    if (m < M && n < N)
+                        *reinterpret_cast<gf_f32x4_t*>(a.out + ((int64_t)(blockIdx.y * a.runs + parts_done) * M + m) * (GATED ? 2 * N : N) + (GATED && (u & 1) ? N : 0) + n) = run;
+                } else {
+                    sum[t][u] += run;
+                }
+            }
+        ++parts_done;
+    }
+    gf_wait<0>();       // (no load may arrive after the workgroup's LDS is another's)
+    if (RUNS) return;
+    // (through this thread's own places in LDS, where x was, so that what checks and stores them is there once)
+    gf_f32x4_t* const mine = reinterpret_cast<gf_f32x4_t*>(all) + wave * MT * NT * ZI_WAVE + lane;
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int u = 0; u < NT; ++u) mine[(t * NT + u) * ZI_WAVE] = parts_done > GF_PARTS / 2 ? first[t][u] + sum[t][u] : sum[t][u];
+    constexpr int STEP = GATED ? 2 : 1;
+    uint64_t nan_rows[2] = {0, 0};       // of the tile's first and last 64 rows
+#pragma unroll 1
+    for (int b = 0; b < MT * NT; b += STEP) {
+        const int t = b / NT, m = m0 + t * 16 + r, n = n0 + wave * NW + (GATED ? 0 : b % NT) * 16 + g * 4, m64 = t / 4 * 64;
+        gf_f32x4_t s[STEP];
+#pragma unroll
+        for (int i = 0; i < STEP; ++i) {
+            s[i] = mine[(b + i) * ZI_WAVE];
+            uint64_t nans = t < 4 ? nan_rows[0] : nan_rows[1];
+            gf_finite(s[i], t % 4 * 16 + r, [&](int e) { return m < M && n + e < N; }, [&](int e) { return n + e + (i ? a.up_at : 0); }, a.x + (int64_t)(m0 + m64) * a.ldx,
+                      a.ldx, a.w, a.ldw, K, nans);
+            if (t < 4) nan_rows[0] = nans;
+            else nan_rows[1] = nans;
+        }
+        if (m < M && n < N) {
+            if (GATED) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[0][e] = gf_gate(s[0][e], s[GATED][e]);
+            }
+            gf_store4(a.out + (int64_t)m * a.ldo, GATED ? nullptr : a.bias, s[0], n, N, a.vec_out);
+        }
+    }
+}
+
+// The runs' sums added in the order of this file: a wavefront 256 outputs of a row.
+template <bool GATED>
+__global__ void __launch_bounds__(4 * ZI_WAVE) gf_add_runs_kernel(const float* __restrict__ sums, gf_many_args a, int runs) {
+    const int m = blockIdx.y, n = (blockIdx.x * 4 * ZI_WAVE + threadIdx.x) * 4;
+    const int64_t row = GATED ? 2 * a.N : a.N;
+    const float* const x = a.x + m * a.ldx;
+    gf_f32x4_t s[GATED ? 2 : 1];
+    uint64_t nan_rows = 0;
+#pragma unroll
+    for (int i = 0; i < (GATED ? 2 : 1); ++i) {
+        const float* at = sums + m * row + i * a.N + (n < a.N ? n : 0);
+        gf_f32x4_t v[GF_PARTS];
+#pragma unroll
+        for (int p = 0; p < GF_PARTS; ++p) v[p] = p < runs ? *reinterpret_cast<const gf_f32x4_t*>(at + p * a.M * row) : gf_f32x4_t{0.f, 0.f, 0.f, 0.f};
+        s[i] = v[0];
+        gf_f32x4_t s2 = v[GF_PARTS / 2];
+#pragma unroll
+        for (int p = 1; p < GF_PARTS / 2; ++p) {
+            s[i] += v[p];
+            s2 += v[GF_PARTS / 2 + p];
+        }
+        s[i] += s2;
+        gf_finite(s[i], 0, [&](int) { return n < a.N; }, [&](int e) { return n + e + (i ? a.up_at : 0); }, x, a.ldx, a.w, a.ldw, a.K, nan_rows);
+    }
+    if (n >= a.N) return;
+    if (GATED) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[0][e] = gf_gate(s[0][e], s[GATED][e]);
+    }
+    gf_store4(a.out + m * a.ldo, GATED ? nullptr : a.bias, s[0], n, a.N, a.vec_out);
+}
+
+// Rows of x that are split at a time: their parts and the runs' sums are the workspace, and a tile's parts lie within 2^31 bytes.
+#define GF_MANY_BYTES (256ll << 20)
+#define GF_MANY_LONGEST 65536
+
+// Columns up to `whole` by workgroups that take all of k, in tiles of 16 mt rows; the others by workgroups that take `runs` of its eight runs.
+struct gf_many_plan {
+    int mt, whole, rest_mt, runs;      // (mt 0: columns that are all of the other kind; both 0: not by these kernels)
+    int64_t rows;                      // of x at a time
+    float us;
+};
+
+// us: a start, rounds of workgroups (two a unit at a time where they have the registers) with a time for a step, more of it where all
+// units work, and for the end of a run, and the results' way (a million of them; `runs` < 8: to memory, back, and out).  A fit to 12,000 timed
+// launches, all tiles and cuts of 4,900 products of 33 to 3,000 rows, 512 to 38,000 weight rows, k to 19,000: off by 2 to 6 % in the mean.
+static float gf_many_us(int64_t M, int64_t weight_rows, int chunks, int mt, int runs) {
+    static const struct {
+        float start, step, full, run, out;
+    } fit[2][3] = {{{12.5f, 0.612f, 0.156f, 0.188f, 2.7f}, {13.4f, 0.796f, 0.192f, 0.434f, 1.9f}, {13.3f, 0.914f, 0.213f, 0.585f, 1.8f}},
+                   {{12.2f, 0.511f, 0.809f, 0.62f, 8.6f}, {12.7f, 0.795f, 0.158f, 0.75f, 9.0f}, {12.3f, 0.907f, 0.192f, 1.1f, 9.0f}}};
+    const bool whole = runs == GF_PARTS;
+    const auto& f = fit[!whole][mt / 2 - 2];
+    const int per = (chunks + GF_PARTS - 1) / GF_PARTS, steps = 2 * (runs * per > chunks ? chunks : runs * per);
+    const int64_t places = (!whole && mt == 4 ? 2 : 1) * zi_compute_units();
+    const int64_t units = (M + 16 * mt - 1) / (16 * mt) * ((weight_rows + 127) / 128) * (GF_PARTS / runs), rounds = (units + places - 1) / places;
+    return f.start + (float)rounds * (steps * (f.step + f.full * units / (rounds * places)) + runs * f.run) + f.out * 1e-6f * M * weight_rows;
+}
+
+static bool gf_many_fits(gf_many_plan* p, int M, int N, int K, bool gated) {
+    const int chunks = (K + GF_KB - 1) / GF_KB;
+    if ((p->whole < N && (N % 4 || p->whole % 4 || (p->runs != 4 && p->runs != 2))) || p->whole < 0 || p->whole > N) return false;
+    const int64_t most = GF_MANY_BYTES / ((int64_t)chunks * 384) / 384 * 384, passes = (M + most - 1) / most;      // (whole tiles of every kind)
+    p->rows = passes == 1 ? M : (M + passes * 384 - 1) / (passes * 384) * 384;
+    return (p->rows + 63) / 64 * ((N + 63) / 64) < (1 << 23);
+}
+
+// All columns in one cut, or whole rounds of the chip in the first and what would leave most of it idle in the second.
+static gf_many_plan gf_many_best(int M, int N, int K, bool gated) {
+    gf_many_plan best{0, 0, 0, 0, 0, 0.f};
+    const int chunks = (K + GF_KB - 1) / GF_KB, nc = gated ? 64 : 128, twice = gated ? 2 : 1, cus = zi_compute_units();
+    auto consider = [&](gf_many_plan p) {
+        if (gf_many_fits(&p, M, N, K, gated) && (!best.us || p.us < best.us)) best = p;
+    };
+    gf_many_plan all{0, N, 0, 0, 0, 0.f};
+    gf_many_fits(&all, M, N, K, gated);
+    const int64_t rows = all.rows, passes = (M + rows - 1) / rows;
+    const float split = 1e-6f * rows * K;
+    for (int mt = 4; mt <= 8; mt += 2) {
+        const int64_t m_tiles = (rows + 16 * mt - 1) / (16 * mt), col_tiles = (N + nc - 1) / nc;
+        consider({mt, N, 0, 0, 0, passes * (split + gf_many_us(rows, (int64_t)N * twice, chunks, mt, GF_PARTS))});
+        for (int runs = 2; runs < GF_PARTS; runs *= 2) consider({0, 0, mt, runs, 0, passes * (split + gf_many_us(rows, (int64_t)N * twice, chunks, mt, runs))});
+        const int64_t full = m_tiles * col_tiles / cus * cus / m_tiles;      // tiles of columns in whole rounds
+        if (full == 0 || full >= col_tiles) continue;
+        const int whole = (int)full * nc;
+        const float us = split + gf_many_us(rows, (int64_t)whole * twice, chunks, mt, GF_PARTS);
+        for (int rest = 4; rest <= 8; rest += 2)
+            for (int runs = 2; runs < GF_PARTS; runs *= 2)
+                consider({mt, whole, rest, runs, 0, passes * (us + gf_many_us(rows, (int64_t)(N - whole) * twice, chunks, rest, runs) - 4.f)});      // (the split is launched once)
+    }
+    return best;
+}
+
+static gf_many_plan gf_many_as_told(int M, int N, int K, bool gated, int mt, int runs, int whole) {
+    gf_many_plan p{mt, runs == GF_PARTS ? N : whole, mt, runs, 0, 0.f};
+    if ((mt != 4 && mt != 6 && mt != 8) || !gf_many_fits(&p, M, N, K, gated)) p.mt = p.rest_mt = 0;
+    return p;
+}
+
+static int64_t gf_many_bytes(const gf_many_plan& p, int64_t N, int chunks, bool gated) {
+    return (p.rows + 15) / 16 * chunks * 6144 + GF_PARTS * p.rows * (N - p.whole) * (gated ? 8 : 4);
+}
+
+// Whether these kernels can make the product: operands that the others here take, in tiles that a launch can hold.
+static bool gf_many_sizes(int M, int N, int K, int64_t ldx, int64_t ldw, int gated) {
+    return M > 0 && N > 0 && K > GF_SPLIT_ABOVE && K <= GF_MANY_LONGEST && ldx >= K && ldw >= K && (int64_t)M * N < (1ll << 36) &&
+           (gated ? zi_gemm_f32_swiglu_takes(nullptr, nullptr, M, N, K, ldx, ldw) : zi_gemm_f32_takes(nullptr, nullptr, N, K, ldx, ldw));
+}
+
+// Bytes of workspace with which zi_gemm_f32_many makes the product of M rows of x and N (gated: 2 N) weight rows, mt, runs and whole as
+// there; 0 where it does not, or (mt 0) where it is not the faster way by both fits: of 5,000 products of 33 to 3,000 rows and sizes as above 3,500
+// were given to these kernels and took 0.78 of the time in the mean, eleven of them more than 1.03 of it and 1.11 at worst.
+// us, without and with the workspace, the split included, weights from memory: 17,920 x 1,536 with the activation at 256 / 512 / 2,048 rows 129 and 98,
+// 200 and 170, 775 and 640; 1,536 x 8,960 89 and 67, 114 and 101, 457 and 331; 37,888 x 3,584 with it 465 and 375, 881 and 700, 3,447 and 2,827;
+// 3,584 x 18,944 289 and 195, 531 and 376, 1,830 and 1,420.  Left to the others: few tiles or short runs, 2,048 x 1,536 at 450 rows 30 and 35, and some
+// 60 rows and fewer (two more launches).
+extern "C" int64_t zi_gemm_f32_many_workspace(int M, int N, int K, int64_t ldx, int64_t ldw, int gated, int mt, int runs, int whole) {
+    if (!gf_many_sizes(M, N, K, ldx, ldw, gated)) return 0;
+    const gf_many_plan p = mt ? gf_many_as_told(M, N, K, gated, mt, runs, whole) : gf_many_best(M, N, K, gated);
+    if (!p.mt && !p.rest_mt) return 0;
+    float tiles_us = 0.f;      // of the tiles without a workspace; 0 where other kernels make the product
+    gf_choose(M, (int64_t)N * (gated ? 2 : 1), K, &tiles_us);
+    tiles_us *= M > 512 ? 1.05f : 0.98f;      // (their fit is low, by 10 to 16 % with a standard deviation of 8 to 12 up to 512 rows, by 15 to 18 with one of 7 beyond)
+    return mt || p.us < tiles_us ? gf_many_bytes(p, N, (K + GF_KB - 1) / GF_KB, gated) : 0;
+}
+
+template <int MT, bool GATED>
+static void gf_many_launch(gf_many_args a, int runs, float* sums, hipStream_t stream) {
+    constexpr int TM = 16 * MT, NC = GATED ? 64 : 128;
+    a.m_tiles = (a.M + TM - 1) / TM;
+    a.tiles = a.m_tiles * ((a.N + NC - 1) / NC);
+    const int grid = (a.tiles + 7) / 8 * 8;
+    if (runs == GF_PARTS) {
+        gemm_f32_split_many_kernel<MT, GATED, false><<<grid, 4 * ZI_WAVE, 0, stream>>>(a);
+    } else {
+        gf_many_args b = a;
+        b.out = sums;
+        b.runs = runs;
+        gemm_f32_split_many_kernel<MT, GATED, true><<<dim3(grid, GF_PARTS / runs), 4 * ZI_WAVE, 0, stream>>>(b);
+        gf_add_runs_kernel<GATED><<<dim3((a.N + 1023) / 1024, a.M), 4 * ZI_WAVE, 0, stream>>>(sums, a, (a.chunks + a.per - 1) / a.per);
+    }
+}
+
+// out[M,N] = x . w^T + bias, or (gated) up * silu(gate) of the first and the last N rows of w, through a workspace of
+// zi_gemm_f32_many_workspace bytes; the bits of the kernels without one.  mt 0: as these sizes are made fastest; else blocks of 16 rows of x a
+// tile (4, 6, 8), runs of k a workgroup of the columns from `whole` on (4 or 2, N and whole multiples of four), or 8: all columns whole.
+extern "C" int zi_gemm_f32_many(float* out, const float* x, const float* w, const float* bias, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo,
+                                int gated, int mt, int runs, int whole, void* workspace, int64_t bytes, hipStream_t stream) {
+    ZI_REQUIRE(out && x && w && workspace, "gemm_f32_many: null operand");
+    ZI_REQUIRE(gf_many_sizes(M, N, K, ldx, ldw, gated) && ldo >= N && ((uintptr_t)x | (uintptr_t)w | (uintptr_t)workspace) % 16 == 0 && !(gated && bias),
+               "gemm_f32_many: M=%d N=%d K=%d is not taken, or not with these strides, alignment or bias", M, N, K);
+    const gf_many_plan p = mt ? gf_many_as_told(M, N, K, gated, mt, runs, whole) : gf_many_best(M, N, K, gated);
+    const int chunks = (K + GF_KB - 1) / GF_KB, per = (chunks + GF_PARTS - 1) / GF_PARTS;
+    ZI_REQUIRE(p.mt || p.rest_mt, "gemm_f32_many: no tiles of %d blocks with %d runs from column %d on", mt, runs, whole);
+    ZI_REQUIRE(bytes >= gf_many_bytes(p, N, chunks, gated), "gemm_f32_many: the workspace is too small");
+    for (int64_t m = 0; m < M; m += p.rows) {
+        const int rows = (int)(M - m < p.rows ? M - m : p.rows), blocks = (rows + 15) / 16;
+        gf_many_args a{out + m * ldo, (const gf_u32x4_t*)workspace, x + m * ldx, w, bias, rows, p.whole, K, ldx, ldw, ldo, chunks, per,
+                       ldo % 4 == 0 && (uintptr_t)out % 16 == 0, 0, 0, 0, N};
+        float* const sums = (float*)((char*)workspace + (int64_t)blocks * chunks * 6144);
+        gf_parts_kernel<<<dim3((2 * chunks + 3) / 4, blocks), 4 * ZI_WAVE, 0, stream>>>((gf_u32x4_t*)workspace, a.x, rows, K, ldx, chunks, per);
+        auto go = [&](int blocks_of_rows, int runs_a_group) {
+#define GF_GO(MT)                                                                  \
+    if (blocks_of_rows == MT) {                                                    \
+        if (gated) gf_many_launch<MT, true>(a, runs_a_group, sums, stream);        \
+        else gf_many_launch<MT, false>(a, runs_a_group, sums, stream);             \
+    }
+            GF_GO(4) GF_GO(6) GF_GO(8)
+#undef GF_GO
+        };
+        if (p.whole > 0) go(p.mt, GF_PARTS);
+        if (p.whole < N) {
+            a.N = N - p.whole;
+            a.out += p.whole;
+            a.w += p.whole * ldw;
+            if (bias) a.bias += p.whole;
+            go(p.rest_mt, p.runs);
+        }
+    }
+    return zi_check_launch("gemm_f32_many");
 }

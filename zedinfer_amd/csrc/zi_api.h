@@ -104,6 +104,9 @@ int zi_gemm_generic(void* out, int out_dt, const void* x, int x_dt, const void* 
 // gemm_f32.hip
 int zi_gemm_f32_swiglu(float* out, const float* x, const float* w, int M, int inter, int K, int64_t ldx, int64_t ldw,
     int64_t ldo, hipStream_t stream);
+// gemm_f32_split.hip
+int zi_gemm_f32_many(float* out, const float* x, const float* w, const float* bias, int M, int N, int K, int64_t ldx,
+    int64_t ldw, int64_t ldo, int gated, int mt, int runs, int whole, void* workspace, int64_t bytes, hipStream_t stream);
 // gemm_lt.hip
 int zi_gemm_lt(void* out, int out_dt, const void* x, const void* weight, const void* bias, int transposed, int64_t M,
     int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldo, void* workspace, int64_t workspace_bytes, hipStream_t
@@ -424,6 +427,7 @@ int zi_sample(int32_t* out, const float* logits, int64_t ld, float* work, int ro
     X(zi_swiglu) \
     X(zi_gemm_generic) \
     X(zi_gemm_f32_swiglu) \
+    X(zi_gemm_f32_many) \
     X(zi_gemm_lt) \
     X(zi_gemm_tiles) \
     X(zi_gemm_skinny) \

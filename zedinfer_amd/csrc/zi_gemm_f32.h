@@ -25,6 +25,8 @@ typedef __attribute__((ext_vector_type(8))) __bf16 gf_bf16x8_t;
 enum gf_kernel { GF_PAIRS, GF_ROWS16, GF_ROWS32, GF_HELD_PAIRS, GF_HELD_ROWS16, GF_TILE_64, GF_TILE_32, GF_TILE_32_HALVES, GF_TILE_96_HALVES, GF_TILE_64_QUARTERS };
 
 gf_kernel zi_gemm_f32_split_kernel(int M, int64_t N, int K);
+bool zi_gemm_f32_takes(const void* x, const void* w, int N, int K, int64_t ldx, int64_t ldw);
+extern "C" int zi_gemm_f32_swiglu_takes(const void* x, const void* w, int M, int inter, int K, int64_t ldx, int64_t ldw);
 int zi_gemm_f32_split_launch(bool gated, float* out, const float* x, const float* w, const float* bias, int M, int N, int K, int64_t ldx,
                              int64_t ldw, int64_t ldo, hipStream_t stream);
 

@@ -65,6 +65,8 @@ _PROTOTYPES = {
     "zi_gemm_generic": [P, I, P, I, P, I, P, I, I, I, I, L, L, L, P],
     "zi_gemm_f32_swiglu": [P, P, P, I, I, I, L, L, L, P],
     "zi_gemm_f32_kernel": [I, I, I],
+    "zi_gemm_f32_many": [P, P, P, P, I, I, I, L, L, L, I, I, I, I, P, L, P],
+    "zi_gemm_f32_many_workspace": [I, I, I, L, L, I, I, I, I],
     "zi_gemm_f32_swiglu_takes": [P, P, I, I, I, L, L],
     "zi_gemm_skinny": [P, I, I, P, P, P, I, I, I, L, L, L, P, L, P],
     "zi_gemm_skinny_act": [P, I, I, P, P, P, I, I, I, L, L, L, P, L, F, P],
@@ -209,6 +211,7 @@ def load() -> ctypes.CDLL:
             fn.restype = c_int
         lib.zi_gemm_skinny_workspace.argtypes = [I, I, I]
         lib.zi_gemm_skinny_workspace.restype = c_int64
+        lib.zi_gemm_f32_many_workspace.restype = c_int64
         lib.zi_delta_rule_workspace.argtypes = [I, I, I, I, I]
         lib.zi_delta_rule_workspace.restype = c_int64
         lib.zi_attention_decode_workspace.argtypes = [I, I, I]

@@ -918,7 +918,8 @@ def attention_prefill(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tenso
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
-           out: Optional[torch.Tensor] = None, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
+           out: Optional[torch.Tensor] = None, out_dtype: Optional[torch.dtype] = None,
+           workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out[M,N] = x[M,K] . weight[N,K]^T + bias[N], accumulated in float32
     (reference: src/backend/ops/linear/op.cpp:57-58).
 
@@ -930,7 +931,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     six products of the operands' three bfloat16 parts each, which hold all their bits, summed in float32 (the three products
     left out reach 2^-25, 2^-25 and 2^-34 of a single one; sums are no further from 64 bits than the float32 instruction's but
     where few products make them, 3.4e-8 against 2.5e-8 for one, or half of every 64 columns is empty, up to 1.04e-7 against
-    7.7e-8); either way one order of the sums whatever the number of rows; every other pairing, and float32 rows that are no whole 16-byte pieces, to the plain FMA kernel."""
+    7.7e-8); either way one order of the sums whatever the number of rows, and the same bits with a ``workspace`` of
+    ``linear_many_workspace`` bytes, in which x of many rows is split once; every other pairing, and float32 rows that are no whole 16-byte pieces, to the plain FMA kernel."""
     _gpu("linear", x, weight, bias, out)
     ldx, K = _rows(x, "linear x")
     ldw, Kw = _rows(weight, "linear weight")
@@ -945,6 +947,9 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     if tuple(out.shape) != (M, N):
         raise ValueError(f"linear: out must be [{M}, {N}], got {tuple(out.shape)}")
     if M == 0:
+        return out
+    if workspace is not None and out.dtype == torch.float32 and (bias is None or bias.dtype == torch.float32) \
+            and _linear_many("linear", x, weight, bias, out, N, False, workspace):
         return out
     bf = torch.bfloat16
     all_bf = x.dtype == bf and weight.dtype == bf and (bias is None or bias.dtype == bf)
@@ -1259,9 +1264,35 @@ def linear_swiglu_halves_supported(x: torch.Tensor, weight: torch.Tensor) -> boo
     return bool(_lib.load().zi_gemm_f32_swiglu_takes(_p(x), _p(weight), M, weight.shape[0] // 2, K, x.stride(0), weight.stride(0)))
 
 
-def linear_swiglu_halves(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+def linear_many_workspace(x: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> int:
+    """Bytes of workspace with which ``linear`` (``gated``: ``linear_swiglu_halves``) makes this product faster than without: float32
+    products of many rows and more than 1,408 columns, whose x is split into its parts once, in the workspace; 0 for all others."""
+    if not all(t.is_cuda and t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1 and t.data_ptr() % 16 == 0 for t in (x, weight)):
+        return 0
+    M, K = x.shape
+    if K != weight.shape[1] or max(M, K, weight.shape[0]) >= 1 << 31 or min(M, K, weight.shape[0]) < 1 or (gated and weight.shape[0] % 2):
+        return 0
+    return int(_lib.load().zi_gemm_f32_many_workspace(M, weight.shape[0] // (2 if gated else 1), K, x.stride(0), weight.stride(0), int(gated), 0, 0, 0))
+
+
+def _linear_many(who: str, x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor, N: int, gated: bool,
+                 workspace: torch.Tensor) -> bool:
+    """The product through ``workspace``, which no other call may use until this one's kernels are done; False where it is not made so."""
+    need = linear_many_workspace(x, weight, gated)
+    if not need:
+        return False
+    have = workspace.numel() * workspace.element_size()
+    if workspace.device != x.device or not workspace.is_contiguous() or workspace.data_ptr() % 16 or have < need:
+        raise ValueError(f"{who}: the workspace must be {need} contiguous bytes on {x.device}, 16-byte aligned")
+    _lib.call("zi_gemm_f32_many", _p(out), _p(x), _p(weight), _p(bias), x.shape[0], N, x.shape[1], x.stride(0), weight.stride(0), out.stride(0),
+              int(gated), 0, 0, 0, _p(workspace), have, _stream())
+    return True
+
+
+def linear_swiglu_halves(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None,
+                         workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     """up * silu(gate) of x . weight^T in one kernel, float32, for a weight [2I, K] of I gate rows and the I up rows; out [M, I].
-    The bits of ``linear`` and ``swiglu`` one after the other."""
+    The bits of ``linear`` and ``swiglu`` one after the other, with a ``workspace`` of ``linear_many_workspace`` bytes too."""
     _gpu("linear_swiglu_halves", x, weight, out)
     if not linear_swiglu_halves_supported(x, weight):
         raise ValueError("linear_swiglu_halves: float32 matrices with rows of whole 16-byte pieces are needed")
@@ -1272,6 +1303,8 @@ def linear_swiglu_halves(x: torch.Tensor, weight: torch.Tensor, out: Optional[to
     ldo, wo = _rows(out, "linear_swiglu_halves out")
     if tuple(out.shape) != (M, inter) or out.dtype != torch.float32:
         raise ValueError(f"linear_swiglu_halves: out must be float32 [{M}, {inter}]")
+    if workspace is not None and _linear_many("linear_swiglu_halves", x, weight, None, out, inter, True, workspace):
+        return out
     _lib.call("zi_gemm_f32_swiglu", _p(out), _p(x), _p(weight), M, inter, K, x.stride(0), weight.stride(0), ldo, _stream())
     return out
 

@@ -88,6 +88,12 @@ class Runtime:
         view = self._views[vkey] = buf[:n].view(tuple(shape))
         return view
 
+    def product_workspace(self, name: str, x: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> Optional[torch.Tensor]:
+        """What ``ops.linear`` (``gated``: ``ops.linear_swiglu_halves``) is to be given as its workspace for this product, or None."""
+        from .. import ops
+        need = ops.linear_many_workspace(x, weight, gated)
+        return self.buffer(name, (need,), torch.uint8) if need else None
+
     def poison(self) -> None:
         """Make every floating-point workspace NaN (a check that a replay writes all it reads; integer workspaces
         may hold indices and are left alone)."""
