@@ -508,9 +508,12 @@ moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restr
 
 // The tiles of 128 rows x 256 columns where k is whole steps: the same loads, places in LDS and sums as the kernel above, but a step is two
 // halves, and while the products of one run, the operands of the next are read from LDS and a share of a later step's loads is issued; the step's
-// one barrier stands between the halves.  Above, a step's reads, products and loads follow each other and only the second wavefront of a SIMD
-// stands beside them: 1.5 us a step where this takes @@STEP@@.  (Past the last step that one is loaded again, so that every step waits alike.)
-// Measured with 32 experts of 1,536 x 1,536, 8,000 pairs, the first product and the second: @@US@@.
+// one barrier stands between the halves.  Above, a step's loads, reads and products follow each other and only the second wavefront of a SIMD
+// stands beside them.  (Past the last step that one is loaded again, so that every step waits alike.)  Bound by the weights' way from memory
+// where an expert has few tiles, by LDS otherwise (its reads and loads are 1,280 cycles of a step, the products 1,024).
+// us, the kernel above and this one, the first product and the second, everything from memory and the launch's 15 us included: 32 experts of
+// 1,536 x 1,536, 8,000 pairs 101 and 101 to 97 and 97, 9,200 118 and 110 to 109 and 103, 16,384 159 and 163 to 145 and 151; of 2,560 x 3,584,
+// 8,192 pairs 342 and 324 to 315 and 303; 8 of 4,096 x 14,336, 2,000 pairs 538 and 539 to 515 and 491.  Taken for every k of whole steps from three on.
 template <typename TO>
 __global__ void __launch_bounds__(8 * ZI_WAVE, 1)
 moe_linear_halves_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restrict__ x, int64_t ldx, const zi_bf16* __restrict__ w,
