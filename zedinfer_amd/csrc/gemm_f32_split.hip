@@ -1172,7 +1172,8 @@ __global__ void __launch_bounds__(4 * ZI_WAVE) gf_add_runs_kernel(const float* _
     gf_store4(a.out + m * a.ldo, GATED ? nullptr : a.bias, s[0], n, a.N, a.vec_out);
 }
 
-// Rows of x that are split at a time: their parts and the runs' sums are the workspace, and a tile's parts lie within 2^31 bytes.
+// What the parts of the rows of x that are split at a time may take, and half of what the runs' sums may: the workspace is both.  A tile's parts lie
+// within 2^31 bytes for every k up to the longest.
 #define GF_MANY_BYTES (256ll << 20)
 #define GF_MANY_LONGEST 65536
 
@@ -1204,7 +1205,7 @@ static bool gf_many_fits(gf_many_plan* p, int M, int N, int K, bool gated) {
     if ((p->whole < N && (N % 4 || p->whole % 4 || (p->runs != 4 && p->runs != 2))) || p->whole < 0 || p->whole > N) return false;
     const int64_t most = GF_MANY_BYTES / ((int64_t)chunks * 384) / 384 * 384, passes = (M + most - 1) / most;      // (whole tiles of every kind)
     p->rows = passes == 1 ? M : (M + passes * 384 - 1) / (passes * 384) * 384;
-    return (p->rows + 63) / 64 * ((N + 63) / 64) < (1 << 23);
+    return (p->rows + 63) / 64 * ((N + 63) / 64) < (1 << 23) && GF_PARTS * p->rows * (N - p->whole) * (gated ? 8 : 4) <= 2 * GF_MANY_BYTES;
 }
 
 // All columns in one cut, or whole rounds of the chip in the first and what would leave most of it idle in the second.
