@@ -1,0 +1,35 @@
+"""Which products of many rows ``ops.linear`` gives to the tiles' kernel, with the launches recorded instead of made: on the CPU."""
+import pytest
+import torch
+
+from zedinfer_amd import ops
+from zedinfer_amd.ops import functional
+
+
+@pytest.fixture
+def launches(monkeypatch):
+    """Names of the library's launches, none of which is made."""
+    calls = []
+    monkeypatch.setattr(functional, "_gpu", lambda *a: None)
+    monkeypatch.setattr(functional, "_stream", lambda: None)
+    monkeypatch.setattr(functional._lib, "call", lambda name, *a: calls.append(name))
+    return calls
+
+
+def operands(M, N, K):
+    return torch.zeros(M, K, dtype=torch.bfloat16), torch.zeros(N, K, dtype=torch.bfloat16)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float64, torch.int32, torch.int16, torch.int8, torch.uint8, torch.bool])
+def test_a_result_of_another_type_is_refused(dtype, launches):
+    """257 rows at sizes that the tiles take: a type that they do not store raises, as for fewer rows, and nothing is launched."""
+    x, w = operands(257, 1536, 1536)
+    ops.linear(x, w)
+    ops.linear(x, w, out_dtype=torch.float32)
+    assert launches == ["zi_gemm_tiles"] * 2
+    launches.clear()
+    for call in (lambda: ops.linear(x, w, out_dtype=dtype), lambda: ops.linear(x, w, out=torch.zeros(257, 1536, dtype=dtype)),
+                 lambda: ops.linear(x[:256], w, out_dtype=dtype), lambda: ops.linear_tune(x, w, out_dtype=dtype)):
+        with pytest.raises(TypeError):
+            call()
+    assert not launches

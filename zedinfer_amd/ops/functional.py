@@ -954,7 +954,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     bf = torch.bfloat16
     all_bf = x.dtype == bf and weight.dtype == bf and (bias is None or bias.dtype == bf)
     if all_bf and _tiles_take(x, weight, out, bias, TILES_PLAIN):
-        _lib.call("zi_gemm_tiles", _p(out), int(out.dtype == torch.float32), _p(x), _p(weight), _p(bias), M, N, K, ldx, ldw, ldo,
+        _lib.call("zi_gemm_tiles", _p(out), TILES_EPILOGUE[out.dtype], _p(x), _p(weight), _p(bias), M, N, K, ldx, ldw, ldo,
                   0, 0, 1, -1, _stream())
         return out
     if all_bf and out.dtype == torch.float32 and M > SKINNY_MAX_ROWS and bias is None and _library_ok(x, weight, out):
@@ -1000,6 +1000,7 @@ def linear_transposed(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch
 
 TILES_PLAIN, TILES_GATES, TILES_SUMS = 0, 1, 2      # what of a product ``zi_gemm_tiles_pays`` is asked about
 TILES_ABOVE = 256                                    # rows up to which it says no
+TILES_EPILOGUE = {torch.bfloat16: 0, torch.float32: 1}      # the types that a whole product can be stored as, and the ends of the kernel that do
 
 
 def _tiles_operands(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -1018,7 +1019,7 @@ def _tiles_pay(M: int, N: int, K: int, kind: int) -> bool:
 def _tiles_take(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, bias: Optional[torch.Tensor], kind: int) -> bool:
     """Whether ``linear`` gives the product to the tiles' kernel: operands and a result it can load and store, and sizes at which it
     was measured to be faster than the library's product."""
-    return (_tiles_operands(x, weight) and out.stride(1) == 1 and out.data_ptr() % 16 == 0
+    return (_tiles_operands(x, weight) and out.dtype in TILES_EPILOGUE and out.stride(1) == 1 and out.data_ptr() % 16 == 0
             and out.stride(0) % (4 if out.dtype == torch.float32 else 8) == 0 and (bias is None or bias.dtype == torch.bfloat16)
             and _tiles_pay(x.shape[0], weight.shape[0], x.shape[1], kind))
 
