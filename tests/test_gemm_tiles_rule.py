@@ -33,3 +33,13 @@ def test_a_result_of_another_type_is_refused(dtype, launches):
         with pytest.raises(TypeError):
             call()
     assert not launches
+
+
+def test_gate_and_up_rows_that_are_no_whole_blocks_are_refused(launches):
+    """8 gate rows, then 8 up rows, and so on: a weight with a row more has no place for it."""
+    x, w = operands(2048, 2 * 8960 + 1, 1536)
+    ops.linear_tiles_swiglu(x, w[:-1])
+    assert launches == ["zi_gemm_tiles"]
+    with pytest.raises(ValueError):
+        ops.linear_tiles_swiglu(x, w)
+    assert launches == ["zi_gemm_tiles"]

@@ -1046,6 +1046,8 @@ def _gates_out(what: str, x: torch.Tensor, weight: torch.Tensor, inter: int, out
 def linear_tiles_swiglu(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """up * silu(gate) of x . weight^T in one kernel for more than 256 rows (``linear_tiles_gates_pay``), for a weight [2I, K]
     whose rows are 8 gate rows, then the 8 up rows of the same columns, and so on; out [M, I] bfloat16."""
+    if weight.dim() != 2 or weight.shape[0] % 16:
+        raise ValueError("linear_tiles_swiglu: the weight's rows must be whole blocks of 8 gate and 8 up rows")
     inter = weight.shape[0] // 2
     out, ldo = _gates_out("linear_tiles_swiglu", x, weight, inter, out)
     _lib.call("zi_gemm_tiles", _p(out), 2, _p(x), _p(weight), c_void_p(0), x.shape[0], inter, x.shape[1], x.stride(0), weight.stride(0),
