@@ -88,11 +88,13 @@ class Runtime:
         view = self._views[vkey] = buf[:n].view(tuple(shape))
         return view
 
-    def product_workspace(self, name: str, x: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> Optional[torch.Tensor]:
-        """What ``ops.linear`` (``gated``: ``ops.linear_swiglu_halves``) is to be given as its workspace for this product, or None."""
+    def product_workspace(self, x: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> Optional[torch.Tensor]:
+        """What ``ops.linear`` (``gated``: ``ops.linear_swiglu_halves``) is to be given as its workspace for this product, or None: one
+        allocation for all of a model's products, which follow each other on one stream.  The float32 steps that were measured pass it, dense
+        attention and SwiGLU; other parts make their float32 products without."""
         from .. import ops
         need = ops.linear_many_workspace(x, weight, gated)
-        return self.buffer(name, (need,), torch.uint8) if need else None
+        return self.buffer("product_parts", (-(-need // 4),), torch.float32) if need else None
 
     def poison(self) -> None:
         """Make every floating-point workspace NaN (a check that a replay writes all it reads; integer workspaces

@@ -155,7 +155,7 @@ class SwiGLU(FeedForward):
             else:
                 self._gate_up_many_rows(x, act)
         elif not self.interleave and self.gate_up is not None and ops.linear_swiglu_halves_supported(x, self.gate_up):
-            ops.linear_swiglu_halves(x, self.gate_up, out=act, workspace=self.rt.product_workspace("ffn_parts", x, self.gate_up, gated=True))
+            ops.linear_swiglu_halves(x, self.gate_up, out=act, workspace=self.rt.product_workspace(x, self.gate_up, gated=True))
         else:
             gu = self.rt.buffer("ffn_gate_up", (n, 2 * I))
             if self.gate_up is not None:
@@ -171,7 +171,7 @@ class SwiGLU(FeedForward):
             S = ops.linear_splits(n, self.hidden, I)
             return ops.linear_sums(act, self.down, out=self.rt.buffer("ffn_out_sums", (S, n, self.hidden), torch.float32))
         out = self.rt.buffer("ffn_out", (n, self.hidden))
-        return ops.linear(act, self.down, out=out, workspace=self.rt.product_workspace("ffn_parts", act, self.down))
+        return ops.linear(act, self.down, out=out, workspace=self.rt.product_workspace(act, self.down))
 
 
 @register_feed_forward("none")

@@ -349,7 +349,7 @@ class Attention(Mixer):
             qkv = self.rt.buffer("attn_qkv", (n, self.qd + 2 * self.kvd))
             q, k, v = qkv[:, :self.qd], qkv[:, self.qd:self.qd + self.kvd], qkv[:, self.qd + self.kvd:]
             if self.qkv is not None:
-                ops.linear(x, self.qkv, self.bias, out=qkv, workspace=self.rt.product_workspace("attn_parts", x, self.qkv))
+                ops.linear(x, self.qkv, self.bias, out=qkv, workspace=self.rt.product_workspace(x, self.qkv))
             else:
                 for dst, m, b in zip((q, k, v), self.mats, self.biases or (None, None, None)):
                     ops.linear(x, m, b, out=dst)
@@ -374,7 +374,7 @@ class Attention(Mixer):
             S = ops.linear_splits(n, self.hidden, self.qd)
             return ops.linear_sums(att, self.o, out=self.rt.buffer("attn_proj_sums", (S, n, self.hidden), torch.float32))
         out = self.rt.buffer("attn_proj", (n, self.hidden))
-        return ops.linear(att, self.o, out=out, workspace=self.rt.product_workspace("attn_parts", att, self.o))
+        return ops.linear(att, self.o, out=out, workspace=self.rt.product_workspace(att, self.o))
 
     def decode_from_sums(self, sums, batch, view, memory: LayerMemory) -> Optional[torch.Tensor]:
         """A pure decode step (one token a sequence): rotation, cache store and attention in one kernel,
