@@ -37,7 +37,7 @@ union gt_pack {
 
 // what the kernel ends with
 #define GT_BF16 0          // bfloat16 results, with a bias
-#define GT_F32 1           // float32 results with a bias, or partial sums [split][M][N]
+#define GT_F32 1           // float32 results, with a bias
 #define GT_SWIGLU 2        // gate and up rows of the weights alternate in blocks of 8; bfloat16
 #define GT_GATED 3         // the gate rows come first, the up rows from row `up_at` on; an activation by its code; bfloat16
 #define GT_ERF 4           // the same with the error function's GELU (a kernel of its own: the function is 40 instructions)
@@ -73,7 +73,7 @@ struct gt_args {
     int M, N, K;                   // N: columns of the result (gate and up make one)
     int64_t ldx, ldw, ldo;
     int up_at, act;
-    int row_tiles, col_tiles, splits, steps, steps_a_split, units;      // units: tiles x splits
+    int row_tiles, col_tiles, steps, units;      // units: tiles
 };
 
 // Where row q of a wavefront's 16 NW rows of LDS comes from, as (column of the result, gate or up).  Blocks of 16 go to the matrix
@@ -93,12 +93,9 @@ __device__ __forceinline__ int gt_unit(const gt_args& g, int b, int i) {
     return count > 0 && b / GT_XCDS < share && id < count ? base + id : -1;
 }
 
-// A unit's place: splits one after the other, in each GT_GROUP tiles of rows at a time, the rows fastest, so that 32 units are about a
-// square of tiles.
-__device__ __forceinline__ void gt_place(const gt_args& g, int unit, int* m, int* n, int* split) {
-    const int tiles = g.row_tiles * g.col_tiles;
-    *split = unit / tiles;
-    const int id = unit - *split * tiles, per = GT_GROUP * g.col_tiles, group = id / per, in = id - group * per;
+// A unit's place: GT_GROUP tiles of rows at a time, the rows fastest, so that 32 units are about a square of tiles.
+__device__ __forceinline__ void gt_place(const gt_args& g, int unit, int* m, int* n) {
+    const int per = GT_GROUP * g.col_tiles, group = unit / per, in = unit - group * per;
     const int rows = g.row_tiles - group * GT_GROUP < GT_GROUP ? g.row_tiles - group * GT_GROUP : GT_GROUP;
     *n = in / rows;
     *m = group * GT_GROUP + in - *n * rows;
@@ -163,14 +160,14 @@ __global__ void __launch_bounds__(128 * WM, 1) gemm_tiles_kernel(gt_args g) {
         work f{g.x, g.w, 0, 0, 64};
         const int unit = gt_unit(g, blockIdx.x, round);
         if (unit >= 0) {
-            int m, n, s;
-            gt_place(g, unit, &m, &n, &s);
-            const int k = s * g.steps_a_split * GT_KB, row = n * (EPI == GT_SWIGLU ? BN : COLS);
-            f.steps = g.steps - s * g.steps_a_split < g.steps_a_split ? g.steps - s * g.steps_a_split : g.steps_a_split;
-            f.x = g.x + (int64_t)m * BM * g.ldx + k;
-            f.w = g.w + (int64_t)row * g.ldw + k;
-            f.x_bytes = (int)(((int64_t)((g.M - m * BM < BM ? g.M - m * BM : BM) - 1) * g.ldx + g.K - k) * 2);
-            f.w_bytes = (int)(((int64_t)(last_row - row - 1) * g.ldw + g.K - k) * 2);
+            int m, n;
+            gt_place(g, unit, &m, &n);
+            const int row = n * (EPI == GT_SWIGLU ? BN : COLS);
+            f.steps = g.steps;
+            f.x = g.x + (int64_t)m * BM * g.ldx;
+            f.w = g.w + (int64_t)row * g.ldw;
+            f.x_bytes = (int)(((int64_t)((g.M - m * BM < BM ? g.M - m * BM : BM) - 1) * g.ldx + g.K) * 2);
+            f.w_bytes = (int)(((int64_t)(last_row - row - 1) * g.ldw + g.K) * 2);
         }
         return f;
     };
@@ -269,8 +266,8 @@ __global__ void __launch_bounds__(128 * WM, 1) gemm_tiles_kernel(gt_args g) {
             for (int m = 0; m < MW; ++m) GT_KEEP(acc[n][m]);
         // C[n][m] of a block: row 4 j + e of the weights, row r of x.  Stores are counted like loads and in the same order: they only
         // make the next steps' waits for loads that are older longer.
-        int tm, tn, split;
-        gt_place(g, unit, &tm, &tn, &split);
+        int tm, tn;
+        gt_place(g, unit, &tm, &tn);
         const int col0 = tn * COLS + wn * (GATES ? 8 * NW : 16 * NW), row0 = tm * BM + wm * MW * 16 + r;
         constexpr int BLOCKS = GATES ? 4 : 2;         // of which a lane's outputs are eight columns; fewer blocks left make four
 #pragma unroll
@@ -296,7 +293,7 @@ __global__ void __launch_bounds__(128 * WM, 1) gemm_tiles_kernel(gt_args g) {
                     }
                 if (row < g.M && col < g.N) {
                     if (EPI == GT_F32) {
-                        float* to = (float*)g.out + ((int64_t)split * g.M + row) * g.ldo + col;
+                        float* to = (float*)g.out + (int64_t)row * g.ldo + col;
                         *reinterpret_cast<gt_f32x4_t*>(to) = gt_f32x4_t{v[0], v[1], v[2], v[3]};
                         if (eight) *reinterpret_cast<gt_f32x4_t*>(to + 4) = gt_f32x4_t{v[4], v[5], v[6], v[7]};
                     } else {
@@ -314,7 +311,7 @@ __global__ void __launch_bounds__(128 * WM, 1) gemm_tiles_kernel(gt_args g) {
     gt_wait<0>();       // (no load may arrive after the workgroup's LDS is another's)
 }
 
-// ---- the tile and the cut of a product ------------------------------------------------------------------------------------
+// ---- the tile of a product ------------------------------------------------------------------------------------------------
 // WM, MW, NW, and what a step of 64 columns takes in ns: c0 where few workgroups run, c0 + c1 where the chip is full of them.
 struct gt_tile {
     int wm, mw, nw, c0, c1;
@@ -327,40 +324,34 @@ static const gt_tile gt_tiles[] = {
 #undef GT_ROW
 };
 #define GT_TILE_COUNT ((int)(sizeof(gt_tiles) / sizeof(gt_tiles[0])))
-#define GT_MOST_SPLITS 8
-#define GT_FEWEST_STEPS 5       // of a unit: no fewer than a kernel has buffers
+#define GT_FEWEST_STEPS 5       // no fewer than a kernel has buffers
 #define GT_ABOVE 256            // rows of x up to which products are the few-rows kernels' or the library's
 
 #define GT_NARROW 512           // columns of the result and of x up to which they are as well: launches, whoever makes them
 
-enum gt_kind { GT_PLAIN, GT_GATES, GT_SUMS };      // what may be made of a product: whole, gate and up, partial sums
+enum gt_kind { GT_PLAIN, GT_GATES };      // what is made of a product
 
 struct gt_plan {
-    int tile, splits, steps_a_split;
+    int tile;
     double ns;
 };
 
-// Tile and cut by the time they take: a launch, for each round of workgroups its steps and its epilogue, the results' way to memory, and,
-// of partial sums, what the kernel that adds them reads more.  The constants are a fit to 9,000 timed launches (10 tiles and up to 8 cuts of
-// 500 products, 129 to 9,000 rows, 512 to 49,888 columns, k 512 to 27,648, weights from memory): off by 6 % in the mean, and the choice by
-// them is within 0.3 % of the best in the mean, 9 % at worst.
+// The tile by the time it takes: a launch, for each round of workgroups its steps and its epilogue, the results' way to memory.  The constants
+// are a fit to 9,000 timed launches (10 tiles and, of products in up to 8 cuts of k that no kernel here makes any more, each cut; 500 products, 129 to
+// 9,000 rows, 512 to 49,888 columns, k 512 to 27,648, weights from memory): off by 6 % in the mean, and the choice by them is within 0.3 % of the
+// best in the mean, 9 % at worst.
 static gt_plan gt_best(int M, int64_t N, int K, int kind) {
-    gt_plan best{-1, 1, 0, 0.0};
+    gt_plan best{-1, 0.0};
     const int cus = zi_compute_units(), steps = K / GT_KB;
     for (int i = 0; i < GT_TILE_COUNT; ++i) {
         const gt_tile& t = gt_tiles[i];
         if (kind == GT_GATES && t.nw % 2) continue;
         const int rows = 16 * t.wm * t.mw, wrows = 32 * t.nw, cols = kind == GT_GATES ? wrows / 2 : wrows;
-        const int64_t tiles = (int64_t)((M + rows - 1) / rows) * ((N + cols - 1) / cols);
-        for (int s0 = 1; s0 <= (kind == GT_SUMS ? GT_MOST_SPLITS : 1); ++s0) {
-            const int per = (steps + s0 - 1) / s0, s = (steps + per - 1) / per;
-            if (s != s0 || steps - (s - 1) * per < GT_FEWEST_STEPS || tiles * s > (1 << 24)) continue;
-            const int64_t units = tiles * s, rounds = (units + cus - 1) / cus;
-            const double fill = (double)units / (double)(rounds * cus), out = (double)M * (double)N;
-            const double ns = 4300.0 + rounds * (per * (t.c0 + t.c1 * fill) + 0.084 * rows * wrows) + out * (s > 1 ? 4 * s : 2) * 0.000116 +
-                              (s > 1 ? out * (4 * s - 2) / 4500.0 : 0.0);
-            if (best.tile < 0 || ns < best.ns) best = gt_plan{i, s, per, ns};
-        }
+        const int64_t tiles = (int64_t)((M + rows - 1) / rows) * ((N + cols - 1) / cols), rounds = (tiles + cus - 1) / cus;
+        if (tiles > (1 << 24)) continue;
+        const double fill = (double)tiles / (double)(rounds * cus);
+        const double ns = 4300.0 + rounds * (steps * (t.c0 + t.c1 * fill) + 0.084 * rows * wrows) + (double)M * (double)N * 0.000232;
+        if (best.tile < 0 || ns < best.ns) best = gt_plan{i, ns};
     }
     return best;
 }
@@ -371,22 +362,17 @@ static bool gt_sizes(int64_t M, int64_t N, int64_t K) {
 
 // 1 when a product of more than 256 rows is to be made by the kernel here: where its time by the fit is below what the library's tuned
 // product takes (with the launch of the activation, for gate and up), 16 us, 10 more from 10 GFLOP on, and 1.3 PFLOP/s.  Of the 500
-// products own time of the library's, geometric mean: gate and up 0.73 to 0.88 up to 160 GFLOP and 0.94 beyond, products that may be
-// partial sums 0.80 to 0.88 and 0.96 to 1.0, plain ones 0.91 to 1.0 and 1.03 to 1.07; with this rule 0.907 over all of them.  us,
-// own and the library's: gate/up with SwiGLU of 8,960 columns x 1,536 at 320 / 1,024 / 2,048 rows 28 and 35, 64 and 75, 111 and 129, of
-// 18,944 x 3,584 104 and 121, 266 and 283, 461 and 523; 1,536 x 8,960 as partial sums 19 and 31, 33 and 47, 55 and 70; 3,584 x 18,944 55 and 107,
-// 135 and 163, and at 2,048 rows 255 and 237: the library's.
+// products own time of the library's, geometric mean: gate and up 0.73 to 0.88 up to 160 GFLOP and 0.94 beyond, plain ones 0.91 to 1.0 and 1.03
+// to 1.07.  us, own and the library's: gate/up with SwiGLU of 8,960 columns x 1,536 at 320 / 1,024 / 2,048 rows 28 and 35, 64 and 75, 111 and 129, of
+// 18,944 x 3,584 104 and 121, 266 and 283, 461 and 523.
 extern "C" int zi_gemm_tiles_pays(int M, int N, int K, int kind) {
-    if (M <= GT_ABOVE || N <= GT_NARROW || K <= GT_NARROW || kind < GT_PLAIN || kind > GT_SUMS || !gt_sizes(M, N, K)) return 0;
+    if (M <= GT_ABOVE || N <= GT_NARROW || K <= GT_NARROW || kind < GT_PLAIN || kind > GT_GATES || !gt_sizes(M, N, K)) return 0;
     const gt_plan p = gt_best(M, N, K, kind);
     const double flops = 2.0 * M * (kind == GT_GATES ? 2.0 : 1.0) * N * K;
     double library = 16000.0 + 10000.0 * (flops < 1e10 ? flops / 1e10 : 1.0) + flops / 1.3e6;
     if (kind == GT_GATES) library += 4000.0 + 6.0 * M * N / 4500.0;
     return p.tile >= 0 && p.ns < library;
 }
-
-// The partial sums that the product leaves as it is made fastest for a kernel that adds them; 1: make it whole.
-extern "C" int zi_gemm_tiles_splits(int M, int N, int K) { return gt_sizes(M, N, K) ? gt_best(M, N, K, GT_SUMS).splits : 1; }
 
 extern "C" int zi_gemm_tiles_count() { return GT_TILE_COUNT; }
 
@@ -396,7 +382,7 @@ static int gt_launch(gt_args g, int epi, hipStream_t stream) {
     const int cols = epi >= GT_SWIGLU ? Z::WROWS / 2 : Z::WROWS, cus = zi_compute_units();
     g.row_tiles = (g.M + Z::ROWS - 1) / Z::ROWS;
     g.col_tiles = (g.N + cols - 1) / cols;
-    const int64_t units = (int64_t)g.row_tiles * g.col_tiles * g.splits;
+    const int64_t units = (int64_t)g.row_tiles * g.col_tiles;
     ZI_REQUIRE(units <= (1 << 24), "gemm_tiles: too many tiles");
     g.units = (int)units;
     const int most = cus / GT_XCDS * GT_XCDS > 0 ? cus / GT_XCDS * GT_XCDS : GT_XCDS;
@@ -413,12 +399,11 @@ static int gt_launch(gt_args g, int epi, hipStream_t stream) {
     return zi_check_launch("gemm_tiles");
 }
 
-// epi 0: out [M,N] bfloat16, bias (bfloat16 [N] or null); 1: the same in float32, or with `splits` > 1 float32 partial sums
-// [splits][M][N] (no bias); 2: w [2 N, K] holds gate and up rows in turn, 8 each, out = up * silu(gate); 3: w holds the gate rows, then from
+// epi 0: out [M,N] bfloat16, bias (bfloat16 [N] or null); 1: the same in float32; 2: w [2 N, K] holds gate and up rows in turn, 8 each, out = up * silu(gate); 3: w holds the gate rows, then from
 // row up_at >= N on the up rows, out = act(gate) * up, act 0 SiLU, 1 GELU in its tanh form, 2 with the error function.
 // tile: a number below zi_gemm_tiles_count(), or -1 for the one that is taken for these sizes.
 extern "C" int zi_gemm_tiles(void* out, int epi, const void* x, const void* w, const void* bias, int M, int N, int K, int64_t ldx,
-                             int64_t ldw, int64_t ldo, int up_at, int act, int splits, int tile, hipStream_t stream) {
+                             int64_t ldw, int64_t ldo, int up_at, int act, int tile, hipStream_t stream) {
     ZI_REQUIRE(out && x && w, "gemm_tiles: null operand");
     ZI_REQUIRE(epi >= GT_BF16 && epi <= GT_GATED, "gemm_tiles: unknown epilogue %d", epi);
     ZI_REQUIRE(gt_sizes(M, N, K), "gemm_tiles: unsupported sizes M=%d N=%d K=%d (N a multiple of 8, K of 64 and at least %d)", M, N, K,
@@ -432,16 +417,8 @@ extern "C" int zi_gemm_tiles(void* out, int epi, const void* x, const void* w, c
     ZI_REQUIRE(epi != GT_GATED || (up_at >= N && act >= ZI_ACT_SILU && act <= ZI_ACT_GELU_ERF), "gemm_tiles: bad rows of up or activation %d", act);
     ZI_REQUIRE(epi < GT_SWIGLU || !bias, "gemm_tiles: gate and up take no bias");
     ZI_REQUIRE(tile >= -1 && tile < GT_TILE_COUNT, "gemm_tiles: no tile %d", tile);
-    ZI_REQUIRE(splits >= 1 && splits <= GT_MOST_SPLITS && (splits == 1 || (epi == GT_F32 && !bias && ldo == N)),
-               "gemm_tiles: partial sums are contiguous float32 without a bias");
-    const int steps = K / GT_KB, per = (steps + splits - 1) / splits;
-    ZI_REQUIRE((steps + per - 1) / per == splits && steps - (splits - 1) * per >= GT_FEWEST_STEPS, "gemm_tiles: k of %d steps is not cut into %d", steps, splits);
-    if (tile < 0) {
-        const gt_plan p = gt_best(M, N, K, epi >= GT_SWIGLU ? GT_GATES : splits > 1 ? GT_SUMS : GT_PLAIN);
-        ZI_REQUIRE(p.tile >= 0 && (splits == 1 || p.splits == splits), "gemm_tiles: not the cut that these sizes are made with");
-        tile = p.tile;
-    }
-    gt_args g{out, (const zi_bf16*)x, (const zi_bf16*)w, (const zi_bf16*)bias, M, N, K, ldx, ldw, ldo, up_at, act, 0, 0, splits, steps, per, 0};
+    if (tile < 0) tile = gt_best(M, N, K, epi >= GT_SWIGLU ? GT_GATES : GT_PLAIN).tile;
+    gt_args g{out, (const zi_bf16*)x, (const zi_bf16*)w, (const zi_bf16*)bias, M, N, K, ldx, ldw, ldo, up_at, act, 0, 0, K / GT_KB, 0};
     int at = 0;
 #define GT_GO(WM, MW, NW, C0, C1) \
     if (tile == at++) return gt_launch<WM, MW, NW>(g, epi, stream);

@@ -113,7 +113,7 @@ int zi_gemm_lt(void* out, int out_dt, const void* x, const void* weight, const v
     stream);
 // gemm_tiles.hip
 int zi_gemm_tiles(void* out, int epi, const void* x, const void* w, const void* bias, int M, int N, int K, int64_t ldx,
-    int64_t ldw, int64_t ldo, int up_at, int act, int splits, int tile, hipStream_t stream);
+    int64_t ldw, int64_t ldo, int up_at, int act, int tile, hipStream_t stream);
 // gemm_skinny.hip
 int zi_gemm_skinny(void* out, int out_dt, int mode, const void* x, const void* w, const void* bias, int M, int N, int
     K, int64_t ldx, int64_t ldw, int64_t ldo, float* workspace, int64_t workspace_floats, hipStream_t stream);

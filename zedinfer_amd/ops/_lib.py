@@ -72,9 +72,8 @@ _PROTOTYPES = {
     "zi_gemm_skinny_act": [P, I, I, P, P, P, I, I, I, L, L, L, P, L, F, P],
     "zi_clamped_glu_il8": [P, L, P, L, I, I, F, F, P],
     "zi_gemm_skinny_splits": [I, I, I],
-    "zi_gemm_tiles": [P, I, P, P, P, I, I, I, L, L, L, I, I, I, I, P],
+    "zi_gemm_tiles": [P, I, P, P, P, I, I, I, L, L, L, I, I, I, P],
     "zi_gemm_tiles_pays": [I, I, I, I],
-    "zi_gemm_tiles_splits": [I, I, I],
     "zi_gemm_tiles_count": [],
     "zi_gemm_lt": [P, I, P, P, P, I, L, L, L, L, L, L, P, L, P],
     "zi_gemm_lt_tune": [P, I, P, P, P, I, L, L, L, L, L, L, P, L, I, I, P, P, P, P],

@@ -955,7 +955,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     all_bf = x.dtype == bf and weight.dtype == bf and (bias is None or bias.dtype == bf)
     if all_bf and _tiles_take(x, weight, out, bias, TILES_PLAIN):
         _lib.call("zi_gemm_tiles", _p(out), TILES_EPILOGUE[out.dtype], _p(x), _p(weight), _p(bias), M, N, K, ldx, ldw, ldo,
-                  0, 0, 1, -1, _stream())
+                  0, 0, -1, _stream())
         return out
     if all_bf and out.dtype == torch.float32 and M > SKINNY_MAX_ROWS and bias is None and _library_ok(x, weight, out):
         # float32 output for many rows (logits of a large decode batch or of every place of a prompt): the
@@ -998,7 +998,7 @@ def linear_transposed(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch
     return out
 
 
-TILES_PLAIN, TILES_GATES, TILES_SUMS = 0, 1, 2      # what of a product ``zi_gemm_tiles_pays`` is asked about
+TILES_PLAIN, TILES_GATES = 0, 1                      # what of a product ``zi_gemm_tiles_pays`` is asked about
 TILES_ABOVE = 256                                    # rows up to which it says no
 TILES_EPILOGUE = {torch.bfloat16: 0, torch.float32: 1}      # the types that a whole product can be stored as, and the ends of the kernel that do
 
@@ -1051,7 +1051,7 @@ def linear_tiles_swiglu(x: torch.Tensor, weight: torch.Tensor, out: Optional[tor
     inter = weight.shape[0] // 2
     out, ldo = _gates_out("linear_tiles_swiglu", x, weight, inter, out)
     _lib.call("zi_gemm_tiles", _p(out), 2, _p(x), _p(weight), c_void_p(0), x.shape[0], inter, x.shape[1], x.stride(0), weight.stride(0),
-              ldo, 0, 0, 1, -1, _stream())
+              ldo, 0, 0, -1, _stream())
     return out
 
 
@@ -1068,7 +1068,7 @@ def linear_tiles_gated(x: torch.Tensor, weight: torch.Tensor, inter: int, up_at:
         raise ValueError("linear_tiles_gated: the up rows must follow the gate rows within the weight")
     out, ldo = _gates_out("linear_tiles_gated", x, weight, inter, out)
     _lib.call("zi_gemm_tiles", _p(out), 3, _p(x), _p(weight), c_void_p(0), x.shape[0], int(inter), x.shape[1], x.stride(0),
-              weight.stride(0), ldo, int(up_at), GATED_ACTIVATIONS[activation], 1, -1, _stream())
+              weight.stride(0), ldo, int(up_at), GATED_ACTIVATIONS[activation], -1, _stream())
     return out
 
 
