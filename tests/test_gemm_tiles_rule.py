@@ -43,3 +43,15 @@ def test_gate_and_up_rows_that_are_no_whole_blocks_are_refused(launches):
     with pytest.raises(ValueError):
         ops.linear_tiles_swiglu(x, w)
     assert launches == ["zi_gemm_tiles"]
+
+
+def pays(M, N, K, gates=False):
+    return ops.load().zi_gemm_tiles_pays(M, N, K, int(gates))
+
+
+def test_the_rule_is_bounded_to_where_it_tells_the_ways_apart():
+    assert [pays(M, 1536, 1536) for M in (256, 257)] == [0, 1] and pays(300, 512, 4608) == pays(300, 4608, 512) == pays(300, 1536, 1528) == 0
+    assert pays(640, 2048, 1536, True) == pays(257, 1000, 640, True) == pays(2048, 8960, 1536, True) == 1
+    # large products, among them those of a prompt of 16,384 tokens at 32B sizes: the library was a quarter faster at some
+    assert pays(4096, 16384, 4096) == pays(2048, 3584, 18944) == 0
+    assert [pays(16384, N, K) for N, K in ((7168, 5120), (5120, 5120), (5120, 27648))] == [0, 0, 0] and pays(16384, 27648, 5120, True) == 0

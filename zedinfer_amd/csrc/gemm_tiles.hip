@@ -361,17 +361,24 @@ static bool gt_sizes(int64_t M, int64_t N, int64_t K) {
 }
 
 // 1 when a product of more than 256 rows is to be made by the kernel here: where its time by the fit is below what the library's tuned
-// product takes (with the launch of the activation, for gate and up), 16 us, 10 more from 10 GFLOP on, and 1.3 PFLOP/s.  Of the 500
-// products own time of the library's, geometric mean: gate and up 0.73 to 0.88 up to 160 GFLOP and 0.94 beyond, plain ones 0.91 to 1.0 and 1.03
-// to 1.07.  us, own and the library's: gate/up with SwiGLU of 8,960 columns x 1,536 at 320 / 1,024 / 2,048 rows 28 and 35, 64 and 75, 111 and 129, of
-// 18,944 x 3,584 104 and 121, 266 and 283, 461 and 523.
+// product takes (with the launch of the activation, for gate and up), 16 us, 10 more from 10 GFLOP on, and 1.5 PFLOP/s, up to 30 GFLOP of a
+// plain product and 3 TFLOP of a gate/up product.  18,680 products timed both ways, weights from memory (257 to 20,000 rows, 520 to 30,000 columns, k 576 to 27,648, up
+// to 10 TFLOP): own time of the library's, geometric mean and one in twenty, where it says 1: plain 0.944 and 1.11 up to 10 GFLOP, 0.951 and 1.09
+// up to 30; gate and up 0.69 and 0.91, 0.79 and 1.03, 0.80 and 0.97 up to 100, 0.82 and 0.98 up to 1,000, 0.91 and 1.00 up to 3,000.  Beyond the bounds either is as fast as the other in the mean (plain 1.00 to 1.05 of the library's time, gate and
+// up 1.03) and 1.25 times as fast at single sizes, the library 0.9 to 1.5 PFLOP/s by how its tiles come out: no rule on the sizes that was tried
+// tells them apart, and the library keeps them.  us, own and the library's: gate/up with SwiGLU of 8,960 columns x 1,536 at 320 / 1,024 / 2,048 rows 28 and 35, 64 and 75, 111 and 129, of
+// 18,944 x 3,584 104 and 121, 266 and 283, 461 and 523, of 27,648 x 5,120 at 12,736 rows 5,664 and 5,371; 5,120 x 27,648 at 4,864 / 8,194 rows 1,119 and 1,388,
+// 1,859 and 1,715; 320 x 536 x 1,792, the worst that it says 1 of, 9.5 and 6.7.
+#define GT_PLAIN_MOST 3e10
+#define GT_GATES_MOST 3e12
+
 extern "C" int zi_gemm_tiles_pays(int M, int N, int K, int kind) {
     if (M <= GT_ABOVE || N <= GT_NARROW || K <= GT_NARROW || kind < GT_PLAIN || kind > GT_GATES || !gt_sizes(M, N, K)) return 0;
     const gt_plan p = gt_best(M, N, K, kind);
     const double flops = 2.0 * M * (kind == GT_GATES ? 2.0 : 1.0) * N * K;
-    double library = 16000.0 + 10000.0 * (flops < 1e10 ? flops / 1e10 : 1.0) + flops / 1.3e6;
+    double library = 16000.0 + 10000.0 * (flops < 1e10 ? flops / 1e10 : 1.0) + flops / 1.5e6;
     if (kind == GT_GATES) library += 4000.0 + 6.0 * M * N / 4500.0;
-    return p.tile >= 0 && p.ns < library;
+    return p.tile >= 0 && p.ns < library && flops <= (kind == GT_GATES ? GT_GATES_MOST : GT_PLAIN_MOST);
 }
 
 extern "C" int zi_gemm_tiles_count() { return GT_TILE_COUNT; }
