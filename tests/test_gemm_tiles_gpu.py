@@ -193,3 +193,44 @@ def test_feed_forwards_of_many_rows(kind, activation, n, H, I, monkeypatch):
     ref = (fn(X @ w["gate"].double().t()) * (X @ w["up"].double().t())) @ w["down"].double().t()
     # the activation and the result are rounded to bfloat16 once each, evenly: 2^-8 / sqrt(3) at most of every value, less of a sum
     assert float((got - ref).norm() / ref.norm()) <= 2 * 2.0 ** -8 / 3 ** 0.5
+
+
+@pytest.mark.parametrize("kind", ["swiglu", "gated_mlp"])
+def test_what_no_rule_tells_apart_is_measured_once(kind, monkeypatch):
+    """``tune`` times the tiles against the library's products and records the faster, the forward pass follows the record, and a part that
+    is given the record times nothing."""
+    from zedinfer_amd import ops
+    from zedinfer_amd.config.forward_config import PartSpec
+    from zedinfer_amd.ops import _lib
+    from zedinfer_amd.parts import FEED_FORWARDS
+    from zedinfer_amd.parts.base import Runtime
+    n, H, I = 1024, 2048, 5120
+    w = {"gate": rnd(I, H, seed=1, scale=0.05), "up": rnd(I, H, seed=2, scale=0.05), "down": rnd(H, I, seed=3, scale=0.05)}
+    x, params = rnd(n, H, seed=4), {"hidden_size": H, "intermediate_size": I, "activation": "silu"}
+    parts = [FEED_FORWARDS.get(kind)(PartSpec(kind, params, {k: k for k in w}), w, Runtime("cuda", torch.bfloat16)) for _ in range(2)]
+    assert 0 < ops.linear_tiles_gates_rule(x, parts[0].gate_up, I) < ops.TILES_SURELY
+    calls, real = [], _lib.call
+    monkeypatch.setattr(_lib, "call", lambda name, *a: (calls.append(name), real(name, *a))[1])
+    choices = parts[0].rt.choices
+    parts[0].rt.buffer("norm_out", (n, H)).copy_(x)
+    parts[0].tune(n)
+    tiles = choices[("tiles_gates", n, 2 * I, H, False, False, "bfloat16")]
+    assert isinstance(tiles, bool) and calls.count("zi_gemm_lt_tune") >= 1 and "zi_gemm_tiles" in calls
+    if kind == "swiglu":         # (its down product is tuned too)
+        assert isinstance(choices[("tiles_product", n, H, I, False, False, "bfloat16")], bool)
+    parts[1].rt.choices.update(choices)
+    outs = []
+    for part in parts:
+        calls.clear()
+        part.tune(n)
+        assert "zi_gemm_lt_tune" not in calls and "zi_gemm_tiles" not in calls and part.rt.choices == choices
+        outs.append(part.forward(x).clone())
+        made = [c for c in calls if c in ("zi_gemm_tiles", "zi_gemm_lt")]
+        assert (made[0] == "zi_gemm_tiles") == tiles
+        assert kind != "swiglu" or (made[1] == "zi_gemm_tiles") == choices[("tiles_product", n, H, I, False, False, "bfloat16")]
+    assert torch.equal(outs[0], outs[1])
+    # either record, the same result but for rounding
+    for way in (False, True):
+        parts[0].rt.choices[("tiles_gates", n, 2 * I, H, False, False, "bfloat16")] = way
+        got = parts[0].forward(x).double()
+        assert float((got - outs[1].double()).norm() / outs[1].double().norm()) <= 2 * 2.0 ** -8

@@ -360,25 +360,35 @@ static bool gt_sizes(int64_t M, int64_t N, int64_t K) {
     return M >= 1 && N >= 8 && N % 8 == 0 && K % GT_KB == 0 && K >= GT_KB * GT_FEWEST_STEPS && M * N < ((int64_t)1 << 40);
 }
 
-// 1 when a product of more than 256 rows is to be made by the kernel here: where its time by the fit is below what the library's tuned
-// product takes (with the launch of the activation, for gate and up), 16 us, 10 more from 10 GFLOP on, and 1.5 PFLOP/s, up to 30 GFLOP of a
-// plain product and 3 TFLOP of a gate/up product.  18,680 products timed both ways, weights from memory (257 to 20,000 rows, 520 to 30,000 columns, k 576 to 27,648, up
-// to 10 TFLOP): own time of the library's, geometric mean and one in twenty, where it says 1: plain 0.944 and 1.11 up to 10 GFLOP, 0.951 and 1.09
-// up to 30; gate and up 0.69 and 0.91, 0.79 and 1.03, 0.80 and 0.97 up to 100, 0.82 and 0.98 up to 1,000, 0.91 and 1.00 up to 3,000.  Beyond the bounds either is as fast as the other in the mean (plain 1.00 to 1.05 of the library's time, gate and
-// up 1.03) and 1.25 times as fast at single sizes, the library 0.9 to 1.5 PFLOP/s by how its tiles come out: no rule on the sizes that was tried
-// tells them apart, and the library keeps them.  us, own and the library's: gate/up with SwiGLU of 8,960 columns x 1,536 at 320 / 1,024 / 2,048 rows 28 and 35, 64 and 75, 111 and 129, of
-// 18,944 x 3,584 104 and 121, 266 and 283, 461 and 523, of 27,648 x 5,120 at 12,736 rows 5,664 and 5,371; 5,120 x 27,648 at 4,864 / 8,194 rows 1,119 and 1,388,
-// 1,859 and 1,715; 320 x 536 x 1,792, the worst that it says 1 of, 9.5 and 6.7.
-#define GT_PLAIN_MOST 3e10
+// The kernel here or the library's product (with the launch of the activation, for gate and up) for more than 256 rows.  0: not taken here;
+// 1: taken, but the library is the faster by the rule; 2: the kernel here is; 3: and surely (a gate/up product).  The rule holds the time by the fit
+// against 16 us, 10 more from 10 GFLOP on, and 1.3 PFLOP/s, and says 2 up to 100 GFLOP of a plain product and 3 TFLOP of a gate/up product, 3 from
+// 0.7 of the library's time down.  18,680 products timed both ways, the library's the fastest of its proposals, and 13,541 with its first one (which runs where
+// nothing was measured), weights from memory, 257 to 20,000 rows, 520 to 30,000 columns, k 576 to 27,648, up to 10 TFLOP.  Own time of the
+// library's, geometric mean and one in twenty, where the rule says 2:
+//                        up to 10 GFLOP     30             100            1,000          3,000          beyond, all of them
+//   plain, first         0.89 and 1.06      0.92 and 1.11  0.97 and 1.14                                0.93 and 1.18
+//   plain, fastest       0.94 and 1.11      0.96 and 1.13  1.01 and 1.15                                1.02 and 1.19
+//   gate/up, first       0.68 and 0.89      0.76 and 1.01  0.76 and 0.94  0.83 and 1.04  0.95 and 1.04  1.00 and 1.10
+//   gate/up, fastest     0.68 and 0.91      0.79 and 1.03  0.82 and 0.99  0.88 and 1.09  0.97 and 1.07  1.03 and 1.12
+// Beyond the bounds single sizes are up to 1.25 times as fast either way, the library 0.9 to 1.5 PFLOP/s by how its tiles come out, which no rule on the
+// sizes that was tried tells apart, so an engine times both (the faster one takes 0.955 of the library's time in the mean, plain, and 0.873), and
+// where nothing was measured the library keeps them.  Where the rule says 3, 0.72, above 1 in one of a thousand.  us, own and the library's fastest: gate/up with
+// SwiGLU of 8,960 columns x 1,536 at 320 / 1,024 / 2,048 rows 28 and 35, 64 and 75, 111 and 129, of 18,944 x 3,584 104 and 121, 266 and 283, 461 and 523, of
+// 27,648 x 5,120 at 12,736 rows 5,664 and 5,371; 5,120 x 27,648 at 4,864 / 8,194 rows 1,119 and 1,388, 1,859 and 1,715; 320 x 536 x 1,792, the worst that the
+// rule says 2 of, 9.5 and 6.7.
+#define GT_PLAIN_MOST 1e11
 #define GT_GATES_MOST 3e12
 
 extern "C" int zi_gemm_tiles_pays(int M, int N, int K, int kind) {
     if (M <= GT_ABOVE || N <= GT_NARROW || K <= GT_NARROW || kind < GT_PLAIN || kind > GT_GATES || !gt_sizes(M, N, K)) return 0;
     const gt_plan p = gt_best(M, N, K, kind);
+    if (p.tile < 0) return 0;
     const double flops = 2.0 * M * (kind == GT_GATES ? 2.0 : 1.0) * N * K;
-    double library = 16000.0 + 10000.0 * (flops < 1e10 ? flops / 1e10 : 1.0) + flops / 1.5e6;
+    double library = 16000.0 + 10000.0 * (flops < 1e10 ? flops / 1e10 : 1.0) + flops / 1.3e6;
     if (kind == GT_GATES) library += 4000.0 + 6.0 * M * N / 4500.0;
-    return p.tile >= 0 && p.ns < library && flops <= (kind == GT_GATES ? GT_GATES_MOST : GT_PLAIN_MOST);
+    if (p.ns >= library || flops > (kind == GT_GATES ? GT_GATES_MOST : GT_PLAIN_MOST)) return 1;
+    return kind == GT_GATES && p.ns < 0.7 * library ? 3 : 2;
 }
 
 extern "C" int zi_gemm_tiles_count() { return GT_TILE_COUNT; }

@@ -15,10 +15,11 @@ from .functional import (add, add_rms_norm, argmax, attention, attention_decode,
                          decode_layer_workspace, device_synchronize, embedding, gather_rows, kv_store,
                          has_cuda, has_gpu, linear, linear_choose, linear_f32_kernel, linear_many_workspace, linear_splits, linear_sums,
                          linear_out_sums, linear_sums_supported, linear_clamped_glu, linear_swiglu, linear_swiglu_halves,
-                         linear_swiglu_halves_supported, linear_swiglu_many, linear_swiglu_many_pays, linear_tiles_gated, linear_tiles_gates_pay, linear_tiles_swiglu, linear_swiglu_pays, linear_swiglu_supported,
+                         linear_swiglu_halves_supported, linear_swiglu_many, linear_swiglu_many_pays, linear_tiles_gated, linear_tiles_gates_rule, linear_tiles_rule, linear_tiles_swiglu,
+                         linear_swiglu_pays, linear_swiglu_supported,
                          linear_transposed, linear_tune, reduce_sums, rms_norm, rope, rope_inv_freq,
                          rope_kv_store, rope_kv_store_sums, rope_table, sample, swiglu, swiglu_t,
-                         DECODE_LAYER_SPIN_LIMIT, FEW_ROWS, SUMS_MAX_ROWS)
+                         DECODE_LAYER_SPIN_LIMIT, FEW_ROWS, SUMS_MAX_ROWS, TILES_ABOVE, TILES_FASTER, TILES_SURELY)
 from .mixing import (delta_conv_state, delta_prepare, delta_rule, delta_rule_chunks_pay, delta_rule_step, delta_rule_steps, delta_rule_workspace, delta_state_floats, gated_act, gated_rms_norm,
                      latent_attention, latent_attention_cores, latent_attention_cores_plan,
                      latent_attention_cores_supported, latent_attention_cores_workspace, latent_inputs, latent_query, latent_query_cores, latent_store, latent_value, latent_value_gates,
@@ -50,7 +51,7 @@ __all__ = [
     "attention_prefill_workspace", "compute_units", "decode_layer", "decode_layer_stamps", "decode_layer_supported", "decode_layer_sync_words",
     "decode_layer_workspace", "device_synchronize", "embedding", "gather_rows", "has_cuda", "kv_store", "has_gpu",
     "linear", "linear_choose", "linear_f32_kernel", "linear_many_workspace", "linear_splits", "linear_out_sums", "linear_sums", "linear_sums_supported", "linear_swiglu",
-    "linear_swiglu_halves", "linear_swiglu_halves_supported", "linear_swiglu_many", "linear_swiglu_many_pays", "linear_tiles_gated", "linear_tiles_gates_pay", "linear_tiles_swiglu", "linear_swiglu_pays", "linear_swiglu_supported", "linear_transposed", "linear_tune", "reduce_sums", "rms_norm", "rope",
+    "linear_swiglu_halves", "linear_swiglu_halves_supported", "linear_swiglu_many", "linear_swiglu_many_pays", "linear_tiles_gated", "linear_tiles_gates_rule", "linear_tiles_rule", "linear_tiles_swiglu", "linear_swiglu_pays", "linear_swiglu_supported", "linear_transposed", "linear_tune", "reduce_sums", "rms_norm", "rope",
     "rope_inv_freq", "rope_kv_store", "rope_kv_store_sums", "rope_table", "sample", "swiglu", "swiglu_t",
     "delta_conv_state", "delta_prepare", "delta_rule", "delta_rule_chunks_pay", "delta_rule_step", "delta_rule_steps", "delta_rule_workspace", "delta_state_floats", "gated_act", "gated_rms_norm",
     "latent_attention", "latent_attention_cores", "latent_attention_cores_plan", "latent_attention_cores_supported",

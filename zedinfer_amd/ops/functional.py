@@ -2,6 +2,7 @@
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from ctypes import c_float, c_int, c_void_p
 from typing import Optional, Tuple
@@ -919,13 +920,13 @@ def attention_prefill(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tenso
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
            out: Optional[torch.Tensor] = None, out_dtype: Optional[torch.dtype] = None,
-           workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
+           workspace: Optional[torch.Tensor] = None, tiles: Optional[bool] = None) -> torch.Tensor:
     """out[M,N] = x[M,K] . weight[N,K]^T + bias[N], accumulated in float32
     (reference: src/backend/ops/linear/op.cpp:57-58).
 
     bfloat16 inputs with bfloat16 weights and output (or float32 output and more than 64 rows) go, of
-    more than 256 rows, to the tiles of ``csrc/gemm_tiles.hip`` where those were measured to be faster, else
-    to the library matrix product, as the reference sends them to its vendor library (reference:
+    more than 256 rows, to the tiles of ``csrc/gemm_tiles.hip`` by a rule on the sizes (``tiles`` True: wherever those take them,
+    False: never), else to the library matrix product, as the reference sends them to its vendor library (reference:
     src/backend/ops/linear/nvidia/linear_cublas.cu:134-231); float32 operands go to the
     matrix cores: up to 1,408 columns to their float32 instruction (products and sums in float32), beyond to the bfloat16 one as
     six products of the operands' three bfloat16 parts each, which hold all their bits, summed in float32 (the three products
@@ -953,7 +954,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
         return out
     bf = torch.bfloat16
     all_bf = x.dtype == bf and weight.dtype == bf and (bias is None or bias.dtype == bf)
-    if all_bf and _tiles_take(x, weight, out, bias, TILES_PLAIN):
+    if all_bf and _tiles_take(x, weight, out, bias, tiles):
         _lib.call("zi_gemm_tiles", _p(out), TILES_EPILOGUE[out.dtype], _p(x), _p(weight), _p(bias), M, N, K, ldx, ldw, ldo,
                   0, 0, -1, _stream())
         return out
@@ -998,8 +999,9 @@ def linear_transposed(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch
     return out
 
 
-TILES_PLAIN, TILES_GATES = 0, 1                      # what of a product ``zi_gemm_tiles_pays`` is asked about
-TILES_ABOVE = 256                                    # rows up to which it says no
+TILES_PLAIN, TILES_GATES = 0, 1                      # what of a product ``zi_gemm_tiles_pays`` is asked about ...
+TILES_TAKEN, TILES_FASTER, TILES_SURELY = 1, 2, 3    # ... and its answers, beside 0
+TILES_ABOVE = 256                                    # rows up to which it says 0
 TILES_EPILOGUE = {torch.bfloat16: 0, torch.float32: 1}      # the types that a whole product can be stored as, and the ends of the kernel that do
 
 
@@ -1012,28 +1014,41 @@ def _tiles_operands(x: torch.Tensor, weight: torch.Tensor) -> bool:
         and x.stride(0) <= 1 << 21 and weight.shape[0] * weight.stride(0) < 1 << 30
 
 
-def _tiles_pay(M: int, N: int, K: int, kind: int) -> bool:
-    return bool(_lib.load().zi_gemm_tiles_pays(int(M), int(N), int(K), kind))
+@functools.lru_cache(maxsize=4096)
+def _tiles_pay(M: int, N: int, K: int, kind: int) -> int:
+    return int(_lib.load().zi_gemm_tiles_pays(M, N, K, kind))
 
 
-def _tiles_take(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, bias: Optional[torch.Tensor], kind: int) -> bool:
-    """Whether ``linear`` gives the product to the tiles' kernel: operands and a result it can load and store, and sizes at which it
-    was measured to be faster than the library's product."""
-    return (_tiles_operands(x, weight) and out.dtype in TILES_EPILOGUE and out.stride(1) == 1 and out.data_ptr() % 16 == 0
-            and out.stride(0) % (4 if out.dtype == torch.float32 else 8) == 0 and (bias is None or bias.dtype == torch.bfloat16)
-            and _tiles_pay(x.shape[0], weight.shape[0], x.shape[1], kind))
+def _tiles_take(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, bias: Optional[torch.Tensor], tiles: Optional[bool] = None) -> bool:
+    """Whether ``linear`` gives the product to the tiles' kernel: operands and a result it can load and store, and sizes at which it is as
+    fast as the library's product by the rule, or for which the caller says so."""
+    if tiles is False or not (_tiles_operands(x, weight) and out.dtype in TILES_EPILOGUE and out.stride(1) == 1 and out.data_ptr() % 16 == 0
+                              and out.stride(0) % (4 if out.dtype == torch.float32 else 8) == 0 and (bias is None or bias.dtype == torch.bfloat16)):
+        return False
+    return _tiles_pay(x.shape[0], weight.shape[0], x.shape[1], TILES_PLAIN) >= (TILES_TAKEN if tiles else TILES_FASTER)
 
 
-def linear_tiles_gates_pay(x: torch.Tensor, weight: torch.Tensor, inter: int) -> bool:
-    """Whether the gate/up product of more than 256 rows with ``inter`` columns each is one that the tiles' kernel takes, the activation
-    in its end, and was measured to make faster than the library's product and the activation's launch."""
-    return int(inter) % 8 == 0 and _tiles_operands(x, weight) and _tiles_pay(x.shape[0], inter, x.shape[1], TILES_GATES)
+def linear_tiles_rule(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                      out_dtype: Optional[torch.dtype] = None) -> int:
+    """What the kernel library says of the tiles for ``linear`` of these operands and a contiguous result: 0, not taken; TILES_TAKEN, taken with
+    ``tiles=True``; TILES_FASTER, and by ``linear`` itself."""
+    if (out_dtype or torch.bfloat16) not in TILES_EPILOGUE or (bias is not None and bias.dtype != torch.bfloat16) \
+            or not _tiles_operands(x, weight) or weight.shape[0] % 8:
+        return 0
+    return _tiles_pay(x.shape[0], weight.shape[0], x.shape[1], TILES_PLAIN)
+
+
+def linear_tiles_gates_rule(x: torch.Tensor, weight: torch.Tensor, inter: int) -> int:
+    """What it says of the gate/up product of more than 256 rows with ``inter`` columns each and the activation in its end: 0, not taken;
+    TILES_TAKEN; TILES_FASTER than the library's product and the activation's launch; TILES_SURELY, by so much that measuring
+    both is not worth its time."""
+    return _tiles_pay(x.shape[0], int(inter), x.shape[1], TILES_GATES) if int(inter) % 8 == 0 and _tiles_operands(x, weight) else 0
 
 
 def _gates_out(what: str, x: torch.Tensor, weight: torch.Tensor, inter: int, out: Optional[torch.Tensor]):
     _gpu(what, x, weight, out)
-    if not linear_tiles_gates_pay(x, weight, inter):
-        raise ValueError(f"{what}: not a product of more than 256 rows that it is for")
+    if not linear_tiles_gates_rule(x, weight, inter):
+        raise ValueError(f"{what}: not a product of more than 256 rows that it takes")
     M = x.shape[0]
     if out is None:
         out = torch.empty((M, inter), dtype=torch.bfloat16, device=x.device)
@@ -1044,7 +1059,7 @@ def _gates_out(what: str, x: torch.Tensor, weight: torch.Tensor, inter: int, out
 
 
 def linear_tiles_swiglu(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """up * silu(gate) of x . weight^T in one kernel for more than 256 rows (``linear_tiles_gates_pay``), for a weight [2I, K]
+    """up * silu(gate) of x . weight^T in one kernel for more than 256 rows (``linear_tiles_gates_rule``), for a weight [2I, K]
     whose rows are 8 gate rows, then the 8 up rows of the same columns, and so on; out [M, I] bfloat16."""
     if weight.dim() != 2 or weight.shape[0] % 16:
         raise ValueError("linear_tiles_swiglu: the weight's rows must be whole blocks of 8 gate and 8 up rows")
@@ -1060,7 +1075,7 @@ GATED_ACTIVATIONS = {"silu": 0, "gelu_tanh": 1, "gelu_erf": 2}
 
 def linear_tiles_gated(x: torch.Tensor, weight: torch.Tensor, inter: int, up_at: int, activation: str,
                        out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """activation(gate) * up of x . weight^T in one kernel for more than 256 rows (``linear_tiles_gates_pay``): the first ``inter``
+    """activation(gate) * up of x . weight^T in one kernel for more than 256 rows (``linear_tiles_gates_rule``): the first ``inter``
     rows of the weight are the gates', those from row ``up_at`` on the ups'; out [M, inter] bfloat16."""
     if activation not in GATED_ACTIVATIONS:
         raise ValueError(f"linear_tiles_gated: unknown activation {activation!r}")
@@ -1095,10 +1110,11 @@ def _library_product(out, x, weight, bias, transposed) -> None:
 
 
 def linear_tune(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, transposed: bool = False,
-                out_dtype: Optional[torch.dtype] = None, candidates: Optional[int] = None, rounds: Optional[int] = None):
+                out_dtype: Optional[torch.dtype] = None, candidates: Optional[int] = None, rounds: Optional[int] = None,
+                tiles: Optional[bool] = None):
     """Let the library time its proposals for the product ``linear`` (``linear_transposed``) makes of these operands
     and keep the fastest for every later call of the shape; returns (chosen, proposed, microseconds), or None when
-    the product is not the library's (few rows, float32 operands, many rows that the tiles' kernel takes).  Waits for the device.  ``candidates``: how
+    the product is not the library's (few rows, float32 operands, many rows that ``linear`` with this ``tiles`` gives to the tiles' kernel).  Waits for the device.  ``candidates``: how
     many of the proposals are timed (None: the first 16, the first 8 of a product of about 250 us and more);
     ``rounds``: timed runs of each (None: five of a short product, fewer of one that takes long enough for the
     clock: three beyond about 50 us, two beyond 250)."""
@@ -1115,7 +1131,7 @@ def linear_tune(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     if M <= (SKINNY_MAX_ROWS if out_dtype == torch.float32 else FEW_ROWS) or (out_dtype == torch.float32 and bias is not None):
         return None
     out = torch.empty((N, M) if transposed else (M, N), dtype=out_dtype, device=x.device)
-    if not _library_ok(x, weight, out) or (not transposed and _tiles_take(x, weight, out, bias, TILES_PLAIN)):
+    if not _library_ok(x, weight, out) or (not transposed and _tiles_take(x, weight, out, bias, tiles)):
         return None
     chosen, proposed, us = c_int(0), c_int(0), c_float(0.0)
     _lib.call("zi_gemm_lt_tune", *_library_args(out, x, weight, bias, transposed), int(candidates), int(rounds),
@@ -1267,6 +1283,11 @@ def linear_swiglu_halves_supported(x: torch.Tensor, weight: torch.Tensor) -> boo
     return bool(_lib.load().zi_gemm_f32_swiglu_takes(_p(x), _p(weight), M, weight.shape[0] // 2, K, x.stride(0), weight.stride(0)))
 
 
+@functools.lru_cache(maxsize=4096)
+def _many_workspace(M: int, N: int, K: int, ldx: int, ldw: int, gated: int) -> int:
+    return int(_lib.load().zi_gemm_f32_many_workspace(M, N, K, ldx, ldw, gated, 0, 0, 0))
+
+
 def linear_many_workspace(x: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> int:
     """Bytes of workspace with which ``linear`` (``gated``: ``linear_swiglu_halves``) makes this product faster than without: float32
     products of many rows and more than 1,408 columns, whose x is split into its parts once, in the workspace; 0 for all others."""
@@ -1275,7 +1296,7 @@ def linear_many_workspace(x: torch.Tensor, weight: torch.Tensor, gated: bool = F
     M, K = x.shape
     if K != weight.shape[1] or max(M, K, weight.shape[0]) >= 1 << 31 or min(M, K, weight.shape[0]) < 1 or (gated and weight.shape[0] % 2):
         return 0
-    return int(_lib.load().zi_gemm_f32_many_workspace(M, weight.shape[0] // (2 if gated else 1), K, x.stride(0), weight.stride(0), int(gated), 0, 0, 0))
+    return _many_workspace(M, weight.shape[0] // (2 if gated else 1), K, x.stride(0), weight.stride(0), int(gated))
 
 
 def _linear_many(who: str, x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor, N: int, gated: bool,

@@ -17,6 +17,18 @@ from ..config.forward_config import PartSpec
 from ..weights.loader import WeightSpec
 
 
+def clock(fn: Callable[[], object], rounds: int = 3) -> float:
+    """Microseconds of a call, of ``rounds`` calls after one that does not count.  Waits for the device."""
+    fn()
+    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    a.record()
+    for _ in range(rounds):
+        fn()
+    b.record()
+    b.synchronize()
+    return a.elapsed_time(b) * 1000.0 / rounds
+
+
 class Runtime:
     """Device, activation type and reusable workspaces.
 
@@ -39,12 +51,63 @@ class Runtime:
         # the deciding part chooses.  They are made outside of steps (``Part.tune``, ``Engine.warm_up``)
         # or given by the caller, never while a step runs: a run with the same choices gives the same bits.
         self.choices: Dict[tuple, object] = {}
+        given = os.environ.get("ZEDINFER_PRODUCT_TILES", "")
+        self.product_tiles: Optional[bool] = given == "1" if given in ("0", "1") else None
+
+    @staticmethod
+    def _product_key(what: str, x: torch.Tensor, weight: torch.Tensor, bias: bool, transposed: bool, out_dtype: Optional[torch.dtype]) -> tuple:
+        return (what, int(x.shape[0]), int(weight.shape[0]), int(x.shape[1]), bias, transposed,
+                "float32" if out_dtype == torch.float32 else "bfloat16")
+
+    def tiles_recorded(self, what: str, x: torch.Tensor, weight: torch.Tensor, bias: bool = False,
+                       out_dtype: Optional[torch.dtype] = None) -> Optional[bool]:
+        """Whether the product of more than 256 rows (``what``: "tiles_product", or "tiles_gates" of a gate/up product) is made in tiles:
+        as ``choices`` says, where a record of the library's algorithm alone is an earlier run's that had it from the library; without one as
+        ZEDINFER_PRODUCT_TILES=0/1 says (1: wherever the tiles take it); None: by the rule of the kernel library."""
+        known = self.choices.get(self._product_key(what, x, weight, bias, False, out_dtype))
+        if known is None and self._product_key("library_product", x, weight, bias, False, out_dtype) in self.choices:
+            return False
+        if known is None:
+            return self.product_tiles
+        return bool(known)
+
+    def tiles_measured(self, what: str, x: torch.Tensor, weight: torch.Tensor, bias: bool = False, out_dtype: Optional[torch.dtype] = None) -> bool:
+        """Whether ``record_tiles`` left a record, now or in the run that the choices are of."""
+        return self._product_key(what, x, weight, bias, False, out_dtype) in self.choices
+
+    def linear(self, x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None,
+               workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """``ops.linear`` made as ``choices`` says where ``tune_linear`` left a record of it."""
+        from .. import ops
+        tiles = None
+        if x.shape[0] > ops.TILES_ABOVE and x.dtype == torch.bfloat16:
+            tiles = self.tiles_recorded("tiles_product", x, weight, bias is not None, out.dtype if out is not None else None)
+        return ops.linear(x, weight, bias, out=out, workspace=workspace, tiles=tiles)
+
+    def fill(self, x: torch.Tensor) -> torch.Tensor:
+        """Normal values in a workspace that a product is about to be timed with: on zeros and on what else a new allocation holds the chip runs
+        faster, some kernels more so than others (2,048 rows of 4,608 x 3,584: the library's 51 us instead of 60, the tiles' 57 instead of 61)."""
+        if x.device.type == "cuda":
+            x.normal_(generator=torch.Generator(device=x.device).manual_seed(1))
+        return x
+
+    def record_tiles(self, what: str, x: torch.Tensor, weight: torch.Tensor, rule: bool, library: Callable[[], object],
+                     tiles: Callable[[], object], bias: bool = False, out_dtype: Optional[torch.dtype] = None) -> None:
+        """Outside of any step: time both ways to a product and record the faster.  What the rule says stays unless the other is 3 % faster
+        (a choice that flips from run to run changes the rounding for nothing)."""
+        if x.device.type != "cuda":
+            return
+        us = [min(clock(fn), clock(fn)) for fn in (tiles, library)]
+        self.choices[self._product_key(what, x, weight, bias, False, out_dtype)] = bool(us[0] < us[1] / 0.97 if rule else us[0] < 0.97 * us[1])
 
     def tune_linear(self, x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
-                    transposed: bool = False, out_dtype: Optional[torch.dtype] = None, sums: bool = False) -> None:
+                    transposed: bool = False, out_dtype: Optional[torch.dtype] = None, sums: bool = False, tiles: bool = True) -> None:
         """Outside of any step: let the library choose, by timing its proposals, the algorithm of the product
         ``ops.linear`` (``ops.linear_transposed``) makes of operands of these shapes, and record the choice in
-        ``choices``; a choice already recorded there (an earlier run's) is put in force instead.  Nothing happens
+        ``choices``; a choice already recorded there (an earlier run's) is put in force instead.  Products of more than 256 rows
+        that the kernels in tiles take as well (``tiles``: of a caller that makes them with ``linear``) are then timed both ways, and
+        the faster is recorded too: at single sizes either is up to a third ahead of the other, which no rule on the sizes tells apart.
+        Nothing happens
         for products that are not the library's (few rows, float32; with ``sums``, of a caller that asks
         ``ops.linear_sums_supported`` first, more than 128 rows that it takes: up to there it takes every size, and
         ``choices`` would hold no record of having measured one) or with ZEDINFER_TUNE_LIBRARY=0."""
@@ -53,15 +116,27 @@ class Runtime:
         from .. import ops
         if sums and x.shape[0] > 128 and ops.linear_sums_supported(x, weight):
             return
-        key = ("library_product", int(x.shape[0]), int(weight.shape[0]), int(x.shape[1]), bias is not None,
-               bool(transposed), "float32" if out_dtype == torch.float32 else "bfloat16")
+        rule = ops.linear_tiles_rule(x, weight, bias, out_dtype) if tiles and not transposed else 0
+        tiles = rule > 0
+        given = self.tiles_recorded("tiles_product", x, weight, bias is not None, out_dtype) if tiles else None
+        if given:
+            return
+        key = self._product_key("library_product", x, weight, bias is not None, bool(transposed), out_dtype)
         known = self.choices.get(key)
         if known is not None:
             ops.linear_choose(x, weight, int(known), bias, transposed, out_dtype)
             return
-        found = ops.linear_tune(x, weight, bias, transposed, out_dtype)
-        if found is not None:
-            self.choices[key] = found[0]
+        if tiles and given is None:
+            self.fill(x)
+        found = ops.linear_tune(x, weight, bias, transposed, out_dtype, tiles=False)
+        if found is None:
+            return
+        if tiles and given is None:
+            out = torch.empty((x.shape[0], weight.shape[0]), dtype=out_dtype or torch.bfloat16, device=x.device)
+            self.record_tiles("tiles_product", x, weight, rule >= ops.TILES_FASTER,
+                              lambda: ops.linear(x, weight, bias, out=out, tiles=False),
+                              lambda: ops.linear(x, weight, bias, out=out, tiles=True), bias is not None, out_dtype)
+        self.choices[key] = found[0]
 
     def buffer(self, name: str, shape: Tuple[int, ...], dtype: Optional[torch.dtype] = None) -> torch.Tensor:
         dtype = dtype or self.dtype

@@ -85,7 +85,7 @@ class GatedDeltaRule(Mixer):
     def forward(self, x: torch.Tensor, batch, memory: LayerMemory, out=None) -> torch.Tensor:
         n, rt, nh, kvh, dim, vdim = x.shape[0], self.rt, self.nh, self.kvh, self.dim, self.vdim
         state = memory.state
-        full = ops.linear(x, self.w_in, out=rt.buffer("delta_proj", (n, self.w_in.shape[0]), torch.float32))
+        full = self.rt.linear(x, self.w_in, out=rt.buffer("delta_proj", (n, self.w_in.shape[0]), torch.float32))
         proj = full[:, :self.width]
         qk = rt.buffer("delta_qk", (n, 2 * kvh * dim), torch.float32)
         v = rt.buffer("delta_v", (n, nh * vdim), torch.float32)
@@ -114,7 +114,7 @@ class GatedDeltaRule(Mixer):
             out = rt.buffer("delta_out", (n, self.hidden))
         if out.dim() == 3:
             return ops.linear_sums(y, self.o, out=out)
-        return ops.linear(y, self.o, out=out)
+        return self.rt.linear(y, self.o, out=out)
 
 
 @register_mixer("channel_delta_rule")
@@ -215,7 +215,7 @@ class ChannelDeltaRule(Mixer):
             proj = ops.linear_sums(x, self.w_in, out=rt.buffer("delta_proj_sums", (S, n, self.width), torch.float32))
             rest = gates = rt.buffer("delta_lowrank", (n, self.b_at - self.a_at), torch.float32)
         else:
-            proj = ops.linear(x, self.w_in, out=rt.buffer("delta_proj", (n, self.width), torch.float32))
+            proj = self.rt.linear(x, self.w_in, out=rt.buffer("delta_proj", (n, self.width), torch.float32))
             gates = proj[:, self.a_at:self.b_at]
         qk = rt.buffer("delta_qk", (n, 2 * kvh * dim), torch.float32)
         v = rt.buffer("delta_v", (n, nh * vdim), torch.float32)
@@ -237,4 +237,4 @@ class ChannelDeltaRule(Mixer):
         if ops.linear_sums_supported(y, self.o):      # few rows: the partial sums go to the norm that follows
             S = ops.linear_splits(n, self.hidden, nh * vdim)
             return ops.linear_sums(y, self.o, out=rt.buffer("delta_out_sums", (S, n, self.hidden), torch.float32))
-        return ops.linear(y, self.o, out=rt.buffer("delta_out", (n, self.hidden)))
+        return self.rt.linear(y, self.o, out=rt.buffer("delta_out", (n, self.hidden)))

@@ -102,7 +102,7 @@ class DifferenceAttention(Attention):
             S = ops.linear_splits(n, rows, self.hidden)
             full = ops.linear_sums(x, self.qkvg, out=rt.buffer("difference_proj_sums", (S, n, rows), torch.float32))
         else:
-            full = ops.linear(x, self.qkvg, out=rt.buffer("difference_proj", (n, rows)))
+            full = self.rt.linear(x, self.qkvg, out=rt.buffer("difference_proj", (n, rows)))
         gate = full[..., self.width:self.width + self.heads] if self.gated else None
         writes, plan = memory.writes, batch.plans[self.plan_key]
         # the rest of the query rows is zeroed unless nobody reads it
@@ -130,4 +130,4 @@ class DifferenceAttention(Attention):
         if ops.linear_sums_supported(att, self.o):
             S = ops.linear_splits(n, self.hidden, self.o.shape[1])
             return ops.linear_sums(att, self.o, out=self.rt.buffer("attn_proj_sums", (S, n, self.hidden), torch.float32))
-        return ops.linear(att, self.o, out=self.rt.buffer("attn_proj", (n, self.hidden)))
+        return self.rt.linear(att, self.o, out=self.rt.buffer("attn_proj", (n, self.hidden)))

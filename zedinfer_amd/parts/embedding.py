@@ -109,7 +109,7 @@ class LinearHead(Part):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         out = self.rt.buffer("logits", (x.shape[0], self.vocab), torch.float32)
-        ops.linear(x, self.weight, out=out)
+        self.rt.linear(x, self.weight, out=out)
         if self.softcap is not None:
             ops.softcap(out, self.softcap)
         return out

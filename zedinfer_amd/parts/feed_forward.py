@@ -9,7 +9,7 @@ import torch
 from .. import ops
 from ..config.forward_config import PartSpec
 from ..weights.loader import WeightSpec
-from .base import FeedForward, Runtime, register_feed_forward
+from .base import FeedForward, Runtime, clock, register_feed_forward
 from .rows import ProductRows
 
 
@@ -40,14 +40,17 @@ class SwiGLU(FeedForward):
 
     graph_safe = True
     tape_safe = True
-    # For many rows the gate/up product is made in tiles that end in the activation (``ops.linear_tiles_swiglu``) or the library's, and at some sizes it makes the transposed
+    # For many rows the gate/up product is made in tiles that end in the activation (``ops.linear_tiles_swiglu``, more than 256 rows)
+    # or the library's, and at some sizes the library makes the transposed
     # result, W . x^T, faster than x . W^T (measured at the 1.5B sizes: 100 against 119 us at 2,048 rows,
     # 31 against 37 at 512, 73 against 67 at 1,024).  The transposed result goes through the activation
-    # kernel that turns it back; the two ways differ by rounding.  Which one a step of n rows takes is
-    # read from ``rt.choices[("gate_up_transposed", n, 2I, H)]``: absent, the straight product (or what
-    # ZEDINFER_GATE_UP_TRANSPOSED=0/1 says).  ``tune(n)`` measures both outside of any step and records
-    # the winner there; nothing is measured while a step runs.  (Up to 256 rows the products at which the few-rows
-    # kernels' epilogue pays are theirs, and neither a choice nor the variable is asked.)
+    # kernel that turns it back; the ways differ by rounding.  Which one a step of n rows takes is
+    # read from ``rt.choices``.  ("tiles_gates", n, 2I, H, ..): tiles or the library; absent, the library where a choice about it
+    # is recorded (an earlier run's) or ZEDINFER_GATE_UP_TRANSPOSED is 0 or 1, else what ZEDINFER_PRODUCT_TILES or the rule on the sizes says.
+    # ("gate_up_transposed", n, 2I, H): the library's way round; absent, the straight product (or what
+    # ZEDINFER_GATE_UP_TRANSPOSED=0/1 says).  ``tune(n)`` measures the ways outside of any step and records
+    # the winners there, but for tiles that are faster by far in any case; nothing is measured while a step runs.  (Up to 256 rows the
+    # products at which the few-rows kernels' epilogue pays are theirs, and neither a choice nor a variable is asked.)
     TRANSPOSED_MIN_ROWS = 128
 
     @staticmethod
@@ -62,13 +65,22 @@ class SwiGLU(FeedForward):
         return (self.interleave == GATE_UP_BLOCK and self.rt.dtype == torch.bfloat16
                 and n >= self.TRANSPOSED_MIN_ROWS and n % 8 == 0)
 
+    def _tiles_given(self, x: torch.Tensor) -> Optional[bool]:
+        """What ``choices`` and the variables say of tiles for the gate/up product of x; None: nothing."""
+        if not self.rt.tiles_measured("tiles_gates", x, self.gate_up) \
+                and (self._choice_key(x.shape[0]) in self.rt.choices or os.environ.get("ZEDINFER_GATE_UP_TRANSPOSED", "") in ("0", "1")):
+            return False
+        return self.rt.tiles_recorded("tiles_gates", x, self.gate_up)
+
     def _tiles(self, x: torch.Tensor) -> bool:
         """Steps of more than 256 rows whose gate/up product is made in tiles that end in the activation."""
-        return self.interleave == GATE_UP_BLOCK and ops.linear_tiles_gates_pay(x, self.gate_up, self.inter)
+        rule = ops.linear_tiles_gates_rule(x, self.gate_up, self.inter) if self.interleave == GATE_UP_BLOCK else 0
+        given = self._tiles_given(x) if rule else False
+        return rule >= ops.TILES_FASTER if given is None else given
 
     def _gate_up_straight(self, x: torch.Tensor, act: torch.Tensor) -> None:
         gu = self.rt.buffer("ffn_gate_up", (x.shape[0], 2 * self.inter))
-        ops.linear(x, self.gate_up, out=gu)
+        ops.linear(x, self.gate_up, out=gu, tiles=False)
         ops.swiglu(gu, out=act, interleave=self.interleave)
 
     def _gate_up_transposed(self, x: torch.Tensor, act: torch.Tensor) -> None:
@@ -95,32 +107,31 @@ class SwiGLU(FeedForward):
     def tune(self, num_tokens: int) -> None:
         """For steps of ``num_tokens`` rows: the library's algorithms for those of the gate/up and down products that it
         makes (up to 128 rows for both), then the orientation of the gate/up product: three runs each of product plus activation; the
-        transposed one must win by 5 %."""
+        transposed one must win by 5 %.  Then that against the tiles, where these take it and the rule is not sure."""
         n, key = int(num_tokens), self._choice_key(num_tokens)
         x = self.rt.buffer("norm_out", (n, self.hidden))
         act = self.rt.buffer("ffn_act", (n, self.inter))
         self.rt.tune_linear(act, self.down, sums=True)
-        if self.interleave and (ops.linear_swiglu_many_pays(x, self.gate_up) or self._tiles(x)):
+        if self.interleave and ops.linear_swiglu_many_pays(x, self.gate_up):
             return
+        rule = ops.linear_tiles_gates_rule(x, self.gate_up, self.inter) if self.interleave == GATE_UP_BLOCK else 0
+        given = self._tiles_given(x) if rule else False
+        if given or (given is None and rule >= ops.TILES_SURELY):
+            return
+        if given is None:
+            self.rt.fill(x)
         # first the library's algorithm, then the way round with it
         if self.gate_up is not None:
-            self.rt.tune_linear(x, self.gate_up)
+            self.rt.tune_linear(x, self.gate_up, tiles=not self.interleave)
             if self._can_transpose(n):
                 self.rt.tune_linear(x, self.gate_up, transposed=True)
         forced = os.environ.get("ZEDINFER_GATE_UP_TRANSPOSED", "")
-        if key in self.rt.choices or not self._can_transpose(n) or forced in ("0", "1"):
-            return
-
-        def clock(fn):
-            fn(x, act)
-            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            a.record()
-            for _ in range(3):
-                fn(x, act)
-            b.record()
-            b.synchronize()
-            return a.elapsed_time(b)
-        self.rt.choices[key] = bool(clock(self._gate_up_transposed) < 0.95 * clock(self._gate_up_straight))
+        if key not in self.rt.choices and self._can_transpose(n) and forced not in ("0", "1"):
+            transposed, straight = (clock(lambda: way(x, act)) for way in (self._gate_up_transposed, self._gate_up_straight))
+            self.rt.choices[key] = bool(transposed < 0.95 * straight)
+        if given is None:
+            self.rt.record_tiles("tiles_gates", x, self.gate_up, rule >= ops.TILES_FASTER,
+                                 lambda: self._gate_up_many_rows(x, act), lambda: ops.linear_tiles_swiglu(x, self.gate_up, out=act))
 
     def __init__(self, spec: PartSpec, weights: Dict[str, torch.Tensor], rt: Runtime):
         super().__init__(spec, weights, rt)
@@ -159,10 +170,10 @@ class SwiGLU(FeedForward):
         else:
             gu = self.rt.buffer("ffn_gate_up", (n, 2 * I))
             if self.gate_up is not None:
-                ops.linear(x, self.gate_up, out=gu)
+                self.rt.linear(x, self.gate_up, out=gu)
             else:
-                ops.linear(x, self.gate, out=gu[:, :I])
-                ops.linear(x, self.up, out=gu[:, I:])
+                self.rt.linear(x, self.gate, out=gu[:, :I])
+                self.rt.linear(x, self.up, out=gu[:, I:])
             if self.interleave:
                 ops.swiglu(gu, out=act, interleave=self.interleave)
             else:
@@ -171,7 +182,7 @@ class SwiGLU(FeedForward):
             S = ops.linear_splits(n, self.hidden, I)
             return ops.linear_sums(act, self.down, out=self.rt.buffer("ffn_out_sums", (S, n, self.hidden), torch.float32))
         out = self.rt.buffer("ffn_out", (n, self.hidden))
-        return ops.linear(act, self.down, out=out, workspace=self.rt.product_workspace(act, self.down))
+        return self.rt.linear(act, self.down, out=out, workspace=self.rt.product_workspace(act, self.down))
 
 
 @register_feed_forward("none")
@@ -225,9 +236,34 @@ class GatedMLP(FeedForward):
         return ProductRows.step_rows(rows, kind)
 
     def tune(self, num_tokens: int) -> None:
-        x = self.rt.buffer("norm_out", (int(num_tokens), self.hidden))
-        if not ops.linear_tiles_gates_pay(x, self.gate_up, self.inter):
-            self.rt.tune_linear(x, self.gate_up)
+        """For steps of ``num_tokens`` rows: the library's algorithm for the gate/up product where it makes that, and the library against the
+        tiles where these take it and the rule is not sure."""
+        n = int(num_tokens)
+        x, act = self.rt.buffer("norm_out", (n, self.hidden)), self.rt.buffer("ffn_act", (n, self.inter))
+        rule = ops.linear_tiles_gates_rule(x, self.gate_up, self.inter)
+        given = self.rt.tiles_recorded("tiles_gates", x, self.gate_up) if rule else False
+        if given or (given is None and rule >= ops.TILES_SURELY):
+            return
+        if given is None:
+            self.rt.fill(x)
+        self.rt.tune_linear(x, self.gate_up, tiles=False)
+        if given is None and os.environ.get("ZEDINFER_TUNE_LIBRARY", "1") != "0":
+            self.rt.record_tiles("tiles_gates", x, self.gate_up, rule >= ops.TILES_FASTER,
+                                 lambda: self._gate_up_apart(x, act), lambda: self._gate_up_tiles(x, act))
+
+    def _gate_up_tiles(self, x: torch.Tensor, act: torch.Tensor) -> None:
+        ops.linear_tiles_gated(x, self.gate_up, self.inter, self.up_at, self.activation, out=act)
+
+    def _gate_up_apart(self, x: torch.Tensor, act: torch.Tensor) -> None:
+        gu = self.rt.buffer("ffn_gate_up", (x.shape[0], self.up_at + self.inter))
+        ops.linear(x, self.gate_up, out=gu, tiles=False)
+        ops.gated_act(gu[:, :self.inter], gu[:, self.up_at:], self.activation, out=act)
+
+    def _tiles(self, x: torch.Tensor) -> bool:
+        """Steps of more than 256 rows whose gate/up product is made in tiles that end in the activation."""
+        rule = ops.linear_tiles_gates_rule(x, self.gate_up, self.inter)
+        given = self.rt.tiles_recorded("tiles_gates", x, self.gate_up) if rule else False
+        return rule >= ops.TILES_FASTER if given is None else given
 
     def out_sums(self, rows: int) -> int:
         return ops.linear_out_sums(self.rt.dtype, rows, self.down)
@@ -235,17 +271,15 @@ class GatedMLP(FeedForward):
     def forward(self, x: torch.Tensor, out=None) -> torch.Tensor:
         n, I = x.shape[0], self.inter
         act = self.rt.buffer("ffn_act", (n, I))
-        if ops.linear_tiles_gates_pay(x, self.gate_up, I):
-            ops.linear_tiles_gated(x, self.gate_up, I, self.up_at, self.activation, out=act)
+        if self._tiles(x):
+            self._gate_up_tiles(x, act)
         else:
-            gu = self.rt.buffer("ffn_gate_up", (n, self.up_at + I))
-            ops.linear(x, self.gate_up, out=gu)
-            ops.gated_act(gu[:, :I], gu[:, self.up_at:], self.activation, out=act)
+            self._gate_up_apart(x, act)
         if out is None:
             out = self.rt.buffer("ffn_out", (n, self.hidden))
         if out.dim() == 3:
             return ops.linear_sums(act, self.down, out=out)
-        return ops.linear(act, self.down, out=out)
+        return self.rt.linear(act, self.down, out=out)
 
 
 @register_feed_forward("routed_experts")
@@ -292,7 +326,7 @@ class RoutedExperts(FeedForward):
     def forward(self, x: torch.Tensor, out=None) -> torch.Tensor:
         n, E, top, rt = x.shape[0], self.experts, self.top, self.rt
         pairs = n * top
-        z = ops.linear(x, self.router, out=rt.buffer("moe_logits", (n, E), torch.float32))
+        z = self.rt.linear(x, self.router, out=rt.buffer("moe_logits", (n, E), torch.float32))
         idx = rt.buffer("moe_choice", (n, top), torch.int32)
         wt = rt.buffer("moe_weight", (n, top), torch.float32)
         ops.moe_route(z, self.correction, top, self.scale, idx, wt)
@@ -317,7 +351,7 @@ def _float_result(rt: Runtime, name: str, x: torch.Tensor, weight: torch.Tensor)
     if ops.linear_sums_supported(x, weight):
         S = ops.linear_splits(n, N, x.shape[1])
         return ops.linear_sums(x, weight, out=rt.buffer(name + "_sums", (S, n, N), torch.float32))
-    return ops.linear(x, weight, out=rt.buffer(name, (n, N), torch.float32))
+    return rt.linear(x, weight, out=rt.buffer(name, (n, N), torch.float32))
 
 
 @register_feed_forward("relu2_mlp")
@@ -354,7 +388,7 @@ class ReluSquaredMLP(FeedForward):
             S = ops.linear_splits(n, I, self.hidden)
             z = ops.linear_sums(x, self.up, out=rt.buffer("ffn_up_sums", (S, n, I), torch.float32))
         else:
-            z = ops.linear(x, self.up, out=rt.buffer("ffn_up", (n, I)))
+            z = self.rt.linear(x, self.up, out=rt.buffer("ffn_up", (n, I)))
         ops.relu_squared(z, out=act)
         return _float_result(rt, "ffn_out_f32", act, self.down)
 
@@ -400,12 +434,12 @@ class ActivatedMLP(FeedForward):
                 S = ops.linear_splits(n, I, self.hidden)
                 z = ops.linear_sums(x, self.up, out=rt.buffer("ffn_up_sums", (S, n, I), torch.float32))
             else:
-                z = ops.linear(x, self.up, out=rt.buffer("ffn_up", (n, I)))
+                z = self.rt.linear(x, self.up, out=rt.buffer("ffn_up", (n, I)))
             ops.activate(z, self.activation, out=act)
         if ops.linear_sums_supported(act, self.down):
             S = ops.linear_splits(n, self.hidden, I)
             return ops.linear_sums(act, self.down, out=rt.buffer("ffn_out_sums", (S, n, self.hidden), torch.float32))
-        return ops.linear(act, self.down, out=rt.buffer("ffn_out", (n, self.hidden)))
+        return self.rt.linear(act, self.down, out=rt.buffer("ffn_out", (n, self.hidden)))
 
 
 class _ClampedGated:
@@ -433,7 +467,7 @@ class _ClampedGated:
             gu = ops.linear_sums(x, self.gate_up, out=rt.buffer(name + "_gate_up_sums", (S, n, self.up_at + I), torch.float32))
             ops.clamped_glu(gu[:, :, :I], gu[:, :, self.up_at:], self.limit, out=act, **self.biases)
         else:
-            gu = ops.linear(x, self.gate_up, out=rt.buffer(name + "_gate_up", (n, self.up_at + I), torch.float32))
+            gu = rt.linear(x, self.gate_up, out=rt.buffer(name + "_gate_up", (n, self.up_at + I), torch.float32))
             ops.clamped_glu(gu[:, :I], gu[:, self.up_at:], self.limit, out=act, **self.biases)
         return act
 
@@ -499,13 +533,13 @@ class ClampedMLP(FeedForward):
             if n <= ops.FEW_ROWS and ops.linear_swiglu_supported(x, self.interleaved):
                 ops.linear_clamped_glu(x, self.interleaved, self.gate_up_bias, self.limit, out=act)
             else:
-                gu = ops.linear(x, self.interleaved, self.gate_up_bias, out=rt.buffer("ffn_gate_up", (n, 2 * self.inter)))
+                gu = self.rt.linear(x, self.interleaved, self.gate_up_bias, out=rt.buffer("ffn_gate_up", (n, 2 * self.inter)))
                 ops.clamped_glu_il8(gu, self.limit, out=act)
         if ops.linear_sums_supported(act, self.down):
             S = ops.linear_splits(n, self.hidden, self.inter)
             return ops.linear_sums(act, self.down, bias=self.down_bias,
                                    out=rt.buffer("ffn_out_sums", (S, n, self.hidden), torch.float32))
-        return ops.linear(act, self.down, self.down_bias, out=rt.buffer("ffn_out", (n, self.hidden)))
+        return self.rt.linear(act, self.down, self.down_bias, out=rt.buffer("ffn_out", (n, self.hidden)))
 
 
 @register_feed_forward("clamped_experts")
@@ -577,7 +611,7 @@ class ClampedExperts(FeedForward):
             probe = rt.buffer("moe_shared_act", (n, self.shared.inter))
             shared_sums = ops.linear_splits(n, self.hidden, self.shared.inter) if ops.linear_sums_supported(probe, self.shared.down) else 0
         terms = rt.buffer("moe_terms", (1 + (shared_sums or (1 if self.shared is not None else 0)), n, self.hidden), torch.float32)
-        z = ops.linear(x, self.router, out=rt.buffer("moe_logits", (n, E), torch.float32))
+        z = self.rt.linear(x, self.router, out=rt.buffer("moe_logits", (n, E), torch.float32))
         idx = rt.buffer("moe_choice", (n, top), torch.int32)
         wt = rt.buffer("moe_weight", (n, top), torch.float32)
         ops.moe_route_top(z, self.router_bias, top, idx, wt)
@@ -599,7 +633,7 @@ class ClampedExperts(FeedForward):
             if shared_sums:
                 ops.linear_sums(act_s, self.shared.down, out=terms[1:])
             else:
-                ops.linear(act_s, self.shared.down, out=terms[1])
+                self.rt.linear(act_s, self.shared.down, out=terms[1])
         return terms
 
 
@@ -738,7 +772,7 @@ class ScoredExperts(FeedForward):
     def forward(self, x: torch.Tensor, out=None) -> torch.Tensor:
         n, E, top, ff, rt = x.shape[0], self.experts, self.top, self.ff, self.rt
         pairs = n * top
-        z = ops.linear(x, self.router, out=rt.buffer("moe_logits", (n, self.router.shape[0]), torch.float32))
+        z = self.rt.linear(x, self.router, out=rt.buffer("moe_logits", (n, self.router.shape[0]), torch.float32))
         idx = rt.buffer("moe_choice", (n, top), torch.int32)
         wt = rt.buffer("moe_weight", (n, top), torch.float32)
         ops.moe_route_sigmoid(z, E, top, idx, wt)

@@ -174,7 +174,7 @@ class LatentAttention(Mixer):
             S = ops.linear_splits(n, rows, self.hidden)
             full = ops.linear_sums(x, self.inputs, out=rt.buffer("latent_inputs_sums", (S, n, rows), torch.float32))
         else:
-            full = ops.linear(x, self.inputs, out=rt.buffer("latent_inputs", (n, rows), self.inputs_dtype()))
+            full = self.rt.linear(x, self.inputs, out=rt.buffer("latent_inputs", (n, rows), self.inputs_dtype()))
         cq = rt.buffer("latent_cq_normed", (n, self.q_rank))
         if memory.writes:
             ops.latent_inputs(full, self.dq_norm, self.eps, cq, self.dkv_at, self.dkv_norm, table, view.slots,
@@ -197,19 +197,19 @@ class LatentAttention(Mixer):
         if self.inputs is not None:
             x, gate = self.gated_inputs(x, batch, view, memory, table)
         elif self.gate is not None:
-            gate = ops.linear(x, self.gate, out=rt.buffer("latent_gate", (n, self.nh * self.vdim), torch.float32))
+            gate = self.rt.linear(x, self.gate, out=rt.buffer("latent_gate", (n, self.nh * self.vdim), torch.float32))
         if memory.writes and self.inputs is None:
-            dkv = ops.linear(x, self.dkv, out=rt.buffer("latent_dkv", (n, self.rank + self.rot), torch.float32))
+            dkv = self.rt.linear(x, self.dkv, out=rt.buffer("latent_dkv", (n, self.rank + self.rot), torch.float32))
             ops.latent_store(dkv, self.dkv_norm, self.eps, table, view.slots, c_cache, kr_cache, self.rank, self.rot)
         if self.q_rank and self.inputs is None:
-            cq = ops.linear(x, self.dq, out=rt.buffer("latent_cq", (n, self.q_rank), torch.float32))
+            cq = self.rt.linear(x, self.dq, out=rt.buffer("latent_cq", (n, self.q_rank), torch.float32))
             x = ops.rms_norm(cq, self.dq_norm, self.eps, out=rt.buffer("latent_cq_normed", (n, self.q_rank)))
         width = self.nh * (self.dim + self.rot)
         if self.short_query and ops.linear_sums_supported(x, self.q):      # few rows: the next kernel adds the partial sums
             S = ops.linear_splits(n, width, self.q.shape[1])
             q = ops.linear_sums(x, self.q, out=rt.buffer("latent_q_sums", (S, n, width), torch.float32))
         else:
-            q = ops.linear(x, self.q, out=rt.buffer("latent_q", (n, width), self.query_dtype()))
+            q = self.rt.linear(x, self.q, out=rt.buffer("latent_q", (n, width), self.query_dtype()))
         # between the products on the matrix cores, rows in bfloat16: what the next product would round them to
         qa = rt.buffer("latent_qa", (n, self.nh, self.rank + self.rot), torch.bfloat16 if self.short_query else torch.float32)
         ops.latent_query(q, self.uk, table, self.nh, self.dim, self.rank, self.rot, out=qa, w_uk_t=self.uk_t)
@@ -237,4 +237,4 @@ class LatentAttention(Mixer):
             out = rt.buffer("latent_out", (n, self.hidden))
         if out.dim() == 3:
             return ops.linear_sums(heads, self.o, out=out)
-        return ops.linear(heads, self.o, out=out)
+        return self.rt.linear(heads, self.o, out=out)

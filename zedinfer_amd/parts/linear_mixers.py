@@ -105,7 +105,7 @@ class ProjectedMixer(Mixer):
     def forward(self, x: torch.Tensor, batch, memory: LayerMemory, out=None) -> torch.Tensor:
         n, rt = x.shape[0], self.rt
         h = self.shifted(x, batch, memory)
-        proj = ops.linear(h, self.w_in, out=rt.buffer("mix_proj", (n, self.w_in.shape[0]), torch.float32))
+        proj = self.rt.linear(h, self.w_in, out=rt.buffer("mix_proj", (n, self.w_in.shape[0]), torch.float32))
         y = rt.buffer("mix_y", (n, self.w_out.shape[1]))
         at = self.hidden if self.shift is not None else 0
         state = memory.state[:, at:at + self.state_floats] if self.state_floats else None
@@ -117,7 +117,7 @@ class ProjectedMixer(Mixer):
                 S = ops.linear_splits(n, self.hidden, self.w_out.shape[1])
                 return ops.linear_sums(y, self.w_out, out=rt.buffer("mix_out_sums", (S, n, self.hidden), torch.float32))
             out = rt.buffer("mix_out", (n, self.hidden), torch.float32)
-        return ops.linear(y, self.w_out, out=out)
+        return self.rt.linear(y, self.w_out, out=out)
 
 
 @register_mixer("lightning_attention")

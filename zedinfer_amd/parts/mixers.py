@@ -330,7 +330,7 @@ class Attention(Mixer):
             q, k, v = (self.rt.buffer(name, (n, width)) for name, width in
                        (("attn_q", self.qd), ("attn_k", self.kvd), ("attn_v", self.kvd)))
             for dst, m, b in zip((q, k, v), self.mats, self.biases or (None, None, None)):
-                ops.linear(x, m, b, out=dst)
+                self.rt.linear(x, m, b, out=dst)
             # every head is a row of head_dim values: normed in place
             ops.rms_norm(q.view(n * self.nh, self.d), self.q_norm, self.qk_norm_eps, out=q.view(n * self.nh, self.d))
             ops.rms_norm(k.view(n * self.nkv, self.d), self.k_norm, self.qk_norm_eps, out=k.view(n * self.nkv, self.d))
@@ -349,10 +349,10 @@ class Attention(Mixer):
             qkv = self.rt.buffer("attn_qkv", (n, self.qd + 2 * self.kvd))
             q, k, v = qkv[:, :self.qd], qkv[:, self.qd:self.qd + self.kvd], qkv[:, self.qd + self.kvd:]
             if self.qkv is not None:
-                ops.linear(x, self.qkv, self.bias, out=qkv, workspace=self.rt.product_workspace(x, self.qkv))
+                self.rt.linear(x, self.qkv, self.bias, out=qkv, workspace=self.rt.product_workspace(x, self.qkv))
             else:
                 for dst, m, b in zip((q, k, v), self.mats, self.biases or (None, None, None)):
-                    ops.linear(x, m, b, out=dst)
+                    self.rt.linear(x, m, b, out=dst)
             self.encode_and_store(q, k, v, batch, view, memory)
         att = self.rt.buffer("attn_out", (n, self.qd))
         self.attend(q, att, batch, view, memory)
@@ -374,7 +374,7 @@ class Attention(Mixer):
             S = ops.linear_splits(n, self.hidden, self.qd)
             return ops.linear_sums(att, self.o, out=self.rt.buffer("attn_proj_sums", (S, n, self.hidden), torch.float32))
         out = self.rt.buffer("attn_proj", (n, self.hidden))
-        return ops.linear(att, self.o, out=out, workspace=self.rt.product_workspace(att, self.o))
+        return self.rt.linear(att, self.o, out=out, workspace=self.rt.product_workspace(att, self.o))
 
     def decode_from_sums(self, sums, batch, view, memory: LayerMemory) -> Optional[torch.Tensor]:
         """A pure decode step (one token a sequence): rotation, cache store and attention in one kernel,
@@ -535,7 +535,7 @@ class ConvAttention(Attention):
         if ops.linear_sums_supported(att, self.o):
             S = ops.linear_splits(n, self.hidden, self.o.shape[1])
             return ops.linear_sums(att, self.o, out=self.rt.buffer("attn_proj_sums", (S, n, self.hidden), torch.float32))
-        return ops.linear(att, self.o, out=self.rt.buffer("attn_proj_f32", (n, self.hidden), torch.float32))
+        return self.rt.linear(att, self.o, out=self.rt.buffer("attn_proj_f32", (n, self.hidden), torch.float32))
 
     def forward(self, x: torch.Tensor, batch, memory: LayerMemory) -> torch.Tensor:
         n, rt = x.shape[0], self.rt
@@ -548,7 +548,7 @@ class ConvAttention(Attention):
             S = ops.linear_splits(n, self.qkv.shape[0], self.hidden)
             full = ops.linear_sums(x, self.qkv, out=rt.buffer("conv_attn_sums", (S, n, self.qkv.shape[0]), torch.float32))
         else:
-            full = ops.linear(x, self.qkv, out=rt.buffer("conv_attn_proj", (n, self.qkv.shape[0]), torch.float32))
+            full = self.rt.linear(x, self.qkv, out=rt.buffer("conv_attn_proj", (n, self.qkv.shape[0]), torch.float32))
         proj = full[..., :self.channels] if self.gated else full
         gate = full[..., self.gate_at:] if self.gated else None
         q = rt.buffer("attn_q", (n, self.qd))

@@ -151,7 +151,7 @@ class PooledWindowAttention(Mixer):
             S = ops.linear_splits(n, self.width, self.hidden)
             proj = ops.linear_sums(x, self.qkv, out=rt.buffer("pooled_qkv_sums", (S, n, self.width), torch.float32))
         else:
-            proj = ops.linear(x, self.qkv, out=rt.buffer("pooled_qkv", (n, self.qkv.shape[0]), torch.float32))[:, :self.width]
+            proj = self.rt.linear(x, self.qkv, out=rt.buffer("pooled_qkv", (n, self.qkv.shape[0]), torch.float32))[:, :self.width]
         q = rt.buffer("pooled_q", (n, self.nh * self.d))
         writes = memory.writes
         ops.norm_rope_store(proj, self.q_gain, self.k_gain, self.eps, table, vtable,
@@ -189,4 +189,4 @@ class PooledWindowAttention(Mixer):
                 S = ops.linear_splits(n, self.hidden, self.nh * self.vd)
                 return ops.linear_sums(heads, self.o, out=rt.buffer("pooled_out_sums", (S, n, self.hidden), torch.float32))
             out = rt.buffer("pooled_out", (n, self.hidden))
-        return ops.linear(heads, self.o, out=out)
+        return self.rt.linear(heads, self.o, out=out)

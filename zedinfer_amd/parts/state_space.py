@@ -82,7 +82,7 @@ class StateSpace(Mixer):
     def forward(self, x: torch.Tensor, batch, memory: LayerMemory, out=None) -> torch.Tensor:
         n, rt, inner, gn = x.shape[0], self.rt, self.inner, self.gn
         state = memory.state
-        full = ops.linear(x, self.w_in, out=rt.buffer("ssm_proj", (n, self.w_in.shape[0]), torch.float32))
+        full = self.rt.linear(x, self.w_in, out=rt.buffer("ssm_proj", (n, self.w_in.shape[0]), torch.float32))
         proj = full[:, :self.width]
         prep = rt.buffer("ssm_prepared", (n, self.width), torch.float32)
         ops.ssm_prepare(proj, self.conv_w, self.conv_b, self.dt_bias, self.a_log, state, batch.tok_seq, batch.entry_start,
@@ -103,4 +103,4 @@ class StateSpace(Mixer):
                 S = ops.linear_splits(n, self.hidden, inner)
                 return ops.linear_sums(g, self.o, out=rt.buffer("ssm_out_sums", (S, n, self.hidden), torch.float32))
             out = rt.buffer("ssm_out", (n, self.hidden))
-        return ops.linear(g, self.o, out=out)
+        return self.rt.linear(g, self.o, out=out)
