@@ -363,20 +363,20 @@ static bool gt_sizes(int64_t M, int64_t N, int64_t K) {
 // The kernel here or the library's product (with the launch of the activation, for gate and up) for more than 256 rows.  0: not taken here;
 // 1: taken, but the library is the faster by the rule; 2: the kernel here is; 3: and surely (a gate/up product).  The rule holds the time by the fit
 // against 16 us, 10 more from 10 GFLOP on, and 1.3 PFLOP/s, and says 2 up to 100 GFLOP of a plain product and 3 TFLOP of a gate/up product, 3 from
-// 0.7 of the library's time down.  18,680 products timed both ways, the library's the fastest of its proposals, and 13,541 with its first one (which runs where
-// nothing was measured), weights from memory, 257 to 20,000 rows, 520 to 30,000 columns, k 576 to 27,648, up to 10 TFLOP.  Own time of the
+// 0.7 of the library's time down.  7,143 products timed both ways, the library's the fastest of its proposals, and 9,027 with its first one (which runs
+// where nothing was measured), weights from memory, 257 to 20,000 rows, 520 to 30,000 columns, k 576 to 27,648, up to 10 TFLOP.  Own time of the
 // library's, geometric mean and one in twenty, where the rule says 2:
 //                        up to 10 GFLOP     30             100            1,000          3,000          beyond, all of them
-//   plain, first         0.89 and 1.06      0.92 and 1.11  0.97 and 1.14                                0.93 and 1.18
-//   plain, fastest       0.94 and 1.11      0.96 and 1.13  1.01 and 1.15                                1.02 and 1.19
-//   gate/up, first       0.68 and 0.89      0.76 and 1.01  0.76 and 0.94  0.83 and 1.04  0.95 and 1.04  1.00 and 1.10
-//   gate/up, fastest     0.68 and 0.91      0.79 and 1.03  0.82 and 0.99  0.88 and 1.09  0.97 and 1.07  1.03 and 1.12
-// Beyond the bounds single sizes are up to 1.25 times as fast either way, the library 0.9 to 1.5 PFLOP/s by how its tiles come out, which no rule on the
-// sizes that was tried tells apart, so an engine times both (the faster one takes 0.955 of the library's time in the mean, plain, and 0.873), and
-// where nothing was measured the library keeps them.  Where the rule says 3, 0.72, above 1 in one of a thousand.  us, own and the library's fastest: gate/up with
-// SwiGLU of 8,960 columns x 1,536 at 320 / 1,024 / 2,048 rows 28 and 35, 64 and 75, 111 and 129, of 18,944 x 3,584 104 and 121, 266 and 283, 461 and 523, of
-// 27,648 x 5,120 at 12,736 rows 5,664 and 5,371; 5,120 x 27,648 at 4,864 / 8,194 rows 1,119 and 1,388, 1,859 and 1,715; 320 x 536 x 1,792, the worst that the
-// rule says 2 of, 9.5 and 6.7.
+//   plain, first         0.83 and 1.02      0.91 and 1.06  0.97 and 1.17                                0.94 and 1.16
+//   plain, fastest       0.88 and 1.10      0.94 and 1.08  1.00 and 1.17                                1.02 and 1.16
+//   gate/up, first       0.64 and 0.87      0.76 and 1.02  0.79 and 0.97  0.85 and 1.06  0.94 and 1.03  0.99 and 1.08
+//   gate/up, fastest     0.64 and 0.87      0.79 and 1.06  0.82 and 0.99  0.89 and 1.09  0.97 and 1.06  1.01 and 1.08
+// Beyond the bounds single sizes are up to 1.25 times as fast either way, the library 0.9 to 1.4 PFLOP/s by how its tiles come out, which no rule on the
+// sizes that was tried tells apart, so an engine times both (the faster one takes 0.945 of the time of the library's fastest in the mean, plain, and 0.874),
+// and where nothing was measured the library keeps them.  Where the rule says 3, 0.72, above 1 in one of eighty and 1.09 at most.  us, own and the library's
+// fastest: gate/up with SwiGLU of 8,960 columns x 1,536 at 320 / 512 / 1,024 / 2,048 rows 27 and 34, 43 and 39, 62 and 76, 115 and 122, of 18,944 x
+// 3,584 105 and 118, 161 and 134, 270 and 260, 465 and 530, of 27,648 x 5,120 at 2,048 / 4,096 950 and 980, 1,980 and 2,020; 1,536 x 8,960 at 320 / 1,024 / 2,048 /
+// 8,192 rows 41 and 31, 54 and 49, 66 and 71, 215 and 171.
 #define GT_PLAIN_MOST 1e11
 #define GT_GATES_MOST 3e12
 
