@@ -864,13 +864,6 @@ __global__ void __launch_bounds__(4 * ZI_WAVE) gf_parts_kernel(gf_u32x4_t* __res
     for (int i = 0; i < 3; ++i) to[i * ZI_WAVE] = p.p[i].u;
 }
 
-// Loads but for the newest n have arrived, and every read of LDS.
-template <int n>
-__device__ __forceinline__ void gf_wait() {
-    static_assert(n < 64, "the counter has six bits");
-    __builtin_amdgcn_s_waitcnt((n & 15) | (7 << 4) | ((n >> 4) << 14));
-}
-
 #define GF_STAGES 4
 
 // The sums stay in the accumulation registers over the loop: without this the compiler moves all of them to other registers and back.
@@ -990,7 +983,7 @@ __global__ void __launch_bounds__(4 * ZI_WAVE, 1) gemm_f32_split_many_kernel(gf_
                 __builtin_amdgcn_sched_barrier(0);
                 asm volatile("" ::: "memory");
                 // the next step's x is there, all wavefronts have read this step's
-                gf_wait<2 * (PW + 2 * NT)>();
+                zi_wait_loads<2 * STEP_LOADS, true>();
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
             }
@@ -1059,7 +1052,7 @@ __global__ void __launch_bounds__(4 * ZI_WAVE, 1) gemm_f32_split_many_kernel(gf_
         __builtin_amdgcn_sched_barrier(0);
     }
     asm volatile("" ::: "memory");
-    gf_wait<(GF_STAGES - 1) * PW + 4 * NT>();
+    zi_wait_loads<(GF_STAGES - 1) * PW + 4 * NT, true>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
@@ -1105,7 +1098,7 @@ __global__ void __launch_bounds__(4 * ZI_WAVE, 1) gemm_f32_split_many_kernel(gf_
             }
         ++parts_done;
     }
-    gf_wait<0>();       // (no load may arrive after the workgroup's LDS is another's)
+    zi_wait_loads<0, true>();       // (no load may arrive after the workgroup's LDS is another's)
     if (RUNS) return;
     // (through this thread's own places in LDS, where x was, so that what checks and stores them is there once)
     gf_f32x4_t* const mine = reinterpret_cast<gf_f32x4_t*>(all) + wave * MT * NT * ZI_WAVE + lane;

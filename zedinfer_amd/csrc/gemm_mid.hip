@@ -308,13 +308,6 @@ gemm_mid_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* __
 // they go to the kernel above, whose addresses have 64 bits, 64 rows a workgroup.
 #define GW_MAX_LD (1 << 22)
 
-// the wavefront's loads but for the newest `n` have arrived (n counts loads; LDS and scalar counters are not waited for)
-template <int n>
-__device__ __forceinline__ void gw_wait() {
-    static_assert(n < 64, "the counter has six bits");
-    __builtin_amdgcn_s_waitcnt((n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14));
-}
-
 // 16 bytes a lane from a buffer into LDS, lane after lane from `to` on; what lies past the buffer's end gives zeros.
 template <int AUX>
 __device__ __forceinline__ void gw_to_lds(__amdgpu_buffer_rsrc_t from, gm_u32x4_t* to, int lane_at) {
@@ -396,7 +389,7 @@ gemm_wide_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* _
     auto step = [&](const gm_u32x4_t* buf, gm_u32x4_t* free, int t) __attribute__((always_inline)) {
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
-        gw_wait<(STAGES - 2) * PW>();
+        zi_wait_loads<(STAGES - 2) * PW>();
         __builtin_amdgcn_s_barrier();          // all wavefronts' loads of the step are there, and all are done with `free`
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
@@ -451,7 +444,7 @@ gemm_wide_kernel(void* __restrict__ out, int mode, int out_f32, const zi_bf16* _
             step(s2, s1, t + 2);
         }
     }
-    gw_wait<0>();       // (no load may arrive after the workgroup's LDS is another's)
+    zi_wait_loads<0>();       // (no load may arrive after the workgroup's LDS is another's)
 #pragma unroll
     for (int n = 0; n < NW; ++n)
         if (n_tile + n < NT)

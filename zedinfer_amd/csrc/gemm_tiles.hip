@@ -13,8 +13,8 @@
 // Which row of the weights stands where in LDS is free, and so chosen that a lane's outputs follow each other in memory (gt_row_of):
 // 16-byte stores, and gate and up of one column in one lane.
 //
-// What bounds it: LDS, which takes a step's loads at 64 bytes a cycle and gives 128 (256 x 192 tiles: 2,176 cycles a step for 1,536 of
-// matrix instructions), the loads in flight where only two buffers fit, and rows of a tile that the XCD's cache has to fetch (tiles
+// What bounds it: LDS, which takes a step's loads at 64 bytes a cycle and gives 128 (256 x 256 tiles: 2,560 cycles a step for 2,048 of
+// matrix instructions, 192 x 192 1,920 for 1,152), the loads in flight where only two buffers fit, and rows of a tile that the XCD's cache has to fetch (tiles
 // that run at a time on an XCD are neighbours).
 #include "zi_common.h"
 #include "zi_activation.h"
@@ -41,13 +41,6 @@ union gt_pack {
 #define GT_SWIGLU 2        // gate and up rows of the weights alternate in blocks of 8; bfloat16
 #define GT_GATED 3         // the gate rows come first, the up rows from row `up_at` on; an activation by its code; bfloat16
 #define GT_ERF 4           // the same with the error function's GELU (a kernel of its own: the function is 40 instructions)
-
-// Loads but for the newest n have arrived, and every read of LDS.
-template <int n>
-__device__ __forceinline__ void gt_wait() {
-    static_assert(n < 64, "the counter has six bits");
-    __builtin_amdgcn_s_waitcnt((n & 15) | (7 << 4) | ((n >> 4) << 14));
-}
 
 __device__ __forceinline__ void gt_to_lds(__amdgpu_buffer_rsrc_t from, gt_u32x4_t* to, int lane_at) {
 #ifdef __HIP_DEVICE_COMPILE__       // (the host's pass knows loads of this size for no target)
@@ -218,7 +211,7 @@ __global__ void __launch_bounds__(128 * WM, 1) gemm_tiles_kernel(gt_args g) {
         }
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("" ::: "memory");
-        gt_wait<(S - 2) * PW>();
+        zi_wait_loads<(S - 2) * PW, true>();
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
@@ -243,7 +236,7 @@ __global__ void __launch_bounds__(128 * WM, 1) gemm_tiles_kernel(gt_args g) {
         __builtin_amdgcn_sched_barrier(0);
     }
     asm volatile("" ::: "memory");
-    gt_wait<(S - 2) * PW + EARLY>();
+    zi_wait_loads<(S - 2) * PW + EARLY, true>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
@@ -308,7 +301,7 @@ __global__ void __launch_bounds__(128 * WM, 1) gemm_tiles_kernel(gt_args g) {
         }
         now = next;
     }
-    gt_wait<0>();       // (no load may arrive after the workgroup's LDS is another's)
+    zi_wait_loads<0, true>();       // (no load may arrive after the workgroup's LDS is another's)
 }
 
 // ---- the tile of a product ------------------------------------------------------------------------------------------------

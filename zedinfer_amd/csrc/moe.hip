@@ -340,13 +340,6 @@ static int moe_turns(int tile_rows, int K) { return tile_rows == 16 ? (K >= 384 
 // the longest row of weights whose tile of rows a buffer's 31-bit offsets reach
 #define MOE_MAX_K (1 << 21)
 
-// the wavefront's loads but for the newest `n` have arrived (n counts loads; LDS and scalar counters are not waited for)
-template <int n>
-__device__ __forceinline__ void moe_wait() {
-    static_assert(n < 64, "the counter has six bits");
-    __builtin_amdgcn_s_waitcnt((n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14));
-}
-
 // 16 bytes a lane into LDS, lane after lane from `to` on: from an address, or from a buffer (zeros past its end).
 __device__ __forceinline__ void moe_to_lds(const zi_bf16* from, moe_u32x4_t* to) {
 #ifdef __HIP_DEVICE_COMPILE__       // (the host's pass knows loads of this size for no target)
@@ -447,8 +440,8 @@ moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restr
         if (TURNS == 1 && t >= steps) return;
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
-        if (TURNS > 1 || steps - 1 - t >= ST - 2) moe_wait<(ST - 2) * PW>();      // the newest steps' loads may still be on their way
-        else moe_wait<0>();
+        if (TURNS > 1 || steps - 1 - t >= ST - 2) zi_wait_loads<(ST - 2) * PW>();      // the newest steps' loads may still be on their way
+        else zi_wait_loads<0>();
         __builtin_amdgcn_s_barrier();          // all wavefronts' loads of the step are there, and all are done with `free`
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
@@ -501,7 +494,7 @@ moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restr
                 }
             }
         }
-        moe_wait<0>();
+        zi_wait_loads<0>();
     }
     moe_store_tile<RW, CT>(out, ldo, acc, act, rows, r0, row0, n0 + wave_c * CT * 16, N, r, j);
 }
@@ -510,7 +503,7 @@ moe_linear_mfma_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __restr
 // halves, and while the products of one run, the operands of the next are read from LDS and a share of a later step's loads is issued; the step's
 // one barrier stands between the halves.  Above, a step's loads, reads and products follow each other and only the second wavefront of a SIMD
 // stands beside them.  (Past the last step that one is loaded again, so that every step waits alike.)  Bound by the weights' way from memory
-// where an expert has few tiles, by LDS otherwise (its reads and loads are 1,280 cycles of a step, the products 1,024).
+// where an expert has few tiles, by LDS otherwise (its reads and loads are 1,792 cycles of a step, the products 1,024).
 // us, the kernel above and this one, the first product and the second, everything from memory and the launch's 15 us included: 32 experts of
 // 1,536 x 1,536, 8,000 pairs 101 and 101 to 97 and 97, 9,200 118 and 110 to 109 and 103, 16,384 159 and 163 to 145 and 151; of 2,560 x 3,584,
 // 8,192 pairs 342 and 324 to 315 and 303; 8 of 4,096 x 14,336, 2,000 pairs 538 and 539 to 515 and 491.  Taken for every k of whole steps from three on.
@@ -586,7 +579,7 @@ moe_linear_halves_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __res
         __builtin_amdgcn_sched_barrier(0);
     }
     asm volatile("" ::: "memory");
-    moe_wait<(ST - 2) * PW + EARLY>();
+    zi_wait_loads<(ST - 2) * PW + EARLY>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
@@ -599,7 +592,7 @@ moe_linear_halves_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __res
         spread(PW - EARLY);
         asm volatile("" ::: "memory");
         // the next step's loads have arrived, all wavefronts have read this step's
-        __builtin_amdgcn_s_waitcnt((((ST - 2) * PW) & 15) | (7 << 4) | ((((ST - 2) * PW) >> 4) << 14));
+        zi_wait_loads<(ST - 2) * PW, true>();
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
@@ -610,7 +603,7 @@ moe_linear_halves_kernel(TO* __restrict__ out, int64_t ldo, const zi_bf16* __res
         multiply(a1, b1);
         spread(EARLY);
     }
-    moe_wait<0>();       // (no load may arrive after the workgroup's LDS is another's)
+    zi_wait_loads<0>();       // (no load may arrive after the workgroup's LDS is another's)
     moe_store_tile<RW, CT>(out, ldo, acc, act, rows, r0, row0, n0 + wave_c * CT * 16, N, r, j);
 }
 

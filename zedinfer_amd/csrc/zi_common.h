@@ -43,12 +43,20 @@ __device__ __forceinline__ float zi_load(const zi_bf16* p) { return zi_bf16_to_f
 __device__ __forceinline__ void zi_store(float* p, float v) { *p = v; }
 __device__ __forceinline__ void zi_store(zi_bf16* p, float v) { p->bits = zi_float_to_bf16(v); }
 
+// The wavefront's loads but for the newest `n` have arrived (n counts loads, and stores, which are counted with them; LDS and scalar counters
+// are not waited for), and with `lds` every read of LDS.
+template <int n, bool lds = false>
+__device__ __forceinline__ void zi_wait_loads() {
+    static_assert(n < 64, "the counter has six bits");
+    __builtin_amdgcn_s_waitcnt((n & 15) | (7 << 4) | ((lds ? 0 : 15) << 8) | ((n >> 4) << 14));
+}
+
 // A barrier behind which every wavefront's loads into LDS (global_load_lds) have arrived.  The wait is asked for by name: the one that
 // __syncthreads() brings along was found missing at the head of a loop whose only reads of the loaded tile a wavefront may skip.
 __device__ __forceinline__ void zi_barrier_loaded() {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));      // vector loads 0; the other counters are the barrier's matter
+    zi_wait_loads<0>();      // (the other counters are the barrier's matter)
     __syncthreads();
 }
 
